@@ -23,7 +23,8 @@
 // two of its blocks fit a CU.
 //
 // Layouts (rows = 16 * RPL, y fastest everywhere):
-//   factors   att[v][z'][x'][rows]  e^{-A(x', y, z')}, A the inclusive sum of mu'
+//   factors   att[v][z'][x'][rows]  e^{-A(x', y, z')}, A the inclusive sum of mu' (none without
+//             attenuation: att null, every factor 1)
 //   partials  part[d][v][x'][rows]  projection of depth chunk d
 //   measured counts and ratio       [v][x'][rows]
 //   U         u + v*ustride + y + rows*((x'+1) + xp*(z'+1))  (zero border in x', z')
@@ -274,6 +275,29 @@ __device__ __forceinline__ Samp yl_samp_from(const YlSamp &h, int src)
     return s;
 }
 
+// Factors e^{-A} of plane z for the columns col(r), r < N (those inside the
+// volume): streamed from a.att, or 1 without attenuation (a.att null; one
+// uniform branch per plane).
+template <int RPL, int N, class Col>
+__device__ __forceinline__ void yl_plane_factors(const EtSweepArgs &a, int v, int z, int row0, Col col,
+                                                 float (*e)[RPL])
+{
+    constexpr int rows = 16 * RPL;
+    if (a.att) {
+#pragma unroll
+        for (int r = 0; r < N; r++) {
+            const int xc = col(r);
+            if (xc >= 0 && xc < a.nx)
+                yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e[r]);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < N; r++)
+#pragma unroll
+            for (int i = 0; i < RPL; i++) e[r][i] = 1.f;
+    }
+}
+
 // ------------------------------------------------------------------------------
 // Projection with cached attenuation factors.  Block (d, v): depth chunk d of
 // view v, all columns.  part[d][v][x'][rows] = sum over the chunk's planes of
@@ -323,11 +347,7 @@ __device__ __forceinline__ void yl_project_body(const EtSweepArgs &a, const Blk 
         // gather and the column pass (every wave of the block reaches the
         // accumulation at the same time, after the barrier)
         float e[NR][RPL];
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const int xc = r * W + slot;
-            if (xc < a.nx) yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e[r]);
-        }
+        yl_plane_factors<RPL, NR>(a, v, z, row0, [&](int r) { return r * W + slot; }, e);
         if constexpr (R > 0) {
             float *plane = lds + (a.yl_nbuf == 2 ? (z & 1) * PF : 0);
 #pragma unroll
@@ -373,10 +393,10 @@ __device__ __forceinline__ void yl_project_body(const EtSweepArgs &a, const Blk 
         if (xc >= a.nx) continue;
         if (d == a.D - 1 && a.bg_line != 0.f) {
             // e^{-A} along the whole ray = the factor of the last plane
-            float e[RPL];
-            yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + a.nz - 1) * a.nx + xc) * rows + row0, e);
+            float e[1][RPL];
+            yl_plane_factors<RPL, 1>(a, v, a.nz - 1, row0, [&](int) { return xc; }, e);
 #pragma unroll
-            for (int i = 0; i < RPL; i++) kahan(r, i, a.bg_line, e[i]);
+            for (int i = 0; i < RPL; i++) kahan(r, i, a.bg_line, e[0][i]);
         }
         float out[RPL];
 #pragma unroll
@@ -588,11 +608,7 @@ __device__ __forceinline__ void yl_project_tile_body(const EtSweepArgs &a, const
             sb = yl_samp_of(fast_sample(fv, (float)col(lane % NRR), z + lane / NRR, a.nx, a.nz, dx, dz));
         // the owned columns' factors first (their latency passes under the gathers)
         float e[NR][RPL];
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const int xc = col(r);
-            if (valid(xc)) yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e[r]);
-        }
+        yl_plane_factors<RPL, NR>(a, v, z, row0, col, e);
         float *plane = lds + (z & 1) * PF;
 #pragma unroll
         for (int r = 0; r < NRR; r++) {
@@ -622,10 +638,10 @@ __device__ __forceinline__ void yl_project_tile_body(const EtSweepArgs &a, const
         const int xc = col(r);
         if (!valid(xc)) continue;
         if (d == a.D - 1 && a.bg_line != 0.f) {
-            float e[RPL];
-            yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + a.nz - 1) * a.nx + xc) * rows + row0, e);
+            float e[1][RPL];
+            yl_plane_factors<RPL, 1>(a, v, a.nz - 1, row0, [&](int) { return xc; }, e);
 #pragma unroll
-            for (int i = 0; i < RPL; i++) kahan(r, i, a.bg_line, e[i]);
+            for (int i = 0; i < RPL; i++) kahan(r, i, a.bg_line, e[0][i]);
         }
         float out[RPL];
 #pragma unroll
@@ -792,10 +808,16 @@ __device__ __forceinline__ void yl_bpu_body(const EtSweepArgs &a, const Blk &b)
         for (int r = 0; r < NR; r++) {
             const int xc = r * W + slot;
             if (xc < a.nx) {
-                float w[RPL], e[RPL];
-                yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e);
+                float w[RPL];
+                if (a.att) {
+                    float e[RPL];
+                    yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e);
 #pragma unroll
-                for (int i = 0; i < RPL; i++) w[i] = sv[r][i] * e[i];
+                    for (int i = 0; i < RPL; i++) w[i] = sv[r][i] * e[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) w[i] = sv[r][i];
+                }
                 if constexpr (R > 0) {
                     float cp[RPL];
                     yl_column_pass<R, RPL>(w, kz + K, cp);
