@@ -487,6 +487,7 @@ struct SweepCtx {
     size_t P;
     float fxp;
     FastView fv;
+    const float *act, *mu;  // this view's source volumes
 };
 
 // Logical block of a launch: linear id (the dispatcher deals linear ids to the
@@ -573,7 +574,9 @@ __device__ __forceinline__ SweepCtx sweep_ctx(const EtSweepArgs &a, bool chunked
     c.xin = c.tx < a.nx;
     c.P = (size_t)a.nx * a.ny;
     c.bufsz = (c.nthr + 2 * R) * (TS + 4);
-    c.fv = load_fast_view(a.views + (size_t)c.v * ET_VIEW_REC);
+    c.fv = load_fast_view(a.views + (size_t)c.v * a.rec_stride);
+    c.act = a.act + (size_t)c.v * a.act_vs;
+    c.mu = a.mu + (size_t)c.v * a.mu_vs;
     c.dx = a.yp;
     c.dz = a.yp * a.xp;
     c.fxp = (float)c.tx;

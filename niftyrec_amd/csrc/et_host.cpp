@@ -565,6 +565,7 @@ EtSweepArgs base_args(et_plan *p)
     a.slabs = p->slabs;
     a.K = p->K;
     a.psf = p->K > 0 ? p->d_sep.p : nullptr;
+    a.rec_stride = ET_VIEW_REC;
     a.bg_act = p->bg;
     a.bg_mu = p->bga;
     a.bg_line = p->bg;
@@ -627,11 +628,17 @@ void pack(et_plan *p, const float *abi, DevBuf &yf)
 
 // Attenuation at the start of every depth chunk (D > 1) and along whole rays
 // for `nv` views whose records start at `recs`; results in p->astart / p->atot.
+// general: the views are rotated copies in mu_yf, yf_elems floats apart, with
+// one identity record.
 void mu_prefix(et_plan *p, const float *recs, int nv, int D, const float *mu_yf, bool want_start, bool want_tot,
-               float *astart_out = nullptr, float *atot_out = nullptr)
+               bool general = false)
 {
     EtSweepArgs a = base_args(p);
     a.views = recs;
+    if (general) {
+        a.rec_stride = 0;
+        a.mu_vs = p->yf_elems;
+    }
     a.V = nv;
     a.D = D;
     a.zlen = (p->nz + D - 1) / D;
@@ -645,9 +652,9 @@ void mu_prefix(et_plan *p, const float *recs, int nv, int D, const float *mu_yf,
         check_launch(et_launch_sweep(ET_MODE_MUSUM, 0, 1, 0, a, (et_stream_t)p->st));
     }
     float *as = nullptr, *at = nullptr, *atl = nullptr;
-    if (want_start) as = astart_out ? astart_out : p->astart.ensure((size_t)nv * D * p->P, false);
+    if (want_start) as = p->astart.ensure((size_t)nv * D * p->P, false);
     if (want_tot) {
-        at = atot_out ? atot_out : p->atot.ensure((size_t)nv * p->P, false);
+        at = p->atot.ensure((size_t)nv * p->P, false);
         atl = p->atot_lo.ensure((size_t)nv * p->P, false);
     }
     ProfScope ps(p, ET_PROF_OTHER, 0);
@@ -774,75 +781,96 @@ void pull_fast(et_plan *p, const float *recs, int nv, const float *u, bool adjoi
     check_launch(et_launch_pull(a, (et_stream_t)p->st));
 }
 
-// ---- general path: one view at a time ------------------------------------------
+// ---- general path: rotated copies of a batch of views ----------------------------
+// A view of the general path has slabs x chunks blocks: 64^3 x 32 views taken
+// one view after another projected in 11.1 ms (329 us per view, 4 blocks of one
+// wave on 256 CUs).  A batch of views shares every launch, with one rotated
+// copy per view.
 
-// Rotated copy of an ABI volume for view v in the YF layout (+ PSF when the
-// radius is too large for the sweep kernels).
-void rotate_general(et_plan *p, const float *abi, int v, float bg, DevBuf &dst, bool psf, bool flip)
+// Views per batch: the rotated copies of the activity, the map and the
+// rotated-frame volume of a batch stay within 256 MiB.
+int general_batch(const et_plan *p)
 {
-    dst.ensure(p->yf_elems, true, p->st);
+    if (p->tune_vb > 0) return std::min(p->tune_vb, p->V);
+    const size_t per_view = (2 * p->yf_elems + p->ustride) * sizeof(float);
+    return (int)std::max<size_t>(1, std::min<size_t>((256ull << 20) / std::max<size_t>(per_view, 1), p->V));
+}
+
+// Depth chunks of the general path's projection and backprojection: powers of
+// two, chunks of at least 4 planes, up to about four waves per SIMD (64^3 x 32
+// views: 16 chunks, 2,048 waves).  Chunks of at least 16 planes, as choose_D
+// takes them, would leave a quarter of that.
+int general_D(const et_plan *p, int nv)
+{
+    if (p->tune_D > 0) return std::min(p->tune_D, p->nz);
+    const long waves = (long)p->slabs * nv * (nthreads_for(p->nx) / 64);
+    int D = 1;
+    while (D < 32 && waves * D < 4096 && p->nz / (2 * D) >= 4) D *= 2;
+    return D;
+}
+
+// Sweep arguments of nv rotated views (identity record) in D chunks.
+EtSweepArgs general_args(et_plan *p, int nv, int D, bool act, bool mu)
+{
+    EtSweepArgs a = base_args(p);
+    a.views = p->d_ident.p;
+    a.rec_stride = 0;
+    a.V = nv;
+    a.D = D;
+    a.zlen = (p->nz + D - 1) / D;
+    a.act = act ? p->rot_act.p : nullptr;
+    a.mu = mu ? p->rot_mu.p : nullptr;
+    a.act_vs = act ? p->yf_elems : 0;
+    a.mu_vs = mu ? p->yf_elems : 0;
+    a.bg_act = 0.f;
+    a.bg_mu = 0.f;
+    return a;
+}
+
+// Rotated copies of an ABI volume for views [v0, v0 + nv) in the YF layout (+
+// PSF when the radius is too large for the sweep kernels).
+void rotate_general(et_plan *p, const float *abi, int v0, int nv, float bg, DevBuf &dst, bool psf)
+{
+    const size_t vs = p->yf_elems;
+    dst.ensure(nv * vs, true, p->st);
     {
-        ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
-        check_launch(et_launch_resample_general(abi, p->nx, p->ny, p->nz, p->d_recs.p + (size_t)v * ET_VIEW_REC, bg,
-                                                dst.p, 1, p->yp, p->gy, (et_stream_t)p->st));
+        ProfScope ps(p, ET_PROF_OTHER, nv * 8.0 * p->nvox);
+        check_launch(et_launch_resample_general(abi, p->nx, p->ny, p->nz, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, bg,
+                                                dst.p, 1, p->yp, p->gy, nv, vs, (et_stream_t)p->st));
     }
     if (psf && p->K > 0 && p->R > ET_RMAX) {
         // row (x) pass then column (y) pass, emission-lib/_et_convolveSeparable2D.cpp:43-75
-        p->tmp.ensure(p->yf_elems, true, p->st);
+        p->tmp.ensure(nv * vs, true, p->st);
         const long sx = p->yp, sy = 1, sz = (long)p->yp * p->xp, off = p->gy + (long)p->yp * (1 + p->xp);
-        const float *sep = flip ? p->d_sep_flip.p : p->d_sep.p;
-        check_launch(et_launch_conv_axis(dst.p, p->tmp.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 0, sep, p->K, 0,
-                                         (et_stream_t)p->st));
-        check_launch(et_launch_conv_axis(p->tmp.p, dst.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 1, sep, p->K, 0,
-                                         (et_stream_t)p->st));
+        check_launch(et_launch_conv_axis(dst.p, p->tmp.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 0, p->d_sep.p, p->K, 0,
+                                         nv, vs, (et_stream_t)p->st));
+        check_launch(et_launch_conv_axis(p->tmp.p, dst.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 1, p->d_sep.p, p->K, 0,
+                                         nv, vs, (et_stream_t)p->st));
     }
 }
 
 // Sweep radius used on the general path (0 when the PSF is applied separately).
 int general_R(et_plan *p) { return p->R > ET_RMAX ? 0 : p->R; }
 
-void conv_u_general(et_plan *p, float *u, bool flip)
+void conv_u_general(et_plan *p, float *u, int nv, bool flip)
 {
     if (!(p->K > 0 && p->R > ET_RMAX)) return;
-    p->tmp2.ensure(p->ustride, true, p->st);
+    const size_t vs = p->ustride;
+    p->tmp2.ensure(nv * vs, true, p->st);
     const long sx = p->yu, sy = 1, sz = (long)p->yu * p->xp, off = (long)p->yu * (1 + p->xp);
     const float *sep = flip ? p->d_sep_flip.p : p->d_sep.p;
-    if (!flip) {
-        check_launch(et_launch_conv_axis(u, p->tmp2.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 0, sep, p->K, 0,
-                                         (et_stream_t)p->st));
-        check_launch(et_launch_conv_axis(p->tmp2.p, u, p->nx, p->ny, p->nz, sx, sy, sz, off, 1, sep, p->K, 0,
-                                         (et_stream_t)p->st));
-    } else {
-        check_launch(et_launch_conv_axis(u, p->tmp2.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 1, sep, p->K, 0,
-                                         (et_stream_t)p->st));
-        check_launch(et_launch_conv_axis(p->tmp2.p, u, p->nx, p->ny, p->nz, sx, sy, sz, off, 0, sep, p->K, 0,
-                                         (et_stream_t)p->st));
-    }
+    // row pass then column pass; the transpose takes them in the other order
+    check_launch(et_launch_conv_axis(u, p->tmp2.p, p->nx, p->ny, p->nz, sx, sy, sz, off, flip ? 1 : 0, sep, p->K, 0,
+                                     nv, vs, (et_stream_t)p->st));
+    check_launch(et_launch_conv_axis(p->tmp2.p, u, p->nx, p->ny, p->nz, sx, sy, sz, off, flip ? 0 : 1, sep, p->K, 0,
+                                     nv, vs, (et_stream_t)p->st));
 }
 
-void pull_general(et_plan *p, int v, const float *u, bool adjoint, bool accumulate, bool truncate, float *out,
-                  int epi)
+void pull_general(et_plan *p, int v0, int nv, const float *u, bool adjoint, bool accumulate, bool truncate, float *out)
 {
-    EtPullArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.nx = p->nx;
-    a.ny = p->ny;
-    a.nz = p->nz;
-    a.yu = p->yu;
-    a.xp = p->xp;
-    a.ustride = (int)p->ustride;
-    a.V = 1;
-    a.views = p->d_recs.p + (size_t)v * ET_VIEW_REC;
-    a.u = u;
-    a.bg = p->bg;
-    a.adjoint = adjoint;
-    a.epilogue = epi;
-    a.accumulate = accumulate;
-    a.truncate = truncate;
-    a.out = out;
-    a.yp = p->yp;
-    a.gy = p->gy;
-    ProfScope ps(p, ET_PROF_PULL, 4.0 * p->nvox + (accumulate ? 8.0 : 4.0) * p->nvox);
+    const EtPullArgs a = pull_args(p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, u, adjoint, ET_EPI_ABI_STORE,
+                                   accumulate, truncate, out, nullptr, nullptr);
+    ProfScope ps(p, ET_PROF_PULL, nv * 4.0 * p->nvox + (accumulate ? 8.0 : 4.0) * p->nvox);
     check_launch(et_launch_pull_general(a, (et_stream_t)p->st));
 }
 
@@ -891,28 +919,32 @@ void op_project(et_plan *p, const float *act, const float *mu, float *sino, int 
         return;
     }
     // general path
-    const int R = general_R(p);
-    for (int v = 0; v < p->V; v++) {
-        float *sv = sino + (size_t)v * p->P;
-        if (mu) rotate_general(p, mu, v, p->bga, p->rot_mu, false, false);
+    const int R = general_R(p), vb = general_batch(p);
+    for (int v0 = 0; v0 < p->V; v0 += vb) {
+        const int nv = std::min(vb, p->V - v0);
+        float *sv = sino + (size_t)v0 * p->P;
+        if (mu) rotate_general(p, mu, v0, nv, p->bga, p->rot_mu, false);
         if (!act) {
-            mu_prefix(p, p->d_ident.p, 1, 1, p->rot_mu.p, false, true);
-            check_launch(et_launch_bg_only(p->atot.p, p->atot_lo.p, p->bg, (int)p->P, sv, truncate,
+            mu_prefix(p, p->d_ident.p, nv, 1, p->rot_mu.p, false, true, true);
+            check_launch(et_launch_bg_only(p->atot.p, p->atot_lo.p, p->bg, (int)(nv * p->P), sv, truncate,
                                            (et_stream_t)p->st));
             continue;
         }
-        rotate_general(p, act, v, p->bg, p->rot_act, true, false);
-        EtSweepArgs a = base_args(p);
-        a.views = p->d_ident.p;
-        a.V = 1;
-        a.act = p->rot_act.p;
-        a.mu = mu ? p->rot_mu.p : nullptr;
-        a.bg_act = 0.f;
-        a.bg_mu = 0.f;
-        a.part = sv;
-        a.truncate = truncate;
-        ProfScope ps(p, ET_PROF_PROJECT, (mu ? 8.0 : 4.0) * p->nvox + 4.0 * p->P);
-        check_launch(et_launch_sweep(ET_MODE_PROJECT, R, mu != nullptr, 1, a, (et_stream_t)p->st));
+        rotate_general(p, act, v0, nv, p->bg, p->rot_act, true);
+        const int D = general_D(p, nv);
+        if (mu && D > 1) mu_prefix(p, p->d_ident.p, nv, D, p->rot_mu.p, true, false, true);
+        EtSweepArgs a = general_args(p, nv, D, true, mu != nullptr);
+        a.astart = mu && D > 1 ? p->astart.p : nullptr;
+        a.part = D == 1 ? sv : p->part.ensure((size_t)D * nv * p->P, false);
+        a.truncate = D == 1 ? truncate : 0;
+        {
+            ProfScope ps(p, ET_PROF_PROJECT, nv * ((mu ? 8.0 : 4.0) * p->nvox + 4.0 * p->P));
+            check_launch(et_launch_sweep(ET_MODE_PROJECT, R, mu != nullptr, 1, a, (et_stream_t)p->st));
+        }
+        if (D > 1) {
+            ProfScope ps(p, ET_PROF_OTHER, 0);
+            check_launch(et_launch_reduce_parts(a.part, D, nv, (int)p->P, sv, truncate, (et_stream_t)p->st));
+        }
     }
 }
 
@@ -943,25 +975,25 @@ void op_backproject(et_plan *p, const float *sino, const float *mu, float *out, 
         }
         return;
     }
-    const int R = general_R(p);
-    p->u.ensure(p->ustride, true, p->st);
-    for (int v = 0; v < p->V; v++) {
-        if (mu) rotate_general(p, mu, v, p->bga, p->rot_mu, false, false);
-        EtSweepArgs a = base_args(p);
-        a.views = p->d_ident.p;
-        a.V = 1;
-        a.mu = mu ? p->rot_mu.p : nullptr;
-        a.bg_mu = 0.f;
+    const int R = general_R(p), vb = general_batch(p);
+    p->u.ensure((size_t)vb * p->ustride, true, p->st);
+    for (int v0 = 0; v0 < p->V; v0 += vb) {
+        const int nv = std::min(vb, p->V - v0);
+        if (mu) rotate_general(p, mu, v0, nv, p->bga, p->rot_mu, false);
+        const int D = general_D(p, nv);
+        if (mu && D > 1) mu_prefix(p, p->d_ident.p, nv, D, p->rot_mu.p, true, false, true);
+        EtSweepArgs a = general_args(p, nv, D, false, mu != nullptr);
+        a.astart = mu && D > 1 ? p->astart.p : nullptr;
         a.src = ET_SRC_SINO;
-        a.sino = sino + (size_t)v * p->P;
+        a.sino = sino + (size_t)v0 * p->P;
         a.u = p->u.p;
         if (p->K > 0) a.psf = adjoint ? p->d_sep_flip.p : p->d_sep.p;
         {
-            ProfScope ps(p, ET_PROF_BPU, (mu ? 8.0 : 4.0) * p->nvox + 4.0 * p->P);
+            ProfScope ps(p, ET_PROF_BPU, nv * ((mu ? 8.0 : 4.0) * p->nvox + 4.0 * p->P));
             check_launch(et_launch_sweep(ET_MODE_BPU, R, mu != nullptr, 0, a, (et_stream_t)p->st));
         }
-        conv_u_general(p, p->u.p, adjoint);
-        pull_general(p, v, p->u.p, adjoint, v > 0, truncate && v == p->V - 1, out, ET_EPI_ABI_STORE);
+        conv_u_general(p, p->u.p, nv, adjoint);
+        pull_general(p, v0, nv, p->u.p, adjoint, v0 > 0, truncate && v0 + nv >= p->V, out);
     }
 }
 
@@ -998,30 +1030,25 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
         }
         return;
     }
-    const int R = general_R(p);
-    p->u.ensure(p->ustride, true, p->st);
-    for (int v = 0; v < p->V; v++) {
-        rotate_general(p, mu, v, p->bga, p->rot_mu, false, false);
-        rotate_general(p, act, v, p->bg, p->rot_act, exact, false);
-        mu_prefix(p, p->d_ident.p, 1, 1, p->rot_mu.p, false, true);
-        EtSweepArgs a = base_args(p);
-        a.views = p->d_ident.p;
-        a.V = 1;
-        a.act = p->rot_act.p;
-        a.mu = p->rot_mu.p;
-        a.bg_act = 0.f;
-        a.bg_mu = 0.f;
+    const int R = general_R(p), vb = general_batch(p);
+    p->u.ensure((size_t)vb * p->ustride, true, p->st);
+    for (int v0 = 0; v0 < p->V; v0 += vb) {
+        const int nv = std::min(vb, p->V - v0);
+        rotate_general(p, mu, v0, nv, p->bga, p->rot_mu, false);
+        rotate_general(p, act, v0, nv, p->bg, p->rot_act, exact);
+        mu_prefix(p, p->d_ident.p, nv, 1, p->rot_mu.p, false, true, true);
+        EtSweepArgs a = general_args(p, nv, 1, true, true);
         a.atot = p->atot.p;
         a.atot_lo = p->atot_lo.p;
         a.src = ET_SRC_SINO;
-        a.sino = sino + (size_t)v * p->P;
+        a.sino = sino + (size_t)v0 * p->P;
         a.u = p->u.p;
         {
-            ProfScope ps(p, ET_PROF_GRAD, 12.0 * p->nvox + 4.0 * p->P);
+            ProfScope ps(p, ET_PROF_GRAD, nv * (12.0 * p->nvox + 4.0 * p->P));
             check_launch(et_launch_sweep(mode, R, 1, 1, a, (et_stream_t)p->st));
         }
-        if (!exact) conv_u_general(p, p->u.p, false);
-        pull_general(p, v, p->u.p, exact, v > 0, truncate && v == p->V - 1, out, ET_EPI_ABI_STORE);
+        if (!exact) conv_u_general(p, p->u.p, nv, false);
+        pull_general(p, v0, nv, p->u.p, exact, v0 > 0, truncate && v0 + nv >= p->V, out);
     }
 }
 
@@ -3129,7 +3156,7 @@ int et_array_rotate(float *image, int *size, float *rotated_image, float *angles
         const float *d_in = hc.upload(image, n);
         float *d_M = hc.upload(M, 12);
         float *d_out = hc.alloc(n);
-        check_launch(et_launch_resample_general(d_in, size[0], size[1], size[2], d_M, background, d_out, 0, 0, 0,
+        check_launch(et_launch_resample_general(d_in, size[0], size[1], size[2], d_M, background, d_out, 0, 0, 0, 1, 0,
                                                 (et_stream_t)hc.st));
         hc.download(rotated_image, d_out, n);
         return niftyrec_success;
@@ -3156,7 +3183,7 @@ int et_array_affine(float *image, int *image_size, float *transformed_image, int
         float *d_M = hc.upload(affine, 12);
         float *d_out = hc.alloc(n);
         check_launch(et_launch_resample_general(d_in, image_size[0], image_size[1], image_size[2], d_M, background,
-                                                d_out, 0, 0, 0, (et_stream_t)hc.st));
+                                                d_out, 0, 0, 0, 1, 0, (et_stream_t)hc.st));
         hc.download(transformed_image, d_out, n);
         return niftyrec_success;
     });
@@ -3252,19 +3279,19 @@ int et_array_project_partial(float *activity, int *activity_size, float *sinogra
         for (int v = 0; v < V; v++) {
             const float *Mf = d_M + (size_t)24 * v, *Mi = Mf + 12;
             if (d_act) {
-                check_launch(et_launch_resample_general(d_act, nx, ny, nz, Mf, background, rot_act, 0, 0, 0, s));
+                check_launch(et_launch_resample_general(d_act, nx, ny, nz, Mf, background, rot_act, 0, 0, 0, 1, 0, s));
                 if (d_sep) {
-                    check_launch(et_launch_conv_axis(rot_act, tmp, nx, ny, nz, 1, nx, (long)P, 0, 0, d_sep, h, 0, s));
-                    check_launch(et_launch_conv_axis(tmp, rot_act, nx, ny, nz, 1, nx, (long)P, 0, 1, d_sep, h, 0, s));
+                    check_launch(et_launch_conv_axis(rot_act, tmp, nx, ny, nz, 1, nx, (long)P, 0, 0, d_sep, h, 0, 1, 0, s));
+                    check_launch(et_launch_conv_axis(tmp, rot_act, nx, ny, nz, 1, nx, (long)P, 0, 1, d_sep, h, 0, 1, 0, s));
                 }
             }
             if (d_mu)
                 check_launch(
-                    et_launch_resample_general(d_mu, nx, ny, nz, Mf, background_attenuation, rot_mu, 0, 0, 0, s));
+                    et_launch_resample_general(d_mu, nx, ny, nz, Mf, background_attenuation, rot_mu, 0, 0, 0, 1, 0, s));
             check_launch(et_launch_partial_line(rot_act, rot_mu, d_bgimg, background, nx, ny, nz, d_sino + P * v,
                                                 part, s));
             if (do_rotate_partial)
-                check_launch(et_launch_resample_general(part, nx, ny, nz, Mi, background, pout, 0, 0, 0, s));
+                check_launch(et_launch_resample_general(part, nx, ny, nz, Mi, background, pout, 0, 0, 0, 1, 0, s));
             hc.download(partialsum + n * v, pout, n);
         }
         if (truncate_negative_values) check_launch(et_launch_truncate(d_sino, P * V, s));
@@ -3300,9 +3327,9 @@ int et_array_convolve(float *image, int *image_size, float *out, int *out_size, 
         const float *d_sep = hc.upload(sep.data(), sep.size());
         float *d_tmp = hc.alloc(n);
         float *d_out = hc.alloc(n);
-        check_launch(et_launch_conv_axis(d_in, d_tmp, nx, ny, nz, 1, nx, (long)nx * ny, 0, 0, d_sep, h, 0,
+        check_launch(et_launch_conv_axis(d_in, d_tmp, nx, ny, nz, 1, nx, (long)nx * ny, 0, 0, d_sep, h, 0, 1, 0,
                                          (et_stream_t)hc.st));
-        check_launch(et_launch_conv_axis(d_tmp, d_out, nx, ny, nz, 1, nx, (long)nx * ny, 0, 1, d_sep, h, 0,
+        check_launch(et_launch_conv_axis(d_tmp, d_out, nx, ny, nz, 1, nx, (long)nx * ny, 0, 1, d_sep, h, 0, 1, 0,
                                          (et_stream_t)hc.st));
         hc.download(out, d_out, n);
         return niftyrec_success;

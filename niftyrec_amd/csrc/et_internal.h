@@ -53,9 +53,11 @@ struct EtSweepArgs {
     int yu, ustride;         // U layout of the output volumes (per view stride)
     int V, D, zlen;          // views in launch, depth chunks, z' per chunk
     int slabs;               // ceil(ny / ET_T)
-    const float *views;      // [V][ET_VIEW_REC]
-    const float *act;        // YF
-    const float *mu;         // YF or null
+    const float *views;      // view v's record at views + v * rec_stride
+    int rec_stride;          // ET_VIEW_REC; 0 on the general path: one identity record for every view
+    const float *act;        // YF; view v reads act + v * act_vs
+    const float *mu;         // YF or null; view v reads mu + v * mu_vs
+    size_t act_vs, mu_vs;    // 0: one volume for every view; the general path's rotated copies: one per view
     const float *psf;        // [nz][2K] row kernel, column kernel (null when R == 0)
     int K;
     float bg_act, bg_mu;     // padding used when resampling act / mu
@@ -140,8 +142,9 @@ int et_launch_pack_yf(const float *abi, float *yf, int nx, int ny, int nz, int y
                       et_stream_t stream);
 int et_launch_unpack_yf(const float *yf, float *abi, int nx, int ny, int nz, int yp, int gy,
                         et_stream_t stream);
+// nv views: view v samples src with the matrix at M12 + v * ET_VIEW_REC into dst + v * dst_vs.
 int et_launch_resample_general(const float *src, int nx, int ny, int nz, const float *M12,
-                               float bg, float *dst, int dst_yf, int yp, int gy,
+                               float bg, float *dst, int dst_yf, int yp, int gy, int nv, size_t dst_vs,
                                et_stream_t stream);
 // Attenuation at the start of every chunk (astart, rounded) and along whole
 // rays (atot + atot_lo), compensated sums of the chunk sums csum + csum_lo.
@@ -151,8 +154,9 @@ int et_launch_reduce_parts(const float *part, int D, int V, int P, float *sino, 
                            et_stream_t stream);
 int et_launch_bg_only(const float *atot, const float *atot_lo, float bg, int n, float *sino, int truncate,
                       et_stream_t stream);
+// nv volumes, vs floats apart in src and dst.
 int et_launch_conv_axis(const float *src, float *dst, int nx, int ny, int nz, long sx, long sy,
-                        long sz, long off, int axis, const float *sep, int K, int flip,
+                        long sz, long off, int axis, const float *sep, int K, int flip, int nv, size_t vs,
                         et_stream_t stream);
 int et_launch_truncate(float *buf, size_t n, et_stream_t stream);
 int et_launch_fill(float *buf, size_t n, float value, et_stream_t stream);

@@ -295,12 +295,15 @@ __device__ float trilinear_ref(const Acc &src, int nx, int ny, int nz, float px,
     return intensity;
 }
 
-// dst(v) = src(M v) for every voxel v of the grid; dst in YF (dst_yf) or ABI layout.
+// dst(v) = src(M v) for every voxel v of the grid; dst in YF (dst_yf) or ABI
+// layout; grid (voxel blocks, views).
 __global__ void __launch_bounds__(256) k_resample_general(const float *__restrict__ src, int nx,
                                                           int ny, int nz, const float *__restrict__ M,
                                                           float bg, float *__restrict__ dst, int dst_yf,
-                                                          int yp, int gy)
+                                                          int yp, int gy, size_t dst_vs)
 {
+    M += (size_t)blockIdx.y * ET_VIEW_REC;
+    dst += (size_t)blockIdx.y * dst_vs;
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t n = (size_t)nx * ny * nz;
     if (i >= n) return;
@@ -326,7 +329,9 @@ __global__ void __launch_bounds__(256) k_resample_general(const float *__restric
         dst[x + (size_t)nx * (y + (size_t)ny * z)] = val;
 }
 
-// General pull of one view into the output (accumulating in place).
+// General pull of a.V views into the output, added in view order (onto the
+// previous content when accumulating).  One launch for a batch of views: a
+// view alone has too few voxels to fill the device at small sizes.
 // Reference mode: inverse matrix (record[12..23]) with the reference borders.
 // Adjoint mode: transpose of k_resample_general's pull with the forward matrix.
 template <int EPI>
@@ -339,65 +344,68 @@ __global__ void __launch_bounds__(256) k_pull_general(EtPullArgs a)
     const size_t r = i / a.nx;
     const int y = (int)(r % a.ny);
     const int z = (int)(r / a.ny);
-    const float *rec = a.views;
-    const float *uv = a.u;
-    float val = 0.f;
-    if (!a.adjoint) {
-        const float *Mi = rec + 12;
-        const float fx = (float)x, fy = (float)y, fz = (float)z;
-        UAccess acc{uv, a.yu, a.xp};
-        val = trilinear_ref(acc, a.nx, a.ny, a.nz, pos3(Mi, fx, fy, fz), pos3(Mi + 4, fx, fy, fz),
-                            pos3(Mi + 8, fx, fy, fz), a.bg);
-    } else {
-        const float *F = rec;
-        const float *Fi = rec + 24;
-        const float rv[3] = {(float)x - F[3], (float)y - F[7], (float)z - F[11]};
-        int lo[3], hi[3];
-        const int nn[3] = {a.nx, a.ny, a.nz};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const float c = Fi[3 * k] * rv[0] + Fi[3 * k + 1] * rv[1] + Fi[3 * k + 2] * rv[2];
-            const float h = fabsf(Fi[3 * k]) + fabsf(Fi[3 * k + 1]) + fabsf(Fi[3 * k + 2]) + 0.01f;
-            lo[k] = max(0, (int)ceilf(c - h));
-            hi[k] = min(nn[k] - 1, (int)floorf(c + h));
-        }
-        const float o[3] = {(float)x, (float)y, (float)z};
-        for (int zc = lo[2]; zc <= hi[2]; zc++)
-            for (int yc = lo[1]; yc <= hi[1]; yc++)
-                for (int xc = lo[0]; xc <= hi[0]; xc++) {
-                    const float p[3] = {pos3(F, (float)xc, (float)yc, (float)zc),
-                                        pos3(F + 4, (float)xc, (float)yc, (float)zc),
-                                        pos3(F + 8, (float)xc, (float)yc, (float)zc)};
-                    float w = 1.f;
-#pragma unroll
-                    for (int k = 0; k < 3; k++) {
-                        const float f = floorf(p[k]), rr = p[k] - f;
-                        w *= (f == o[k]) ? 1.f - rr : ((f == o[k] - 1.f) ? rr : 0.f);
+    float *o;
+    if constexpr (EPI == ET_EPI_ABI_STORE)
+        o = a.out + i;
+    else
+        o = a.out + (a.gy + y) + (size_t)a.yp * ((x + 1) + (size_t)(a.nx + 2) * (z + 1));
+    float res = a.accumulate ? *o : 0.f;
+    for (int v = 0; v < a.V; v++) {
+        const float *rec = a.views + (size_t)v * ET_VIEW_REC;
+        const float *uv = a.u + (size_t)v * a.ustride;
+        float val = 0.f;
+        if (!a.adjoint) {
+            const float *Mi = rec + 12;
+            const float fx = (float)x, fy = (float)y, fz = (float)z;
+            UAccess acc{uv, a.yu, a.xp};
+            val = trilinear_ref(acc, a.nx, a.ny, a.nz, pos3(Mi, fx, fy, fz), pos3(Mi + 4, fx, fy, fz),
+                                pos3(Mi + 8, fx, fy, fz), a.bg);
+        } else {
+            const float *F = rec;
+            const float *Fi = rec + 24;
+            const float rv[3] = {(float)x - F[3], (float)y - F[7], (float)z - F[11]};
+            int lo[3], hi[3];
+            const int nn[3] = {a.nx, a.ny, a.nz};
+    #pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const float c = Fi[3 * k] * rv[0] + Fi[3 * k + 1] * rv[1] + Fi[3 * k + 2] * rv[2];
+                const float h = fabsf(Fi[3 * k]) + fabsf(Fi[3 * k + 1]) + fabsf(Fi[3 * k + 2]) + 0.01f;
+                lo[k] = max(0, (int)ceilf(c - h));
+                hi[k] = min(nn[k] - 1, (int)floorf(c + h));
+            }
+            const float o[3] = {(float)x, (float)y, (float)z};
+            for (int zc = lo[2]; zc <= hi[2]; zc++)
+                for (int yc = lo[1]; yc <= hi[1]; yc++)
+                    for (int xc = lo[0]; xc <= hi[0]; xc++) {
+                        const float p[3] = {pos3(F, (float)xc, (float)yc, (float)zc),
+                                            pos3(F + 4, (float)xc, (float)yc, (float)zc),
+                                            pos3(F + 8, (float)xc, (float)yc, (float)zc)};
+                        float w = 1.f;
+    #pragma unroll
+                        for (int k = 0; k < 3; k++) {
+                            const float f = floorf(p[k]), rr = p[k] - f;
+                            w *= (f == o[k]) ? 1.f - rr : ((f == o[k] - 1.f) ? rr : 0.f);
+                        }
+                        if (w != 0.f) val = fmaf(w, uv[yc + (size_t)a.yu * ((xc + 1) + (size_t)a.xp * (zc + 1))], val);
                     }
-                    if (w != 0.f) val = fmaf(w, uv[yc + (size_t)a.yu * ((xc + 1) + (size_t)a.xp * (zc + 1))], val);
-                }
+        }
+        res += val;
     }
-    if constexpr (EPI == ET_EPI_ABI_STORE) {
-        float *o = a.out + i;
-        float res = a.accumulate ? *o + val : val;
-        if (a.truncate && res < 0.f) res = 0.f;
-        *o = res;
-    } else {
-        float *o = a.out + (a.gy + y) + (size_t)a.yp * ((x + 1) + (size_t)(a.nx + 2) * (z + 1));
-        float res = a.accumulate ? *o + val : val;
-        if (a.truncate && res < 0.f) res = 0.f;
-        *o = res;
-    }
+    if (a.truncate && res < 0.f) res = 0.f;
+    *o = res;
 }
 
 // One axis of the depth-dependent separable convolution with a runtime radius
 // (general path, PSF radius beyond ET_RMAX).  axis 0: row kernel along x,
-// axis 1: column kernel along y.  flip: correlation (adjoint).
+// axis 1: column kernel along y.  flip: correlation (adjoint).  grid (voxel
+// blocks, volumes).
 __global__ void __launch_bounds__(256) k_conv_axis(const float *__restrict__ src, float *__restrict__ dst,
                                                    int nx, int ny, int nz, long sx, long sy, long sz,
                                                    long off, int axis, const float *__restrict__ sep,
-                                                   int K, int flip)
+                                                   int K, int flip, size_t vs)
 {
+    src += (size_t)blockIdx.y * vs;
+    dst += (size_t)blockIdx.y * vs;
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t n = (size_t)nx * ny * nz;
     if (i >= n) return;
@@ -844,11 +852,12 @@ int et_launch_unpack_yf(const float *yf, float *abi, int nx, int ny, int nz, int
 }
 
 int et_launch_resample_general(const float *src, int nx, int ny, int nz, const float *M12, float bg, float *dst,
-                               int dst_yf, int yp, int gy, et_stream_t stream)
+                               int dst_yf, int yp, int gy, int nv, size_t dst_vs, et_stream_t stream)
 {
     const size_t n = (size_t)nx * ny * nz;
-    hipLaunchKernelGGL(k_resample_general, dim3(nblk(n, 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                       src, nx, ny, nz, M12, bg, dst, dst_yf, yp, gy);
+    if (nv <= 0 || nv > 65535) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_resample_general, dim3(nblk(n, 256), nv), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), src, nx, ny, nz, M12, bg, dst, dst_yf, yp, gy, dst_vs);
     return (int)hipGetLastError();
 }
 
@@ -877,11 +886,12 @@ int et_launch_bg_only(const float *atot, const float *atot_lo, float bg, int n, 
 }
 
 int et_launch_conv_axis(const float *src, float *dst, int nx, int ny, int nz, long sx, long sy, long sz, long off,
-                        int axis, const float *sep, int K, int flip, et_stream_t stream)
+                        int axis, const float *sep, int K, int flip, int nv, size_t vs, et_stream_t stream)
 {
     const size_t n = (size_t)nx * ny * nz;
-    hipLaunchKernelGGL(k_conv_axis, dim3(nblk(n, 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), src,
-                       dst, nx, ny, nz, sx, sy, sz, off, axis, sep, K, flip);
+    if (nv <= 0 || nv > 65535) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_conv_axis, dim3(nblk(n, 256), nv), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), src,
+                       dst, nx, ny, nz, sx, sy, sz, off, axis, sep, K, flip, vs);
     return (int)hipGetLastError();
 }
 

@@ -74,11 +74,11 @@ __device__ __forceinline__ void project_body(const EtSweepArgs &a, const Blk &b)
         float yc[TS];
         if constexpr (COOP) {
             float rows[NA];
-            coop_rows<NA, LA, SA, OPA>(a.act + (a.gy + c.y0 - R4), c.dx, c.dz, s, tab, stage,
+            coop_rows<NA, LA, SA, OPA>(c.act + (a.gy + c.y0 - R4), c.dx, c.dz, s, tab, stage,
                                        [](int, float v) { return v; }, rows);
             column_pass<TS, R>(rows, kz + K, yc);
         } else {
-            resample_column<TS, R, NA, LA, SA>(a.act + s.off + (a.gy + c.y0 - R4), c.dx, c.dz, s, kz + K,
+            resample_column<TS, R, NA, LA, SA>(c.act + s.off + (a.gy + c.y0 - R4), c.dx, c.dz, s, kz + K,
                                                [](int, float v) { return v; }, yc);
         }
         if constexpr (HAS_MU && AM != 2) {
@@ -89,9 +89,9 @@ __device__ __forceinline__ void project_body(const EtSweepArgs &a, const Blk &b)
             };
             if constexpr (COOP) {
                 float dummy[TS];
-                coop_rows<TS, TS, 0, OPM>(a.mu + (a.gmu + c.y0), c.dx, c.dz, s, tab, stage, cum, dummy);
+                coop_rows<TS, TS, 0, OPM>(c.mu + (a.gmu + c.y0), c.dx, c.dz, s, tab, stage, cum, dummy);
             } else {
-                bilinear_map<TS, TS, 0>(a.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s,
+                bilinear_map<TS, TS, 0>(c.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s,
                                         [&](int i, float m) { comp_add(A[i], Al[i], m); });
             }
         }
@@ -213,10 +213,10 @@ __device__ __forceinline__ void bpu_body(const EtSweepArgs &a, const Blk &b)
             };
             if constexpr (COOP) {
                 float rows[NA];
-                coop_rows<NA, LA, SA, OPA>(a.mu + (a.gmu + c.y0 - R4), c.dx, c.dz, s, tab, stage, wfun, rows);
+                coop_rows<NA, LA, SA, OPA>(c.mu + (a.gmu + c.y0 - R4), c.dx, c.dz, s, tab, stage, wfun, rows);
                 column_pass<TS, R>(rows, kz + K, yc);
             } else {
-                resample_column<TS, R, NA, LA, SA>(a.mu + s.off + (a.gmu + c.y0 - R4), c.dx, c.dz, s, kz + K, wfun,
+                resample_column<TS, R, NA, LA, SA>(c.mu + s.off + (a.gmu + c.y0 - R4), c.dx, c.dz, s, kz + K, wfun,
                                                    yc);
             }
         } else if constexpr (R == 0) {
@@ -319,12 +319,12 @@ __global__ void __launch_bounds__(512) k_grad_ref(EtSweepArgs a)
         const float *kz = psf_plane<R>(a.psf, z);  // never read when R == 0
         // mu rows first: tail needs A(z') before this plane's mu joins the suffix
         float Az[NA];
-        bilinear_map<NA, LA, SA>(a.mu + s.off + (a.gmu + c.y0 - R4), c.dx, c.dz, s, [&](int j, float m) {
+        bilinear_map<NA, LA, SA>(c.mu + s.off + (a.gmu + c.y0 - R4), c.dx, c.dz, s, [&](int j, float m) {
             Az[j] = (At[j] - suf[j]) + (Atl[j] - sufl[j]);
             comp_add(suf[j], sufl[j], m);
         });
         float yc[TS];
-        resample_column<TS, R, NA, LA, SA>(a.act + s.off + (a.gy + c.y0 - R4), c.dx, c.dz, s, kz + K,
+        resample_column<TS, R, NA, LA, SA>(c.act + s.off + (a.gy + c.y0 - R4), c.dx, c.dz, s, kz + K,
                                            [&](int j, float v) {
                                                tail[j] = fmaf(v, exp_neg(Az[j]), tail[j]);
                                                return sv[j] * tail[j];
@@ -373,7 +373,7 @@ __global__ void __launch_bounds__(512) k_grad_mu(EtSweepArgs a)
         float h[TS];
         {
             float yc[TS];
-            resample_column<TS, R, NA, LA, SA>(a.act + s.off + (a.gy + c.y0 - R4), c.dx, c.dz, s, kz + K,
+            resample_column<TS, R, NA, LA, SA>(c.act + s.off + (a.gy + c.y0 - R4), c.dx, c.dz, s, kz + K,
                                                [](int, float v) { return v; }, yc);
             if constexpr (R == 0) {
 #pragma unroll
@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(512) k_grad_mu(EtSweepArgs a)
             }
         }
         float out[TS];
-        bilinear_map<TS, TS, 0>(a.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s, [&](int i, float m) {
+        bilinear_map<TS, TS, 0>(c.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s, [&](int i, float m) {
             const float Az = (At[i] - suf[i]) + (Atl[i] - sufl[i]);
             comp_add(suf[i], sufl[i], m);
             tail[i] = fmaf(h[i], exp_neg(Az), tail[i]);
@@ -414,7 +414,7 @@ __global__ void __launch_bounds__(512) k_att_factors(EtSweepArgs a)
     }
     for (int z = 0; z < a.nz; z++) {
         const Samp s = fast_sample(c.fv, c.fxp, z, a.nx, a.nz, c.dx, c.dz);
-        bilinear_map<TS, TS, 0>(a.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s,
+        bilinear_map<TS, TS, 0>(c.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s,
                                 [&](int i, float m) { comp_add(A[i], Al[i], m); });
         float *ez = a.att + (((size_t)c.v * a.nz + z) * a.yu + c.y0) * c.nthr + c.tx;
 #pragma unroll
@@ -437,7 +437,7 @@ __global__ void __launch_bounds__(512) k_musum(EtSweepArgs a)
     }
     for (int z = c.zb; z < c.ze; z++) {
         const Samp s = fast_sample(c.fv, c.fxp, z, a.nx, a.nz, c.dx, c.dz);
-        bilinear_map<TS, TS, 0>(a.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s,
+        bilinear_map<TS, TS, 0>(c.mu + s.off + (a.gmu + c.y0), c.dx, c.dz, s,
                                 [&](int i, float m) { comp_add(acc[i], lo[i], m); });
     }
     const size_t off = ((size_t)c.v * a.D + c.d) * c.P;
