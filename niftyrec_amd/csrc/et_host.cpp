@@ -827,25 +827,49 @@ EtSweepArgs general_args(et_plan *p, int nv, int D, bool act, bool mu)
     return a;
 }
 
-// Rotated copies of an ABI volume for views [v0, v0 + nv) in the YF layout (+
-// PSF when the radius is too large for the sweep kernels).
-void rotate_general(et_plan *p, const float *abi, int v0, int nv, float bg, DevBuf &dst, bool psf)
+// Source volumes of an operation in the YF layout, once per operation, where the
+// rotation reads that (zero background); the others are read as the caller's.
+void general_sources(et_plan *p, const float *act, const float *mu)
+{
+    if (act && p->bg == 0.f) pack(p, act, p->act_yf);
+    if (mu && p->bga == 0.f) pack(p, mu, p->mu_yf);
+}
+
+// Rotated copies of act and mu (either may be null) for views [v0, v0 + nv) in
+// the YF layout, into rot_act (+ the PSF when asked for and its radius is too
+// large for the sweep kernels) and rot_mu; after general_sources.
+void rotate_general(et_plan *p, const float *act, const float *mu, int v0, int nv, bool psf)
 {
     const size_t vs = p->yf_elems;
-    dst.ensure(nv * vs, true, p->st);
+    const float *recs = p->d_recs.p + (size_t)v0 * ET_VIEW_REC;
+    const et_stream_t st = (et_stream_t)p->st;
+    if (act) p->rot_act.ensure(nv * vs, true, p->st);
+    if (mu) p->rot_mu.ensure(nv * vs, true, p->st);
+    const bool act_yf = act && p->bg == 0.f, mu_yf = mu && p->bga == 0.f;
     {
-        ProfScope ps(p, ET_PROF_OTHER, nv * 8.0 * p->nvox);
-        check_launch(et_launch_resample_general(abi, p->nx, p->ny, p->nz, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, bg,
-                                                dst.p, 1, p->yp, p->gy, nv, vs, (et_stream_t)p->st));
+        ProfScope ps(p, ET_PROF_OTHER, nv * ((act ? 8.0 : 0.0) + (mu ? 8.0 : 0.0)) * p->nvox);
+        if (act_yf || mu_yf)
+            check_launch(et_launch_rotate_yf(act_yf ? p->act_yf.p : p->mu_yf.p, act_yf && mu_yf ? p->mu_yf.p : nullptr,
+                                             p->nx, p->ny, p->nz, recs, p->yp, p->gy,
+                                             act_yf ? p->rot_act.p : p->rot_mu.p,
+                                             act_yf && mu_yf ? p->rot_mu.p : nullptr, vs, nv, st));
+        // a background takes the reference's border rule
+        if (act && !act_yf)
+            check_launch(et_launch_resample_general(act, p->nx, p->ny, p->nz, recs, p->bg, p->rot_act.p, 1, p->yp,
+                                                    p->gy, nv, vs, st));
+        if (mu && !mu_yf)
+            check_launch(et_launch_resample_general(mu, p->nx, p->ny, p->nz, recs, p->bga, p->rot_mu.p, 1, p->yp,
+                                                    p->gy, nv, vs, st));
     }
-    if (psf && p->K > 0 && p->R > ET_RMAX) {
+    if (act && psf && p->K > 0 && p->R > ET_RMAX) {
         // row (x) pass then column (y) pass, emission-lib/_et_convolveSeparable2D.cpp:43-75
+        float *dst = p->rot_act.p;
         p->tmp.ensure(nv * vs, true, p->st);
         const long sx = p->yp, sy = 1, sz = (long)p->yp * p->xp, off = p->gy + (long)p->yp * (1 + p->xp);
-        check_launch(et_launch_conv_axis(dst.p, p->tmp.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 0, p->d_sep.p, p->K, 0,
-                                         nv, vs, (et_stream_t)p->st));
-        check_launch(et_launch_conv_axis(p->tmp.p, dst.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 1, p->d_sep.p, p->K, 0,
-                                         nv, vs, (et_stream_t)p->st));
+        check_launch(et_launch_conv_axis(dst, p->tmp.p, p->nx, p->ny, p->nz, sx, sy, sz, off, 0, p->d_sep.p, p->K, 0,
+                                         nv, vs, st));
+        check_launch(et_launch_conv_axis(p->tmp.p, dst, p->nx, p->ny, p->nz, sx, sy, sz, off, 1, p->d_sep.p, p->K, 0,
+                                         nv, vs, st));
     }
 }
 
@@ -919,18 +943,18 @@ void op_project(et_plan *p, const float *act, const float *mu, float *sino, int 
         return;
     }
     // general path
+    general_sources(p, act, mu);
     const int R = general_R(p), vb = general_batch(p);
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
         float *sv = sino + (size_t)v0 * p->P;
-        if (mu) rotate_general(p, mu, v0, nv, p->bga, p->rot_mu, false);
+        rotate_general(p, act, mu, v0, nv, true);
         if (!act) {
             mu_prefix(p, p->d_ident.p, nv, 1, p->rot_mu.p, false, true, true);
             check_launch(et_launch_bg_only(p->atot.p, p->atot_lo.p, p->bg, (int)(nv * p->P), sv, truncate,
                                            (et_stream_t)p->st));
             continue;
         }
-        rotate_general(p, act, v0, nv, p->bg, p->rot_act, true);
         const int D = general_D(p, nv);
         if (mu && D > 1) mu_prefix(p, p->d_ident.p, nv, D, p->rot_mu.p, true, false, true);
         EtSweepArgs a = general_args(p, nv, D, true, mu != nullptr);
@@ -975,11 +999,12 @@ void op_backproject(et_plan *p, const float *sino, const float *mu, float *out, 
         }
         return;
     }
+    general_sources(p, nullptr, mu);
     const int R = general_R(p), vb = general_batch(p);
     p->u.ensure((size_t)vb * p->ustride, true, p->st);
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
-        if (mu) rotate_general(p, mu, v0, nv, p->bga, p->rot_mu, false);
+        if (mu) rotate_general(p, nullptr, mu, v0, nv, false);
         const int D = general_D(p, nv);
         if (mu && D > 1) mu_prefix(p, p->d_ident.p, nv, D, p->rot_mu.p, true, false, true);
         EtSweepArgs a = general_args(p, nv, D, false, mu != nullptr);
@@ -1030,12 +1055,12 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
         }
         return;
     }
+    general_sources(p, act, mu);
     const int R = general_R(p), vb = general_batch(p);
     p->u.ensure((size_t)vb * p->ustride, true, p->st);
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
-        rotate_general(p, mu, v0, nv, p->bga, p->rot_mu, false);
-        rotate_general(p, act, v0, nv, p->bg, p->rot_act, exact);
+        rotate_general(p, act, mu, v0, nv, exact);
         mu_prefix(p, p->d_ident.p, nv, 1, p->rot_mu.p, false, true, true);
         EtSweepArgs a = general_args(p, nv, 1, true, true);
         a.atot = p->atot.p;

@@ -146,6 +146,11 @@ int et_launch_unpack_yf(const float *yf, float *abi, int nx, int ny, int nz, int
 int et_launch_resample_general(const float *src, int nx, int ny, int nz, const float *M12,
                                float bg, float *dst, int dst_yf, int yp, int gy, int nv, size_t dst_vs,
                                et_stream_t stream);
+// Rotated copies of s0 into d0 and (when not null) s1 into d1 for nv views with
+// records recs: YF volumes with zero borders (at least one guard row on either
+// side), dst volumes vs floats apart.
+int et_launch_rotate_yf(const float *s0, const float *s1, int nx, int ny, int nz, const float *recs, int yp, int gy,
+                        float *d0, float *d1, size_t vs, int nv, et_stream_t stream);
 // Attenuation at the start of every chunk (astart, rounded) and along whole
 // rays (atot + atot_lo), compensated sums of the chunk sums csum + csum_lo.
 int et_launch_chunk_scan(const float *csum, const float *csum_lo, float *astart, float *atot, float *atot_lo,

@@ -19,7 +19,8 @@ def _t(a):
 
 
 @pytest.mark.parametrize("batch, chunks", [(1, 0), (3, 0), (0, 0), (3, 1), (2, 5)])
-@pytest.mark.parametrize("shape, K, bg", [((18, 21, 18), 5, 0.0), ((26, 9, 26), 23, 0.0), ((12, 17, 12), 0, 0.3)])
+@pytest.mark.parametrize("shape, K, bg", [((18, 21, 18), 5, 0.0), ((26, 9, 26), 23, 0.0), ((12, 17, 12), 0, 0.3),
+                                          ((10, 70, 10), 3, 0.0)])
 def test_general_path_in_batches(shape, K, bg, batch, chunks):
     from niftyrec_amd.api import Plan
     rng = np.random.default_rng(11)
