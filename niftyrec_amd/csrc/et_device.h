@@ -410,6 +410,34 @@ __device__ __forceinline__ Samp fast_sample(const FastView &fv, float fxp, int z
     return make_samp(px, pz, nx, nz, dx, dz);
 }
 
+// 64-bit mix of one element of a content fingerprint (bits in the upper half,
+// index times an odd constant folded in): the fingerprint of an array is the sum
+// modulo 2^64 over its elements, so any partition into blocks gives the same key.
+__device__ __forceinline__ unsigned long long fp_mix(unsigned long long h)
+{
+    h ^= h >> 33;
+    h *= 0xff51afd7ed558ccdull;
+    h ^= h >> 33;
+    h *= 0xc4ceb9fe1a85ec53ull;
+    h ^= h >> 33;
+    return h;
+}
+__device__ __forceinline__ unsigned long long fp_element(unsigned bits, size_t i)
+{
+    return fp_mix(((unsigned long long)bits << 32) ^ (i * 0x9e3779b97f4a7c15ull));
+}
+
+// Sum of h over a block of 256 threads (every thread gets it); `part` holds 4 words.
+__device__ __forceinline__ unsigned long long block_sum_256(unsigned long long h, unsigned long long *part)
+{
+    for (int o = 32; o >= 1; o >>= 1) h += __shfl_xor(h, o, 64);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = h;
+    __syncthreads();
+    h = part[0] + part[1] + part[2] + part[3];
+    __syncthreads();
+    return h;
+}
+
 // Sum over d < D of part[d * stride + i], added in order of d with TwoSum
 // compensation.  The loads go out eight at a time: a loop that adds each value
 // as it arrives waits out one memory latency per term.

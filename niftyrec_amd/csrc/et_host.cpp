@@ -284,18 +284,20 @@ struct et_plan {
     DevBuf fac, sino_t, op_acc, op_acc2;  // (op_acc, op_acc2: pull accumulators, YF layout)
     DevBuf op_tables[YL_OP_SLOTS];        // per operation: its last table, and that table's bytes
     std::vector<char> op_tables_h[YL_OP_SLOTS];
-    bool fac_valid = false;
-    unsigned long long fac_key = 0;
-    // the last projection's partial sums [fwd_D][V][x'][rows] and the content
-    // keys of its activity and map: an exact gradient of the same pair seeds
-    // its reverse sweeps from them instead of projecting again
+    // content keys on the device (EtKeys), and what the host knows: key_gen the
+    // operations so far, fac_built / fwd_built whether the factors / the forward
+    // sums hold those of the last keys
+    DevBuf keys;
+    unsigned key_gen = 0;
+    bool fac_built = false, fwd_built = false;
+    // the last projection's partial sums [D][V][x'][rows] (D chunks as asked of
+    // yl_chunks, the projector's tiles): an exact gradient of the same activity
+    // and map seeds its reverse sweeps from them instead of projecting again
     DevBuf fwd_part;
-    bool fwd_valid = false;
-    unsigned long long fwd_act = 0, fwd_mu = 0;
-    int fwd_D = 0, fwd_tiles = 0;  // (fwd_D: the depth chunks the projection asked yl_chunks for)
+    int fwd_D = 0, fwd_tiles = 0;
     std::vector<struct YlLaunch> yl_launches;          // per subset: projection, ratio, backprojection, pull
     std::vector<const void *> osem_sig;                // buffers yl_launches refer to
-    DevBuf fp_dev;                  // fingerprint partial sums (two arrays of ET_FP_BLOCKS)
+    DevBuf fp_dev;                  // fingerprint partial sums (ET_FP_BLOCKS)
     unsigned long long *fp_host = nullptr;  // their pinned host copy
     // tuning
     int tune_D = 0, tune_vb = 0;
@@ -904,19 +906,17 @@ void pull_general(et_plan *p, int v0, int nv, const float *u, bool adjoint, bool
 
 // Row-lane versions (defined with the row-lane kernels' host code); false when
 // the plan does not take them.
-bool yl_op_project(et_plan *p, const float *act, const float *act_yf, const float *mu, const float *mu_yf, float *sino,
-                   int truncate);
-bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, const float *mu_yf, float *out, bool adjoint,
-                       int truncate);
-bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float *act_yf, const float *mu,
-                    const float *mu_yf, float *out, int truncate);
-bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float *act_yf, const float *mu,
-                    const float *mu_yf, float *out_act, float *out_mu, int truncate);
+bool yl_op_project(et_plan *p, const float *act, const float *mu, float *sino, int truncate);
+bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate);
+bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate);
+bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float *mu, float *out_act, float *out_mu,
+                    int truncate);
 
 void op_project(et_plan *p, const float *act, const float *mu, float *sino, int truncate)
 {
-    const float *act_yf = nullptr, *mu_yf = nullptr;
     if (p->fast) {
+        if (yl_op_project(p, act, mu, sino, truncate)) return;
+        const float *act_yf = nullptr, *mu_yf = nullptr;
         if (act) {
             pack(p, act, p->act_yf);
             act_yf = p->act_yf.p;
@@ -932,7 +932,6 @@ void op_project(et_plan *p, const float *act, const float *mu, float *sino, int 
                                            (et_stream_t)p->st));
             return;
         }
-        if (yl_op_project(p, act, act_yf, mu, mu_yf, sino, truncate)) return;
         const int D = mu ? choose_D(p, p->V) : std::max(1, choose_D(p, p->V));
         const float *astart = nullptr;
         if (mu && D > 1) {
@@ -975,12 +974,12 @@ void op_project(et_plan *p, const float *act, const float *mu, float *sino, int 
 void op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate)
 {
     if (p->fast) {
+        if (yl_op_backproject(p, sino, mu, out, adjoint, truncate)) return;
         const float *mu_yf = nullptr;
         if (mu) {
             pack(p, mu, p->mu_yf);
             mu_yf = p->mu_yf.p;
         }
-        if (yl_op_backproject(p, sino, mu, mu_yf, out, adjoint, truncate)) return;
         const int vb = view_batch(p);
         p->u.ensure((size_t)vb * p->ustride, true, p->st);
         for (int v0 = 0; v0 < p->V; v0 += vb) {
@@ -1027,9 +1026,9 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
 {
     const int mode = exact ? ET_MODE_GRAD_MU : ET_MODE_GRAD_REF;
     if (p->fast) {
+        if (exact && yl_op_gradient(p, sino, act, mu, out, truncate)) return;
         pack(p, act, p->act_yf);
         pack(p, mu, p->mu_yf);
-        if (exact && yl_op_gradient(p, sino, act, p->act_yf.p, mu, p->mu_yf.p, out, truncate)) return;
         const int vb = grad_view_batch(p);
         p->u.ensure((size_t)vb * p->ustride, true, p->st);
         for (int v0 = 0; v0 < p->V; v0 += vb) {
@@ -1079,16 +1078,11 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
 
 // Both gradients of <sino, project(act, mu)>: the exact adjoint backprojection
 // of sino (activity) and the exact attenuation gradient (mu).  Row-lane plans
-// after a projection of the same pair take one pass (yl_op_backward); otherwise
-// the two operations in turn.
+// take one pass (yl_op_backward), others the two operations in turn.
 void op_backward(et_plan *p, const float *sino, const float *act, const float *mu, float *out_act, float *out_mu,
                  int truncate)
 {
-    if (p->fast && p->yl_ops && p->yl) {
-        pack(p, act, p->act_yf);
-        pack(p, mu, p->mu_yf);
-        if (yl_op_backward(p, sino, act, p->act_yf.p, mu, p->mu_yf.p, out_act, out_mu, truncate)) return;
-    }
+    if (yl_op_backward(p, sino, act, mu, out_act, out_mu, truncate)) return;
     op_backproject(p, sino, mu, out_act, true, truncate);
     op_gradient(p, sino, act, mu, out_mu, true, truncate);
 }
@@ -1265,50 +1259,33 @@ int tune_depth_chunks(et_plan *p, int mode, const float *recs, int nv, const flo
 // into the YF layout), osem_subset (one subset update on the YF iterate) and
 // osem_finish (x unpacked).  The subset layout stays in the plan between them.
 // Key of the attenuation map for the OSEM caches: mu_key_launch queues its
-// content fingerprint (copied to pinned host memory) on the plan's stream;
-// mu_key_read returns it once the stream has reached that point (or mu's
-// address when the plan's mu_check is off and `content` is not asked for, 0
-// without attenuation).
-// Queues the fingerprints of a and (when not null) b, n = nvox floats each,
-// and the copy of their partial sums to pinned host memory.
-void fp_launch(et_plan *p, const float *a, const float *b)
+// content fingerprint (partial sums copied to pinned host memory) on the plan's
+// stream; mu_key_read returns it once the stream has reached that point (or
+// mu's address when the plan's mu_check is off, 0 without attenuation).
+void mu_key_launch(et_plan *p, const float *mu)
 {
-    p->fp_dev.ensure(2 * 2 * ET_FP_BLOCKS, false);  // (floats: two arrays of 8-byte partials)
-    if (!p->fp_host && hipHostMalloc((void **)&p->fp_host, 2 * ET_FP_BLOCKS * sizeof(unsigned long long),
+    if (!mu || !p->mu_check) return;
+    p->fp_dev.ensure(2 * ET_FP_BLOCKS, false);  // (8-byte partials)
+    if (!p->fp_host && hipHostMalloc((void **)&p->fp_host, ET_FP_BLOCKS * sizeof(unsigned long long),
                                      hipHostMallocDefault) != hipSuccess) {
         p->fp_host = nullptr;
         throw EtError{niftyrec_error_alloccpu};
     }
     const int nb = et_fingerprint_blocks(p->nvox);
     unsigned long long *d = reinterpret_cast<unsigned long long *>(p->fp_dev.p);
-    ProfScope ps(p, ET_PROF_OTHER, (b ? 8.0 : 4.0) * p->nvox);
-    check_launch(et_launch_fingerprints(a, b, p->nvox, d, (et_stream_t)p->st));
-    check_hip(hipMemcpyAsync(p->fp_host, d, (b ? 2 : 1) * nb * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                             p->st),
+    ProfScope ps(p, ET_PROF_OTHER, 4.0 * p->nvox);
+    check_launch(et_launch_fingerprint(mu, p->nvox, d, (et_stream_t)p->st));
+    check_hip(hipMemcpyAsync(p->fp_host, d, nb * sizeof(unsigned long long), hipMemcpyDeviceToHost, p->st),
               niftyrec_error_transfergpu);
 }
 
-// Key of array k (0: a, 1: b) of the last fp_launch, once the stream has
-// reached it: the sum modulo 2^64 of its partials.
-unsigned long long fp_key(const et_plan *p, int k)
-{
-    const int nb = et_fingerprint_blocks(p->nvox);
-    unsigned long long key = 0;
-    for (int i = 0; i < nb; i++) key += p->fp_host[(size_t)k * nb + i];
-    return key;
-}
-
-void mu_key_launch(et_plan *p, const float *mu, bool content = false)
-{
-    if (!mu || !(p->mu_check || content)) return;
-    fp_launch(p, mu, nullptr);
-}
-
-unsigned long long mu_key_read(const et_plan *p, const float *mu, bool content = false)
+unsigned long long mu_key_read(const et_plan *p, const float *mu)
 {
     if (!mu) return 0;
-    if (!(p->mu_check || content)) return (unsigned long long)(uintptr_t)mu;
-    return fp_key(p, 0);
+    if (!p->mu_check) return (unsigned long long)(uintptr_t)mu;
+    unsigned long long key = 0;  // the sum modulo 2^64 of the partials
+    for (int i = 0, nb = et_fingerprint_blocks(p->nvox); i < nb; i++) key += p->fp_host[i];
+    return key;
 }
 
 
@@ -1344,6 +1321,7 @@ EtSweepArgs yl_sweep_args(const et_plan *p, const float *recs, int nv, int D, co
     a.D = Deff;
     a.zlen = zlen;
     a.att = const_cast<float *>(att);
+    a.part_V = nv;
     a.yl_nbuf = p->yl_nbuf;
     a.yl_tiles = p->yl_tiles;
     return a;
@@ -1533,36 +1511,78 @@ void yl_upload(DevBuf &buf, const YlTable &t, hipStream_t st)
 // projector, and the rotated-frame volumes go to the sweep kernels' pulls
 // (same u layout).
 
-// Content fingerprints of the map mu and (when given) the activity act, with
-// one stream synchronisation.  The single operations key their caches on
-// content whatever the plan's mu_check (which keys the OSEM caches): they may
-// see other maps between OSEM calls, and a map rewritten in place is caught.
-void content_keys(et_plan *p, const float *mu, const float *act, unsigned long long &kmu, unsigned long long &kact)
+// Sources of a single operation: the YF copies of act and mu (either may be
+// null) and, with a map, the factors of every view in view order
+// ([v][z'][x'][rows], null without a map).  The factors and the forward sums are
+// keyed on content, whatever the plan's mu_check (which keys the OSEM caches):
+// the operations may see other maps between OSEM calls, and a map rewritten in
+// place is caught.  The keys are formed where the volumes are packed and compared
+// on the device: the factor kernel of an unchanged map ends at once, a
+// projection that the forward sums make superfluous likewise (EtSweepArgs.skip),
+// and no call waits for the stream (32 x 24 x 32, 16 views: projection 33.6 ->
+// 19.4 us).  fwd: as EtKeys.
+const float *yl_sources(et_plan *p, const float *act, const float *mu, int fwd)
 {
-    kmu = kact = 0;
-    if (!mu && !act) return;
-    fp_launch(p, mu ? mu : act, mu ? act : nullptr);  // one launch for both
-    check_hip(hipStreamSynchronize(p->st), niftyrec_error_kernel);
-    if (mu) kmu = fp_key(p, 0);
-    if (act) kact = fp_key(p, mu ? 1 : 0);
+    EtPackArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.nx = p->nx;
+    a.ny = p->ny;
+    a.nz = p->nz;
+    a.yp = p->yp;
+    int n = 0;
+    if (mu) {
+        a.src[n] = mu;
+        a.guard[n] = p->gmu;
+        a.dst[n++] = p->mu_yf.ensure(p->yf_elems + ET_YF_SLACK, true, p->st);
+    }
+    if (act) {
+        a.src[n] = act;
+        a.guard[n] = p->gy;
+        a.dst[n++] = p->act_yf.ensure(p->yf_elems, true, p->st);
+    }
+    if (n == 0) return nullptr;
+    EtKeys k;
+    std::memset(&k, 0, sizeof(k));
+    if (mu) {
+        // (8-byte words: the state, which starts out unread, then the partial sums)
+        k.np = et_pack_keys_blocks(p->nx, p->ny, p->nz);
+        k.st = reinterpret_cast<unsigned long long *>(p->keys.ensure(2 * (ET_KEY_WORDS + 2 * (size_t)k.np), false));
+        a.parts = k.st + ET_KEY_WORDS;
+        k.mu = a.parts;
+        k.act = act ? a.parts + k.np : nullptr;
+        k.cur = (int)(p->key_gen & 1u);
+        k.fac_built = p->fac_built;
+        k.fwd = fwd;
+    }
+    {
+        ProfScope ps(p, ET_PROF_OTHER, n * 8.0 * p->nvox);
+        check_launch(et_launch_pack_keys(a, n, (et_stream_t)p->st));
+    }
+    if (!mu) return nullptr;
+    p->fac_built = false;  // until the launch is queued
+    p->fac.ensure(yl_att_elems(p, p->V), false);
+    EtSweepArgs f = yl_sweep_args(p, p->d_recs.p, p->V, 1, p->fac.p);
+    f.mu = p->mu_yf.p;
+    ProfScope ps(p, ET_PROF_OTHER, (double)p->V * 8.0 * p->nvox);
+    check_launch(et_launch_yl_factors(p->yl_rpl, f, k, (et_stream_t)p->st));
+    p->fac_built = true;
+    p->key_gen++;
+    return p->fac.p;
 }
 
-// Factors of every view in view order ([v][z'][x'][rows]) for the map mu (mu_yf
-// its YF copy; key its content key), rebuilt when the key changes.
-const float *yl_view_factors(et_plan *p, const float *mu_yf, unsigned long long key)
+// Rotated-frame volumes for up to `want` views in p->u (`per` volumes a view):
+// fewer views where the device has no room for them.
+int yl_u_views(et_plan *p, int want, int per)
 {
-    if (p->fac_valid && p->fac_key == key) return p->fac.p;
-    p->fac_valid = false;
-    p->fac.ensure(yl_att_elems(p, p->V), false);
-    EtSweepArgs a = yl_sweep_args(p, p->d_recs.p, p->V, 1, p->fac.p);
-    a.mu = mu_yf;
-    {
-        ProfScope ps(p, ET_PROF_OTHER, (double)p->V * 8.0 * p->nvox);
-        check_launch(et_launch_yl_factors(p->yl_rpl, a, (et_stream_t)p->st));
+    for (int nv = want;; nv = (nv + 1) / 2) {
+        try {
+            p->u.ensure((size_t)nv * per * p->ustride, true, p->st);
+            return nv;
+        } catch (const EtError &) {
+            if (nv <= 1) throw;
+            (void)hipGetLastError();
+        }
     }
-    p->fac_valid = true;
-    p->fac_key = key;
-    return p->fac.p;
 }
 
 // Depth chunks of a row-lane launch of `per_chunk` blocks per chunk: the fewest
@@ -1627,49 +1647,56 @@ void yl_pull_into(YlTable &t, et_plan *p, const float *recs, int nv, bool adjoin
                           });
 }
 
-bool yl_op_project(et_plan *p, const float *act, const float *act_yf, const float *mu, const float *mu_yf, float *sino,
-                   int truncate)
+// Adds to t the projection of every view into the forward sums p->fwd_part (D
+// chunks asked for), not done where *skip is set.
+float *yl_forward(YlTable &t, et_plan *p, const float *fac, int D, const int *skip)
 {
-    if (!p->yl_ops || !p->yl || !act_yf) return false;
-    // without attenuation there are no factors to cache and no gradient to
-    // keep the chunk sums for: no keys
-    unsigned long long kmu = 0, kact = 0;
-    if (mu) content_keys(p, mu, act, kmu, kact);
-    const float *fac = mu ? yl_view_factors(p, mu_yf, kmu) : nullptr;
-    const int D = !mu && p->tune_D > 0 ? p->tune_D : yl_op_chunks(p, (long)p->V * p->yl_tiles);
     int Deff, zlen;
     yl_chunks(p, D, Deff, zlen);
-    p->fwd_valid = false;
     float *part = p->fwd_part.ensure((size_t)Deff * p->V * yl_plane_elems(p), false);
-    YlTable t;
     t.grouped<EtSweepArgs>(YL_PROJECT, {p}, YlTable::project_key, [&](int, int &gx, int &gy, double &bytes) {
-        bytes += (double)p->V * ((mu ? 8.0 : 4.0) * p->nvox + 4.0 * p->P);
+        bytes += (double)p->V * ((fac ? 8.0 : 4.0) * p->nvox + 4.0 * p->P);
         EtSweepArgs a = yl_sweep_args(p, p->d_recs.p, p->V, D, fac);
-        a.act = const_cast<float *>(act_yf);
+        a.act = p->act_yf.p;
         a.part = part;
+        a.skip = skip;
         gx = a.D * p->yl_tiles;
         gy = p->V;
         return a;
     });
+    return part;
+}
+
+// Depth chunks of the projection of every view (the forward sums' chunking).
+int yl_forward_chunks(const et_plan *p, bool mu)
+{
+    return !mu && p->tune_D > 0 ? p->tune_D : yl_op_chunks(p, (long)p->V * p->yl_tiles);
+}
+
+bool yl_op_project(et_plan *p, const float *act, const float *mu, float *sino, int truncate)
+{
+    if (!p->yl_ops || !p->yl || !act) return false;
+    p->fwd_built = false;  // until the sums are queued
+    const float *fac = yl_sources(p, act, mu, 1);
+    const int D = yl_forward_chunks(p, mu != nullptr);
+    int Deff, zlen;
+    yl_chunks(p, D, Deff, zlen);
+    YlTable t;
+    const float *part = yl_forward(t, p, fac, D, nullptr);
     yl_run(p, t, YL_OP_PROJECT);
     ProfScope ps(p, ET_PROF_OTHER, (Deff + 1.0) * 4.0 * p->V * p->P);
     check_launch(
         et_launch_yl_parts_to_sino(part, Deff, p->V, p->nx, p->ny, p->yu, truncate, sino, (et_stream_t)p->st));
-    p->fwd_valid = mu != nullptr;
-    p->fwd_act = kact;
-    p->fwd_mu = kmu;
-    p->fwd_D = D;  // the chunking as requested: yl_chunks maps it to the same chunks again
+    p->fwd_built = mu != nullptr;  // (without a map there is no gradient to seed, and no key)
+    p->fwd_D = D;
     p->fwd_tiles = p->yl_tiles;
     return true;
 }
 
-bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, const float *mu_yf, float *out, bool adjoint,
-                       int truncate)
+bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate)
 {
     if (!p->yl_ops || !p->yl) return false;
-    unsigned long long kmu = 0, kact;
-    if (mu) content_keys(p, mu, nullptr, kmu, kact);
-    const float *fac = mu ? yl_view_factors(p, mu_yf, kmu) : nullptr;
+    const float *fac = yl_sources(p, nullptr, mu, 0);
     const size_t pe = yl_plane_elems(p);
     const float *st = yl_sino_t(p, sino);
     const int vb = view_batch(p);
@@ -1699,96 +1726,97 @@ bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, const flo
     return true;
 }
 
-// Exact attenuation gradient: per view batch, the projection's partial sums
-// (the plan's projector kind, the gradient sweep's chunking), the gradient
-// sweep of the same kind (tiled or full width) and the exact adjoint pull.
-bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float *act_yf, const float *mu,
-                    const float *mu_yf, float *out, int truncate)
+// Adds to t the forward sums that the gradient sweeps of this activity and map
+// start from: the last projection's, or formed here (the device decides by the
+// keys of yl_sources with fwd = 2).
+float *yl_gradient_forward(YlTable &t, et_plan *p, const float *fac, int D)
 {
-    if (!p->yl_ops || !p->yl) return false;
-    unsigned long long kmu, kact;
-    content_keys(p, mu, act, kmu, kact);
-    const float *fac = yl_view_factors(p, mu_yf, kmu);
-    const size_t pe = yl_plane_elems(p);
+    const bool same = p->fwd_built && p->fwd_D == D && p->fwd_tiles == p->yl_tiles;
+    p->fwd_built = false;  // until the sums are queued
+    return yl_forward(t, p, fac, D,
+                      same ? reinterpret_cast<const int *>(
+                                 reinterpret_cast<const unsigned long long *>(p->keys.p) + ET_KEY_SKIP_FWD)
+                           : nullptr);
+}
+
+void yl_forward_kept(et_plan *p, int D)
+{
+    p->fwd_built = true;
+    p->fwd_D = D;
+    p->fwd_tiles = p->yl_tiles;
+}
+
+// Gradient sweep of nv views from view v0 on (their forward sums in `part`) into
+// u, with the plan's projector kind and the forward sums' chunking.
+void yl_gradient_sweep(YlTable &t, et_plan *p, int v0, int nv, const float *fac, const float *st, float *part, int D,
+                       float *u)
+{
+    t.grouped<EtSweepArgs>(YL_GRAD, {p}, YlTable::project_key, [&](int, int &gx, int &gy, double &bytes) {
+        bytes += (double)nv * (8.0 * p->nvox + 4.0 * p->P);
+        EtSweepArgs a = yl_sweep_args(p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, D, yl_att_at(p, fac, v0));
+        a.act = p->act_yf.p;
+        a.part = part + (size_t)v0 * yl_plane_elems(p);
+        a.part_V = p->V;
+        a.sino = st + (size_t)v0 * yl_plane_elems(p);
+        a.u = u;
+        gx = a.D * p->yl_tiles;
+        gy = nv;
+        return a;
+    });
+}
+
+// Largest rotated-frame buffer of the gradient and the joint backward: 4 GiB
+// (128^3 x 120 views hold 1.0 GiB each).
+constexpr size_t ET_YL_U_BYTES = 4ull << 30;
+
+// Exact attenuation gradient: the forward sums of every view (kept from the last
+// projection or formed here), then per view batch the gradient sweep and the
+// exact adjoint pull.
+bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate)
+{
+    if (!p->yl_ops || !p->yl || !act || !mu) return false;
+    const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
-    const int tiles = p->yl_tiles;
-    // the last projection's partial sums, when it projected this activity
-    // through this map with this projector: all views in one batch at its
-    // chunking, no projection pass
-    const bool reuse = p->fwd_valid && p->fwd_act == kact && p->fwd_mu == kmu && p->fwd_tiles == tiles;
-    const int vb = reuse ? p->V : view_batch(p);
-    p->u.ensure((size_t)vb * p->ustride, true, p->st);
+    const int D = yl_forward_chunks(p, true);
+    const long fit = (long)std::max<size_t>(1, ET_YL_U_BYTES / (p->ustride * sizeof(float)));
+    const int vb = yl_u_views(p, p->tune_vb > 0 ? std::min(p->tune_vb, p->V) : (int)std::min<long>(fit, p->V), 1);
     float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
-    // every batch in one table (the batches reuse part and u in stream order);
-    // the partial sums take the most chunks any batch uses
-    float *part = nullptr;
-    if (reuse) {
-        part = p->fwd_part.p;
-    } else {
-        int Dmax = 1;
-        for (int v0 = 0; v0 < p->V; v0 += vb) {
-            int Deff, zlen;
-            yl_chunks(p, yl_op_chunks(p, (long)std::min(vb, p->V - v0) * tiles), Deff, zlen);
-            Dmax = std::max(Dmax, Deff);
-        }
-        part = p->part.ensure((size_t)Dmax * vb * pe, false);
-    }
-    YlTable t;
+    YlTable t;  // every batch in one table: the batches reuse u in stream order
+    float *part = yl_gradient_forward(t, p, fac, D);
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
-        const int D = reuse ? p->fwd_D : yl_op_chunks(p, (long)nv * tiles);
-        const float *recs = p->d_recs.p + (size_t)v0 * ET_VIEW_REC;
-        auto args = [&](int &gx, int &gy, double &bytes) {
-            bytes += (double)nv * (8.0 * p->nvox + 4.0 * p->P);
-            EtSweepArgs a = yl_sweep_args(p, recs, nv, D, yl_att_at(p, fac, v0));
-            a.act = const_cast<float *>(act_yf);
-            a.part = part;
-            a.sino = st + (size_t)v0 * pe;
-            a.u = p->u.p;
-            gx = a.D * tiles;
-            gy = nv;
-            return a;
-        };
-        // the tiled kernels where the plan projects with them (key NR 0)
-        if (!reuse)
-            t.grouped<EtSweepArgs>(YL_PROJECT, {p}, YlTable::project_key,
-                                   [&](int, int &gx, int &gy, double &bytes) { return args(gx, gy, bytes); });
-        t.grouped<EtSweepArgs>(YL_GRAD, {p}, YlTable::project_key,
-                               [&](int, int &gx, int &gy, double &bytes) { return args(gx, gy, bytes); });
-        yl_pull_into(t, p, recs, nv, true, v0 > 0, v0 + nv >= p->V && truncate, acc);
+        yl_gradient_sweep(t, p, v0, nv, fac, st, part, D, p->u.p);
+        yl_pull_into(t, p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, true, v0 > 0, v0 + nv >= p->V && truncate, acc);
     }
     yl_run(p, t, YL_OP_GRADIENT);
+    yl_forward_kept(p, D);
     ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc, out, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
     return true;
 }
 
-// Both gradients in one pass over the views, after a projection of the same
-// activity through the same map (the forward partial sums are reused, as
-// yl_op_gradient does): the adjoint backprojection sweep writes its rotated-frame
-// volumes into the first half of u, the gradient sweep into the second, and one
-// exact adjoint pull (YL_PULL_ADJ2), whose candidate weights serve both, adds
-// them up.  Each output equals its operation's on its own with all views in one
-// batch (the view batch set to the view count).  False (nothing issued) without
-// the forward sums or when the two volumes of every view would exceed 4 GiB.
-bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float *act_yf, const float *mu,
-                    const float *mu_yf, float *out_act, float *out_mu, int truncate)
+// Both gradients in one pass over the views: the forward sums as for the
+// gradient, the adjoint backprojection sweep's rotated-frame volumes into the
+// first half of u, the gradient sweep's into the second, and one exact adjoint
+// pull (YL_PULL_ADJ2), whose candidate weights serve both, adds them up.  Each
+// output equals its operation's on its own with all views in one batch (the
+// view batch set to the view count).  False (nothing issued) when the two
+// volumes of every view would exceed 4 GiB or the device's memory.
+bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float *mu, float *out_act, float *out_mu,
+                    int truncate)
 {
     if (!p->yl_ops || !p->yl || !act || !mu) return false;
     const int V = p->V;
-    if (2.0 * V * p->ustride * sizeof(float) > 4.0 * (1ull << 30)) return false;
-    unsigned long long kmu, kact;
-    content_keys(p, mu, act, kmu, kact);
-    const int tiles = p->yl_tiles;
-    if (!(p->fwd_valid && p->fwd_act == kact && p->fwd_mu == kmu && p->fwd_tiles == tiles)) return false;
-    const float *fac = yl_view_factors(p, mu_yf, kmu);
+    if (2 * (size_t)V * p->ustride * sizeof(float) > ET_YL_U_BYTES || yl_u_views(p, V, 2) < V) return false;
+    const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
-    p->u.ensure((size_t)2 * V * p->ustride, true, p->st);
     float *ub = p->u.p, *ug = p->u.p + (size_t)V * p->ustride;
     float *acc_a = p->op_acc.ensure(p->yf_elems, true, p->st);
     float *acc_m = p->op_acc2.ensure(p->yf_elems, true, p->st);
     const float *recs = p->d_recs.p;
+    const int D = yl_forward_chunks(p, true);
     YlTable t;
+    float *part = yl_gradient_forward(t, p, fac, D);
     const int Db = yl_op_chunks(p, V);
     t.grouped<EtSweepArgs>(YL_BPU, {p}, YlTable::sweep_key, [&](int, int &gx, int &gy, double &bytes) {
         bytes += (double)V * (8.0 * p->nvox + 4.0 * p->P);
@@ -1801,17 +1829,7 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
         gy = V;
         return a;
     });
-    t.grouped<EtSweepArgs>(YL_GRAD, {p}, YlTable::project_key, [&](int, int &gx, int &gy, double &bytes) {
-        bytes += (double)V * (8.0 * p->nvox + 4.0 * p->P);
-        EtSweepArgs a = yl_sweep_args(p, recs, V, p->fwd_D, fac);
-        a.act = const_cast<float *>(act_yf);
-        a.part = p->fwd_part.p;
-        a.sino = st;
-        a.u = ug;
-        gx = a.D * tiles;
-        gy = V;
-        return a;
-    });
+    yl_gradient_sweep(t, p, 0, V, fac, st, part, D, ug);
     t.grouped<EtPullArgs>(YL_PULL_ADJ2, {p}, YlTable::pull_key, [&](int, int &gx, int &gy, double &bytes) {
         bytes += (double)V * 8.0 * p->nvox + 8.0 * p->nvox;
         gx = yl_pull_tiles(p);
@@ -1822,6 +1840,7 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
         return a;
     });
     yl_run(p, t, YL_OP_BACKWARD);
+    yl_forward_kept(p, D);
     ProfScope ps(p, ET_PROF_OTHER, 16.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc_a, out_act, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
     check_launch(et_launch_unpack_yf(acc_m, out_mu, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
@@ -1943,7 +1962,7 @@ void yl_osem_build(et_plan *p, const float *mu_yf, int S, float eps, const std::
         EtSweepArgs a = yl_sweep_args(p, p->osem_recs.p, p->V, 1, p->osem_E.p);
         a.mu = mu_yf;
         ProfScope ps(p, ET_PROF_OTHER, (double)p->V * 8.0 * p->nvox);
-        check_launch(et_launch_yl_factors(p->yl_rpl, a, (et_stream_t)p->st));
+        check_launch(et_launch_yl_factors(p->yl_rpl, a, EtKeys{}, (et_stream_t)p->st));
     }
     p->u.ensure((size_t)maxsub * p->ustride, true, p->st);
     p->ratio.ensure((size_t)maxsub * yl_plane_elems(p), true, p->st);
@@ -3596,8 +3615,8 @@ int et_plan_invalidate(et_plan *plan)
 {
     if (!plan) return niftyrec_error_parameters;
     plan->osem_valid = false;
-    plan->fac_valid = false;
-    plan->fwd_valid = false;
+    plan->fac_built = false;
+    plan->fwd_built = false;
     return niftyrec_success;
 }
 

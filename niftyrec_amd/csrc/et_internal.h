@@ -78,6 +78,8 @@ struct EtSweepArgs {
     float *att;              // attenuation factors e^{-A(x',y,z')} of the views, [V][nz][yu][nthr] with
                              // nthr = roundup(nx, 64) (the block width); see et_launch_sweep's has_mu
                              // (row-lane kernels: [V][nz][nx][yu])
+    int part_V;              // row-lane sweeps: views per depth chunk of `part` (V, or more in a view batch)
+    const int *skip;         // row-lane projector: nothing to do when *skip is set (null: never)
     int yl_nbuf;             // row-lane sweeps: LDS planes (2: alternate, one barrier per plane; 1: two)
     int yl_tiles;            // row-lane projector: column tiles per plane (1: the whole width per block)
 };
@@ -191,15 +193,44 @@ int et_launch_ratio_group(const EtRatioArgs *args, const void *tab, int n, int b
 // what lies beyond plane z, sino = the whole ray; act or mu may be null.
 int et_launch_partial_line(const float *act, const float *mu, const float *bgimg, float bg, int nx, int ny, int nz,
                            float *sino, float *part, et_stream_t stream);
-// Content fingerprints of p0 and (when not null) p1, n floats each: the keys
-// under which the caches remember the attenuation map and the activity.  The
-// launch stores et_fingerprint_blocks(n) partial sums per array in parts (p0's,
-// then p1's; at most 2 * ET_FP_BLOCKS); a key is the sum modulo 2^64 of its
-// array's partials.
+// Content fingerprint of n floats: the key under which the OSEM caches remember
+// the attenuation map.  The launch stores et_fingerprint_blocks(n) (at most
+// ET_FP_BLOCKS) partial sums in parts; the key is their sum modulo 2^64.
 #define ET_FP_BLOCKS 1024
 int et_fingerprint_blocks(size_t n);
-int et_launch_fingerprints(const float *p0, const float *p1, size_t n, unsigned long long *parts,
-                           et_stream_t stream);
+int et_launch_fingerprint(const float *p, size_t n, unsigned long long *parts, et_stream_t stream);
+// Caller volumes (ABI layout) into YF copies and the fingerprints of what was
+// read, in one pass: src[k] into dst[k] (guard[k] guard rows), k < n (1 or 2);
+// volume k's partial sums in parts[k * np .. (k + 1) * np), np =
+// et_pack_keys_blocks(nx, ny, nz); parts null: no fingerprints.  The keys are
+// et_launch_fingerprint's.
+struct EtPackArgs {
+    const float *src[2];
+    float *dst[2];
+    int guard[2];
+    unsigned long long *parts;
+    int nx, ny, nz, yp;
+};
+int et_pack_keys_blocks(int nx, int ny, int nz);
+int et_launch_pack_keys(const EtPackArgs &a, int n, et_stream_t stream);
+
+// Content keys of a plan's single operations, kept and compared on the device
+// (no host synchronisation).  mu, act: the operation's partial sums (np each;
+// act null when the operation reads none).  st: ET_KEY_WORDS words, two slots
+// per key; the operation reads slot cur ^ 1, which the one before it wrote, and
+// writes slot cur, so that no block of the launch reads a word that another
+// block of it writes.
+enum { ET_KEY_MU = 0, ET_KEY_FWD_MU = 2, ET_KEY_FWD_ACT = 4, ET_KEY_SKIP_FWD = 6, ET_KEY_WORDS = 8 };
+struct EtKeys {
+    const unsigned long long *mu, *act;
+    int np;
+    unsigned long long *st;
+    int cur;
+    int fac_built;  // the factor buffer holds the factors of slot cur ^ 1's map
+    int fwd;        // 0: the forward sums stay as they are; 1: this operation forms them;
+                    // 2: formed again unless those of slot cur ^ 1 are this pair's (st[ET_KEY_SKIP_FWD])
+};
+
 // Row-lane kernels of the OSEM subset loop (et_yl.h).  Grouped launches only
 // (tab as et_launch_sweep_group): sweeps kind 0 projection, 1 rotated-frame
 // backprojection, 3 exact attenuation gradient (reads the projection's partial
@@ -228,8 +259,9 @@ int et_launch_att_factors(const EtSweepArgs &a, et_stream_t stream);
 // a.u into a.out and a.u2 into a.out2 with one set of candidate weights.
 int et_launch_yl_pull_adj(int RPL, int nsrc, const EtPullArgs *args, const void *tab, int n, int blocks,
                           et_stream_t stream);
-// Attenuation factors of a.V views into a.att (row-lane layout) from a.mu (YF).
-int et_launch_yl_factors(int RPL, const EtSweepArgs &a, et_stream_t stream);
+// Attenuation factors of a.V views into a.att (row-lane layout) from a.mu (YF);
+// with keys (st not null): only if the map is another one than the factors' own.
+int et_launch_yl_factors(int RPL, const EtSweepArgs &a, const EtKeys &k, et_stream_t stream);
 // sino[v][y][x] = sum over d < D of part[d][v][x][y] (compensated), truncated
 // at 0 if asked: row-lane partial sums (V views, rows per column) in the ABI layout.
 int et_launch_yl_parts_to_sino(const float *part, int D, int V, int nx, int ny, int rows, int truncate, float *sino,

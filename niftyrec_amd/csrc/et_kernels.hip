@@ -494,6 +494,47 @@ __global__ void __launch_bounds__(256) k_pack_yf(const float *__restrict__ abi, 
     }
 }
 
+// k_pack_yf for up to two volumes with the fingerprints of what it reads
+// (EtPackArgs): a single operation's sources and their content keys in one
+// launch (at 32 x 24 x 32 three launches, a copy and a stream synchronisation
+// before).  grid (ceil(nx/32), ceil(ny/32), volumes x zb), each block every
+// zb-th plane of its volume.
+__global__ void __launch_bounds__(256) k_pack_keys(EtPackArgs a, int zb)
+{
+    __shared__ float tile[32][33];
+    __shared__ unsigned long long part[4];
+    const int vol = (int)blockIdx.z / zb, z0 = (int)blockIdx.z - vol * zb;
+    const float *__restrict__ src = a.src[vol];
+    float *__restrict__ dst = a.dst[vol];
+    const int xb = blockIdx.x * 32, yb = blockIdx.y * 32, guard = a.guard[vol];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    unsigned long long h = 0;
+    for (int z = z0; z < a.nz; z += zb) {
+        for (int k = ty; k < 32; k += 8) {
+            const int x = xb + tx, y = yb + k;
+            float v = 0.f;
+            if (x < a.nx && y < a.ny) {
+                const size_t i = x + (size_t)a.nx * (y + (size_t)a.ny * z);
+                v = src[i];
+                if (a.parts) h += fp_element(__float_as_uint(v), i);
+            }
+            tile[k][tx] = v;
+        }
+        __syncthreads();
+        for (int k = ty; k < 32; k += 8) {
+            const int y = yb + tx, x = xb + k;
+            if (x < a.nx && y < a.ny)
+                dst[(guard + y) + (size_t)a.yp * ((x + 1) + (size_t)(a.nx + 2) * (z + 1))] = tile[tx][k];
+        }
+        __syncthreads();
+    }
+    if (a.parts) {
+        h = block_sum_256(h, part);
+        if (threadIdx.x == 0)
+            a.parts[blockIdx.x + (size_t)gridDim.x * (blockIdx.y + (size_t)gridDim.y * blockIdx.z)] = h;
+    }
+}
+
 __global__ void __launch_bounds__(256) k_unpack_yf(const float *__restrict__ yf, float *__restrict__ abi,
                                                    int nx, int ny, int nz, int yp, int gy)
 {
@@ -672,32 +713,15 @@ __global__ void __launch_bounds__(256) k_ratio_parts(const float *__restrict__ m
     out[i] = (p < eps) ? meas[i] / eps : meas[i] / p;
 }
 
-// Content fingerprint of n floats: the sum modulo 2^64 of a 64-bit mix of
-// (bits, index) per element (order-independent: any partition into blocks
-// gives the same sum).  Any change of one element changes the sum.
-__device__ __forceinline__ unsigned long long fp_mix(unsigned long long h)
-{
-    h ^= h >> 33;
-    h *= 0xff51afd7ed558ccdull;
-    h ^= h >> 33;
-    h *= 0xc4ceb9fe1a85ec53ull;
-    h ^= h >> 33;
-    return h;
-}
-
-// Fingerprints of one or two arrays of n floats (p0, p1): blocks [0, nb) hash
-// p0, blocks [nb, 2 nb) p1, and block b stores its partial sum in parts[b] (no
-// atomics, nothing to clear first); an array's key is the sum modulo 2^64 of
-// its nb partials.  16-byte loads where both arrays are 16-byte aligned (VEC4).
+// Fingerprint of n floats: block b stores its partial sum in parts[b] (no
+// atomics, nothing to clear first).  16-byte loads where the array is 16-byte
+// aligned (VEC4).
 template <bool VEC4>
-__global__ void __launch_bounds__(256) k_fingerprint(const unsigned *__restrict__ p0, const unsigned *__restrict__ p1,
-                                                     size_t n, int nb, unsigned long long *__restrict__ parts)
+__global__ void __launch_bounds__(256) k_fingerprint(const unsigned *__restrict__ p, size_t n,
+                                                     unsigned long long *__restrict__ parts)
 {
-    constexpr unsigned long long G = 0x9e3779b97f4a7c15ull;
-    const int arr = (int)blockIdx.x / nb, lb = (int)blockIdx.x - arr * nb;
-    const unsigned *__restrict__ p = arr ? p1 : p0;
     unsigned long long h = 0;
-    const size_t t0 = (size_t)lb * blockDim.x + threadIdx.x, stride = (size_t)nb * blockDim.x;
+    const size_t t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
     size_t done = 0;
     if constexpr (VEC4) {
         const size_t n4 = n / 4;
@@ -705,19 +729,14 @@ __global__ void __launch_bounds__(256) k_fingerprint(const unsigned *__restrict_
         for (size_t j = t0; j < n4; j += stride) {
             const uint4 v = p4[j];
             const size_t i = 4 * j;
-            h += fp_mix(((unsigned long long)v.x << 32) ^ (i * G)) +
-                 fp_mix(((unsigned long long)v.y << 32) ^ ((i + 1) * G)) +
-                 fp_mix(((unsigned long long)v.z << 32) ^ ((i + 2) * G)) +
-                 fp_mix(((unsigned long long)v.w << 32) ^ ((i + 3) * G));
+            h += fp_element(v.x, i) + fp_element(v.y, i + 1) + fp_element(v.z, i + 2) + fp_element(v.w, i + 3);
         }
         done = 4 * n4;
     }
-    for (size_t i = done + t0; i < n; i += stride) h += fp_mix(((unsigned long long)p[i] << 32) ^ (i * G));
-    for (int o = 32; o >= 1; o >>= 1) h += __shfl_xor(h, o, 64);
+    for (size_t i = done + t0; i < n; i += stride) h += fp_element(p[i], i);
     __shared__ unsigned long long part[4];
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = h;
-    __syncthreads();
-    if (threadIdx.x == 0) parts[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+    h = block_sum_256(h, part);
+    if (threadIdx.x == 0) parts[blockIdx.x] = h;
 }
 
 // dst[v][x][y] = src[order[v]][y][x] for y < ny, 0 for ny <= y < rows: the
@@ -886,6 +905,28 @@ int et_launch_pack_yf(const float *abi, float *yf, int nx, int ny, int nz, int y
 {
     dim3 g((nx + 31) / 32, (ny + 31) / 32, nz);
     hipLaunchKernelGGL(k_pack_yf, g, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), abi, yf, nx, ny, nz, yp, gy);
+    return (int)hipGetLastError();
+}
+
+// Planes of a volume per pack launch: at most about 2,048 blocks per volume, so
+// that the partial sums, which every block of the factor kernel adds up, stay few.
+static int pack_keys_zb(int nx, int ny, int nz)
+{
+    const int per = (int)(nblk(nx, 32) * nblk(ny, 32));
+    return std::max(1, std::min(nz, 2048 / std::max(per, 1)));
+}
+
+int et_pack_keys_blocks(int nx, int ny, int nz)
+{
+    return (int)(nblk(nx, 32) * nblk(ny, 32)) * pack_keys_zb(nx, ny, nz);
+}
+
+int et_launch_pack_keys(const EtPackArgs &a, int n, et_stream_t stream)
+{
+    if (n < 1 || n > 2 || !a.src[0] || (n > 1 && !a.src[1])) return (int)hipErrorInvalidValue;
+    const int zb = pack_keys_zb(a.nx, a.ny, a.nz);
+    const dim3 g(nblk(a.nx, 32), nblk(a.ny, 32), n * zb);
+    hipLaunchKernelGGL(k_pack_keys, g, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a, zb);
     return (int)hipGetLastError();
 }
 
@@ -1091,18 +1132,16 @@ bool et_withdraw_launch_events()
 
 int et_fingerprint_blocks(size_t n) { return (int)std::max<size_t>(1, std::min<size_t>(nblk(n, 1024), ET_FP_BLOCKS)); }
 
-int et_launch_fingerprints(const float *p0, const float *p1, size_t n, unsigned long long *parts, et_stream_t stream)
+int et_launch_fingerprint(const float *p, size_t n, unsigned long long *parts, et_stream_t stream)
 {
-    if (!p0) return (int)hipErrorInvalidValue;
+    if (!p) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const int nb = et_fingerprint_blocks(n);
-    const unsigned *q0 = reinterpret_cast<const unsigned *>(p0), *q1 = reinterpret_cast<const unsigned *>(p1);
-    const bool vec4 = (reinterpret_cast<uintptr_t>(p0) & 15) == 0 && (reinterpret_cast<uintptr_t>(p1) & 15) == 0;
-    const dim3 grid(p1 ? 2 * nb : nb);
-    if (vec4)
-        hipLaunchKernelGGL(k_fingerprint<true>, grid, dim3(256), 0, st, q0, q1, n, nb, parts);
+    const dim3 grid(et_fingerprint_blocks(n));
+    const unsigned *q = reinterpret_cast<const unsigned *>(p);
+    if ((reinterpret_cast<uintptr_t>(p) & 15) == 0)
+        hipLaunchKernelGGL(k_fingerprint<true>, grid, dim3(256), 0, st, q, n, parts);
     else
-        hipLaunchKernelGGL(k_fingerprint<false>, grid, dim3(256), 0, st, q0, q1, n, nb, parts);
+        hipLaunchKernelGGL(k_fingerprint<false>, grid, dim3(256), 0, st, q, n, parts);
     return (int)hipGetLastError();
 }
 
@@ -1171,13 +1210,13 @@ int et_launch_yl_pull_adj(int RPL, int nsrc, const EtPullArgs *args, const void 
     return (int)hipErrorInvalidValue;
 }
 
-int et_launch_yl_factors(int RPL, const EtSweepArgs &a, et_stream_t stream)
+int et_launch_yl_factors(int RPL, const EtSweepArgs &a, const EtKeys &k, et_stream_t stream)
 {
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const dim3 g((a.nx + 15) / 16, a.V);
 #define ET_YLF(rpl)                                                                   \
     if (RPL == rpl) {                                                                 \
-        hipLaunchKernelGGL((k_yl_factors<rpl>), g, dim3(256), 0, st, a);              \
+        hipLaunchKernelGGL((k_yl_factors<rpl>), g, dim3(256), 0, st, a, k);            \
         return (int)hipGetLastError();                                                \
     }
     ET_YLF(2) ET_YLF(4) ET_YLF(6) ET_YLF(8)

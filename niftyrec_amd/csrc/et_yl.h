@@ -401,7 +401,7 @@ __device__ __forceinline__ void yl_project_body(const EtSweepArgs &a, const Blk 
         float out[RPL];
 #pragma unroll
         for (int i = 0; i < RPL; i++) out[i] = acc[r][i] - cmp[r][i];
-        yl_store<RPL>(a.part + (((size_t)d * a.V + v) * a.nx + xc) * rows + row0, out);
+        yl_store<RPL>(a.part + (((size_t)d * a.part_V + v) * a.nx + xc) * rows + row0, out);
     }
 }
 
@@ -452,7 +452,7 @@ __device__ __forceinline__ void yl_grad_body(const EtSweepArgs &a, const Blk &b)
         }
         for (int d2 = d + 1; d2 < a.D; d2++) {
             float t[RPL];
-            yl_load<RPL>(a.part + (((size_t)d2 * a.V + v) * a.nx + xc) * rows + row0, t);
+            yl_load<RPL>(a.part + (((size_t)d2 * a.part_V + v) * a.nx + xc) * rows + row0, t);
 #pragma unroll
             for (int i = 0; i < RPL; i++) comp_add(hi[i], lo[i], t[i]);
         }
@@ -646,7 +646,7 @@ __device__ __forceinline__ void yl_project_tile_body(const EtSweepArgs &a, const
         float out[RPL];
 #pragma unroll
         for (int i = 0; i < RPL; i++) out[i] = acc[r][i] - cmp[r][i];
-        yl_store<RPL>(a.part + (((size_t)d * a.V + v) * a.nx + xc) * rows + row0, out);
+        yl_store<RPL>(a.part + (((size_t)d * a.part_V + v) * a.nx + xc) * rows + row0, out);
     }
 }
 
@@ -702,7 +702,7 @@ __device__ __forceinline__ void yl_grad_tile_body(const EtSweepArgs &a, const Bl
         }
         for (int d2 = d + 1; d2 < a.D; d2++) {
             float t[RPL];
-            yl_load<RPL>(a.part + (((size_t)d2 * a.V + v) * a.nx + xc) * rows + row0, t);
+            yl_load<RPL>(a.part + (((size_t)d2 * a.part_V + v) * a.nx + xc) * rows + row0, t);
 #pragma unroll
             for (int i = 0; i < RPL; i++) comp_add(hi[i], lo[i], t[i]);
         }
@@ -851,6 +851,7 @@ __global__ void __launch_bounds__(1024) k_yl_project(const EtSweepArgs *__restri
     int j;
     if (!group_block(tab, n, b, j)) return;
     const EtSweepArgs a = ((ET_CONST_AS const EtSweepArgs *)args)[j];
+    if (a.skip && *a.skip) return;
     yl_project_body<R, RPL, NR>(a, b);
 }
 
@@ -875,6 +876,7 @@ __global__ void __launch_bounds__(512, 4) k_yl_project_tile(const EtSweepArgs *_
     int j;
     if (!group_block(tab, n, b, j)) return;
     const EtSweepArgs a = ((ET_CONST_AS const EtSweepArgs *)args)[j];
+    if (a.skip && *a.skip) return;
     yl_project_tile_body<R, RPL>(a, b);
 }
 
@@ -941,9 +943,35 @@ __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
     }
 }
 
+// Keys of a single operation (EtKeys; the OSEM caches pass none): every block
+// adds up the map's partial fingerprints and stops if its key is the one the
+// factors were formed from; block (0, 0) writes the keys of this operation and
+// whether its forward sums are there already.  At 128^3 the launch takes about
+// 8 us where the factors stay; a host that read the keys waited for the stream.
 template <int RPL>
-__global__ void __launch_bounds__(256) k_yl_factors(EtSweepArgs a)
+__global__ void __launch_bounds__(256) k_yl_factors(EtSweepArgs a, EtKeys k)
 {
+    if (k.st) {
+        __shared__ unsigned long long part[4];
+        unsigned long long h = 0;
+        for (int i = threadIdx.x; i < k.np; i += 256) h += k.mu[i];
+        const unsigned long long km = block_sum_256(h, part);
+        const int prev = k.cur ^ 1;
+        if (blockIdx.x == 0 && blockIdx.y == 0) {
+            h = 0;
+            if (k.act)
+                for (int i = threadIdx.x; i < k.np; i += 256) h += k.act[i];
+            const unsigned long long ka = block_sum_256(h, part);
+            if (threadIdx.x == 0) {
+                const unsigned long long fm = k.st[ET_KEY_FWD_MU + prev], fa = k.st[ET_KEY_FWD_ACT + prev];
+                k.st[ET_KEY_MU + k.cur] = km;
+                k.st[ET_KEY_FWD_MU + k.cur] = k.fwd ? km : fm;
+                k.st[ET_KEY_FWD_ACT + k.cur] = k.fwd ? ka : fa;
+                *reinterpret_cast<int *>(k.st + ET_KEY_SKIP_FWD) = k.fwd == 2 && fm == km && fa == ka;
+            }
+        }
+        if (k.fac_built && k.st[ET_KEY_MU + prev] == km) return;
+    }
     yl_factor_body<RPL>(a);
 }
 
