@@ -233,10 +233,13 @@ struct YlLaunch {
 };
 enum {
     YL_PROJECT = 0, YL_RATIO = 1, YL_BPU = 2, YL_PULL_OSEM = 3, YL_PULL_STORE = 4, YL_GRAD = 5, YL_PULL_ADJ = 6,
-    YL_PULL_ADJ2 = 7  // exact adjoint pull of two volumes (u, u2) into two outputs
+    YL_PULL_ADJ2 = 7,  // exact adjoint pull of two volumes (u, u2) into two outputs
+    YL_GREF = 8,       // reference attenuation gradient
 };
 // Table slots of the single operations (each keeps its last upload).
-enum { YL_OP_PROJECT = 0, YL_OP_BACKPROJECT = 1, YL_OP_GRADIENT = 2, YL_OP_BACKWARD = 3, YL_OP_SLOTS = 4 };
+enum {
+    YL_OP_PROJECT = 0, YL_OP_BACKPROJECT = 1, YL_OP_GRADIENT = 2, YL_OP_BACKWARD = 3, YL_OP_GREF = 4, YL_OP_SLOTS = 5
+};
 
 struct et_plan {
     int device = 0;
@@ -909,6 +912,7 @@ void pull_general(et_plan *p, int v0, int nv, const float *u, bool adjoint, bool
 bool yl_op_project(et_plan *p, const float *act, const float *mu, float *sino, int truncate);
 bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate);
 bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate);
+bool yl_op_gradient_ref(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate);
 bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float *mu, float *out_act, float *out_mu,
                     int truncate);
 
@@ -1026,7 +1030,9 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
 {
     const int mode = exact ? ET_MODE_GRAD_MU : ET_MODE_GRAD_REF;
     if (p->fast) {
-        if (exact && yl_op_gradient(p, sino, act, mu, out, truncate)) return;
+        if (exact ? yl_op_gradient(p, sino, act, mu, out, truncate)
+                  : yl_op_gradient_ref(p, sino, act, mu, out, truncate))
+            return;
         pack(p, act, p->act_yf);
         pack(p, mu, p->mu_yf);
         const int vb = grad_view_batch(p);
@@ -1355,7 +1361,9 @@ struct YlTable {
                 const et_plan *q = plans[i];
                 // tiled projector (key NR 0, R > 0), full-width sweeps, backprojection
                 const bool tiled = (kind == YL_PROJECT || kind == YL_GRAD) && std::get<2>(g.first) == 0 && q->R > 0;
-                lds = std::max(lds, kind == YL_BPU ? q->yl_lds_bpu : (tiled ? q->yl_lds_tile : q->yl_lds_full));
+                if (std::get<0>(g.first) > 0)  // (no PSF: no LDS plane)
+                    lds = std::max(lds, kind == YL_BPU || kind == YL_GREF ? q->yl_lds_bpu
+                                                                          : (tiled ? q->yl_lds_tile : q->yl_lds_full));
             }
             const auto &k = g.first;
             L.push_back({kind, std::get<0>(k), std::get<1>(k), std::get<2>(k), std::get<3>(k), lds, tb.put(args),
@@ -1462,10 +1470,11 @@ void yl_issue(const float *dev, const std::vector<YlLaunch> &L, size_t from, siz
         switch (l.kind) {
         case YL_PROJECT:
         case YL_BPU:
-        case YL_GRAD: {
+        case YL_GRAD:
+        case YL_GREF: {
             ProfScope ps(prof, l.kind == YL_PROJECT ? ET_PROF_PROJECT : (l.kind == YL_BPU ? ET_PROF_BPU : ET_PROF_GRAD),
                          l.bytes);
-            const int k = l.kind == YL_BPU ? 1 : (l.kind == YL_GRAD ? (l.NR == 0 ? 4 : 3) : (l.NR == 0 ? 2 : 0));
+            const int k = l.kind == YL_BPU ? 1 : l.kind == YL_GREF ? 5 : (l.kind == YL_GRAD ? (l.NR == 0 ? 4 : 3) : (l.NR == 0 ? 2 : 0));
             check_launch(et_launch_yl_sweep(k, l.R, l.RPL, l.NR, l.nthr, l.lds, static_cast<const EtSweepArgs *>(args),
                                             tab, l.n, l.blocks, s));
             break;
@@ -1790,6 +1799,50 @@ bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float
     }
     yl_run(p, t, YL_OP_GRADIENT);
     yl_forward_kept(p, D);
+    ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
+    check_launch(et_launch_unpack_yf(acc, out, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
+    return true;
+}
+
+// Reference attenuation gradient: the chunk sums of act' e^{-A} (a projection
+// without PSF) of every view, then per view batch the reverse sweep and the
+// reference pull.
+bool yl_op_gradient_ref(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate)
+{
+    if (!p->yl_ops || !p->yl || !act || !mu) return false;
+    const float *fac = yl_sources(p, act, mu, 0);
+    const size_t pe = yl_plane_elems(p);
+    const float *st = yl_sino_t(p, sino);
+    const int vb = yl_u_views(p, view_batch(p), 1);
+    const int D = yl_op_chunks(p, vb);
+    int Deff, zlen;
+    yl_chunks(p, D, Deff, zlen);
+    float *part = p->part.ensure((size_t)Deff * p->V * pe, false);
+    float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
+    YlTable t;
+    auto sweep = [&](int kind, int v0, int nv, auto key) {
+        t.grouped<EtSweepArgs>(kind, {p}, key, [&](int, int &gx, int &gy, double &bytes) {
+            bytes += (double)nv * (8.0 * p->nvox + 4.0 * p->P);
+            EtSweepArgs a = yl_sweep_args(p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, D, yl_att_at(p, fac, v0));
+            a.act = p->act_yf.p;
+            a.part = part + (size_t)v0 * pe;
+            a.part_V = p->V;
+            a.sino = st + (size_t)v0 * pe;
+            a.u = p->u.p;
+            gx = a.D;
+            gy = nv;
+            return a;
+        });
+    };
+    if (Deff > 1)  // (one chunk: no later chunks to sum)
+        sweep(YL_PROJECT, 0, p->V,
+              [](const et_plan *q) { return std::make_tuple(0, q->yl_rpl, q->yl_nr, 16 * q->yl_w); });
+    for (int v0 = 0; v0 < p->V; v0 += vb) {
+        const int nv = std::min(vb, p->V - v0);
+        sweep(YL_GREF, v0, nv, YlTable::sweep_key);
+        yl_pull_into(t, p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, false, v0 > 0, v0 + nv >= p->V && truncate, acc);
+    }
+    yl_run(p, t, YL_OP_GREF);
     ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc, out, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
     return true;

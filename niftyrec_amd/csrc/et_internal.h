@@ -233,8 +233,8 @@ struct EtKeys {
 
 // Row-lane kernels of the OSEM subset loop (et_yl.h).  Grouped launches only
 // (tab as et_launch_sweep_group): sweeps kind 0 projection, 1 rotated-frame
-// backprojection, 3 exact attenuation gradient (reads the projection's partial
-// sums of the same chunking), gx = depth chunks, gy = views, nthr = 16 * W
+// backprojection, 3 exact and 5 reference attenuation gradient (read a projection's
+// partial sums of the same chunking), gx = depth chunks, gy = views, nthr = 16 * W
 // threads, `lds` bytes of LDS; kinds 2 and 4 the tiled projection and the tiled
 // gradient (R > 0), gx = depth chunks x tiles (tile fastest), 512 threads, NR
 // unused; pull gx = ceil(nx * nz / 16),

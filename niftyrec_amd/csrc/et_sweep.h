@@ -598,7 +598,7 @@ static int launch_sweep_r(int mode, int has_mu, const EtSweepArgs &a, hipStream_
 
 // Row-lane sweeps (et_yl.h) of PSF radius R: kind 0 projection, 1 rotated-frame
 // backprojection, 2 tiled projection, 3 exact attenuation gradient, 4 its tiled
-// variant; a grouped launch of `blocks` blocks of nthr = 16 * W threads
+// variant, 5 reference attenuation gradient; a grouped launch of `blocks` blocks of nthr = 16 * W threads
 // with `lds` bytes of dynamic LDS (two planes of the widest problem).
 // A row-lane projector launch, timed by its own dispatch (start and end
 // recorded in the events a profiling scope offered) where there is an offer.
@@ -641,6 +641,9 @@ static int launch_yl_r(int kind, int RPL, int NR, int nthr, size_t lds, const Et
         } else if (kind == 3) {                                                                                   \
             allow_lds(k_yl_grad<R, rpl, nr>, lds);                                                                \
             hipLaunchKernelGGL((k_yl_grad<R, rpl, nr>), dim3(blocks), dim3(nthr), lds, st, args, tab, n);         \
+        } else if (kind == 5) {                                                                                   \
+            allow_lds(k_yl_gref<R, rpl, nr>, lds);                                                                \
+            hipLaunchKernelGGL((k_yl_gref<R, rpl, nr>), dim3(blocks), dim3(nthr), lds, st, args, tab, n);         \
         } else {                                                                                                  \
             allow_lds(k_yl_bpu<R, rpl, nr>, lds);                                                                 \
             hipLaunchKernelGGL((k_yl_bpu<R, rpl, nr>), dim3(blocks), dim3(nthr), lds, st, args, tab, n);          \

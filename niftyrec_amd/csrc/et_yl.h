@@ -843,6 +843,104 @@ __device__ __forceinline__ void yl_bpu_body(const EtSweepArgs &a, const Blk &b)
     }
 }
 
+// ------------------------------------------------------------------------------
+// Reference attenuation gradient in the rotated frame, with cached factors:
+//   u(x', y, z') = PSF_z'( s(x', y) sum_{k >= z'} act'(x', y, k) e^{-A(k)} )
+// (emission-lib_gpu/_et_attenuation_gradient_gpu_kernels.cu:15-42, then the PSF
+// of emission-lib/_et.cpp:1829-1843).  Block (d, v) sweeps its chunk's planes
+// from the far end toward the detector, as yl_grad_body; the later chunks' sums
+// come from a projection without PSF (k_yl_project<0>) of the same chunking, the
+// running sum is Kahan-compensated.  The PSF passes and the LDS plane are the
+// backprojection's.  The sweep kernel k_grad_ref runs a whole ray per block in
+// slabs of 4 to 8 rows with 2R halo rows each and forms A again: at 64^3 x 64
+// views, PSF 7, it took 192 us, after 74 us of sums of mu.
+// ------------------------------------------------------------------------------
+template <int R, int RPL, int NR>
+__device__ __forceinline__ void yl_gref_body(const EtSweepArgs &a, const Blk &b)
+{
+    constexpr int K = 2 * R + 1;
+    extern __shared__ float lds[];
+    const int lane = threadIdx.x & 15, slot = threadIdx.x >> 4, W = blockDim.x >> 4;
+    const int d = b.x, v = b.y;
+    const int zb = d * a.zlen, ze = min(a.nz, zb + a.zlen);
+    constexpr int rows = 16 * RPL, CS = rows + 4;  // == a.yu
+    const int row0 = RPL * lane;
+    const int dx = a.yp, dz = a.yp * a.xp;
+    const FastView fv = load_fast_view(a.views + (size_t)v * ET_VIEW_REC);
+    if constexpr (R > 0) yl_zero_lds(lds, yl_plane_floats(a.nx, R, rows));
+    const float *act = a.act + a.gy + row0;
+    float *uv = a.u + (size_t)v * a.ustride + row0;
+
+    float acc[NR][RPL], cmp[NR][RPL];  // the running sum is acc - cmp
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const int xc = r * W + slot;
+#pragma unroll
+        for (int i = 0; i < RPL; i++) {
+            acc[r][i] = 0.f;
+            cmp[r][i] = 0.f;
+        }
+        if (xc >= a.nx) continue;
+        for (int d2 = d + 1; d2 < a.D; d2++) {
+            float t[RPL];
+            yl_load<RPL>(a.part + (((size_t)d2 * a.part_V + v) * a.nx + xc) * rows + row0, t);
+#pragma unroll
+            for (int i = 0; i < RPL; i++) {
+                float lo = -cmp[r][i];
+                comp_add(acc[r][i], lo, t[i]);
+                cmp[r][i] = -lo;
+            }
+        }
+    }
+    constexpr int PB = 16 / NR;  // planes per sample batch (descending)
+    YlSamp sb;
+    int kb = 0;
+    for (int z = ze - 1; z >= zb; z--, kb = kb + 1 == PB ? 0 : kb + 1) {
+        const float *kz = psf_plane<R>(a.psf, z);  // never read when R == 0
+        if (kb == 0)  // (planes before the chunk and columns past the end give samples no round takes)
+            sb = yl_samp_of(fast_sample(fv, (float)((lane % NR) * W + slot), z - lane / NR, a.nx, a.nz, dx, dz));
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int xc = r * W + slot;
+            if (xc < a.nx) {
+                const Samp s = yl_samp_from(sb, kb * NR + r);
+                float bl[RPL], e[RPL], sv[RPL];
+                yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e);
+                yl_bilinear<RPL>(act + s.off, dx, dz, s, bl);
+                yl_load<RPL>(a.sino + ((size_t)v * a.nx + xc) * rows + row0, sv);  // (a cache hit after the first plane)
+#pragma unroll
+                for (int i = 0; i < RPL; i++) {
+                    const float y = fmaf(bl[i], e[i], -cmp[r][i]);
+                    const float t = acc[r][i] + y;
+                    cmp[r][i] = (t - acc[r][i]) - y;
+                    acc[r][i] = t;
+                    bl[i] = sv[i] * (t - cmp[r][i]);
+                }
+                if constexpr (R > 0) {
+                    float cp[RPL];
+                    yl_column_pass<R, RPL>(bl, kz + K, cp);
+                    lds_store<RPL>(lds + (xc + R) * CS + row0, cp);
+                } else {
+                    yl_store<RPL>(uv + (size_t)rows * ((xc + 1) + (size_t)a.xp * (z + 1)), bl);
+                }
+            }
+        }
+        if constexpr (R > 0) {
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                const int xc = r * W + slot;
+                if (xc < a.nx) {
+                    float o[RPL];
+                    yl_row_pass<R, RPL>(lds, CS, xc, row0, kz, o);
+                    yl_store<RPL>(uv + (size_t)rows * ((xc + 1) + (size_t)a.xp * (z + 1)), o);
+                }
+            }
+            __syncthreads();  // the next plane's writes wait for these reads
+        }
+    }
+}
+
 template <int R, int RPL, int NR>
 __global__ void __launch_bounds__(1024) k_yl_project(const EtSweepArgs *__restrict__ args, const int4 *__restrict__ tab,
                                                      int n)
@@ -853,6 +951,17 @@ __global__ void __launch_bounds__(1024) k_yl_project(const EtSweepArgs *__restri
     const EtSweepArgs a = ((ET_CONST_AS const EtSweepArgs *)args)[j];
     if (a.skip && *a.skip) return;
     yl_project_body<R, RPL, NR>(a, b);
+}
+
+template <int R, int RPL, int NR>
+__global__ void __launch_bounds__(1024) k_yl_gref(const EtSweepArgs *__restrict__ args, const int4 *__restrict__ tab,
+                                                  int n)
+{
+    Blk b;
+    int j;
+    if (!group_block(tab, n, b, j)) return;
+    const EtSweepArgs a = ((ET_CONST_AS const EtSweepArgs *)args)[j];
+    yl_gref_body<R, RPL, NR>(a, b);
 }
 
 template <int R, int RPL>
