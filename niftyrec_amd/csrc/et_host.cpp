@@ -259,7 +259,7 @@ struct et_plan {
     // OSEM caches (valid while osem_valid; keyed on the subset count, the
     // chunking, eps and the attenuation map's key: its content fingerprint, or
     // its address when mu_check is off)
-    DevBuf x_yf, sens, osem_recs, osem_meas, osem_E, osem_order;
+    DevBuf x_yf, sens, osem_recs, osem_meas, osem_E, osem_order;  // (osem_E: the sweep kernels' factors)
     bool osem_valid = false;
     bool osem_yl = false;           // the cached data are the row-lane kernels'
     int osem_S = 0, osem_D = 0, osem_Dp = 0, osem_Db = 0;
@@ -279,6 +279,8 @@ struct et_plan {
     int yl_tiles = 1;                                  // projector column tiles (> 1: the tiled projector)
     int yl_tile_n = 1;                                 // tiles of the tiled projector where it applies, else 1
     size_t yl_lds_full = 0, yl_lds_tile = 0;           // LDS of a full-width / tiled projector block
+    int yt_L = 0, yt_cols = 0;                         // wide or tall plans (tile kernels): lanes per column (else 0),
+                                                       // columns per tile
     DevBuf osem_tables;                                // argument records and block tables of the OSEM launches
     // row-lane kernels for the single operations of a created plan (projection,
     // backprojection, exact attenuation gradient with attenuation): factors of
@@ -300,6 +302,9 @@ struct et_plan {
     int fwd_D = 0, fwd_tiles = 0;
     std::vector<struct YlLaunch> yl_launches;          // per subset: projection, ratio, backprojection, pull
     std::vector<const void *> osem_sig;                // buffers yl_launches refer to
+    bool osem_struct = false;   // row-lane plans: records, chunking and tables are those of osem_S, osem_has_mu and
+    int osem_tune_D = 0;        // tune_D = osem_tune_D (they do not depend on the map's content)
+    unsigned osem_key_gen = 0;  // key_gen when the factors were last known to be the OSEM map's
     DevBuf fp_dev;                  // fingerprint partial sums (ET_FP_BLOCKS)
     unsigned long long *fp_host = nullptr;  // their pinned host copy
     // tuning
@@ -334,6 +339,55 @@ namespace {
 
 int nthreads_for(int nx) { return ((nx + 63) / 64) * 64; }
 
+// Wide or tall plans on the tile kernels (k_yt_*): more than 192 columns or 128
+// rows.  16 lanes hold a column of up to 128 rows, 32 lanes one of up to 256.
+// The sweep kernels keep
+//   - tall volumes of at most 64 columns: one tile, whose halo columns and 1,024
+//     thread blocks buy nothing there;
+//   - wide volumes of at most 16 rows: one slab of theirs, against rows padded to 32;
+//   - more than 256 rows.
+void yt_plan(et_plan *p)
+{
+    const int nx = p->nx, ny = p->ny;
+    const bool tall = ny > 128 && ny <= 256 && nx > ET_YL_TILE, wide = ny > 16 && ny <= 128 && nx > 192;
+    if (!tall && !wide) return;
+    const int L = tall ? 32 : 16, rpl = tall ? (ny + 63) / 64 * 2 : (ny + 31) / 32 * 2;
+    int dev = 0, lim = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        return;
+    // Columns per tile: as few tiles as possible with two LDS planes per block, the
+    // columns spread evenly over them (blocks of up to 512 threads, 16 lanes per
+    // column, share a CU by two, those of up to 1,024 have it to themselves); one
+    // plane of the widest tile where two would leave tiles narrower than 40
+    // columns.  The slots of a tile, C / 2, cover its 2R halo columns, and its
+    // threads are whole waves: C a multiple of 4 (L = 32) or 8, at least 4R.
+    const int blocks = tall ? 1 : 2, step = 128 / L, R = p->R;
+    const int least = (std::max(4 * R, step) + step - 1) / step * step;
+    auto fits = [&](int C, int nbuf) {
+        return R == 0 || nbuf * blocks * et_yt_plane_bytes(C, R, L * rpl) <= (size_t)lim;
+    };
+    int widest = ET_YL_TILE, nbuf = 2;
+    while (widest > 40 && !fits(widest, 2)) widest -= step;
+    if (!fits(widest, 2) || widest < least) {
+        widest = ET_YL_TILE;
+        nbuf = 1;
+        while (widest > least && !fits(widest, 1)) widest -= step;
+        if (!fits(widest, 1) || widest < least) return;
+    }
+    const int T = (nx + widest - 1) / widest;
+    const int C = std::max(least, ((nx + T - 1) / T + step - 1) / step * step);
+    p->yl = true;
+    p->yt_L = L;
+    p->yt_cols = C;
+    p->yl_rpl = rpl;
+    p->yl_nr = 0;
+    p->yl_w = C / 2;
+    p->yl_nbuf = nbuf;
+    p->yl_lds = p->yl_lds_full = p->yl_lds_tile = p->yl_lds_bpu = R == 0 ? 0 : nbuf * et_yt_plane_bytes(C, R, L * rpl);
+    p->yl_tile_n = p->yl_tiles = (nx + C - 1) / C;
+}
+
 int build_plan(et_plan *p, int nx, int ny, int nz, const Cameras &cams, const float *psf, int psf_h,
                float bg, float bga)
 {
@@ -347,6 +401,7 @@ int build_plan(et_plan *p, int nx, int ny, int nz, const Cameras &cams, const fl
     p->R = p->K > 0 ? (p->K - 1) / 2 : 0;
     p->recs.assign((size_t)cams.V * ET_VIEW_REC, 0.f);
     p->fast = true;
+    p->osem_valid = p->osem_struct = p->fac_built = p->fwd_built = false;  // (a plan object built again)
     for (int v = 0; v < cams.V; v++) {
         float M[16], Mi[16];
         const int V = cams.V;
@@ -368,6 +423,8 @@ int build_plan(et_plan *p, int nx, int ny, int nz, const Cameras &cams, const fl
     // at most 3 rounds of up to 64 columns, and one or two LDS planes of
     // (nx + 2R) x (rows + 4) floats within the device's per-block LDS.
     p->yl = false;
+    p->yt_L = 0;
+    p->yl_tile_n = p->yl_tiles = 1;
     if (p->fast) {
         const int rows32 = ((ny + 31) / 32) * 32;
         const int rpl = rows32 / 16, nr = (nx + 63) / 64;
@@ -399,8 +456,9 @@ int build_plan(et_plan *p, int nx, int ny, int nz, const Cameras &cams, const fl
                 }
             }
         }
+        if (!p->yl) yt_plan(p);
     }
-    const int yrows = p->yl ? 16 * p->yl_rpl : p->slabs * ET_T;  // axial rows held per column
+    const int yrows = p->yl ? (p->yt_L ? p->yt_L : 16) * p->yl_rpl : p->slabs * ET_T;  // axial rows held per column
     // YF layout.  Guard rows: the activity-like volumes are gathered in windows
     // of rows y0 - R4 .. y0 + TS + R4 - 1 (R4 = R rounded up to 4); with R4
     // guard rows every 16-row slab's window starts on a 64-byte segment
@@ -1315,6 +1373,10 @@ const float *yl_att_at(const et_plan *p, const float *att, int v0)
     return att ? att + (size_t)v0 * p->nz * yl_plane_elems(p) : nullptr;
 }
 
+// Blocks of a rotated-frame backprojection along x: chunks (and tiles, on the
+// tile kernels).
+int yl_bpu_gx(const et_plan *p, int D) { return D * (p->yt_L ? p->yl_tiles : 1); }
+
 // Arguments of a row-lane sweep over nv views (records recs, factors att; null
 // without attenuation).
 EtSweepArgs yl_sweep_args(const et_plan *p, const float *recs, int nv, int D, const float *att)
@@ -1327,15 +1389,21 @@ EtSweepArgs yl_sweep_args(const et_plan *p, const float *recs, int nv, int D, co
     a.D = Deff;
     a.zlen = zlen;
     a.att = const_cast<float *>(att);
+    a.att_vs = (size_t)p->nz * yl_plane_elems(p);
     a.part_V = nv;
     a.yl_nbuf = p->yl_nbuf;
+    a.yt_cols = p->yt_cols;
     a.yl_tiles = p->yl_tiles;
     return a;
 }
 
 // Blocks of the row-lane pulls (reference and exact adjoint): 4 x 4 tiles of
 // image columns in super-tiles of 8 x 8 tiles.
-int yl_pull_tiles(const et_plan *p) { return (((p->nx + 3) / 4 + 7) / 8) * (((p->nz + 3) / 4 + 7) / 8) * 64; }
+int yl_pull_tiles(const et_plan *p)
+{
+    // (two row halves where 32 lanes hold a column)
+    return (((p->nx + 3) / 4 + 7) / 8) * (((p->nz + 3) / 4 + 7) / 8) * 64 * (p->yt_L == 32 ? 2 : 1);
+}
 
 // Grouped launches of row-lane OSEM work over several plans; the block shapes
 // and templates come from each plan.  Sweeps share a launch when they share
@@ -1343,6 +1411,14 @@ int yl_pull_tiles(const et_plan *p) { return (((p->nx + 3) / 4 + 7) / 8) * (((p-
 struct YlTable {
     TableBytes tb;
     std::vector<YlLaunch> L;
+    int S = 1, sub = 0;  // OSEM launches: subset sub of S (views sub, sub + S, ... of the plans' factors)
+
+    // Factors of the current subset's views: the plan's, in view order.
+    void subset_factors(const et_plan *p, EtSweepArgs &a) const
+    {
+        a.att = p->osem_mu_yf ? p->fac.p + (size_t)sub * a.att_vs : nullptr;
+        a.att_vs *= S;
+    }
 
     template <class Args, class Key, class Fill>
     void grouped(int kind, const std::vector<et_plan *> &plans, Key key, Fill fill)
@@ -1373,13 +1449,15 @@ struct YlTable {
 
     static std::tuple<int, int, int, int> sweep_key(const et_plan *p)
     {
-        return std::make_tuple(p->R, p->yl_rpl, p->yl_nr, 16 * p->yl_w);
+        // (the tile kernels of wide or tall plans: NR = -L)
+        return p->yt_L ? std::make_tuple(p->R, p->yl_rpl, -p->yt_L, p->yl_w * p->yt_L)
+                       : std::make_tuple(p->R, p->yl_rpl, p->yl_nr, 16 * p->yl_w);
     }
     static std::tuple<int, int, int, int> pull_key(const et_plan *p) { return std::make_tuple(0, p->yl_rpl, 0, 256); }
     // projector launches: the tiled kernel is keyed with NR = 0
     static std::tuple<int, int, int, int> project_key(const et_plan *p)
     {
-        return p->yl_tiles > 1 ? std::make_tuple(p->R, p->yl_rpl, 0, 512) : sweep_key(p);
+        return p->yl_tiles > 1 && !p->yt_L ? std::make_tuple(p->R, p->yl_rpl, 0, 512) : sweep_key(p);
     }
 
     // Projection of each plan's views [v0, v0 + nv) of its OSEM records into its
@@ -1390,8 +1468,9 @@ struct YlTable {
         grouped<EtSweepArgs>(YL_PROJECT, plans, project_key, [&](int i, int &gx, int &gy, double &bytes) {
             et_plan *p = plans[i];
             bytes += (double)nv[i] * (8.0 * p->nvox + 4.0 * p->P);  // activity and mu (factors) per view, sinogram
-            EtSweepArgs a = yl_sweep_args(p, p->osem_recs.p + (size_t)v0[i] * ET_VIEW_REC, nv[i], Dp[i],
-                                          yl_att_at(p, p->osem_mu_yf ? p->osem_E.p : nullptr, v0[i]));
+            EtSweepArgs a =
+                yl_sweep_args(p, p->osem_recs.p + (size_t)v0[i] * ET_VIEW_REC, nv[i], Dp[i], nullptr);
+            subset_factors(p, a);
             a.act = p->x_yf.p;
             a.part = p->part.p;
             gx = a.D * p->yl_tiles;
@@ -1426,12 +1505,13 @@ struct YlTable {
         grouped<EtSweepArgs>(YL_BPU, plans, sweep_key, [&](int i, int &gx, int &gy, double &bytes) {
             et_plan *p = plans[i];
             bytes += (double)nv[i] * (8.0 * p->nvox + 4.0 * p->P);  // factors read, u write, sinogram read
-            EtSweepArgs a = yl_sweep_args(p, p->osem_recs.p + (size_t)v0[i] * ET_VIEW_REC, nv[i], Db[i],
-                                          yl_att_at(p, p->osem_mu_yf ? p->osem_E.p : nullptr, v0[i]));
+            EtSweepArgs a =
+                yl_sweep_args(p, p->osem_recs.p + (size_t)v0[i] * ET_VIEW_REC, nv[i], Db[i], nullptr);
+            subset_factors(p, a);
             a.src = ones ? ET_SRC_ONES : ET_SRC_SINO;
             a.sino = p->ratio.p;
             a.u = p->u.p;
-            gx = a.D;
+            gx = yl_bpu_gx(p, a.D);
             gy = nv[i];
             return a;
         });
@@ -1451,6 +1531,8 @@ struct YlTable {
                                                 (*sens_out)[i], nullptr, nullptr)
                                     : pull_args(p, r, nv[i], p->u.p, false, ET_EPI_OSEM, false, false, nullptr,
                                                 p->x_yf.p, sens[i]);
+            // the sensitivity is truncated at 0, then clamped below at epsilon
+            if (sens_out) a.floor = std::max(p->osem_cur_eps, 0.f);
             gx = yl_pull_tiles(p);
             gy = 1;
             return a;
@@ -1474,8 +1556,11 @@ void yl_issue(const float *dev, const std::vector<YlLaunch> &L, size_t from, siz
         case YL_GREF: {
             ProfScope ps(prof, l.kind == YL_PROJECT ? ET_PROF_PROJECT : (l.kind == YL_BPU ? ET_PROF_BPU : ET_PROF_GRAD),
                          l.bytes);
-            const int k = l.kind == YL_BPU ? 1 : l.kind == YL_GREF ? 5 : (l.kind == YL_GRAD ? (l.NR == 0 ? 4 : 3) : (l.NR == 0 ? 2 : 0));
-            check_launch(et_launch_yl_sweep(k, l.R, l.RPL, l.NR, l.nthr, l.lds, static_cast<const EtSweepArgs *>(args),
+            const int k = l.NR < 0 ? (l.kind == YL_PROJECT ? 6 : (l.kind == YL_BPU ? 7 : 8))
+                          : l.kind == YL_BPU ? 1
+                          : l.kind == YL_GREF ? 5
+                                              : (l.kind == YL_GRAD ? (l.NR == 0 ? 4 : 3) : (l.NR == 0 ? 2 : 0));
+            check_launch(et_launch_yl_sweep(k, l.R, l.RPL, std::abs(l.NR), l.nthr, l.lds, static_cast<const EtSweepArgs *>(args),
                                             tab, l.n, l.blocks, s));
             break;
         }
@@ -1519,6 +1604,23 @@ void yl_upload(DevBuf &buf, const YlTable &t, hipStream_t st)
 // attenuation map's key, as the OSEM caches), the activity is gathered by the
 // projector, and the rotated-frame volumes go to the sweep kernels' pulls
 // (same u layout).
+
+// Whether the device has room for the factors of every view (4 bytes per voxel
+// and view: 12 GB at 256^3 x 180 views); a single operation falls back to the
+// sweep kernels, which form them as they go, where it has not.
+bool yl_factor_room(et_plan *p)
+{
+    try {
+        const bool held = p->fac.p != nullptr;
+        p->fac.ensure(yl_att_elems(p, p->V), false);
+        if (!held) p->fac_built = false;
+        return true;
+    } catch (const EtError &) {
+        (void)hipGetLastError();
+        p->fac_built = false;
+        return false;
+    }
+}
 
 // Sources of a single operation: the YF copies of act and mu (either may be
 // null) and, with a map, the factors of every view in view order
@@ -1676,15 +1778,36 @@ float *yl_forward(YlTable &t, et_plan *p, const float *fac, int D, const int *sk
     return part;
 }
 
-// Depth chunks of the projection of every view (the forward sums' chunking).
+// Largest rotated-frame buffer of the gradient and the joint backward: 4 GiB
+// (128^3 x 120 views hold 1.0 GiB each).
+constexpr size_t ET_YL_U_BYTES = 4ull << 30;
+
+// Views per batch of the exact attenuation gradient (rotated-frame volumes of at
+// most ET_YL_U_BYTES).
+int yl_gradient_batch(const et_plan *p)
+{
+    const long fit = (long)std::max<size_t>(1, ET_YL_U_BYTES / (p->ustride * sizeof(float)));
+    return (int)std::min<long>(p->tune_vb > 0 ? p->tune_vb : fit, p->V);
+}
+
+// Depth chunks of the projection of every view (the forward sums' chunking, which
+// the gradient sweeps share).  The blocks of a tall plan have a CU to themselves,
+// so a launch of a few blocks per CU ends in a nearly empty round (256^3, 63
+// views, PSF 21, gradient sweep: 320 blocks in one chunk 5.6 ms, MEASURED_GRAD in
+// eight); its chunks, of at least 16 planes, give eight per CU.
 int yl_forward_chunks(const et_plan *p, bool mu)
 {
-    return !mu && p->tune_D > 0 ? p->tune_D : yl_op_chunks(p, (long)p->V * p->yl_tiles);
+    if (!mu && p->tune_D > 0) return p->tune_D;
+    if (p->yt_L != 32) return yl_op_chunks(p, (long)p->V * p->yl_tiles);
+    const long per_chunk = (long)yl_gradient_batch(p) * p->yl_tiles;
+    int D = 1;
+    while (D < 32 && p->nz / (2 * D) >= 16 && per_chunk * D < 8L * 256) D *= 2;
+    return D;
 }
 
 bool yl_op_project(et_plan *p, const float *act, const float *mu, float *sino, int truncate)
 {
-    if (!p->yl_ops || !p->yl || !act) return false;
+    if (!p->yl_ops || !p->yl || !act || (mu && !yl_factor_room(p))) return false;
     p->fwd_built = false;  // until the sums are queued
     const float *fac = yl_sources(p, act, mu, 1);
     const int D = yl_forward_chunks(p, mu != nullptr);
@@ -1704,7 +1827,7 @@ bool yl_op_project(et_plan *p, const float *act, const float *mu, float *sino, i
 
 bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate)
 {
-    if (!p->yl_ops || !p->yl) return false;
+    if (!p->yl_ops || !p->yl || (mu && !yl_factor_room(p))) return false;
     const float *fac = yl_sources(p, nullptr, mu, 0);
     const size_t pe = yl_plane_elems(p);
     const float *st = yl_sino_t(p, sino);
@@ -1714,7 +1837,7 @@ bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *ou
     YlTable t;  // every batch in one table: the batches reuse u in stream order
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
-        const int D = yl_op_chunks(p, nv);
+        const int D = yl_op_chunks(p, yl_bpu_gx(p, nv));
         const float *recs = p->d_recs.p + (size_t)v0 * ET_VIEW_REC;
         t.grouped<EtSweepArgs>(YL_BPU, {p}, YlTable::sweep_key, [&](int, int &gx, int &gy, double &bytes) {
             bytes += (double)nv * (8.0 * p->nvox + 4.0 * p->P);
@@ -1723,7 +1846,7 @@ bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *ou
             a.sino = st + (size_t)v0 * pe;
             a.u = p->u.p;
             if (p->K > 0 && adjoint) a.psf = p->d_sep_flip.p;  // correlation: the adjoint of the PSF
-            gx = a.D;
+            gx = yl_bpu_gx(p, a.D);
             gy = nv;
             return a;
         });
@@ -1774,21 +1897,16 @@ void yl_gradient_sweep(YlTable &t, et_plan *p, int v0, int nv, const float *fac,
     });
 }
 
-// Largest rotated-frame buffer of the gradient and the joint backward: 4 GiB
-// (128^3 x 120 views hold 1.0 GiB each).
-constexpr size_t ET_YL_U_BYTES = 4ull << 30;
-
 // Exact attenuation gradient: the forward sums of every view (kept from the last
 // projection or formed here), then per view batch the gradient sweep and the
 // exact adjoint pull.
 bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate)
 {
-    if (!p->yl_ops || !p->yl || !act || !mu) return false;
+    if (!p->yl_ops || !p->yl || !act || !mu || !yl_factor_room(p)) return false;
     const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
     const int D = yl_forward_chunks(p, true);
-    const long fit = (long)std::max<size_t>(1, ET_YL_U_BYTES / (p->ustride * sizeof(float)));
-    const int vb = yl_u_views(p, p->tune_vb > 0 ? std::min(p->tune_vb, p->V) : (int)std::min<long>(fit, p->V), 1);
+    const int vb = yl_u_views(p, yl_gradient_batch(p), 1);
     float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
     YlTable t;  // every batch in one table: the batches reuse u in stream order
     float *part = yl_gradient_forward(t, p, fac, D);
@@ -1809,7 +1927,7 @@ bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float
 // reference pull.
 bool yl_op_gradient_ref(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate)
 {
-    if (!p->yl_ops || !p->yl || !act || !mu) return false;
+    if (!p->yl_ops || !p->yl || p->yt_L || !act || !mu || !yl_factor_room(p)) return false;  // (no such tile kernel)
     const float *fac = yl_sources(p, act, mu, 0);
     const size_t pe = yl_plane_elems(p);
     const float *st = yl_sino_t(p, sino);
@@ -1860,7 +1978,8 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
 {
     if (!p->yl_ops || !p->yl || !act || !mu) return false;
     const int V = p->V;
-    if (2 * (size_t)V * p->ustride * sizeof(float) > ET_YL_U_BYTES || yl_u_views(p, V, 2) < V) return false;
+    if (2 * (size_t)V * p->ustride * sizeof(float) > ET_YL_U_BYTES || !yl_factor_room(p) || yl_u_views(p, V, 2) < V)
+        return false;
     const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
     float *ub = p->u.p, *ug = p->u.p + (size_t)V * p->ustride;
@@ -1870,7 +1989,7 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
     const int D = yl_forward_chunks(p, true);
     YlTable t;
     float *part = yl_gradient_forward(t, p, fac, D);
-    const int Db = yl_op_chunks(p, V);
+    const int Db = yl_op_chunks(p, yl_bpu_gx(p, V));
     t.grouped<EtSweepArgs>(YL_BPU, {p}, YlTable::sweep_key, [&](int, int &gx, int &gy, double &bytes) {
         bytes += (double)V * (8.0 * p->nvox + 4.0 * p->P);
         EtSweepArgs a = yl_sweep_args(p, recs, V, Db, fac);
@@ -1878,7 +1997,7 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
         a.sino = st;
         a.u = ub;
         if (p->K > 0) a.psf = p->d_sep_flip.p;  // correlation: the adjoint of the PSF
-        gx = a.D;
+        gx = yl_bpu_gx(p, a.D);
         gy = V;
         return a;
     });
@@ -1904,32 +2023,42 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
 // full-width one.
 void yl_use_tiles(et_plan *p, bool tiled)
 {
+    if (p->yt_L) return;  // (one projector kind)
     tiled = tiled && p->yl_tile_n > 1;
     p->yl_tiles = tiled ? p->yl_tile_n : 1;
     p->yl_lds = tiled ? p->yl_lds_tile : p->yl_lds_full;
 }
 
-// Depth chunking of the row-lane projection (mode ET_MODE_PROJECT, timed with
-// the ratio that reads its partial sums) or backprojection (ET_MODE_BPU, timed
-// behind the chosen projection and ratio) on the first subset: candidates 8,
-// 16, 32 chunks and the count that puts one block per CU, three launches each
-// after a warm-up, in three interleaved rounds; the fastest round decides.
-// Where the tiled projector applies, the projection candidates are timed with
-// both projector kinds, and the plan keeps the kind of the fastest.
-int yl_tune_chunks(et_plan *p, int mode, int nv, int Dp = 0)
+// Depth chunkings of the row-lane OSEM sweeps of nv views that are timed: 8, 16,
+// 32 chunks and the count that puts one block per CU (a fixed tuning: that alone).
+std::vector<int> yl_chunk_candidates(const et_plan *p, int nv)
 {
     int cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
+    const std::vector<int> ask = p->tune_D > 0 ? std::vector<int>{p->tune_D}
+                                               : std::vector<int>{8, 16, 32, cus / std::max(nv, 1)};
     std::vector<int> chunks;
-    for (int D : {8, 16, 32, cus / std::max(nv, 1)}) {
+    for (int D : ask) {
         int Deff, zlen;
         yl_chunks(p, D, Deff, zlen);
-        if (Deff >= 1 && std::find(chunks.begin(), chunks.end(), Deff) == chunks.end()) chunks.push_back(Deff);
+        if (std::find(chunks.begin(), chunks.end(), Deff) == chunks.end()) chunks.push_back(Deff);
     }
+    return chunks;
+}
+
+// Depth chunking of the row-lane projection (mode ET_MODE_PROJECT, timed with
+// the ratio that reads its partial sums) or backprojection (ET_MODE_BPU, timed
+// behind the chosen projection and ratio) on the first of S subsets: the
+// candidate chunkings, three launches each after a warm-up, in three interleaved rounds; the fastest round decides.
+// Where the tiled projector applies, the projection candidates are timed with
+// both projector kinds, and the plan keeps the kind of the fastest.
+int yl_tune_chunks(et_plan *p, int mode, int S, int nv, int Dp = 0)
+{
+    const std::vector<int> chunks = yl_chunk_candidates(p, nv);
     // (depth chunks, tiled projector); the backprojection keeps the projector chosen
-    const bool both = mode == ET_MODE_PROJECT && p->yl_tile_n > 1;
+    const bool both = mode == ET_MODE_PROJECT && p->yl_tile_n > 1 && !p->yt_L;
     const bool tiled_now = p->yl_tiles > 1;
     std::vector<std::pair<int, bool>> cand;
     for (int D : chunks) {
@@ -1950,6 +2079,7 @@ int yl_tune_chunks(et_plan *p, int mode, int nv, int Dp = 0)
             const int D = cand[ci].first;
             yl_use_tiles(p, cand[ci].second);
             YlTable t;
+            t.S = S;
             const std::vector<int> dp{mode == ET_MODE_PROJECT ? D : Dp}, db{D};
             t.project(one, v0, nvv, dp);
             t.ratio(one, v0, nvv, dp);
@@ -1979,79 +2109,126 @@ int yl_tune_chunks(et_plan *p, int mode, int nv, int Dp = 0)
 // the table is then rebuilt.
 std::vector<const void *> yl_osem_sig(const et_plan *p)
 {
-    return {p->x_yf.p, p->osem_meas.p, p->part.p, p->ratio.p, p->u.p, p->sens.p, p->osem_recs.p, p->osem_E.p};
+    return {p->x_yf.p, p->osem_meas.p, p->part.p, p->ratio.p, p->u.p, p->sens.p, p->osem_recs.p, p->fac.p};
 }
 
-// Launch table of one row-lane OSEM iteration: per subset projection, ratio,
-// backprojection, pull with the update.
+// Launch table of a row-lane OSEM run: per subset the sensitivity
+// (backprojection of ones, pull with the clamp), then per subset projection,
+// ratio, backprojection, pull with the update.
 void yl_osem_tables(et_plan *p, int S, const std::vector<int> &start)
 {
     const std::vector<et_plan *> one{p};
     YlTable t;
-    for (int s = 0; s < S; s++) {
-        const std::vector<int> v0{start[s]}, nv{start[s + 1] - start[s]}, dp{p->osem_Dp}, db{p->osem_Db};
-        const std::vector<const float *> sens{p->sens.p + (size_t)s * p->yf_elems};
-        t.project(one, v0, nv, dp);
-        t.ratio(one, v0, nv, dp);
-        t.bpu(one, v0, nv, db, false);
-        t.pull(one, v0, nv, sens, nullptr);
+    t.S = S;
+    for (int pass = 0; pass < 2; pass++) {
+        for (int s = 0; s < S; s++) {
+            const std::vector<int> v0{start[s]}, nv{start[s + 1] - start[s]}, dp{p->osem_Dp}, db{p->osem_Db};
+            float *sens = p->sens.p + (size_t)s * p->yf_elems;
+            t.sub = s;
+            if (pass == 0) {
+                std::vector<float *> out{sens};
+                t.bpu(one, v0, nv, db, true);
+                t.pull(one, v0, nv, {}, &out);
+            } else {
+                t.project(one, v0, nv, dp);
+                t.ratio(one, v0, nv, dp);
+                t.bpu(one, v0, nv, db, false);
+                t.pull(one, v0, nv, {sens}, nullptr);
+            }
+        }
     }
     yl_upload(p->osem_tables, t, p->st);
     p->yl_launches = t.L;
     p->osem_sig = yl_osem_sig(p);
 }
 
-// Row-lane caches of an OSEM rebuild: attenuation factors of every view (one
-// launch), chunkings, subset sensitivities, and the launch table of one
-// iteration.  The measured planes and the iterate are set by the caller.
-void yl_osem_build(et_plan *p, const float *mu_yf, int S, float eps, const std::vector<int> &start)
+// Row-lane OSEM caches, in two parts.  What follows from the plan, the subset
+// count and the tuning (records in subset order, buffers, chunkings, launch
+// table) is built once; what follows from the map's content (factors, subset
+// sensitivities) is formed again for another map without waiting for the stream
+// or timing the chunkings again.  The factors are the single operations' own
+// (view order; a subset's views lie S apart), so that a map that changes between
+// OSEM passes and gradients of it (joint estimation) has its factors formed
+// once: at 256^3 x 180 views they take 12 GB and 5 ms.
+void yl_osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, int S, float eps,
+                     unsigned long long mu_key, const std::vector<int> &order, const std::vector<int> &start)
 {
+    const bool has_mu = mu != nullptr;
+    const bool structure = !p->osem_struct || p->osem_S != S || p->osem_has_mu != has_mu || p->osem_tune_D != p->tune_D;
+    const bool content = structure || !p->osem_valid || p->osem_mu_key != mu_key || p->osem_eps != eps;
+    const size_t pe = yl_plane_elems(p);
     const int maxsub = (p->V + S - 1) / S;
-    // every buffer the launch tables refer to is allocated before they are built
-    p->x_yf.ensure(p->yf_elems, true, p->st);
-    p->osem_meas.ensure((size_t)p->V * yl_plane_elems(p), true, p->st);
-    if (mu_yf) {
-        p->osem_E.ensure(yl_att_elems(p, p->V), false);
-        EtSweepArgs a = yl_sweep_args(p, p->osem_recs.p, p->V, 1, p->osem_E.p);
-        a.mu = mu_yf;
-        ProfScope ps(p, ET_PROF_OTHER, (double)p->V * 8.0 * p->nvox);
-        check_launch(et_launch_yl_factors(p->yl_rpl, a, EtKeys{}, (et_stream_t)p->st));
-    }
-    p->u.ensure((size_t)maxsub * p->ustride, true, p->st);
-    p->ratio.ensure((size_t)maxsub * yl_plane_elems(p), true, p->st);
-    p->part.ensure((size_t)p->nz * maxsub * yl_plane_elems(p), false);
     p->osem_cur_eps = eps;
-    int Dp = p->tune_D, Db = p->tune_D;
-    yl_use_tiles(p, true);  // the tiled projector unless timing prefers the full-width one
-    if (p->tune_D <= 0) {
-        Dp = yl_tune_chunks(p, ET_MODE_PROJECT, start[1] - start[0]);
-        Db = yl_tune_chunks(p, ET_MODE_BPU, start[1] - start[0], Dp);
+    p->osem_mu_yf = has_mu;
+    if (content) p->osem_valid = false;  // until the rebuild is queued
+    // the map's factors; after an OSEM call of the same map only if another
+    // operation has formed factors meanwhile (then it is the device that compares)
+    if (has_mu && (content || p->key_gen != p->osem_key_gen)) {
+        yl_sources(p, nullptr, mu, 0);
+        p->osem_key_gen = p->key_gen;
     }
-    int zlen;
-    yl_chunks(p, Dp, p->osem_Dp, zlen);
-    yl_chunks(p, Db, p->osem_Db, zlen);
-    // sensitivities: backprojection of ones, truncated, clamped below at eps
-    p->sens.ensure((size_t)S * p->yf_elems, true, p->st);
-    const std::vector<et_plan *> one{p};
-    for (int s = 0; s < S; s++) {
-        YlTable t;
-        const std::vector<int> v0{start[s]}, nv{start[s + 1] - start[s]}, db{p->osem_Db};
-        std::vector<float *> out{p->sens.p + (size_t)s * p->yf_elems};
-        t.bpu(one, v0, nv, db, true);
-        t.pull(one, v0, nv, {}, &out);
-        yl_upload(p->osem_tables, t, p->st);
-        yl_issue(p->osem_tables.p, t.L, 0, t.L.size(), p->st, p);
-        ProfScope ps(p, ET_PROF_OTHER, 0);
-        check_launch(et_launch_yf_clamp_min(out[0], p->nx, p->ny, p->nz, p->yp, p->gy, eps, (et_stream_t)p->st));
+    if (structure) {
+        p->osem_struct = false;
+        std::vector<float> recs((size_t)p->V * ET_VIEW_REC);
+        for (int i = 0; i < p->V; i++)
+            std::memcpy(&recs[(size_t)i * ET_VIEW_REC], &p->recs[(size_t)order[i] * ET_VIEW_REC],
+                        sizeof(float) * ET_VIEW_REC);
+        p->osem_recs.ensure(recs.size(), false);
+        check_hip(hipMemcpyAsync(p->osem_recs.p, recs.data(), sizeof(float) * recs.size(), hipMemcpyHostToDevice,
+                                 p->st),
+                  niftyrec_error_transfergpu);
+        p->osem_order.ensure(order.size(), false);
+        check_hip(hipMemcpyAsync(p->osem_order.p, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice,
+                                 p->st),
+                  niftyrec_error_transfergpu);
+        check_hip(hipStreamSynchronize(p->st), niftyrec_error_kernel);  // (the host copies end here)
+        // every buffer the launch table refers to, before it is built
+        p->x_yf.ensure(p->yf_elems, true, p->st);
+        p->osem_meas.ensure((size_t)p->V * pe, true, p->st);
+        p->u.ensure((size_t)maxsub * p->ustride, true, p->st);
+        p->ratio.ensure((size_t)maxsub * pe, true, p->st);
+        p->sens.ensure((size_t)S * p->yf_elems, true, p->st);
+        int Dmax = 1;
+        for (int D : yl_chunk_candidates(p, start[1] - start[0])) Dmax = std::max(Dmax, D);
+        p->part.ensure((size_t)Dmax * maxsub * pe, false);
+        int Dp = p->tune_D, Db = p->tune_D, zlen;
+        yl_use_tiles(p, true);  // the tiled projector unless timing prefers the full-width one
+        if (p->tune_D <= 0) {
+            Dp = yl_tune_chunks(p, ET_MODE_PROJECT, S, start[1] - start[0]);
+            Db = yl_tune_chunks(p, ET_MODE_BPU, S, start[1] - start[0], Dp);
+        }
+        yl_chunks(p, Dp, p->osem_Dp, zlen);
+        yl_chunks(p, Db, p->osem_Db, zlen);
     }
-    yl_osem_tables(p, S, start);
+    // (a single operation may have reallocated a buffer of the table)
+    if (structure || yl_osem_sig(p) != p->osem_sig) yl_osem_tables(p, S, start);
+    p->osem_struct = true;
+    p->osem_S = S;
+    p->osem_has_mu = has_mu;
+    p->osem_tune_D = p->tune_D;
+    if (content) {
+        if (!structure && p->osem_eps != eps) yl_osem_tables(p, S, start);  // (epsilon is in the records)
+        yl_issue(p->osem_tables.p, p->yl_launches, 0, 2 * (size_t)S, p->st, p);  // sensitivities
+        p->osem_mu_key = mu_key;
+        p->osem_eps = eps;
+        p->osem_yl = true;
+        p->osem_valid = true;
+    }
+    // measured data in subset order, transposed to [v][x][rows]
+    {
+        ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->V * p->P);
+        check_launch(et_launch_gather_planes_t(p->osem_meas.p, meas, reinterpret_cast<const int *>(p->osem_order.p),
+                                               p->V, p->nx, p->ny, p->yu, (et_stream_t)p->st));
+    }
+    pack(p, x, p->x_yf);
+    p->osem_start = start;
+    p->osem_cur_mu = has_mu ? p->mu_yf.p : nullptr;
 }
 
 void osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, int S, float eps,
                   unsigned long long mu_key)
 {
     if (S <= 0 || S > p->V || !p->fast) throw EtError{niftyrec_error_parameters};
-    const bool use_yl = p->yl;
     // subset s: views s, s+S, ...; records and measured planes reordered by subset
     std::vector<int> order, start(S + 1, 0);
     for (int s = 0; s < S; s++) {
@@ -2059,10 +2236,11 @@ void osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, int 
         for (int v = s; v < p->V; v += S) order.push_back(v);
     }
     start[S] = (int)order.size();
+    if (p->yl) return yl_osem_prepare(p, x, meas, mu, S, eps, mu_key, order, start);
     const int maxsub = (p->V + S - 1) / S;
     const int D = choose_D(p, maxsub);
     const bool rebuild = !p->osem_valid || p->osem_S != S || p->osem_D != D || p->osem_has_mu != (mu != nullptr) ||
-                         p->osem_mu_key != mu_key || p->osem_eps != eps || p->osem_yl != use_yl;
+                         p->osem_mu_key != mu_key || p->osem_eps != eps;
     // mu in the YF layout is read only to build the caches (the subset loop
     // reads the cached factors), so it is packed only for a rebuild
     if (mu && rebuild) pack(p, mu, p->mu_yf);
@@ -2081,34 +2259,6 @@ void osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, int 
                                  p->st),
                   niftyrec_error_transfergpu);
         p->osem_valid = false;  // until the rebuild completes
-        if (use_yl) {
-            p->osem_mu_yf = mu_yf != nullptr;
-            yl_osem_build(p, mu_yf, S, eps, start);
-            check_hip(hipStreamSynchronize(p->st), niftyrec_error_kernel);
-            p->osem_S = S;
-            p->osem_D = D;
-            p->osem_has_mu = mu != nullptr;
-            p->osem_mu_key = mu_key;
-            p->osem_eps = eps;
-            p->osem_yl = true;
-            p->osem_valid = true;
-        }
-    }
-    if (use_yl) {
-        // measured data in subset order, transposed to [v][x][rows]
-        p->osem_meas.ensure((size_t)p->V * yl_plane_elems(p), false);
-        {
-            ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->V * p->P);
-            check_launch(et_launch_gather_planes_t(p->osem_meas.p, meas, reinterpret_cast<const int *>(p->osem_order.p),
-                                                   p->V, p->nx, p->ny, p->yu, (et_stream_t)p->st));
-        }
-        pack(p, x, p->x_yf);
-        // a single operation reallocated a buffer of the cached table
-        if (yl_osem_sig(p) != p->osem_sig) yl_osem_tables(p, S, start);
-        p->osem_start = start;
-        p->osem_cur_mu = mu_yf;
-        p->osem_cur_eps = eps;
-        return;
     }
     if (rebuild) {
         // chunking: fixed by et_plan_set_tuning, else timed on the first subset
@@ -2168,7 +2318,8 @@ void osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, int 
 void osem_subset(et_plan *p, int s)
 {
     if (p->osem_yl) {
-        yl_issue(p->osem_tables.p, p->yl_launches, 4 * (size_t)s, 4 * (size_t)s + 4, p->st, p);
+        const size_t at = 2 * (size_t)p->osem_S + 4 * (size_t)s;  // (after the sensitivities' launches)
+        yl_issue(p->osem_tables.p, p->yl_launches, at, at + 4, p->st, p);
         return;
     }
     const std::vector<int> &start = p->osem_start;
@@ -2704,7 +2855,7 @@ std::vector<const void *> batch_key(const et_batch *b, int S, float eps)
     k.push_back(reinterpret_cast<const void *>((uintptr_t)e));
     for (const et_plan *p : b->plans) {
         k.insert(k.end(), {p->x_yf.p, p->osem_meas.p, p->part.p, p->ratio.p, p->u.p, p->sens.p, p->osem_recs.p,
-                           p->osem_E.p, p->osem_cur_mu, p->d_sep.p});
+                           p->osem_E.p, p->fac.p, p->osem_cur_mu, p->d_sep.p});
         k.push_back(reinterpret_cast<const void *>((uintptr_t)(p->osem_Dp * 1024 + p->osem_Db)));
         k.push_back(reinterpret_cast<const void *>((uintptr_t)p->osem_yl));
     }
@@ -2730,6 +2881,7 @@ void batch_build(et_batch *b, int S, hipStream_t st)
     std::map<std::tuple<int, int, int, int>, std::vector<et_plan *>> ygroups;
     for (et_plan *p : ylp) ygroups[YlTable::sweep_key(p)].push_back(p);
     YlTable t;
+    t.S = S;
     b->yl_group_begin.clear();
     for (auto &g : ygroups) {
         b->yl_group_begin.push_back(t.L.size());
@@ -2738,6 +2890,7 @@ void batch_build(et_batch *b, int S, hipStream_t st)
         for (int s = 0; s < S; s++) {
             std::vector<int> v0(n), nv(n), dp(n), db(n);
             std::vector<const float *> sens(n);
+            t.sub = s;
             for (size_t i = 0; i < n; i++) {
                 const et_plan *p = gp[i];
                 v0[i] = p->osem_start[s];

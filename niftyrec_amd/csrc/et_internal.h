@@ -77,10 +77,12 @@ struct EtSweepArgs {
     float *u;                // U layout outputs
     float *att;              // attenuation factors e^{-A(x',y,z')} of the views, [V][nz][yu][nthr] with
                              // nthr = roundup(nx, 64) (the block width); see et_launch_sweep's has_mu
-                             // (row-lane kernels: [V][nz][nx][yu])
+                             // (row-lane kernels: [nz][nx][yu] per view, att_vs floats apart)
+    size_t att_vs;           // row-lane kernels
     int part_V;              // row-lane sweeps: views per depth chunk of `part` (V, or more in a view batch)
     const int *skip;         // row-lane projector: nothing to do when *skip is set (null: never)
     int yl_nbuf;             // row-lane sweeps: LDS planes (2: alternate, one barrier per plane; 1: two)
+    int yt_cols;             // tile kernels of wide or tall volumes: columns per tile
     int yl_tiles;            // row-lane projector: column tiles per plane (1: the whole width per block)
 };
 
@@ -101,6 +103,7 @@ struct EtPullArgs {
     int epilogue;            // EtEpilogue
     int accumulate;          // add the previous content of the output
     int truncate;            // clamp negatives after this launch
+    float floor;             // row-lane reference pull: the value they are clamped to (0; the sensitivity's epsilon)
     float *out;              // ABI or YF output
     int yp, gy;              // YF layout of out / x / sens
     float *x;                // ET_EPI_OSEM: activity (YF), updated in place
@@ -239,13 +242,20 @@ struct EtKeys {
 // gradient (R > 0), gx = depth chunks x tiles (tile fastest), 512 threads, NR
 // unused; pull gx = ceil(nx * nz / 16),
 // gy = 1, 256 threads.  RPL (rows per lane) in {2, 4, 6, 8}, NR (column
-// rounds) in {1, 2, 3}.
+// rounds) in {1, 2, 3}.  Tile kernels of wide or tall volumes: kinds 6
+// projection, 7 rotated-frame backprojection, 8 exact attenuation gradient, NR =
+// L the lanes per column (16; 32 with RPL 6 or 8), gx = depth chunks x tiles
+// (tile fastest), C L / 2 threads for tiles of C columns.
 // Tiled row-lane projector: columns per tile, LDS bytes of a block (two
 // planes of 64 + 2R columns of rows + 4 floats).
 #define ET_YL_TILE 64
 inline constexpr size_t et_yl_tile_lds_bytes(int R, int rows)
 {
     return (size_t)2 * (ET_YL_TILE + 2 * R) * (rows + 4) * sizeof(float);
+}
+inline constexpr size_t et_yt_plane_bytes(int cols, int R, int rows)
+{
+    return (size_t)(cols + 2 * R) * (rows + 4) * sizeof(float);
 }
 int et_launch_yl_sweep(int kind, int R, int RPL, int NR, int nthr, size_t lds, const EtSweepArgs *args,
                        const void *tab, int n, int blocks, et_stream_t stream);

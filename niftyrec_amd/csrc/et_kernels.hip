@@ -1213,7 +1213,8 @@ int et_launch_yl_pull_adj(int RPL, int nsrc, const EtPullArgs *args, const void 
 int et_launch_yl_factors(int RPL, const EtSweepArgs &a, const EtKeys &k, et_stream_t stream)
 {
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const dim3 g((a.nx + 15) / 16, a.V);
+    if (a.yu % (16 * RPL) != 0) return (int)hipErrorInvalidValue;
+    const dim3 g((a.nx + 15) / 16 * (a.yu / (16 * RPL)), a.V);
 #define ET_YLF(rpl)                                                                   \
     if (RPL == rpl) {                                                                 \
         hipLaunchKernelGGL((k_yl_factors<rpl>), g, dim3(256), 0, st, a, k);            \

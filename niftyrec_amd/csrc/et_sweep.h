@@ -598,7 +598,8 @@ static int launch_sweep_r(int mode, int has_mu, const EtSweepArgs &a, hipStream_
 
 // Row-lane sweeps (et_yl.h) of PSF radius R: kind 0 projection, 1 rotated-frame
 // backprojection, 2 tiled projection, 3 exact attenuation gradient, 4 its tiled
-// variant, 5 reference attenuation gradient; a grouped launch of `blocks` blocks of nthr = 16 * W threads
+// variant, 5 reference attenuation gradient, 6 to 8 the tile kernels of wide or
+// tall volumes; a grouped launch of `blocks` blocks of nthr = 16 * W threads
 // with `lds` bytes of dynamic LDS (two planes of the widest problem).
 // A row-lane projector launch, timed by its own dispatch (start and end
 // recorded in the events a profiling scope offered) where there is an offer.
@@ -631,6 +632,26 @@ static int launch_yl_r(int kind, int RPL, int NR, int nthr, size_t lds, const Et
             ET_YLT(2) ET_YLT(4) ET_YLT(6) ET_YLT(8)
         }
 #undef ET_YLT
+        return (int)hipErrorInvalidValue;
+    }
+    if (kind >= 6) {  // tile kernels of wide or tall volumes
+#define ET_YT(rpl, l)                                                                                             \
+        if (RPL == rpl && NR == l) {                                                                              \
+            if (kind == 6) {                                                                                      \
+                allow_lds(k_yt_project<R, rpl, l>, lds);                                                          \
+                ET_YL_PROJECTOR_LAUNCH((k_yt_project<R, rpl, l>))                                                 \
+            } else if (kind == 7) {                                                                               \
+                allow_lds(k_yt_bpu<R, rpl, l>, lds);                                                              \
+                hipLaunchKernelGGL((k_yt_bpu<R, rpl, l>), dim3(blocks), dim3(nthr), lds, st, args, tab, n);       \
+            } else {                                                                                              \
+                allow_lds(k_yt_grad<R, rpl, l>, lds);                                                             \
+                hipLaunchKernelGGL((k_yt_grad<R, rpl, l>), dim3(blocks), dim3(nthr), lds, st, args, tab, n);      \
+            }                                                                                                     \
+            return (int)hipGetLastError();                                                                        \
+        }
+        if (nthr > 32 * NR) return (int)hipErrorInvalidValue;
+        ET_YT(2, 16) ET_YT(4, 16) ET_YT(6, 16) ET_YT(8, 16) ET_YT(6, 32) ET_YT(8, 32)
+#undef ET_YT
         return (int)hipErrorInvalidValue;
     }
 #define ET_YL(rpl, nr)                                                                                            \

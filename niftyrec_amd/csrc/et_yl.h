@@ -288,7 +288,7 @@ __device__ __forceinline__ void yl_plane_factors(const EtSweepArgs &a, int v, in
         for (int r = 0; r < N; r++) {
             const int xc = col(r);
             if (xc >= 0 && xc < a.nx)
-                yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e[r]);
+                yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e[r]);
         }
     } else {
 #pragma unroll
@@ -458,7 +458,7 @@ __device__ __forceinline__ void yl_grad_body(const EtSweepArgs &a, const Blk &b)
         }
         if (d == a.D - 1 && a.bg_line != 0.f) {
             float e[RPL];
-            yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + a.nz - 1) * a.nx + xc) * rows + row0, e);
+            yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)(a.nz - 1) * a.nx + xc) * rows + row0, e);
 #pragma unroll
             for (int i = 0; i < RPL; i++) comp_add(hi[i], lo[i], a.bg_line * e[i]);
         }
@@ -495,7 +495,7 @@ __device__ __forceinline__ void yl_grad_body(const EtSweepArgs &a, const Blk &b)
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             const int xc = r * W + slot;
-            if (xc < a.nx) yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e[r]);
+            if (xc < a.nx) yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e[r]);
         }
         if constexpr (R > 0) {
             float *plane = lds + (a.yl_nbuf == 2 ? (z & 1) * PF : 0);
@@ -708,7 +708,7 @@ __device__ __forceinline__ void yl_grad_tile_body(const EtSweepArgs &a, const Bl
         }
         if (d == a.D - 1 && a.bg_line != 0.f) {
             float e[RPL];
-            yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + a.nz - 1) * a.nx + xc) * rows + row0, e);
+            yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)(a.nz - 1) * a.nx + xc) * rows + row0, e);
 #pragma unroll
             for (int i = 0; i < RPL; i++) comp_add(hi[i], lo[i], a.bg_line * e[i]);
         }
@@ -736,7 +736,7 @@ __device__ __forceinline__ void yl_grad_tile_body(const EtSweepArgs &a, const Bl
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             const int xc = col(r);
-            if (valid(xc)) yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e[r]);
+            if (valid(xc)) yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e[r]);
         }
         float *plane = lds + (z & 1) * PF;
 #pragma unroll
@@ -811,7 +811,7 @@ __device__ __forceinline__ void yl_bpu_body(const EtSweepArgs &a, const Blk &b)
                 float w[RPL];
                 if (a.att) {
                     float e[RPL];
-                    yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e);
+                    yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e);
 #pragma unroll
                     for (int i = 0; i < RPL; i++) w[i] = sv[r][i] * e[i];
                 } else {
@@ -905,7 +905,7 @@ __device__ __forceinline__ void yl_gref_body(const EtSweepArgs &a, const Blk &b)
             if (xc < a.nx) {
                 const Samp s = yl_samp_from(sb, kb * NR + r);
                 float bl[RPL], e[RPL], sv[RPL];
-                yl_load_stream<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e);
+                yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e);
                 yl_bilinear<RPL>(act + s.off, dx, dz, s, bl);
                 yl_load<RPL>(a.sino + ((size_t)v * a.nx + xc) * rows + row0, sv);  // (a cache hit after the first plane)
 #pragma unroll
@@ -939,6 +939,372 @@ __device__ __forceinline__ void yl_gref_body(const EtSweepArgs &a, const Blk &b)
             __syncthreads();  // the next plane's writes wait for these reads
         }
     }
+}
+
+// ------------------------------------------------------------------------------
+// Tile kernels of wide or tall volumes: projection, exact attenuation gradient
+// and rotated-frame backprojection on blocks (tile, d, v) that own C =
+// a.yt_cols <= 64 columns of a plane.  A column is held by L lanes of RPL rows:
+// L = 16 (a DPP row, up to 128 rows) or L = 32 (up to 256 rows, whose halo rows
+// come from the neighbour lanes by permutes, masked at the column's ends).  C / 2
+// slots of L lanes own two adjacent columns each, so the x' pass reads 2R + 2 LDS
+// columns for both instead of 2 (2R + 1), and 2R slots take one halo column
+// each; the x' pass comes first, as in the tiled projector.  Two LDS planes
+// alternate (one barrier per plane) wherever a narrower tile lets them fit: the
+// phases of a plane (gathers, x' pass, axial pass) are bound by HBM, the LDS and
+// the VALU in turn, and a single block of 16 waves with one plane runs them one
+// after another (256^3, PSF 21, 18 views: 1,056 us with one plane of 64 columns,
+// MEASURED_TWO with two of 52).
+// ------------------------------------------------------------------------------
+template <int R, int RPL, int L>
+__device__ __forceinline__ void yt_column_pass(const float *in, const float *__restrict__ kc, float *out)
+{
+    if constexpr (L == 16 || R == 0) {
+        yl_column_pass<R, RPL>(in, kc, out);
+    } else {
+        static_assert(L == 32, "lanes per column");
+        const int lane = threadIdx.x & 31, me = threadIdx.x & 63;
+        float ext[RPL + 2 * R];
+#pragma unroll
+        for (int t = 0; t < RPL; t++) ext[R + t] = in[t];
+#pragma unroll
+        for (int t = 0; t < R; t++) {
+            const int kb = (t + RPL) / RPL, ku = 1 + t / RPL;  // lanes below / above that hold the row
+            const float lo = __int_as_float(
+                __builtin_amdgcn_ds_bpermute(4 * (me - kb), __float_as_int(in[kb * RPL - (t + 1)])));
+            const float up = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (me + ku), __float_as_int(in[t % RPL])));
+            ext[R - (t + 1)] = lane >= kb ? lo : 0.f;
+            ext[R + RPL + t] = lane + ku < L ? up : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < RPL; i++) {
+            float t = 0.f;
+#pragma unroll
+            for (int j = 0; j <= 2 * R; j++) t = fmaf(ext[i + j], cload(kc + 2 * R - j), t);
+            out[i] = t;
+        }
+    }
+}
+
+// x' pass of two adjacent columns from the LDS plane: p points at the lane's
+// rows of LDS column c, which holds the first column's leftmost neighbour.
+template <int R, int RPL>
+__device__ __forceinline__ void yt_row_pass2(const float *p, int CS, const float *__restrict__ kr, float (*out)[RPL])
+{
+#pragma unroll
+    for (int i = 0; i < RPL; i++) {
+        out[0][i] = 0.f;
+        out[1][i] = 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k <= 2 * R + 1; k++) {
+        // two columns' loads at a time: the scheduler would issue every column's at
+        // once and spill (263 registers in the backprojection at R = 10)
+        if (k % 2 == 0) ET_CHUNK_FENCE();
+        float t[RPL];
+        lds_load<RPL>(p + k * CS, t);
+        if (k <= 2 * R) {
+            const float c = cload(kr + 2 * R - k);
+#pragma unroll
+            for (int i = 0; i < RPL; i++) out[0][i] = fmaf(t[i], c, out[0][i]);
+        }
+        if (k >= 1) {
+            const float c = cload(kr + 2 * R + 1 - k);
+#pragma unroll
+            for (int i = 0; i < RPL; i++) out[1][i] = fmaf(t[i], c, out[1][i]);
+        }
+    }
+}
+
+// Geometry of a tile block.
+template <int R, int RPL, int L>
+struct YtCtx {
+    static constexpr int rows = L * RPL, CS = rows + 4, NRR = R > 0 ? 3 : 2;
+    int lane, slot, d, v, x_lo, zb, ze, row0, nx, C, PF;  // PF: floats of an LDS plane
+    __device__ __forceinline__ YtCtx(const EtSweepArgs &a, const Blk &b)
+    {
+        lane = threadIdx.x & (L - 1);
+        slot = threadIdx.x / L;
+        // the tiles of one (view, depth chunk) on one XCD, as the tiled projector
+        const int T = a.yl_tiles;
+        const int2 o = xcd_order(b, T, a.D * a.V, b.x % T, b.x / T + a.D * b.y);
+        d = o.y % a.D;
+        v = o.y / a.D;
+        C = a.yt_cols;
+        PF = (C + 2 * R) * CS;
+        x_lo = o.x * C;
+        zb = d * a.zlen;
+        ze = min(a.nz, zb + a.zlen);
+        row0 = RPL * lane;
+        nx = a.nx;
+    }
+    // column of round r: the owned pair, then the halo columns (2R <= C / 2
+    // slots, the host sees to it); -1 where none
+    __device__ __forceinline__ int col(int r) const
+    {
+        if (r < 2) return x_lo + 2 * slot + r;
+        if (slot < R) return x_lo - R + slot;
+        return slot < 2 * R ? x_lo + C + slot - R : -1;
+    }
+    __device__ __forceinline__ bool valid(int xc) const { return xc >= 0 && xc < nx; }
+    // lane's rows of the LDS column of xc
+    __device__ __forceinline__ float *at(float *plane, int xc) const { return plane + (xc - x_lo + R) * CS + row0; }
+    // sample batches: lane k computes plane k / NRR, round k % NRR
+    static constexpr int PB = L / NRR;
+    __device__ __forceinline__ YlSamp batch(const EtSweepArgs &a, const FastView &fv, int z, int dir) const
+    {
+        return yl_samp_of(
+            fast_sample(fv, (float)col(lane % NRR), z + dir * (lane / NRR), a.nx, a.nz, a.yp, a.yp * a.xp));
+    }
+    __device__ __forceinline__ Samp sample(const YlSamp &h, int src) const
+    {
+        const int addr = (((int)threadIdx.x & 63 & ~(L - 1)) + src) * 4;
+        Samp s;
+        s.off = __builtin_amdgcn_ds_bpermute(addr, h.off);
+        s.w00 = __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(h.w00)));
+        s.w01 = __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(h.w01)));
+        s.w10 = __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(h.w10)));
+        s.w11 = __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(h.w11)));
+        return s;
+    }
+};
+
+// Projection (GRAD false) or exact attenuation gradient (true), as
+// yl_project_tile_body and yl_grad_tile_body.
+template <int R, int RPL, int L, bool GRAD>
+__device__ __forceinline__ void yt_project_body(const EtSweepArgs &a, const Blk &b)
+{
+    constexpr int K = 2 * R + 1;
+    typedef YtCtx<R, RPL, L> C;
+    constexpr int rows = C::rows, NRR = C::NRR;
+    extern __shared__ float lds[];
+    const C c(a, b);
+    const int dx = a.yp, dz = a.yp * a.xp, v = c.v, d = c.d, row0 = c.row0;
+    const FastView fv = load_fast_view(a.views + (size_t)v * ET_VIEW_REC);
+    if constexpr (R > 0) yl_zero_lds(lds, a.yl_nbuf * c.PF);
+    const float *act = a.act + a.gy + row0;
+    float *uv = GRAD ? a.u + (size_t)v * a.ustride + row0 : nullptr;
+
+    float acc[2][RPL], cmp[2][RPL];  // the running sum is acc - cmp
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int xc = c.col(r);
+#pragma unroll
+        for (int i = 0; i < RPL; i++) {
+            acc[r][i] = 0.f;
+            cmp[r][i] = 0.f;
+        }
+        if constexpr (GRAD) {
+            if (!c.valid(xc)) continue;
+            for (int d2 = d + 1; d2 < a.D; d2++) {  // the later chunks' sums
+                float t[RPL];
+                yl_load<RPL>(a.part + (((size_t)d2 * a.part_V + v) * a.nx + xc) * rows + row0, t);
+#pragma unroll
+                for (int i = 0; i < RPL; i++) {
+                    float lo = -cmp[r][i];
+                    comp_add(acc[r][i], lo, t[i]);
+                    cmp[r][i] = -lo;
+                }
+            }
+        }
+    }
+    auto kahan = [&](int r, int i, float h, float e) {
+        const float y = fmaf(h, e, -cmp[r][i]);
+        const float t = acc[r][i] + y;
+        cmp[r][i] = (t - acc[r][i]) - y;
+        acc[r][i] = t;
+    };
+
+    YlSamp sb;
+    int kb = 0;
+    const int n = c.ze - c.zb;
+    for (int k = 0; k < n; k++, kb = kb + 1 == C::PB ? 0 : kb + 1) {
+        const int z = GRAD ? c.ze - 1 - k : c.zb + k;
+        const float *kz = psf_plane<R>(a.psf, z);  // never read when R == 0
+        if (kb == 0)  // (planes past the chunk and absent columns give samples no round takes)
+            sb = c.batch(a, fv, z, GRAD ? -1 : 1);
+        // the owned columns' factors first (their latency passes under the gathers)
+        float e[2][RPL], h[2][RPL];
+        if (a.att) {
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+                yl_load_stream<RPL>(
+                    a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + min(c.col(r), a.nx - 1)) * rows + row0, e[r]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int i = 0; i < RPL; i++) e[r][i] = 1.f;
+        }
+        float *plane = lds + (R > 0 && a.yl_nbuf == 2 ? (z & 1) * c.PF : 0);
+#pragma unroll
+        for (int r = 0; r < NRR; r++) {
+            const int xc = c.col(r);
+            if (c.valid(xc)) {
+                const Samp s = c.sample(sb, kb * NRR + r);
+                if constexpr (R > 0) {
+                    float bl[RPL];
+                    yl_bilinear<RPL>(act + s.off, dx, dz, s, bl);
+                    lds_store<RPL>(c.at(plane, xc), bl);
+                } else {
+                    yl_bilinear<RPL>(act + s.off, dx, dz, s, h[r]);
+                }
+            }
+        }
+        if constexpr (R > 0) __syncthreads();
+        if (c.valid(c.col(0))) {
+            if constexpr (R > 0) {
+                float t[2][RPL];
+                yt_row_pass2<R, RPL>(plane + 2 * c.slot * C::CS + row0, C::CS, kz, t);
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    ET_CHUNK_FENCE();
+                    yt_column_pass<R, RPL, L>(t[r], kz + K, h[r]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+#pragma unroll
+                for (int i = 0; i < RPL; i++) kahan(r, i, h[r][i], e[r][i]);
+                if constexpr (GRAD) {
+                    if (r == 1 && !c.valid(c.col(1))) continue;
+                    // s is read again at every plane (a cache hit) rather than held in registers
+                    float sv[RPL], out[RPL];
+                    yl_load<RPL>(a.sino + ((size_t)v * a.nx + c.col(r)) * rows + row0, sv);
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) out[i] = -sv[i] * (acc[r][i] - cmp[r][i]);
+                    yl_store_stream<RPL>(uv + (size_t)rows * ((c.col(r) + 1) + (size_t)a.xp * (z + 1)), out);
+                }
+            }
+        }
+        if constexpr (R > 0)
+            if (a.yl_nbuf == 1) __syncthreads();  // one plane: the next writes wait for these reads
+    }
+    if constexpr (!GRAD) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int xc = c.col(r);
+            if (!c.valid(xc)) continue;
+            float out[RPL];
+#pragma unroll
+            for (int i = 0; i < RPL; i++) out[i] = acc[r][i] - cmp[r][i];
+            yl_store<RPL>(a.part + (((size_t)d * a.part_V + v) * a.nx + xc) * rows + row0, out);
+        }
+    }
+}
+
+// Rotated-frame backprojection, as yl_bpu_body: the halo columns' factors are
+// read as well (cache hits of the neighbour tile's, on the same XCD).
+template <int R, int RPL, int L>
+__device__ __forceinline__ void yt_bpu_body(const EtSweepArgs &a, const Blk &b)
+{
+    constexpr int K = 2 * R + 1;
+    typedef YtCtx<R, RPL, L> C;
+    constexpr int rows = C::rows, NRR = C::NRR;
+    extern __shared__ float lds[];
+    const C c(a, b);
+    const int v = c.v, row0 = c.row0;
+    if constexpr (R > 0) yl_zero_lds(lds, a.yl_nbuf * c.PF);
+    float sv[NRR][RPL];
+#pragma unroll
+    for (int r = 0; r < NRR; r++) {
+        const int xc = c.col(r);
+        if (!c.valid(xc)) continue;
+        if (a.src == ET_SRC_ONES) {
+#pragma unroll
+            for (int i = 0; i < RPL; i++) sv[r][i] = (row0 + i < a.ny) ? 1.f : 0.f;
+        } else {
+            yl_load<RPL>(a.sino + ((size_t)v * a.nx + xc) * rows + row0, sv[r]);
+        }
+    }
+    float *uv = a.u + (size_t)v * a.ustride + row0;
+    // a plane's factors are loaded while the plane before it is convolved
+    float e[NRR][RPL];
+    auto load = [&](int z) {
+        if (!a.att) return;
+#pragma unroll
+        for (int r = 0; r < NRR; r++) {
+            const int xc = c.col(r);
+            if (c.valid(xc))
+                yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e[r]);
+        }
+    };
+    load(c.zb);
+    for (int z = c.zb; z < c.ze; z++) {
+        const float *kz = psf_plane<R>(a.psf, z);  // never read when R == 0
+        float *plane = lds + (R > 0 && a.yl_nbuf == 2 ? (z & 1) * c.PF : 0);
+#pragma unroll
+        for (int r = 0; r < NRR; r++) {
+            const int xc = c.col(r);
+            if (c.valid(xc)) {
+                float w[RPL];
+                if (a.att) {
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) w[i] = sv[r][i] * e[r][i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) w[i] = sv[r][i];
+                }
+                if constexpr (R > 0)
+                    lds_store<RPL>(c.at(plane, xc), w);
+                else
+                    yl_store<RPL>(uv + (size_t)rows * ((xc + 1) + (size_t)a.xp * (z + 1)), w);
+            }
+        }
+        if (z + 1 < c.ze) load(z + 1);
+        if constexpr (R > 0) {
+            __syncthreads();
+            if (c.valid(c.col(0))) {
+                float t[2][RPL];
+                yt_row_pass2<R, RPL>(plane + 2 * c.slot * C::CS + row0, C::CS, kz, t);
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    // (a branch around the second pass made the compiler keep both
+                    // columns' halos: 225 spilled registers at R = 10)
+                    float o[RPL];
+                    ET_CHUNK_FENCE();
+                    yt_column_pass<R, RPL, L>(t[r], kz + K, o);
+                    if (c.valid(c.col(r)))
+                        yl_store<RPL>(uv + (size_t)rows * ((c.col(r) + 1) + (size_t)a.xp * (z + 1)), o);
+                }
+            }
+            if (a.yl_nbuf == 1) __syncthreads();  // one plane: the next writes wait for these reads
+        }
+    }
+}
+
+template <int R, int RPL, int L>
+__global__ void __launch_bounds__(32 * L, 4) k_yt_project(const EtSweepArgs *__restrict__ args,
+                                                       const int4 *__restrict__ tab, int n)
+{
+    Blk b;
+    int j;
+    if (!group_block(tab, n, b, j)) return;
+    const EtSweepArgs a = ((ET_CONST_AS const EtSweepArgs *)args)[j];
+    if (a.skip && *a.skip) return;
+    yt_project_body<R, RPL, L, false>(a, b);
+}
+
+template <int R, int RPL, int L>
+__global__ void __launch_bounds__(32 * L, 4) k_yt_grad(const EtSweepArgs *__restrict__ args,
+                                                    const int4 *__restrict__ tab, int n)
+{
+    Blk b;
+    int j;
+    if (!group_block(tab, n, b, j)) return;
+    const EtSweepArgs a = ((ET_CONST_AS const EtSweepArgs *)args)[j];
+    yt_project_body<R, RPL, L, true>(a, b);
+}
+
+template <int R, int RPL, int L>
+__global__ void __launch_bounds__(32 * L, 4) k_yt_bpu(const EtSweepArgs *__restrict__ args,
+                                                   const int4 *__restrict__ tab, int n)
+{
+    Blk b;
+    int j;
+    if (!group_block(tab, n, b, j)) return;
+    const EtSweepArgs a = ((ET_CONST_AS const EtSweepArgs *)args)[j];
+    yt_bpu_body<R, RPL, L>(a, b);
 }
 
 template <int R, int RPL, int NR>
@@ -1020,16 +1386,18 @@ __global__ void __launch_bounds__(1024) k_yl_bpu(const EtSweepArgs *__restrict__
 // Attenuation factors of every view (no PSF): att[v][z'][x'][rows] =
 // e^{-A(x', y, z')}, A the inclusive sum along depth of the resampled mu,
 // accumulated as a compensated (hi, lo) pair.  Block: 16 columns of one view,
-// all planes.  grid (ceil(nx / 16), V), 256 threads.
+// all planes, one run of 16 RPL rows.  grid (ceil(nx / 16) x rows / (16 RPL), V),
+// 256 threads.
 // ------------------------------------------------------------------------------
 template <int RPL>
 __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
 {
     const int lane = threadIdx.x & 15, slot = threadIdx.x >> 4;
-    const int xc = blockIdx.x * 16 + slot, v = blockIdx.y;
+    const int ncb = (a.nx + 15) >> 4, half = (int)blockIdx.x / ncb;  // (columns of 32 RPL rows: two row halves)
+    const int xc = ((int)blockIdx.x - half * ncb) * 16 + slot, v = blockIdx.y;
     if (xc >= a.nx) return;  // the whole 16-lane row
-    constexpr int rows = 16 * RPL;  // == a.yu
-    const int row0 = RPL * lane;
+    const int rows = a.yu;
+    const int row0 = RPL * (lane + 16 * half);
     const int dx = a.yp, dz = a.yp * a.xp;
     const FastView fv = load_fast_view(a.views + (size_t)v * ET_VIEW_REC);
     const float *mu = a.mu + a.gmu + row0;
@@ -1048,7 +1416,7 @@ __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
             comp_add(A[i], Al[i], m[i]);
             e[i] = exp_neg(A[i] + Al[i]);
         }
-        yl_store<RPL>(a.att + (((size_t)v * a.nz + z) * a.nx + xc) * rows + row0, e);
+        yl_store<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e);
     }
 }
 
@@ -1093,19 +1461,22 @@ __global__ void __launch_bounds__(256) k_yl_factors(EtSweepArgs a, EtKeys k)
 // columns (x, z), x fastest; tiles numbered in 8 x 8-tile super-tiles (x-major
 // within and between them), contiguous per XCD, so that an XCD covers a
 // compact image region (32 x 32 columns per super-tile).  256 threads; grid
-// 64 * ceil(nx/32) * ceil(nz/32), blocks past the image exit at once.
+// 64 * ceil(nx/32) * ceil(nz/32) * rows / (16 RPL), blocks past the image exit at
+// once.
 // ------------------------------------------------------------------------------
 template <int RPL, int EPI>
 __device__ __forceinline__ void yl_pull_body(const EtPullArgs &a, const Blk &b)
 {
     const int lane = threadIdx.x & 15, slot = threadIdx.x >> 4;
-    const int cb = ((b.gx & 7) == 0) ? (b.lin & 7) * (b.gx >> 3) + (b.lin >> 3) : b.lin;
+    int cb = ((b.gx & 7) == 0) ? (b.lin & 7) * (b.gx >> 3) + (b.lin >> 3) : b.lin;
     const int ntx = (a.nx + 3) >> 2, nsx = (ntx + 7) >> 3;
+    const int tiles = nsx * ((((a.nz + 3) >> 2) + 7) >> 3) * 64, half = cb / tiles;  // (two row halves above 128 rows)
+    cb -= half * tiles;
     const int sup = cb >> 6, t = cb & 63;
     const int x = ((sup % nsx) * 8 + (t & 7)) * 4 + (slot & 3), z = ((sup / nsx) * 8 + (t >> 3)) * 4 + (slot >> 2);
     if (x >= a.nx || z >= a.nz) return;
-    constexpr int rows = 16 * RPL;  // == a.yu
-    const int row0 = RPL * lane;
+    const int rows = a.yu;
+    const int row0 = RPL * (lane + 16 * half);
     const int dx = rows, dz = rows * a.xp;
     float acc[RPL];
 #pragma unroll
@@ -1145,7 +1516,7 @@ __device__ __forceinline__ void yl_pull_body(const EtPullArgs &a, const Blk &b)
 #pragma unroll
         for (int i = 0; i < RPL; i++) {
             float val = a.accumulate ? ov[i] + acc[i] : acc[i];
-            if (a.truncate && val < 0.f) val = 0.f;
+            if (a.truncate && val < a.floor) val = a.floor;
             o[i] = (row0 + i < a.ny) ? val : ov[i];
         }
         yl_store<RPL>(a.out + base, o);
@@ -1175,13 +1546,15 @@ __device__ __forceinline__ void yl_pull_adj_body(const EtPullArgs &a, const Blk 
     static_assert(NS == 1 || NS == 2, "one or two volumes");
     constexpr int HB = 4 / NS;  // hits per batch
     const int lane = threadIdx.x & 15, slot = threadIdx.x >> 4;
-    const int cb = ((b.gx & 7) == 0) ? (b.lin & 7) * (b.gx >> 3) + (b.lin >> 3) : b.lin;
+    int cb = ((b.gx & 7) == 0) ? (b.lin & 7) * (b.gx >> 3) + (b.lin >> 3) : b.lin;
     const int ntx = (a.nx + 3) >> 2, nsx = (ntx + 7) >> 3;
+    const int tiles = nsx * ((((a.nz + 3) >> 2) + 7) >> 3) * 64, half = cb / tiles;  // (two row halves above 128 rows)
+    cb -= half * tiles;
     const int sup = cb >> 6, t = cb & 63;
     const int x = ((sup % nsx) * 8 + (t & 7)) * 4 + (slot & 3), z = ((sup / nsx) * 8 + (t >> 3)) * 4 + (slot >> 2);
     if (x >= a.nx || z >= a.nz) return;  // (the whole 16-lane row)
-    constexpr int rows = 16 * RPL;  // == a.yu
-    const int row0 = RPL * lane;
+    const int rows = a.yu;
+    const int row0 = RPL * (lane + 16 * half);
     const float fxo = (float)x, fzo = (float)z;
     __shared__ float hit_w[16][16];  // per row: the weights and offsets of its non-zero candidates
     __shared__ int hit_o[16][16];
