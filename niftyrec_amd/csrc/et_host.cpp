@@ -286,6 +286,7 @@ struct et_plan {
     // backprojection, exact attenuation gradient with attenuation): factors of
     // every view in view order, cached on the attenuation map's key
     bool yl_ops = false;
+    bool yl_osem = false;                 // OSEM on the row-lane kernels
     DevBuf fac, sino_t, op_acc, op_acc2;  // (op_acc, op_acc2: pull accumulators, YF layout)
     DevBuf op_tables[YL_OP_SLOTS];        // per operation: its last table, and that table's bytes
     std::vector<char> op_tables_h[YL_OP_SLOTS];
@@ -458,6 +459,12 @@ int build_plan(et_plan *p, int nx, int ny, int nz, const Cameras &cams, const fl
         }
         if (!p->yl) yt_plan(p);
     }
+    // OSEM on tall plans: the tile kernels move and convolve the rows that pad a
+    // column to 32 lanes; below 7/8 real rows the sweep kernels (16-row slabs) are
+    // faster (PSF 11, 30 views of 128 columns, 4 subsets: 190 of 192 rows 1,133 us
+    // against 1,236, 240 of 256 1,471 / 1,524, 216 of 256 1,470 / 1,394, 140 of 192
+    // 1,133 / 915).  The single operations, on cached factors, gain at any height.
+    p->yl_osem = p->yl && !(p->yt_L == 32 && 8 * ny < 7 * 32 * p->yl_rpl);
     const int yrows = p->yl ? (p->yt_L ? p->yt_L : 16) * p->yl_rpl : p->slabs * ET_T;  // axial rows held per column
     // YF layout.  Guard rows: the activity-like volumes are gathered in windows
     // of rows y0 - R4 .. y0 + TS + R4 - 1 (R4 = R rounded up to 4); with R4
@@ -1793,7 +1800,7 @@ int yl_gradient_batch(const et_plan *p)
 // Depth chunks of the projection of every view (the forward sums' chunking, which
 // the gradient sweeps share).  The blocks of a tall plan have a CU to themselves,
 // so a launch of a few blocks per CU ends in a nearly empty round (256^3, 63
-// views, PSF 21, gradient sweep: 320 blocks in one chunk 5.6 ms, MEASURED_GRAD in
+// views, PSF 21, gradient sweep: 320 blocks in one chunk 5.6 ms, 4.0 ms in
 // eight); its chunks, of at least 16 planes, give eight per CU.
 int yl_forward_chunks(const et_plan *p, bool mu)
 {
@@ -2236,7 +2243,7 @@ void osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, int 
         for (int v = s; v < p->V; v += S) order.push_back(v);
     }
     start[S] = (int)order.size();
-    if (p->yl) return yl_osem_prepare(p, x, meas, mu, S, eps, mu_key, order, start);
+    if (p->yl_osem) return yl_osem_prepare(p, x, meas, mu, S, eps, mu_key, order, start);
     const int maxsub = (p->V + S - 1) / S;
     const int D = choose_D(p, maxsub);
     const bool rebuild = !p->osem_valid || p->osem_S != S || p->osem_D != D || p->osem_has_mu != (mu != nullptr) ||

@@ -954,7 +954,7 @@ __device__ __forceinline__ void yl_gref_body(const EtSweepArgs &a, const Blk &b)
 // phases of a plane (gathers, x' pass, axial pass) are bound by HBM, the LDS and
 // the VALU in turn, and a single block of 16 waves with one plane runs them one
 // after another (256^3, PSF 21, 18 views: 1,056 us with one plane of 64 columns,
-// MEASURED_TWO with two of 52).
+// 838 us with two of 52; the sweep kernel 926 us).
 // ------------------------------------------------------------------------------
 template <int R, int RPL, int L>
 __device__ __forceinline__ void yt_column_pass(const float *in, const float *__restrict__ kc, float *out)
@@ -1047,6 +1047,18 @@ struct YtCtx {
         return slot < 2 * R ? x_lo + C + slot - R : -1;
     }
     __device__ __forceinline__ bool valid(int xc) const { return xc >= 0 && xc < nx; }
+    // Zeroes the LDS columns of every plane that lie outside the volume; the
+    // others are written at every plane.  (Clearing whole planes, up to 150 KB a
+    // block, cost as much as two planes' work.)
+    __device__ __forceinline__ void zero_outside(float *lds, int planes) const
+    {
+        const int lo = max(0, R - x_lo), hi = max(lo, min(C + 2 * R, nx - x_lo + R));
+        for (int p = 0; p < planes; p++)
+            for (int k = 4 * (int)threadIdx.x; k < PF; k += 4 * (int)blockDim.x)
+                if (k < lo * CS || k >= hi * CS)
+                    *reinterpret_cast<float4 *>(lds + p * PF + k) = make_float4(0.f, 0.f, 0.f, 0.f);
+        __syncthreads();
+    }
     // lane's rows of the LDS column of xc
     __device__ __forceinline__ float *at(float *plane, int xc) const { return plane + (xc - x_lo + R) * CS + row0; }
     // sample batches: lane k computes plane k / NRR, round k % NRR
@@ -1081,7 +1093,7 @@ __device__ __forceinline__ void yt_project_body(const EtSweepArgs &a, const Blk 
     const C c(a, b);
     const int dx = a.yp, dz = a.yp * a.xp, v = c.v, d = c.d, row0 = c.row0;
     const FastView fv = load_fast_view(a.views + (size_t)v * ET_VIEW_REC);
-    if constexpr (R > 0) yl_zero_lds(lds, a.yl_nbuf * c.PF);
+    if constexpr (R > 0) c.zero_outside(lds, a.yl_nbuf);
     const float *act = a.act + a.gy + row0;
     float *uv = GRAD ? a.u + (size_t)v * a.ustride + row0 : nullptr;
 
@@ -1194,7 +1206,8 @@ __device__ __forceinline__ void yt_project_body(const EtSweepArgs &a, const Blk 
 }
 
 // Rotated-frame backprojection, as yl_bpu_body: the halo columns' factors are
-// read as well (cache hits of the neighbour tile's, on the same XCD).
+// read as well, with cached loads (the neighbour tile, on the same XCD, reads
+// them too: 782 us per 18 views at 256^3, PSF 21, against 806 us streamed).
 template <int R, int RPL, int L>
 __device__ __forceinline__ void yt_bpu_body(const EtSweepArgs &a, const Blk &b)
 {
@@ -1204,7 +1217,7 @@ __device__ __forceinline__ void yt_bpu_body(const EtSweepArgs &a, const Blk &b)
     extern __shared__ float lds[];
     const C c(a, b);
     const int v = c.v, row0 = c.row0;
-    if constexpr (R > 0) yl_zero_lds(lds, a.yl_nbuf * c.PF);
+    if constexpr (R > 0) c.zero_outside(lds, a.yl_nbuf);
     float sv[NRR][RPL];
 #pragma unroll
     for (int r = 0; r < NRR; r++) {
@@ -1226,7 +1239,7 @@ __device__ __forceinline__ void yt_bpu_body(const EtSweepArgs &a, const Blk &b)
         for (int r = 0; r < NRR; r++) {
             const int xc = c.col(r);
             if (c.valid(xc))
-                yl_load_stream<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e[r]);
+                yl_load<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e[r]);
         }
     };
     load(c.zb);

@@ -2,7 +2,7 @@
 kernels: projection, both backprojections, the exact gradients and ordered
 subsets against the oracle, at the edges of the tiles, of the rows a column's
 lanes hold and of the halo (the permutes across a column's lanes), with and
-without attenuation; and the sizes the sweep kernels keep."""
+without attenuation; and the sizes whose OSEM the sweep kernels keep (0 tiles)."""
 import numpy as np
 import pytest
 
@@ -20,8 +20,8 @@ def _t(a):
 
 
 @pytest.mark.parametrize("shape, V, K, attenuated, tiles", [
-    ((65, 129, 65), 3, 21, True, 2), ((70, 192, 70), 3, 7, True, 2), ((66, 193, 66), 2, 0, True, 2),
-    ((129, 256, 129), 2, 17, True, 3), ((72, 140, 72), 3, 19, False, 2), ((193, 17, 193), 2, 21, True, 4),
+    ((65, 129, 65), 3, 21, True, 0), ((70, 192, 70), 3, 7, True, 2), ((66, 193, 66), 2, 0, True, 0),
+    ((129, 256, 129), 2, 17, True, 3), ((72, 168, 72), 3, 19, False, 2), ((72, 167, 72), 3, 19, False, 0), ((193, 17, 193), 2, 21, True, 4),
     ((200, 33, 200), 2, 0, False, 4), ((257, 65, 257), 2, 5, True, 5), ((194, 128, 194), 2, 11, True, 4),
     ((64, 129, 64), 2, 5, True, 0), ((200, 16, 200), 2, 3, True, 0), ((70, 257, 70), 2, 3, True, 0)])
 def test_wide_and_tall_plans(shape, V, K, attenuated, tiles):
@@ -70,7 +70,7 @@ def test_osem_with_maps_that_change():
     operation with the other map in between, another epsilon, then the first
     map again, each bit-identical to a fresh plan's with the same chunking."""
     from niftyrec_amd.api import Plan
-    shape, V = (72, 130, 72), 6
+    shape, V = (72, 180, 72), 6
     gen = torch.Generator(device="cuda").manual_seed(9)
     rand = lambda *s: torch.rand(s, device="cuda", generator=gen)  # noqa: E731
     cams = np.linspace(0, 5, V).astype(np.float32)
