@@ -235,6 +235,7 @@ enum {
     YL_PROJECT = 0, YL_RATIO = 1, YL_BPU = 2, YL_PULL_OSEM = 3, YL_PULL_STORE = 4, YL_GRAD = 5, YL_PULL_ADJ = 6,
     YL_PULL_ADJ2 = 7,  // exact adjoint pull of two volumes (u, u2) into two outputs
     YL_GREF = 8,       // reference attenuation gradient
+    YL_PROJECT_IF = 9, // projection that the device may skip
 };
 // Table slots of the single operations (each keeps its last upload).
 enum {
@@ -1443,7 +1444,8 @@ struct YlTable {
                 bt.add(gx, gy);
                 const et_plan *q = plans[i];
                 // tiled projector (key NR 0, R > 0), full-width sweeps, backprojection
-                const bool tiled = (kind == YL_PROJECT || kind == YL_GRAD) && std::get<2>(g.first) == 0 && q->R > 0;
+                const bool tiled = (kind == YL_PROJECT || kind == YL_PROJECT_IF || kind == YL_GRAD) &&
+                                   std::get<2>(g.first) == 0 && q->R > 0;
                 if (std::get<0>(g.first) > 0)  // (no PSF: no LDS plane)
                     lds = std::max(lds, kind == YL_BPU || kind == YL_GREF ? q->yl_lds_bpu
                                                                           : (tiled ? q->yl_lds_tile : q->yl_lds_full));
@@ -1558,17 +1560,19 @@ void yl_issue(const float *dev, const std::vector<YlLaunch> &L, size_t from, siz
         const et_stream_t s = (et_stream_t)st;
         switch (l.kind) {
         case YL_PROJECT:
+        case YL_PROJECT_IF:
         case YL_BPU:
         case YL_GRAD:
         case YL_GREF: {
-            ProfScope ps(prof, l.kind == YL_PROJECT ? ET_PROF_PROJECT : (l.kind == YL_BPU ? ET_PROF_BPU : ET_PROF_GRAD),
-                         l.bytes);
-            const int k = l.NR < 0 ? (l.kind == YL_PROJECT ? 6 : (l.kind == YL_BPU ? 7 : 8))
+            const bool project = l.kind == YL_PROJECT || l.kind == YL_PROJECT_IF;
+            ProfScope ps(prof, project ? ET_PROF_PROJECT : (l.kind == YL_BPU ? ET_PROF_BPU : ET_PROF_GRAD), l.bytes);
+            const int k = l.NR < 0 ? (project ? 6 : (l.kind == YL_BPU ? 7 : 8))
                           : l.kind == YL_BPU ? 1
                           : l.kind == YL_GREF ? 5
                                               : (l.kind == YL_GRAD ? (l.NR == 0 ? 4 : 3) : (l.NR == 0 ? 2 : 0));
-            check_launch(et_launch_yl_sweep(k, l.R, l.RPL, std::abs(l.NR), l.nthr, l.lds, static_cast<const EtSweepArgs *>(args),
-                                            tab, l.n, l.blocks, s));
+            check_launch(et_launch_yl_sweep(k + (l.kind == YL_PROJECT_IF ? ET_YL_COND : 0), l.R, l.RPL,
+                                            std::abs(l.NR), l.nthr, l.lds, static_cast<const EtSweepArgs *>(args), tab,
+                                            l.n, l.blocks, s));
             break;
         }
         case YL_RATIO: {
@@ -1772,7 +1776,8 @@ float *yl_forward(YlTable &t, et_plan *p, const float *fac, int D, const int *sk
     int Deff, zlen;
     yl_chunks(p, D, Deff, zlen);
     float *part = p->fwd_part.ensure((size_t)Deff * p->V * yl_plane_elems(p), false);
-    t.grouped<EtSweepArgs>(YL_PROJECT, {p}, YlTable::project_key, [&](int, int &gx, int &gy, double &bytes) {
+    t.grouped<EtSweepArgs>(skip ? YL_PROJECT_IF : YL_PROJECT, {p}, YlTable::project_key,
+                           [&](int, int &gx, int &gy, double &bytes) {
         bytes += (double)p->V * ((fac ? 8.0 : 4.0) * p->nvox + 4.0 * p->P);
         EtSweepArgs a = yl_sweep_args(p, p->d_recs.p, p->V, D, fac);
         a.act = p->act_yf.p;

@@ -80,7 +80,7 @@ struct EtSweepArgs {
                              // (row-lane kernels: [nz][nx][yu] per view, att_vs floats apart)
     size_t att_vs;           // row-lane kernels
     int part_V;              // row-lane sweeps: views per depth chunk of `part` (V, or more in a view batch)
-    const int *skip;         // row-lane projector: nothing to do when *skip is set (null: never)
+    const int *skip;         // conditional row-lane projection: nothing to do when *skip is set
     int yl_nbuf;             // row-lane sweeps: LDS planes (2: alternate, one barrier per plane; 1: two)
     int yt_cols;             // tile kernels of wide or tall volumes: columns per tile
     int yl_tiles;            // row-lane projector: column tiles per plane (1: the whole width per block)
@@ -245,7 +245,9 @@ struct EtKeys {
 // rounds) in {1, 2, 3}.  Tile kernels of wide or tall volumes: kinds 6
 // projection, 7 rotated-frame backprojection, 8 exact attenuation gradient, NR =
 // L the lanes per column (16; 32 with RPL 6 or 8), gx = depth chunks x tiles
-// (tile fastest), C L / 2 threads for tiles of C columns.
+// (tile fastest), C L / 2 threads for tiles of C columns.  A projection kind +
+// ET_YL_COND: not done where the record's *skip is set.
+#define ET_YL_COND 16
 // Tiled row-lane projector: columns per tile, LDS bytes of a block (two
 // planes of 64 + 2R columns of rows + 4 floats).
 #define ET_YL_TILE 64

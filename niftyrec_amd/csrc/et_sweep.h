@@ -616,10 +616,15 @@ template <int R>
 static int launch_yl_r(int kind, int RPL, int NR, int nthr, size_t lds, const EtSweepArgs *args, const int4 *tab,
                        int n, int blocks, hipStream_t st)
 {
+    const bool cond = kind >= ET_YL_COND;  // a projection that the device may skip
+    if (cond) kind -= ET_YL_COND;
     if (kind == 2 || kind == 4) {  // tiled projector, tiled attenuation gradient (R > 0)
 #define ET_YLT(rpl)                                                                                               \
         if (RPL == rpl) {                                                                                         \
-            if (kind == 2) {                                                                                      \
+            if (cond) {                                                                                           \
+                allow_lds(k_yl_project_tile_if<R, rpl>, lds);                                                     \
+                ET_YL_PROJECTOR_LAUNCH((k_yl_project_tile_if<R, rpl>))                                            \
+            } else if (kind == 2) {                                                                               \
                 allow_lds(k_yl_project_tile<R, rpl>, lds);                                                        \
                 ET_YL_PROJECTOR_LAUNCH((k_yl_project_tile<R, rpl>))                                               \
             } else {                                                                                              \
@@ -637,7 +642,10 @@ static int launch_yl_r(int kind, int RPL, int NR, int nthr, size_t lds, const Et
     if (kind >= 6) {  // tile kernels of wide or tall volumes
 #define ET_YT(rpl, l)                                                                                             \
         if (RPL == rpl && NR == l) {                                                                              \
-            if (kind == 6) {                                                                                      \
+            if (cond) {                                                                                           \
+                allow_lds(k_yt_project_if<R, rpl, l>, lds);                                                       \
+                ET_YL_PROJECTOR_LAUNCH((k_yt_project_if<R, rpl, l>))                                              \
+            } else if (kind == 6) {                                                                               \
                 allow_lds(k_yt_project<R, rpl, l>, lds);                                                          \
                 ET_YL_PROJECTOR_LAUNCH((k_yt_project<R, rpl, l>))                                                 \
             } else if (kind == 7) {                                                                               \
@@ -656,7 +664,10 @@ static int launch_yl_r(int kind, int RPL, int NR, int nthr, size_t lds, const Et
     }
 #define ET_YL(rpl, nr)                                                                                            \
     if (RPL == rpl && NR == nr) {                                                                                 \
-        if (kind == 0) {                                                                                          \
+        if (cond) {                                                                                               \
+            allow_lds(k_yl_project_if<R, rpl, nr>, lds);                                                          \
+            ET_YL_PROJECTOR_LAUNCH((k_yl_project_if<R, rpl, nr>))                                                 \
+        } else if (kind == 0) {                                                                                   \
             allow_lds(k_yl_project<R, rpl, nr>, lds);                                                             \
             ET_YL_PROJECTOR_LAUNCH((k_yl_project<R, rpl, nr>))                                                    \
         } else if (kind == 3) {                                                                                   \
