@@ -1782,6 +1782,7 @@ float *yl_forward(YlTable &t, et_plan *p, const float *fac, int D, const int *sk
         EtSweepArgs a = yl_sweep_args(p, p->d_recs.p, p->V, D, fac);
         a.act = p->act_yf.p;
         a.part = part;
+        a.near_views = 1;
         a.skip = skip;
         gx = a.D * p->yl_tiles;
         gy = p->V;
@@ -1901,6 +1902,7 @@ void yl_gradient_sweep(YlTable &t, et_plan *p, int v0, int nv, const float *fac,
         a.act = p->act_yf.p;
         a.part = part + (size_t)v0 * yl_plane_elems(p);
         a.part_V = p->V;
+        a.near_views = 1;
         a.sino = st + (size_t)v0 * yl_plane_elems(p);
         a.u = u;
         gx = a.D * p->yl_tiles;

@@ -82,6 +82,7 @@ struct EtSweepArgs {
     int part_V;              // row-lane sweeps: views per depth chunk of `part` (V, or more in a view batch)
     const int *skip;         // conditional row-lane projection: nothing to do when *skip is set
     int yl_nbuf;             // row-lane sweeps: LDS planes (2: alternate, one barrier per plane; 1: two)
+    int near_views;          // tiled row-lane sweeps: the views are in order (neighbouring angles), see yl_block_order
     int yt_cols;             // tile kernels of wide or tall volumes: columns per tile
     int yl_tiles;            // row-lane projector: column tiles per plane (1: the whole width per block)
 };

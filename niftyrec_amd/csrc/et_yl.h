@@ -554,6 +554,13 @@ __device__ __forceinline__ void yl_grad_body(const EtSweepArgs &a, const Blk &b)
 // ------------------------------------------------------------------------------
 #define YL_TILE ET_YL_TILE
 
+// (tile, chunk + D view) of a tiled block.
+__device__ __forceinline__ int2 yl_block_order(const EtSweepArgs &a, const Blk &b, int T)
+{
+    const int tile = b.x % T, slow = b.x / T + a.D * b.y;
+    return a.near_views ? xcd_order_contig(b, T, a.D * a.V, tile, slow) : xcd_order(b, T, a.D * a.V, tile, slow);
+}
+
 template <int R, int RPL>
 __device__ __forceinline__ void yl_project_tile_body(const EtSweepArgs &a, const Blk &b)
 {
@@ -564,7 +571,7 @@ __device__ __forceinline__ void yl_project_tile_body(const EtSweepArgs &a, const
     // the T tiles of one (view, depth chunk) on one XCD, dispatched together:
     // each tile's halo columns are the neighbour's owned columns, in the same L2
     const int T = a.yl_tiles;
-    const int2 o = xcd_order(b, T, a.D * a.V, b.x % T, b.x / T + a.D * b.y);
+    const int2 o = yl_block_order(a, b, T);
     const int tile = o.x, d = o.y % a.D, v = o.y / a.D;
     const int x_lo = tile * YL_TILE;
     const int zb = d * a.zlen, ze = min(a.nz, zb + a.zlen);
@@ -665,7 +672,7 @@ __device__ __forceinline__ void yl_grad_tile_body(const EtSweepArgs &a, const Bl
     extern __shared__ float lds[];
     const int lane = threadIdx.x & 15, slot = threadIdx.x >> 4;
     const int T = a.yl_tiles;
-    const int2 o = xcd_order(b, T, a.D * a.V, b.x % T, b.x / T + a.D * b.y);
+    const int2 o = yl_block_order(a, b, T);
     const int tile = o.x, d = o.y % a.D, v = o.y / a.D;
     const int x_lo = tile * YL_TILE;
     const int zb = d * a.zlen, ze = min(a.nz, zb + a.zlen);
@@ -1027,7 +1034,7 @@ struct YtCtx {
         slot = threadIdx.x / L;
         // the tiles of one (view, depth chunk) on one XCD, as the tiled projector
         const int T = a.yl_tiles;
-        const int2 o = xcd_order(b, T, a.D * a.V, b.x % T, b.x / T + a.D * b.y);
+        const int2 o = yl_block_order(a, b, T);
         d = o.y % a.D;
         v = o.y / a.D;
         C = a.yt_cols;
