@@ -1685,8 +1685,9 @@ const float *yl_sources(et_plan *p, const float *act, const float *mu, int fwd)
     p->fac.ensure(yl_att_elems(p, p->V), false);
     EtSweepArgs f = yl_sweep_args(p, p->d_recs.p, p->V, 1, p->fac.p);
     f.mu = p->mu_yf.p;
+    const bool stream_out = yl_att_elems(p, p->V) * sizeof(float) > (256ull << 20);  // (the Infinity Cache)
     ProfScope ps(p, ET_PROF_OTHER, (double)p->V * 8.0 * p->nvox);
-    check_launch(et_launch_yl_factors(p->yl_rpl, f, k, (et_stream_t)p->st));
+    check_launch(et_launch_yl_factors(p->yl_rpl, stream_out, f, k, (et_stream_t)p->st));
     p->fac_built = true;
     p->key_gen++;
     return p->fac.p;

@@ -274,7 +274,8 @@ int et_launch_yl_pull_adj(int RPL, int nsrc, const EtPullArgs *args, const void 
                           et_stream_t stream);
 // Attenuation factors of a.V views into a.att (row-lane layout) from a.mu (YF);
 // with keys (st not null): only if the map is another one than the factors' own.
-int et_launch_yl_factors(int RPL, const EtSweepArgs &a, const EtKeys &k, et_stream_t stream);
+// stream_out: store past the caches (factors larger than they are).
+int et_launch_yl_factors(int RPL, bool stream_out, const EtSweepArgs &a, const EtKeys &k, et_stream_t stream);
 // sino[v][y][x] = sum over d < D of part[d][v][x][y] (compensated), truncated
 // at 0 if asked: row-lane partial sums (V views, rows per column) in the ABI layout.
 int et_launch_yl_parts_to_sino(const float *part, int D, int V, int nx, int ny, int rows, int truncate, float *sino,

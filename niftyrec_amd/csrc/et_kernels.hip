@@ -1210,15 +1210,18 @@ int et_launch_yl_pull_adj(int RPL, int nsrc, const EtPullArgs *args, const void 
     return (int)hipErrorInvalidValue;
 }
 
-int et_launch_yl_factors(int RPL, const EtSweepArgs &a, const EtKeys &k, et_stream_t stream)
+int et_launch_yl_factors(int RPL, bool stream_out, const EtSweepArgs &a, const EtKeys &k, et_stream_t stream)
 {
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (a.yu % (16 * RPL) != 0) return (int)hipErrorInvalidValue;
     const dim3 g((a.nx + 15) / 16 * (a.yu / (16 * RPL)), a.V);
-#define ET_YLF(rpl)                                                                   \
-    if (RPL == rpl) {                                                                 \
-        hipLaunchKernelGGL((k_yl_factors<rpl>), g, dim3(256), 0, st, a, k);            \
-        return (int)hipGetLastError();                                                \
+#define ET_YLF(rpl)                                                                 \
+    if (RPL == rpl) {                                                               \
+        if (stream_out)                                                             \
+            hipLaunchKernelGGL((k_yl_factors<rpl, true>), g, dim3(256), 0, st, a, k); \
+        else                                                                        \
+            hipLaunchKernelGGL((k_yl_factors<rpl, false>), g, dim3(256), 0, st, a, k); \
+        return (int)hipGetLastError();                                              \
     }
     ET_YLF(2) ET_YLF(4) ET_YLF(6) ET_YLF(8)
 #undef ET_YLF

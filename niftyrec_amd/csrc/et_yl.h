@@ -176,6 +176,64 @@ __device__ __forceinline__ void yl_bilinear(const float *p00, int dx, int dz, co
     for (int i = 0; i < RPL; i++) out[i] = c[0][i] * s.w00 + c[1][i] * s.w01 + c[2][i] * s.w10 + c[3][i] * s.w11;
 }
 
+// Interleaved rows, for kernels (and phases) that use no neighbouring rows: the
+// row's 16 lanes take the column's leading 64 rows four at a time, then the rest
+// (RPL 8: four, RPL 6: two at a time), so that a load of the 16 lanes is one
+// contiguous run.  With RPL consecutive rows per lane each of its 16-byte loads
+// uses every other 16 bytes of the lines it touches.
+template <int RPL>
+__device__ __forceinline__ int yl_irow(int lane, int i)  // row of element i
+{
+    if constexpr (RPL == 2) return 2 * lane + i;
+    if constexpr (RPL == 6) return i < 4 ? 4 * lane + i : 64 + 2 * lane + i - 4;
+    return (i & ~3) * 16 + 4 * lane + (i & 3);
+}
+template <int RPL>
+__device__ __forceinline__ void yl_iload(const float *col, int lane, float *v)
+{
+    if constexpr (RPL == 2) {
+        yl_load<2>(col + 2 * lane, v);
+    } else {
+        yl_load<4>(col + 4 * lane, v);
+        if constexpr (RPL == 6) yl_load<2>(col + 64 + 2 * lane, v + 4);
+        if constexpr (RPL == 8) yl_load<4>(col + 64 + 4 * lane, v + 4);
+    }
+}
+template <int RPL>
+__device__ __forceinline__ void yl_istore(float *col, int lane, const float *v)
+{
+    if constexpr (RPL == 2) {
+        yl_store<2>(col + 2 * lane, v);
+    } else {
+        yl_store<4>(col + 4 * lane, v);
+        if constexpr (RPL == 6) yl_store<2>(col + 64 + 2 * lane, v + 4);
+        if constexpr (RPL == 8) yl_store<4>(col + 64 + 4 * lane, v + 4);
+    }
+}
+template <int RPL>
+__device__ __forceinline__ void yl_istore_stream(float *col, int lane, const float *v)
+{
+    if constexpr (RPL == 2) {
+        yl_store_stream<2>(col + 2 * lane, v);
+    } else {
+        yl_store_stream<4>(col + 4 * lane, v);
+        if constexpr (RPL == 6) yl_store_stream<2>(col + 64 + 2 * lane, v + 4);
+        if constexpr (RPL == 8) yl_store_stream<4>(col + 64 + 4 * lane, v + 4);
+    }
+}
+// yl_bilinear of the lane's interleaved rows; p00: the corner column's first row.
+template <int RPL>
+__device__ __forceinline__ void yl_ibilinear(const float *p00, int lane, int dx, int dz, const Samp &s, float *out)
+{
+    float c[4][RPL];
+    yl_iload<RPL>(p00, lane, c[0]);
+    yl_iload<RPL>(p00 + dx, lane, c[1]);
+    yl_iload<RPL>(p00 + dz, lane, c[2]);
+    yl_iload<RPL>(p00 + dz + dx, lane, c[3]);
+#pragma unroll
+    for (int i = 0; i < RPL; i++) out[i] = c[0][i] * s.w00 + c[1][i] * s.w01 + c[2][i] * s.w10 + c[3][i] * s.w11;
+}
+
 // The R rows on either side of a lane's run, from its row neighbours:
 // ext[R - t] = row -t (lane l - ceil(t / RPL)), ext[R + RPL + t] = row RPL + t
 // (lane l + 1 + t / RPL).  The DPP controls are immediates, hence the recursion.
@@ -1441,7 +1499,7 @@ __global__ void __launch_bounds__(32 * L, 4) k_yt_project_if(const EtSweepArgs *
 // all planes, one run of 16 RPL rows.  grid (ceil(nx / 16) x rows / (16 RPL), V),
 // 256 threads.
 // ------------------------------------------------------------------------------
-template <int RPL>
+template <int RPL, bool STREAM>
 __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
 {
     const int lane = threadIdx.x & 15, slot = threadIdx.x >> 4;
@@ -1449,7 +1507,7 @@ __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
     const int xc = ((int)blockIdx.x - half * ncb) * 16 + slot, v = blockIdx.y;
     if (xc >= a.nx) return;  // the whole 16-lane row
     const int rows = a.yu;
-    const int row0 = RPL * (lane + 16 * half);
+    const int row0 = 16 * RPL * half;
     const int dx = a.yp, dz = a.yp * a.xp;
     const FastView fv = load_fast_view(a.views + (size_t)v * ET_VIEW_REC);
     const float *mu = a.mu + a.gmu + row0;
@@ -1459,16 +1517,41 @@ __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
         A[i] = 0.f;
         Al[i] = 0.f;
     }
+    // Bound by the stores and by the L1: factors that exceed the Infinity Cache are
+    // stored past the caches, which keeps mu in them (290 -> 228 us at 128^3 x 120
+    // views, 1 GB, 4.6 TB/s; 256^3 x 60 views 1,704 -> 1,201), interleaved rows make
+    // every gather one run (315 -> 290 us); lane k computes the sample of plane z0 +
+    // k, and a plane's corners are loaded while the plane before it is summed (318
+    // -> 315 us).
+    YlSamp sb = {};
+    float c[4][RPL];
+    Samp s;
+    auto load = [&](int z) {
+        if ((z & 15) == 0) sb = yl_samp_of(fast_sample(fv, (float)xc, z + lane, a.nx, a.nz, dx, dz));
+        s = yl_samp_from(sb, z & 15);
+        const float *p = mu + s.off;
+        yl_iload<RPL>(p, lane, c[0]);
+        yl_iload<RPL>(p + dx, lane, c[1]);
+        yl_iload<RPL>(p + dz, lane, c[2]);
+        yl_iload<RPL>(p + dz + dx, lane, c[3]);
+    };
+    load(0);
     for (int z = 0; z < a.nz; z++) {
-        const Samp s = fast_sample(fv, (float)xc, z, a.nx, a.nz, dx, dz);
         float m[RPL], e[RPL];
-        yl_bilinear<RPL>(mu + s.off, dx, dz, s, m);
+#pragma unroll
+        for (int i = 0; i < RPL; i++)
+            m[i] = c[0][i] * s.w00 + c[1][i] * s.w01 + c[2][i] * s.w10 + c[3][i] * s.w11;
+        if (z + 1 < a.nz) load(z + 1);
 #pragma unroll
         for (int i = 0; i < RPL; i++) {
             comp_add(A[i], Al[i], m[i]);
             e[i] = exp_neg(A[i] + Al[i]);
         }
-        yl_store<RPL>(a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0, e);
+        float *o = a.att + (size_t)v * a.att_vs + ((size_t)z * a.nx + xc) * rows + row0;
+        if constexpr (STREAM)
+            yl_istore_stream<RPL>(o, lane, e);
+        else
+            yl_istore<RPL>(o, lane, e);
     }
 }
 
@@ -1477,7 +1560,7 @@ __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
 // factors were formed from; block (0, 0) writes the keys of this operation and
 // whether its forward sums are there already.  At 128^3 the launch takes about
 // 8 us where the factors stay; a host that read the keys waited for the stream.
-template <int RPL>
+template <int RPL, bool STREAM>
 __global__ void __launch_bounds__(256) k_yl_factors(EtSweepArgs a, EtKeys k)
 {
     if (k.st) {
@@ -1501,7 +1584,7 @@ __global__ void __launch_bounds__(256) k_yl_factors(EtSweepArgs a, EtKeys k)
         }
         if (k.fac_built && k.st[ET_KEY_MU + prev] == km) return;
     }
-    yl_factor_body<RPL>(a);
+    yl_factor_body<RPL, STREAM>(a);
 }
 
 // ------------------------------------------------------------------------------
@@ -1528,7 +1611,7 @@ __device__ __forceinline__ void yl_pull_body(const EtPullArgs &a, const Blk &b)
     const int x = ((sup % nsx) * 8 + (t & 7)) * 4 + (slot & 3), z = ((sup / nsx) * 8 + (t >> 3)) * 4 + (slot >> 2);
     if (x >= a.nx || z >= a.nz) return;
     const int rows = a.yu;
-    const int row0 = RPL * (lane + 16 * half);
+    const int row0 = 16 * RPL * half;  // (the lane's rows: row0 + yl_irow)
     const int dx = rows, dz = rows * a.xp;
     float acc[RPL];
 #pragma unroll
@@ -1546,7 +1629,7 @@ __device__ __forceinline__ void yl_pull_body(const EtPullArgs &a, const Blk &b)
         }
         const Samp s = yl_samp_from(sb, v & 15);
         float t[RPL];
-        yl_bilinear<RPL>(a.u + (size_t)v * a.ustride + row0 + s.off, dx, dz, s, t);
+        yl_ibilinear<RPL>(a.u + (size_t)v * a.ustride + row0 + s.off, lane, dx, dz, s, t);
 #pragma unroll
         for (int i = 0; i < RPL; i++) acc[i] += t[i];
     }
@@ -1554,24 +1637,24 @@ __device__ __forceinline__ void yl_pull_body(const EtPullArgs &a, const Blk &b)
     float o[RPL];
     if constexpr (EPI == ET_EPI_OSEM) {
         float xv[RPL], sv[RPL];
-        yl_load<RPL>(a.x + base, xv);
-        yl_load<RPL>(a.sens + base, sv);
+        yl_iload<RPL>(a.x + base, lane, xv);
+        yl_iload<RPL>(a.sens + base, lane, sv);
 #pragma unroll
         for (int i = 0; i < RPL; i++) {
             const float bb = acc[i] < 0.f ? 0.f : acc[i];
-            o[i] = (row0 + i < a.ny) ? xv[i] * (bb / sv[i]) : xv[i];
+            o[i] = (row0 + yl_irow<RPL>(lane, i) < a.ny) ? xv[i] * (bb / sv[i]) : xv[i];
         }
-        yl_store<RPL>(a.x + base, o);
+        yl_istore<RPL>(a.x + base, lane, o);
     } else {
         float ov[RPL];
-        yl_load<RPL>(a.out + base, ov);
+        yl_iload<RPL>(a.out + base, lane, ov);
 #pragma unroll
         for (int i = 0; i < RPL; i++) {
             float val = a.accumulate ? ov[i] + acc[i] : acc[i];
             if (a.truncate && val < a.floor) val = a.floor;
-            o[i] = (row0 + i < a.ny) ? val : ov[i];
+            o[i] = (row0 + yl_irow<RPL>(lane, i) < a.ny) ? val : ov[i];
         }
-        yl_store<RPL>(a.out + base, o);
+        yl_istore<RPL>(a.out + base, lane, o);
     }
 }
 
@@ -1606,7 +1689,7 @@ __device__ __forceinline__ void yl_pull_adj_body(const EtPullArgs &a, const Blk 
     const int x = ((sup % nsx) * 8 + (t & 7)) * 4 + (slot & 3), z = ((sup / nsx) * 8 + (t >> 3)) * 4 + (slot >> 2);
     if (x >= a.nx || z >= a.nz) return;  // (the whole 16-lane row)
     const int rows = a.yu;
-    const int row0 = RPL * (lane + 16 * half);
+    const int row0 = 16 * RPL * half;  // (the lane's rows: row0 + yl_irow)
     const float fxo = (float)x, fzo = (float)z;
     __shared__ float hit_w[16][16];  // per row: the weights and offsets of its non-zero candidates
     __shared__ int hit_o[16][16];
@@ -1662,7 +1745,7 @@ __device__ __forceinline__ void yl_pull_adj_body(const EtPullArgs &a, const Blk 
                     w[q] = hit_w[slot][h];
                     const int o = hit_o[slot][h];
 #pragma unroll
-                    for (int s = 0; s < NS; s++) yl_load<RPL>(uv[s] + o, t[q][s]);
+                    for (int s = 0; s < NS; s++) yl_iload<RPL>(uv[s] + o, lane, t[q][s]);
                 }
 #pragma unroll
                 for (int q = 0; q < HB; q++) {
@@ -1681,14 +1764,14 @@ __device__ __forceinline__ void yl_pull_adj_body(const EtPullArgs &a, const Blk 
     for (int s = 0; s < NS; s++) {
         float *out = s == 0 ? a.out : a.out2;
         float ov[RPL], o[RPL];
-        yl_load<RPL>(out + base, ov);
+        yl_iload<RPL>(out + base, lane, ov);
 #pragma unroll
         for (int i = 0; i < RPL; i++) {
             float val = a.accumulate ? ov[i] + acc[s][i] : acc[s][i];
             if (a.truncate && val < 0.f) val = 0.f;
-            o[i] = (row0 + i < a.ny) ? val : ov[i];
+            o[i] = (row0 + yl_irow<RPL>(lane, i) < a.ny) ? val : ov[i];
         }
-        yl_store<RPL>(out + base, o);
+        yl_istore<RPL>(out + base, lane, o);
     }
 }
 
