@@ -185,16 +185,232 @@ int odd_segments(int n)
 // Device buffers
 // ---------------------------------------------------------------------------
 
+// Device memory kept between the calls on host arrays.  Each such call builds a
+// plan, runs it and drops it, and a plan's buffers are large: of an MLEM update at
+// 96^3 x 60 views two are 212 MB.  hipMalloc and hipFree map and unmap them on
+// every call, and hipFree waits for the device: that update took 2.9 ms in a fresh
+// process and 12-28 ms in one that holds other memory; with its blocks kept 1.37 ms
+// in either (the kernels take 0.4 ms, the copies 0.9).  A call
+// therefore takes its blocks and its stream from here and gives them back when it
+// ends, after its stream has been waited for, so no kernel of it is in flight when
+// another call or thread takes them.  Contents are whatever the last call left:
+// buffers that need zeros are filled by their owner, as fresh memory is.
+//   LIMIT  bounds what is kept, per process: the two large buffers of a call of
+//          ordinary size; blocks that do not fit it are freed as before.
+//   AGE    a block that this many ended calls did not take is freed.
+// et_array_reset_gpu gives everything back, and so does a failed allocation
+// (here or for a plan of the caller's own), which is then tried once more.
+class CallPool {
+public:
+    struct Block {
+        void *p;
+        size_t bytes;
+        int device;
+        unsigned long long stamp;
+    };
+    static CallPool &get()
+    {
+        static CallPool *pool = new CallPool;  // not destroyed: the runtime may end before static objects do
+        return *pool;
+    }
+    // A kept block of `device` that holds `bytes` with at most a quarter (small
+    // ones: 64 KiB) to spare, or a new one.
+    Block take(size_t bytes, int device)
+    {
+        const size_t need = (std::max<size_t>(bytes, 1) + GRAIN - 1) / GRAIN * GRAIN;
+        {
+            std::lock_guard<std::mutex> lk(m_);
+            size_t best = kept_.size();
+            for (size_t i = 0; i < kept_.size(); i++) {
+                const Block &b = kept_[i];
+                if (b.device != device || b.bytes < need || b.bytes > need + std::max<size_t>(need / 4, 65536)) continue;
+                if (best == kept_.size() || b.bytes < kept_[best].bytes) best = i;
+            }
+            if (best < kept_.size()) {
+                const Block b = kept_[best];
+                kept_[best] = kept_.back();
+                kept_.pop_back();
+                held_ -= b.bytes;
+                return b;
+            }
+        }
+        return Block{device_malloc(need), need, device, 0};
+    }
+    // A call ends: its blocks are kept, newest last, up to LIMIT.
+    void give(std::vector<Block> &blocks) noexcept
+    {
+        std::vector<Block> out;  // to free, outside the lock
+        try {
+            std::lock_guard<std::mutex> lk(m_);
+            out.reserve(kept_.size() + blocks.size());
+            kept_.reserve(kept_.size() + blocks.size());  // nothing below throws
+            calls_++;
+            for (size_t i = 0; i < kept_.size();)
+                if (calls_ - kept_[i].stamp > AGE) drop(i, out);
+                else i++;
+            for (Block &b : blocks) {
+                if (b.bytes > LIMIT) {
+                    out.push_back(b);
+                    continue;
+                }
+                while (held_ + b.bytes > LIMIT) {  // the least recently used go first
+                    size_t old = 0;
+                    for (size_t i = 1; i < kept_.size(); i++)
+                        if (kept_[i].stamp < kept_[old].stamp) old = i;
+                    if (kept_[old].stamp == calls_) break;  // this call's own: no gain
+                    drop(old, out);
+                }
+                if (held_ + b.bytes > LIMIT) {
+                    out.push_back(b);
+                    continue;
+                }
+                b.stamp = calls_;
+                kept_.push_back(b);
+                held_ += b.bytes;
+            }
+        } catch (...) {  // no host memory for the list: nothing was kept
+            out.swap(blocks);
+        }
+        for (const Block &b : out) (void)hipFree(b.p);
+        blocks.clear();
+    }
+    hipStream_t take_stream(int device)
+    {
+        {
+            std::lock_guard<std::mutex> lk(m_);
+            for (size_t i = 0; i < streams_.size(); i++)
+                if (streams_[i].second == device) {
+                    const hipStream_t st = streams_[i].first;
+                    streams_.erase(streams_.begin() + i);
+                    return st;
+                }
+        }
+        hipStream_t st = nullptr;
+        check_hip(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), niftyrec_error_unspecified);
+        return st;
+    }
+    void give_stream(hipStream_t st, int device) noexcept
+    {
+        {
+            std::lock_guard<std::mutex> lk(m_);
+            if (streams_.size() < STREAMS) {  // (reserved)
+                streams_.emplace_back(st, device);
+                return;
+            }
+        }
+        (void)hipStreamDestroy(st);
+    }
+    bool clear()
+    {
+        std::vector<Block> out;
+        std::vector<std::pair<hipStream_t, int>> st;
+        {
+            std::lock_guard<std::mutex> lk(m_);
+            out.swap(kept_);
+            st.reserve(STREAMS);
+            st.swap(streams_);
+            held_ = 0;
+        }
+        for (const Block &b : out) (void)hipFree(b.p);
+        for (auto &x : st) (void)hipStreamDestroy(x.first);
+        return !out.empty();
+    }
+    static void *device_malloc(size_t bytes)
+    {
+        void *p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        if (get().clear()) {
+            (void)hipGetLastError();
+            if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        }
+        throw EtError{niftyrec_error_allocgpu};
+    }
+
+private:
+    CallPool() { streams_.reserve(STREAMS); }
+    static constexpr size_t GRAIN = 4096, LIMIT = (size_t)2 << 30, STREAMS = 4;
+    static constexpr unsigned long long AGE = 16;
+    void drop(size_t i, std::vector<Block> &out)
+    {
+        out.push_back(kept_[i]);
+        held_ -= kept_[i].bytes;
+        kept_[i] = kept_.back();
+        kept_.pop_back();
+    }
+    std::mutex m_;
+    std::vector<Block> kept_;
+    std::vector<std::pair<hipStream_t, int>> streams_;
+    size_t held_ = 0;
+    unsigned long long calls_ = 0;
+};
+
+// One call on host arrays: its stream and every block that it or its plans take.
+// Declared before the call's plans, so they end before it does; a buffer that a
+// plan drops or outgrows stays with the call until then, for the call's kernels
+// may still use it.
+struct HostCall {
+    hipStream_t st = nullptr;
+    int device = 0;
+    std::vector<CallPool::Block> blocks;
+    HostCall *outer = nullptr;
+    HostCall() : outer(current()) {}
+    HostCall(const HostCall &) = delete;
+    HostCall &operator=(const HostCall &) = delete;
+    ~HostCall()
+    {
+        if (!st) return;
+        current() = outer;
+        if (hipStreamSynchronize(st) == hipSuccess) {
+            CallPool::get().give(blocks);
+            CallPool::get().give_stream(st, device);
+        } else {
+            for (const CallPool::Block &b : blocks) (void)hipFree(b.p);
+            (void)hipStreamDestroy(st);
+        }
+    }
+    // The call that this thread is in, if any: its plans' buffers come from it.
+    static HostCall *&current()
+    {
+        thread_local HostCall *call = nullptr;
+        return call;
+    }
+    void init()
+    {
+        check_hip(hipGetDevice(&device), niftyrec_error_nogpuinstalled);
+        blocks.reserve(64);
+        st = CallPool::get().take_stream(device);
+        current() = this;
+    }
+    float *alloc(size_t n)
+    {
+        blocks.reserve(blocks.size() + 1);
+        blocks.push_back(CallPool::get().take(n * sizeof(float), device));
+        return (float *)blocks.back().p;
+    }
+    float *upload(const float *h, size_t n)
+    {
+        float *d = alloc(n);
+        check_hip(hipMemcpyAsync(d, h, n * sizeof(float), hipMemcpyHostToDevice, st), niftyrec_error_transfergpu);
+        return d;
+    }
+    void download(float *h, const float *d, size_t n)
+    {
+        check_hip(hipMemcpyAsync(h, d, n * sizeof(float), hipMemcpyDeviceToHost, st), niftyrec_error_transfergpu);
+        check_hip(hipStreamSynchronize(st), niftyrec_error_kernel);
+    }
+};
+
 struct DevBuf {
     float *p = nullptr;
     size_t n = 0;
+    bool lent = false;  // of the call on host arrays that the owner runs in
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() { release(); }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p && !lent) (void)hipFree(p);
         p = nullptr;
         n = 0;
     }
@@ -205,10 +421,10 @@ struct DevBuf {
     {
         if (count <= n && p) return p;
         release();
-        if (hipMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(float)) != hipSuccess) {
-            p = nullptr;
-            throw EtError{niftyrec_error_allocgpu};
-        }
+        const size_t m = std::max<size_t>(count, 1);
+        HostCall *call = HostCall::current();
+        lent = call != nullptr;
+        p = call ? call->alloc(m) : (float *)CallPool::device_malloc(m * sizeof(float));
         n = count;
         if (zero) check_launch(et_launch_fill(p, count, 0.f, (et_stream_t)stream));
         return p;
@@ -2371,40 +2587,6 @@ void op_osem(et_plan *p, float *x, const float *meas, const float *mu, int S, in
 // Host-pointer calls: upload, run on a private stream, download.
 // ---------------------------------------------------------------------------
 
-struct HostCall {
-    hipStream_t st = nullptr;
-    std::vector<float *> bufs;
-    ~HostCall()
-    {
-        if (st) (void)hipStreamSynchronize(st);
-        for (float *b : bufs) (void)hipFree(b);
-        if (st) (void)hipStreamDestroy(st);
-    }
-    void init()
-    {
-        check_hip(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), niftyrec_error_unspecified);
-    }
-    float *alloc(size_t n)
-    {
-        float *p = nullptr;
-        if (hipMalloc((void **)&p, std::max<size_t>(n, 1) * sizeof(float)) != hipSuccess)
-            throw EtError{niftyrec_error_allocgpu};
-        bufs.push_back(p);
-        return p;
-    }
-    float *upload(const float *h, size_t n)
-    {
-        float *d = alloc(n);
-        check_hip(hipMemcpyAsync(d, h, n * sizeof(float), hipMemcpyHostToDevice, st), niftyrec_error_transfergpu);
-        return d;
-    }
-    void download(float *h, const float *d, size_t n)
-    {
-        check_hip(hipMemcpyAsync(h, d, n * sizeof(float), hipMemcpyDeviceToHost, st), niftyrec_error_transfergpu);
-        check_hip(hipStreamSynchronize(st), niftyrec_error_kernel);
-    }
-};
-
 template <class F>
 int guarded(F &&f)
 {
@@ -2455,8 +2637,8 @@ int project_host(float *activity, int *activity_size, float *sinogram, int *sino
         Cameras cams;
         int rc = expand_cameras(cameras, V, cols, vs, cams);
         if (rc) return rc;
-        et_plan plan;
         HostCall hc;
+        et_plan plan;
         hc.init();
         plan.st = hc.st;
         rc = build_plan(&plan, nx, ny, nz, cams, no_psf ? nullptr : psf, no_psf ? 0 : psf_size[0], background,
@@ -2625,8 +2807,8 @@ int backproject_host(float *sino, int *sino_size, float *bkpr, int *bkpr_size, f
         Cameras cams;
         int rc = expand_cameras(cameras, V, cols, act_size, cams);
         if (rc) return rc;
-        et_plan plan;
         HostCall hc;
+        et_plan plan;
         hc.init();
         plan.st = hc.st;
         rc = build_plan(&plan, nx, ny, nz, cams, no_psf ? nullptr : psf, no_psf ? 0 : psf_size[0], background,
@@ -2655,13 +2837,14 @@ int em_step_host(float *activity, int size_x, int size_y, const float *sino, int
         Cameras cams;
         int rc = expand_cameras(cams3, V, 3, vs, cams);
         if (rc) return rc;
-        et_plan plan;
         HostCall hc;
+        et_plan plan;
         hc.init();
         plan.st = hc.st;
         rc = build_plan(&plan, nx, ny, nz, cams, psf, psf ? psf_h : 0, bg, bga);
         if (rc) return rc;
-        // one update: the chunking comes from the launch size, not from timing
+        plan.mu_check = false;  // one update: the map cannot change under its caches
+        // ... and the chunking comes from the launch size, not from timing
         plan.tune_D = launch_depth_chunks(&plan, V);
         const size_t n = (size_t)nx * ny * nz;
         float *d_x = hc.upload(activity, n);
@@ -3266,6 +3449,7 @@ int et_array_reset_gpu(void)
 {
     int st = select_device();
     if (st) return st;
+    CallPool::get().clear();  // memory kept between calls on host arrays
     return hipDeviceSynchronize() == hipSuccess ? niftyrec_success : niftyrec_error_kernel;
 }
 
@@ -3387,8 +3571,8 @@ int et_array_gradient_attenuation(float *sino, int *sino_size, float *activity, 
         Cameras cams;
         int rc = expand_cameras(cameras, V, cols, activity_size ? activity_size : gradient_size, cams);
         if (rc) return rc;
-        et_plan plan;
         HostCall hc;
+        et_plan plan;
         hc.init();
         plan.st = hc.st;
         rc = build_plan(&plan, nx, ny, nz, cams, no_psf ? nullptr : psf, no_psf ? 0 : psf_size[0], background,
