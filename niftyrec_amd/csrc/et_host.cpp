@@ -440,7 +440,7 @@ struct DevBuf {
 // One grouped launch of the row-lane OSEM kernels: argument records and block
 // table at byte offsets of a device table buffer.
 struct YlLaunch {
-    int kind;                 // YL_PROJECT, YL_RATIO, YL_BPU, YL_PULL_OSEM, YL_PULL_STORE, YL_GRAD, YL_PULL_ADJ(2)
+    int kind;                 // YL_PROJECT, YL_RATIO, YL_BPU, YL_PULL_OSEM, YL_PULL_STORE, YL_GRAD, YL_PULL_ADJ
     int R, RPL, NR, nthr;     // sweep template and block shape (pull: RPL)
     size_t lds;               // dynamic LDS bytes (sweeps)
     size_t args_off, tab_off;
@@ -449,9 +449,8 @@ struct YlLaunch {
 };
 enum {
     YL_PROJECT = 0, YL_RATIO = 1, YL_BPU = 2, YL_PULL_OSEM = 3, YL_PULL_STORE = 4, YL_GRAD = 5, YL_PULL_ADJ = 6,
-    YL_PULL_ADJ2 = 7,  // exact adjoint pull of two volumes (u, u2) into two outputs
-    YL_GREF = 8,       // reference attenuation gradient
-    YL_PROJECT_IF = 9, // projection that the device may skip
+    YL_GREF = 7,        // reference attenuation gradient
+    YL_PROJECT_IF = 8,  // projection that the device may skip
 };
 // Table slots of the single operations (each keeps its last upload).
 enum {
@@ -878,19 +877,25 @@ int choose_D(et_plan *p, int views)
     return D;
 }
 
+// Views per batch of a backprojection: rotated-frame volumes of at most 208 MiB, so
+// that with the volume they are added into they stay in the 256 MiB Infinity Cache
+// between the sweep that writes them and the pull that reads them; the views are
+// spread evenly over the batches.  128^3 x 120 views, PSF 11: 24 views a batch 452
+// us, 15 494, 30 500, all at once 529; 96^3 x 120, PSF 7: 40 a batch 233, 64 246.
 int view_batch(et_plan *p)
 {
     if (p->tune_vb > 0) return std::min(p->tune_vb, p->V);
     const size_t bytes = p->ustride * sizeof(float);
-    long vb = (long)((256ull << 20) / std::max<size_t>(bytes, 1));
-    return (int)std::max(1L, std::min<long>(vb, p->V));
+    const long vb = std::max(1L, (long)((208ull << 20) / std::max<size_t>(bytes, 1)));
+    const long nb = (p->V + vb - 1) / vb;
+    return (int)((p->V + nb - 1) / nb);
 }
 
 // Views per launch of the gradient sweeps.  They run whole rays (one depth
 // chunk: the reverse sum needs the ray's total), so a launch has only
 // slabs x views blocks: at least two per CU are taken, with rotated-frame
-// volumes of up to 4 GiB (256^3: 32 views, 2.2 GB), where view_batch's 256 MiB
-// would give 3 views (48 blocks).
+// volumes of up to 4 GiB (256^3: 32 views, 2.2 GB), where view_batch would give
+// 3 views (48 blocks).
 int grad_view_batch(et_plan *p)
 {
     if (p->tune_vb > 0) return std::min(p->tune_vb, p->V);
@@ -1796,11 +1801,9 @@ void yl_issue(const float *dev, const std::vector<YlLaunch> &L, size_t from, siz
             check_launch(et_launch_ratio_group(static_cast<const EtRatioArgs *>(args), tab, l.n, l.blocks, s));
             break;
         }
-        case YL_PULL_ADJ:
-        case YL_PULL_ADJ2: {
+        case YL_PULL_ADJ: {
             ProfScope ps(prof, ET_PROF_PULL, l.bytes);
-            check_launch(et_launch_yl_pull_adj(l.RPL, l.kind == YL_PULL_ADJ2 ? 2 : 1,
-                                               static_cast<const EtPullArgs *>(args), tab, l.n, l.blocks, s));
+            check_launch(et_launch_yl_pull_adj(l.RPL, static_cast<const EtPullArgs *>(args), tab, l.n, l.blocks, s));
             break;
         }
         default: {
@@ -1909,13 +1912,13 @@ const float *yl_sources(et_plan *p, const float *act, const float *mu, int fwd)
     return p->fac.p;
 }
 
-// Rotated-frame volumes for up to `want` views in p->u (`per` volumes a view):
-// fewer views where the device has no room for them.
-int yl_u_views(et_plan *p, int want, int per)
+// Rotated-frame volumes for up to `want` views in p->u: fewer views where the
+// device has no room for them.
+int yl_u_views(et_plan *p, int want)
 {
     for (int nv = want;; nv = (nv + 1) / 2) {
         try {
-            p->u.ensure((size_t)nv * per * p->ustride, true, p->st);
+            p->u.ensure((size_t)nv * p->ustride, true, p->st);
             return nv;
         } catch (const EtError &) {
             if (nv <= 1) throw;
@@ -2008,8 +2011,7 @@ float *yl_forward(YlTable &t, et_plan *p, const float *fac, int D, const int *sk
     return part;
 }
 
-// Largest rotated-frame buffer of the gradient and the joint backward: 4 GiB
-// (128^3 x 120 views hold 1.0 GiB each).
+// Largest rotated-frame buffer of the gradient: 4 GiB (128^3 x 120 views hold 1.0).
 constexpr size_t ET_YL_U_BYTES = 4ull << 30;
 
 // Views per batch of the exact attenuation gradient (rotated-frame volumes of at
@@ -2055,16 +2057,11 @@ bool yl_op_project(et_plan *p, const float *act, const float *mu, float *sino, i
     return true;
 }
 
-bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate)
+// Adds to t the backprojection of every view into acc, in batches of vb views that
+// reuse u in stream order.
+void yl_backproject_views(YlTable &t, et_plan *p, const float *fac, const float *st, int vb, bool adjoint,
+                          bool truncate, float *acc)
 {
-    if (!p->yl_ops || !p->yl || (mu && !yl_factor_room(p))) return false;
-    const float *fac = yl_sources(p, nullptr, mu, 0);
-    const size_t pe = yl_plane_elems(p);
-    const float *st = yl_sino_t(p, sino);
-    const int vb = view_batch(p);
-    p->u.ensure((size_t)vb * p->ustride, true, p->st);
-    float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
-    YlTable t;  // every batch in one table: the batches reuse u in stream order
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
         const int D = yl_op_chunks(p, yl_bpu_gx(p, nv));
@@ -2073,7 +2070,7 @@ bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *ou
             bytes += (double)nv * (8.0 * p->nvox + 4.0 * p->P);
             EtSweepArgs a = yl_sweep_args(p, recs, nv, D, yl_att_at(p, fac, v0));
             a.src = ET_SRC_SINO;
-            a.sino = st + (size_t)v0 * pe;
+            a.sino = st + (size_t)v0 * yl_plane_elems(p);
             a.u = p->u.p;
             if (p->K > 0 && adjoint) a.psf = p->d_sep_flip.p;  // correlation: the adjoint of the PSF
             gx = yl_bpu_gx(p, a.D);
@@ -2082,6 +2079,17 @@ bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *ou
         });
         yl_pull_into(t, p, recs, nv, adjoint, v0 > 0, v0 + nv >= p->V && truncate, acc);
     }
+}
+
+bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate)
+{
+    if (!p->yl_ops || !p->yl || (mu && !yl_factor_room(p))) return false;
+    const float *fac = yl_sources(p, nullptr, mu, 0);
+    const float *st = yl_sino_t(p, sino);
+    const int vb = yl_u_views(p, view_batch(p));
+    float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
+    YlTable t;
+    yl_backproject_views(t, p, fac, st, vb, adjoint, truncate != 0, acc);
     yl_run(p, t, YL_OP_BACKPROJECT);
     ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc, out, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
@@ -2108,24 +2116,30 @@ void yl_forward_kept(et_plan *p, int D)
     p->fwd_tiles = p->yl_tiles;
 }
 
-// Gradient sweep of nv views from view v0 on (their forward sums in `part`) into
-// u, with the plan's projector kind and the forward sums' chunking.
-void yl_gradient_sweep(YlTable &t, et_plan *p, int v0, int nv, const float *fac, const float *st, float *part, int D,
-                       float *u)
+// Adds to t the gradient of every view into acc, in batches of vb views: the sweep
+// into u with the plan's projector kind and the chunking D of the forward sums
+// `part`, then the exact adjoint pull.
+void yl_gradient_views(YlTable &t, et_plan *p, const float *fac, const float *st, float *part, int D, int vb,
+                       bool truncate, float *acc)
 {
-    t.grouped<EtSweepArgs>(YL_GRAD, {p}, YlTable::project_key, [&](int, int &gx, int &gy, double &bytes) {
-        bytes += (double)nv * (8.0 * p->nvox + 4.0 * p->P);
-        EtSweepArgs a = yl_sweep_args(p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, D, yl_att_at(p, fac, v0));
-        a.act = p->act_yf.p;
-        a.part = part + (size_t)v0 * yl_plane_elems(p);
-        a.part_V = p->V;
-        a.near_views = 1;
-        a.sino = st + (size_t)v0 * yl_plane_elems(p);
-        a.u = u;
-        gx = a.D * p->yl_tiles;
-        gy = nv;
-        return a;
-    });
+    for (int v0 = 0; v0 < p->V; v0 += vb) {
+        const int nv = std::min(vb, p->V - v0);
+        const float *recs = p->d_recs.p + (size_t)v0 * ET_VIEW_REC;
+        t.grouped<EtSweepArgs>(YL_GRAD, {p}, YlTable::project_key, [&](int, int &gx, int &gy, double &bytes) {
+            bytes += (double)nv * (8.0 * p->nvox + 4.0 * p->P);
+            EtSweepArgs a = yl_sweep_args(p, recs, nv, D, yl_att_at(p, fac, v0));
+            a.act = p->act_yf.p;
+            a.part = part + (size_t)v0 * yl_plane_elems(p);
+            a.part_V = p->V;
+            a.near_views = 1;
+            a.sino = st + (size_t)v0 * yl_plane_elems(p);
+            a.u = p->u.p;
+            gx = a.D * p->yl_tiles;
+            gy = nv;
+            return a;
+        });
+        yl_pull_into(t, p, recs, nv, true, v0 > 0, v0 + nv >= p->V && truncate, acc);
+    }
 }
 
 // Exact attenuation gradient: the forward sums of every view (kept from the last
@@ -2137,15 +2151,11 @@ bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float
     const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
     const int D = yl_forward_chunks(p, true);
-    const int vb = yl_u_views(p, yl_gradient_batch(p), 1);
+    const int vb = yl_u_views(p, yl_gradient_batch(p));
     float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
-    YlTable t;  // every batch in one table: the batches reuse u in stream order
+    YlTable t;
     float *part = yl_gradient_forward(t, p, fac, D);
-    for (int v0 = 0; v0 < p->V; v0 += vb) {
-        const int nv = std::min(vb, p->V - v0);
-        yl_gradient_sweep(t, p, v0, nv, fac, st, part, D, p->u.p);
-        yl_pull_into(t, p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, true, v0 > 0, v0 + nv >= p->V && truncate, acc);
-    }
+    yl_gradient_views(t, p, fac, st, part, D, vb, truncate != 0, acc);
     yl_run(p, t, YL_OP_GRADIENT);
     yl_forward_kept(p, D);
     ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
@@ -2162,7 +2172,7 @@ bool yl_op_gradient_ref(et_plan *p, const float *sino, const float *act, const f
     const float *fac = yl_sources(p, act, mu, 0);
     const size_t pe = yl_plane_elems(p);
     const float *st = yl_sino_t(p, sino);
-    const int vb = yl_u_views(p, view_batch(p), 1);
+    const int vb = yl_u_views(p, view_batch(p));
     const int D = yl_op_chunks(p, vb);
     int Deff, zlen;
     yl_chunks(p, D, Deff, zlen);
@@ -2197,51 +2207,26 @@ bool yl_op_gradient_ref(et_plan *p, const float *sino, const float *act, const f
     return true;
 }
 
-// Both gradients in one pass over the views: the forward sums as for the
-// gradient, the adjoint backprojection sweep's rotated-frame volumes into the
-// first half of u, the gradient sweep's into the second, and one exact adjoint
-// pull (YL_PULL_ADJ2), whose candidate weights serve both, adds them up.  Each
-// output equals its operation's on its own with all views in one batch (the
-// view batch set to the view count).  False (nothing issued) when the two
-// volumes of every view would exceed 4 GiB or the device's memory.
+// Both gradients from one set of sources: the adjoint backprojection and the
+// gradient, each output what its operation on its own gives.  One pull of both
+// volumes, with one set of candidate weights, needs both of every view at once, 2
+// GB at 128^3 x 120 views that the Infinity Cache does not hold: it took 629 us
+// where the two pulls take about 500, and a GB more of memory.
 bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float *mu, float *out_act, float *out_mu,
                     int truncate)
 {
-    if (!p->yl_ops || !p->yl || !act || !mu) return false;
-    const int V = p->V;
-    if (2 * (size_t)V * p->ustride * sizeof(float) > ET_YL_U_BYTES || !yl_factor_room(p) || yl_u_views(p, V, 2) < V)
-        return false;
+    if (!p->yl_ops || !p->yl || !act || !mu || !yl_factor_room(p)) return false;
     const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
-    float *ub = p->u.p, *ug = p->u.p + (size_t)V * p->ustride;
+    const int want_b = view_batch(p), want_g = yl_gradient_batch(p);
+    const int room = yl_u_views(p, std::max(want_b, want_g));
     float *acc_a = p->op_acc.ensure(p->yf_elems, true, p->st);
     float *acc_m = p->op_acc2.ensure(p->yf_elems, true, p->st);
-    const float *recs = p->d_recs.p;
     const int D = yl_forward_chunks(p, true);
     YlTable t;
     float *part = yl_gradient_forward(t, p, fac, D);
-    const int Db = yl_op_chunks(p, yl_bpu_gx(p, V));
-    t.grouped<EtSweepArgs>(YL_BPU, {p}, YlTable::sweep_key, [&](int, int &gx, int &gy, double &bytes) {
-        bytes += (double)V * (8.0 * p->nvox + 4.0 * p->P);
-        EtSweepArgs a = yl_sweep_args(p, recs, V, Db, fac);
-        a.src = ET_SRC_SINO;
-        a.sino = st;
-        a.u = ub;
-        if (p->K > 0) a.psf = p->d_sep_flip.p;  // correlation: the adjoint of the PSF
-        gx = yl_bpu_gx(p, a.D);
-        gy = V;
-        return a;
-    });
-    yl_gradient_sweep(t, p, 0, V, fac, st, part, D, ug);
-    t.grouped<EtPullArgs>(YL_PULL_ADJ2, {p}, YlTable::pull_key, [&](int, int &gx, int &gy, double &bytes) {
-        bytes += (double)V * 8.0 * p->nvox + 8.0 * p->nvox;
-        gx = yl_pull_tiles(p);
-        gy = 1;
-        EtPullArgs a = pull_args(p, recs, V, ub, true, ET_EPI_YF_STORE, false, truncate != 0, acc_a, nullptr, nullptr);
-        a.u2 = ug;
-        a.out2 = acc_m;
-        return a;
-    });
+    yl_backproject_views(t, p, fac, st, std::min(want_b, room), true, truncate != 0, acc_a);
+    yl_gradient_views(t, p, fac, st, part, D, std::min(want_g, room), truncate != 0, acc_m);
     yl_run(p, t, YL_OP_BACKWARD);
     yl_forward_kept(p, D);
     ProfScope ps(p, ET_PROF_OTHER, 16.0 * p->nvox);
