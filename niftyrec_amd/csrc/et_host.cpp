@@ -3047,7 +3047,7 @@ std::vector<const void *> batch_key(const et_batch *b, int S, float eps)
 
 // Launch lists of one OSEM iteration.  Plans whose cached data are the
 // row-lane kernels' take those (yl_launches, one table; one chain of all
-// subsets per sweep template, yl_group_begin), the others the sweep kernels
+// subsets per group of plans, yl_group_begin), the others the sweep kernels
 // (launches, subset by subset, subset_begin): per subset, grouped
 // projections, the ratios, grouped rotated-frame backprojections, then the
 // pulls with the multiplicative update, with the same argument records as a
@@ -3058,11 +3058,30 @@ void batch_build(et_batch *b, int S, hipStream_t st)
     std::vector<et_plan *> ylp, oldp;
     for (et_plan *p : b->plans) (p->osem_yl ? ylp : oldp).push_back(p);
     b->subset_begin.assign((size_t)S + 1, 0);
-    // row-lane plans: one group per sweep template (their sweeps share
-    // launches); a group's chain holds all its subsets in order and depends on
-    // no other group's
-    std::map<std::tuple<int, int, int, int>, std::vector<et_plan *>> ygroups;
-    for (et_plan *p : ylp) ygroups[YlTable::sweep_key(p)].push_back(p);
+    // row-lane plans: groups of one sweep template (their sweeps share launches); a
+    // group's chain holds all its subsets in order and depends on no other group's.
+    // A group ends where its subsets' rotated-frame volumes reach 64 MiB, so that the
+    // four chains in flight keep theirs in the Infinity Cache and none is left alone
+    // at the end; the longest start first.  8 problems of 64^3 to 160 x 96 x 160: one
+    // group per template 7.39 ms per iteration, 64 MiB groups 7.15, in this order 7.00
+    // (32 to 300 MB alike); 48 problems 40.7 -> 40.3.
+    constexpr size_t GROUP_U = (size_t)64 << 20;
+    std::map<std::tuple<int, int, int, int>, std::vector<et_plan *>> templates;
+    for (et_plan *p : ylp) templates[YlTable::sweep_key(p)].push_back(p);
+    std::vector<std::pair<double, std::vector<et_plan *>>> ygroups;  // (work, plans)
+    for (auto &g : templates) {
+        size_t held = GROUP_U;
+        for (et_plan *p : g.second) {
+            if (held >= GROUP_U) {
+                ygroups.emplace_back();
+                held = 0;
+            }
+            held += sizeof(float) * p->ustride * (size_t)((p->V + S - 1) / S);
+            ygroups.back().first += (double)p->V * p->nvox * (4 * p->R + 24);  // ~ operations
+            ygroups.back().second.push_back(p);
+        }
+    }
+    std::stable_sort(ygroups.begin(), ygroups.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
     YlTable t;
     t.S = S;
     b->yl_group_begin.clear();
