@@ -67,6 +67,8 @@ int et_array_list_gpus(int *gpu_count, int *gpus_info_array);
 int et_array_set_gpu(int id);
 int et_array_set_gpu_pointer(int *id);
 int et_array_isinstalled(void);
+/* Also frees the device memory and streams kept between calls on host arrays
+ * (at most 2 GiB and 4 streams per process). */
 int et_array_reset_gpu(void);
 /* The kernels accept any volume size: both return values report that
  * (the reference required multiples of 64, emission-lib/_et.cpp:27-36). */
@@ -275,11 +277,10 @@ int et_plan_gradient_attenuation(et_plan *plan, const float *sino, const float *
 /* Both gradients of <sino, project(act, mu)> (sino holds dL/dp): out_act as
  * et_plan_backproject with adjoint 1, out_mu as et_plan_gradient_attenuation
  * with exact 1, one truncate flag for both.  No counterpart in the reference:
- * the backward pass of a differentiable projection.  Right after
- * et_plan_project of the same act and mu, plans on the row-lane kernels run
- * both rotated-frame sweeps and one exact adjoint pull whose candidate weights
- * serve both outputs (rotated-frame volumes of all views twice: at most
- * 4 GiB); otherwise the two operations in turn.  Outputs must not overlap
+ * the backward pass of a differentiable projection.  Plans on the row-lane or
+ * tile kernels form both from one set of packed sources, after et_plan_project
+ * of the same act and mu without another projector pass; others run the two
+ * operations in turn.  Outputs must not overlap
  * each other or an input: an output pointer equal to an input's or to the
  * other output's is rejected (niftyrec_error_parameters); partial overlaps
  * are not detected. */

@@ -1371,7 +1371,7 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
 
 // Both gradients of <sino, project(act, mu)>: the exact adjoint backprojection
 // of sino (activity) and the exact attenuation gradient (mu).  Row-lane plans
-// take one pass (yl_op_backward), others the two operations in turn.
+// take both from one set of sources (yl_op_backward), others run the two in turn.
 void op_backward(et_plan *p, const float *sino, const float *act, const float *mu, float *out_act, float *out_mu,
                  int truncate)
 {

@@ -24,10 +24,10 @@
 //
 // Layouts (rows = 16 * RPL, y fastest everywhere):
 //   factors   att[v][z'][x'][rows]  e^{-A(x', y, z')}, A the inclusive sum of mu' (none without
-//             attenuation: att null, every factor 1)
+//             attenuation: att null, every factor 1), rows in lane order (yl_iload)
 //   partials  part[d][v][x'][rows]  projection of depth chunk d
 //   measured counts and ratio       [v][x'][rows]
-//   U         u + v*ustride + y + rows*((x'+1) + xp*(z'+1))  (zero border in x', z')
+//   U         u + v*ustride + y + rows*((x'+1) + xp*(z'+1))  (zero border in x', z'), rows in lane order
 // Activity, attenuation and sensitivity are in the YF layout of the plan, whose
 // columns hold at least `rows` rows.
 #pragma once
