@@ -978,11 +978,9 @@ EtSweepArgs project_args(et_plan *p, const float *recs, int nv, const float *act
 }
 
 // Fast-path projection of nv views (records recs) into sino [nv][ny][nx].
-// att (with mu): the attenuation factors of the views, stored there by this
-// projection (att_read false) or read from there instead of resampling mu.
+// att (with mu): the attenuation factors of the views, read instead of resampling mu.
 void project_fast(et_plan *p, const float *recs, int nv, const float *act_yf, const float *mu_yf, float *sino,
-                  int truncate, int D, const float *astart, float *parts_out = nullptr, float *att = nullptr,
-                  bool att_read = false)
+                  int truncate, int D, const float *astart, float *parts_out = nullptr, float *att = nullptr)
 {
     float *part = parts_out;
     if (!part) part = (D == 1) ? sino : p->part.ensure((size_t)D * nv * p->P, false);
@@ -991,7 +989,7 @@ void project_fast(et_plan *p, const float *recs, int nv, const float *act_yf, co
     {
         const double bytes = (double)nv * ((mu_yf ? 8.0 : 4.0) * p->nvox + 4.0 * p->P);
         ProfScope ps(p, ET_PROF_PROJECT, bytes);
-        const int hm = mu_yf ? (a.att ? (att_read ? 3 : 2) : 1) : 0;
+        const int hm = mu_yf ? (a.att ? 3 : 1) : 0;
         check_launch(et_launch_sweep(ET_MODE_PROJECT, p->R, hm, 1, a, (et_stream_t)p->st));
     }
     if (D > 1 && !parts_out) {
@@ -1417,7 +1415,7 @@ void em_subset_update(et_plan *p, const float *recs, int nv, float *x_yf, const 
     p->u.ensure((size_t)nv * p->ustride, true, p->st);
     float *parts = p->part.ensure((size_t)Dp * nv * p->P, false);
     float *ratio = p->ratio.ensure((size_t)nv * p->P, false);
-    project_fast(p, recs, nv, x_yf, mu_yf, nullptr, 1, Dp, nullptr, parts, att, true);
+    project_fast(p, recs, nv, x_yf, mu_yf, nullptr, 1, Dp, nullptr, parts, att);
     {
         ProfScope ps(p, ET_PROF_OTHER, (Dp + 2.0) * 4.0 * nv * p->P);
         check_launch(et_launch_ratio_parts(meas, parts, Dp, (size_t)nv * p->P, eps, ratio, (et_stream_t)p->st));
@@ -1518,13 +1516,13 @@ int tune_depth_chunks(et_plan *p, int mode, const float *recs, int nv, const flo
             auto run = [&]() {
                 if (mode == ET_MODE_PROJECT) {
                     // with the ratio kernel, whose reads grow with the number of partial sums
-                    project_fast(p, recs, nv, act, mu_yf, nullptr, 1, D, as, parts, att, true);
+                    project_fast(p, recs, nv, act, mu_yf, nullptr, 1, D, as, parts, att);
                     check_launch(et_launch_ratio_parts(parts, parts, D, (size_t)nv * p->P, 1e-6f, ratio,
                                                        (et_stream_t)p->st));
                 } else {
                     // behind the chosen projection and its ratio, reading that ratio, as in
                     // the subset update (the cache state the backprojection meets there)
-                    project_fast(p, recs, nv, act, mu_yf, nullptr, 1, Dp, as, parts, att, true);
+                    project_fast(p, recs, nv, act, mu_yf, nullptr, 1, Dp, as, parts, att);
                     check_launch(et_launch_ratio_parts(parts, parts, Dp, (size_t)nv * p->P, 1e-6f, ratio,
                                                        (et_stream_t)p->st));
                     bpu_fast(p, recs, nv, mu_yf, ET_SRC_SINO, ratio, nullptr, nullptr, 0, 0.f, D, as, false, p->u.p,

@@ -135,9 +135,8 @@ void et_offer_launch_events(et_event_t start, et_event_t stop);
 bool et_claim_launch_events(et_event_t *start, et_event_t *stop);
 bool et_withdraw_launch_events();
 
-// has_mu: 0 no attenuation; 1 attenuation from the resampled a.mu; 2 (PROJECT)
-// as 1, and the attenuation factors stored in a.att; 3 (PROJECT, BPU) the
-// factors read from a.att instead of resampling mu.
+// has_mu: 0 no attenuation; 1 attenuation from the resampled a.mu; 3 (PROJECT,
+// BPU) the attenuation factors read from a.att instead of resampling mu.
 int et_launch_sweep(int mode, int R, int has_mu, int has_act, const EtSweepArgs &a,
                     et_stream_t stream);
 int et_launch_pull(const EtPullArgs &a, et_stream_t stream);

@@ -18,9 +18,8 @@ namespace {
 // grid: (slabs, V*D); block: nthr >= nx threads, thread tx owns column x' = tx.
 // PROJECT: partial projection of chunk d written to part[d][v][y][x]
 // (the sinogram itself when D == 1).  Reference emission-lib/_et.cpp:218-281.
-// AM (with HAS_MU): 0 attenuation from the resampled mu; 1 the same, and the
-// factors e^{-A} of every plane stored in a.att; 2 the factors read from a.att
-// (mu is not read).
+// AM (with HAS_MU): 0 attenuation from the resampled mu; 2 the factors e^{-A} of
+// every plane read from a.att (mu is not read).
 template <int TS, int R, bool HAS_MU, bool COOP, int AM>
 __device__ __forceinline__ void project_body(const EtSweepArgs &a, const Blk &b)
 {
@@ -107,16 +106,9 @@ __device__ __forceinline__ void project_body(const EtSweepArgs &a, const Blk &b)
             row_pass<TS, R>(lds, c.tx, yc, kz, h);
         }
         // factors of plane z in the padded layout att[v][z][yu][nthr]
-        // (coalesced over x'; every lane stores or loads)
-        float *ez = a.att + (((size_t)c.v * a.nz + z) * a.yu + c.y0) * c.nthr + c.tx;
-        if constexpr (HAS_MU && AM == 1) {
-#pragma unroll
-            for (int i = 0; i < TS; i++) {
-                const float e = exp_neg(A[i] + Al[i]);
-                kahan(i, h[i], e);
-                gstore(ez + i * c.nthr, e);
-            }
-        } else if constexpr (HAS_MU && AM == 2) {
+        // (coalesced over x')
+        const float *ez = a.att + (((size_t)c.v * a.nz + z) * a.yu + c.y0) * c.nthr + c.tx;
+        if constexpr (HAS_MU && AM == 2) {
 #pragma unroll
             for (int i = 0; i < TS; i++) kahan(i, h[i], gload(ez + i * c.nthr));
         } else {
@@ -548,8 +540,6 @@ static int launch_sweep_ts(int mode, int has_mu, const EtSweepArgs &a, hipStream
             dim3 g(slabs, a.V * a.D);
             if (has_mu == 3) {
                 if (coop) ET_LP(true, true, 2) else ET_LP(true, false, 2)
-            } else if (has_mu == 2) {
-                if (coop) ET_LP(true, true, 1) else ET_LP(true, false, 1)
             } else if (has_mu) {
                 if (coop) ET_LP(true, true, 0) else ET_LP(true, false, 0)
             } else {
