@@ -2209,7 +2209,7 @@ bool yl_op_gradient_ref(et_plan *p, const float *sino, const float *act, const f
 // gradient, each output what its operation on its own gives.  One pull of both
 // volumes, with one set of candidate weights, needs both of every view at once, 2
 // GB at 128^3 x 120 views that the Infinity Cache does not hold: it took 629 us
-// where the two pulls take about 500, and a GB more of memory.
+// where the two pulls take 570, and a GB more of memory.
 bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float *mu, float *out_act, float *out_mu,
                     int truncate)
 {
