@@ -2094,13 +2094,22 @@ bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *ou
     return true;
 }
 
-// Adds to t the forward sums that the gradient sweeps of this activity and map
-// start from: the last projection's, or formed here (the device decides by the
-// keys of yl_sources with fwd = 2).
-float *yl_gradient_forward(YlTable &t, et_plan *p, const float *fac, int D)
+// Whether the forward sums kept in the plan have the chunking that a gradient in D
+// chunks asks for.  They count as lost from here until yl_forward_kept: yl_sources
+// with fwd = 2 names them this gradient's on the device, and what comes between
+// (allocations, launches) may throw.  Called before yl_sources.
+bool yl_take_forward(et_plan *p, int D)
 {
     const bool same = p->fwd_built && p->fwd_D == D && p->fwd_tiles == p->yl_tiles;
-    p->fwd_built = false;  // until the sums are queued
+    p->fwd_built = false;
+    return same;
+}
+
+// Adds to t the forward sums that the gradient sweeps of this activity and map
+// start from: formed here, or (same: yl_take_forward) the last projection's where
+// the device finds its keys to be this pair's.
+float *yl_gradient_forward(YlTable &t, et_plan *p, const float *fac, int D, bool same)
+{
     return yl_forward(t, p, fac, D,
                       same ? reinterpret_cast<const int *>(
                                  reinterpret_cast<const unsigned long long *>(p->keys.p) + ET_KEY_SKIP_FWD)
@@ -2146,13 +2155,14 @@ void yl_gradient_views(YlTable &t, et_plan *p, const float *fac, const float *st
 bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float *mu, float *out, int truncate)
 {
     if (!p->yl_ops || !p->yl || !act || !mu || !yl_factor_room(p)) return false;
+    const int D = yl_forward_chunks(p, true);
+    const bool same = yl_take_forward(p, D);
     const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
-    const int D = yl_forward_chunks(p, true);
     const int vb = yl_u_views(p, yl_gradient_batch(p));
     float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
     YlTable t;
-    float *part = yl_gradient_forward(t, p, fac, D);
+    float *part = yl_gradient_forward(t, p, fac, D, same);
     yl_gradient_views(t, p, fac, st, part, D, vb, truncate != 0, acc);
     yl_run(p, t, YL_OP_GRADIENT);
     yl_forward_kept(p, D);
@@ -2214,15 +2224,16 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
                     int truncate)
 {
     if (!p->yl_ops || !p->yl || !act || !mu || !yl_factor_room(p)) return false;
+    const int D = yl_forward_chunks(p, true);
+    const bool same = yl_take_forward(p, D);
     const float *fac = yl_sources(p, act, mu, 2);
     const float *st = yl_sino_t(p, sino);
     const int want_b = view_batch(p), want_g = yl_gradient_batch(p);
     const int room = yl_u_views(p, std::max(want_b, want_g));
     float *acc_a = p->op_acc.ensure(p->yf_elems, true, p->st);
     float *acc_m = p->op_acc2.ensure(p->yf_elems, true, p->st);
-    const int D = yl_forward_chunks(p, true);
     YlTable t;
-    float *part = yl_gradient_forward(t, p, fac, D);
+    float *part = yl_gradient_forward(t, p, fac, D, same);
     yl_backproject_views(t, p, fac, st, std::min(want_b, room), true, truncate != 0, acc_a);
     yl_gradient_views(t, p, fac, st, part, D, std::min(want_g, room), truncate != 0, acc_m);
     yl_run(p, t, YL_OP_BACKWARD);

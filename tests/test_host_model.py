@@ -1,0 +1,124 @@
+"""The host layer (et_host.cpp) on a CPU model of the device
+(host_model/model.cpp): every launch's arguments are checked against the live
+device blocks, and results carry tags of what they were formed from, so that a
+call that used something stale differs from the same call on a fresh plan.
+Failed allocations and launches are forced from here."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+P, I, F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+STREAM = P(0x700)
+NO_LIMIT = (1 << 64) - 1
+ALLOC_FAILED = 4  # niftyrec_error_allocgpu
+
+
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("model") / "libmodel.so")
+    csrc = os.path.join(ROOT, "niftyrec_amd", "csrc")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-w", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                           "-D__align__(x)=__attribute__((aligned(x)))", "-DHIP_SYMBOL(x)=x", "-I/opt/rocm/include",
+                           "-I" + os.path.join(ROOT, "include"), "-I" + csrc, os.path.join(csrc, "et_host.cpp"),
+                           os.path.join(ROOT, "tests", "host_model", "model.cpp"), "-Wl,-Bsymbolic", "-Wl,-z,defs",
+                           "-o", out])
+    m = ctypes.CDLL(out)
+    for name, res, args in (("model_volume", P, [ctypes.c_size_t, ctypes.c_ulonglong]),
+                            ("model_set", None, [P, ctypes.c_ulonglong]), ("model_tag", ctypes.c_ulonglong, [P]),
+                            ("model_violations", ctypes.c_char_p, []), ("model_used", ctypes.c_size_t, []),
+                            ("model_limit", None, [ctypes.c_size_t]), ("model_fail", None, [ctypes.c_char_p, I]),
+                            ("model_count", I, [ctypes.c_char_p]), ("model_begin", None, [P]),
+                            ("model_replay", None, [I]),
+                            ("et_plan_create", I, [P, I, I, I, P, I, I, P, I, F, F]), ("et_plan_destroy", I, [P]),
+                            ("et_plan_project", I, [P, P, P, P, I, P]),
+                            ("et_plan_backproject", I, [P, P, P, P, I, I, P]),
+                            ("et_plan_gradient_attenuation", I, [P, P, P, P, P, I, I, P]),
+                            ("et_plan_project_backward", I, [P, P, P, P, P, P, I, P]),
+                            ("et_plan_osem", I, [P, P, P, P, I, I, F, P]), ("et_plan_set_mu_check", I, [P, I]),
+                            ("et_plan_set_tuning", I, [P, I, I]), ("et_plan_invalidate", I, [P])):
+        getattr(m, name).restype = res
+        getattr(m, name).argtypes = args
+    yield m
+    assert m.model_violations() == b""
+
+
+class Rig:
+    """Plans of one geometry (nx, ny, nz, views) and the volumes they work on."""
+
+    def __init__(self, model, nx, ny, nz, views, psf=0, cols=1, bg=0.0):
+        self.m, self.dims, self.V, self.K, self.cols, self.bg = model, (nx, ny, nz), views, psf, cols, bg
+        model.model_clear()
+        model.model_limit(NO_LIMIT)
+        self.seq = 100
+        self.plans, self.vols = [], []
+
+    def plan(self):
+        nx, ny, nz = self.dims
+        cams = (F * (self.V * self.cols))(*[0.1 + 0.3 * i for i in range(self.V * self.cols)])
+        psf = None if not self.K else (F * (self.K * self.K * nz))(*([0.5] * (self.K * self.K * nz)))
+        h = P()
+        assert self.m.et_plan_create(ctypes.byref(h), nx, ny, nz, cams, self.V, self.cols, psf, self.K, self.bg,
+                                     0.0) == 0
+        assert self.m.et_plan_set_mu_check(h, 0) == 0
+        self.plans.append(h)
+        return h
+
+    def vol(self, sino=False):
+        nx, ny, nz = self.dims
+        self.seq += 1
+        v = P(self.m.model_volume(nx * ny * (self.V if sino else nz), self.seq))
+        self.vols.append(v)
+        return v
+
+    def tag(self, v):
+        return self.m.model_tag(v)
+
+    def project(self, h, a, m, out, truncate=1):
+        return self.m.et_plan_project(h, a, m, out, truncate, STREAM)
+
+    def backproject(self, h, s, m, out, adjoint=0, truncate=1):
+        return self.m.et_plan_backproject(h, s, m, out, adjoint, truncate, STREAM)
+
+    def gradient(self, h, s, a, m, out, exact=1, truncate=1):
+        return self.m.et_plan_gradient_attenuation(h, s, a, m, out, exact, truncate, STREAM)
+
+    def backward(self, h, s, a, m, ga, gm):
+        return self.m.et_plan_project_backward(h, s, a, m, ga, gm, 0, STREAM)
+
+    def osem(self, h, x, y, m, subsets, eps=1e-6, iterations=1):
+        return self.m.et_plan_osem(h, x, y, m, subsets, iterations, eps, STREAM)
+
+    def close(self):
+        for h in self.plans:
+            assert self.m.et_plan_destroy(h) == 0
+        assert self.m.model_violations() == b""
+        for v in self.vols:
+            self.m.hipFree(v)
+
+
+@pytest.mark.parametrize("op", ["gradient", "backward"])
+@pytest.mark.parametrize("spare", [0, 30000, 250000, 500000])
+def test_gradient_after_a_failed_allocation(model, op, spare):
+    """A gradient that ran out of memory leaves no forward sums behind: the next
+    one of the same activity and map forms them, whatever was projected before."""
+    r = Rig(model, 40, 20, 32, 4)
+    A, B, M, S, out, out2 = r.vol(), r.vol(), r.vol(), r.vol(sino=True), r.vol(), r.vol()
+
+    def call(h, a):
+        return r.gradient(h, S, a, M, out) if op == "gradient" else r.backward(h, S, a, M, out2, out)
+
+    plan = r.plan()
+    assert r.project(plan, A, M, S) == 0
+    model.model_set(S, 7)
+    model.model_limit(model.model_used() + spare)
+    assert call(plan, B) == ALLOC_FAILED
+    model.model_limit(NO_LIMIT)
+    assert call(plan, B) == 0
+    got = r.tag(out)
+    assert call(r.plan(), B) == 0
+    assert got == r.tag(out)
+    r.close()
