@@ -1911,10 +1911,21 @@ const float *yl_sources(et_plan *p, const float *act, const float *mu, int fwd)
 }
 
 // Rotated-frame volumes for up to `want` views in p->u: fewer views where the
-// device has no room for them.
+// device has no room for them.  A buffer that holds fewer is kept, without asking
+// for more again at every call, unless there is room for all or for twice as many.
 int yl_u_views(et_plan *p, int want)
 {
-    for (int nv = want;; nv = (nv + 1) / 2) {
+    const int have = (int)std::min<size_t>(p->u.n / p->ustride, want);
+    if (have >= want) return want;
+    int nv = want;
+    if (have > 0) {
+        size_t room = 0, total = 0;
+        if (hipMemGetInfo(&room, &total) != hipSuccess) room = 0;
+        const size_t fit = have + room / (p->ustride * sizeof(float));
+        while ((size_t)nv > fit) nv = (nv + 1) / 2;
+        if (nv < want && nv < 2 * have) return have;
+    }
+    for (;; nv = (nv + 1) / 2) {
         try {
             p->u.ensure((size_t)nv * p->ustride, true, p->st);
             return nv;
@@ -2392,6 +2403,18 @@ void yl_osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, i
         yl_sources(p, nullptr, mu, 0);
         p->osem_key_gen = p->key_gen;
     }
+    // Every buffer the launch table refers to, before it is built, at every call: the
+    // single operations work in u and part too and may have left them smaller, or
+    // none at all, where an allocation failed.
+    auto buffers = [&](int D) {
+        p->x_yf.ensure(p->yf_elems, true, p->st);
+        p->osem_meas.ensure((size_t)p->V * pe, true, p->st);
+        p->u.ensure((size_t)maxsub * p->ustride, true, p->st);
+        p->ratio.ensure((size_t)maxsub * pe, true, p->st);
+        p->sens.ensure((size_t)S * p->yf_elems, true, p->st);
+        p->part.ensure((size_t)D * maxsub * pe, false);
+    };
+    if (!structure) buffers(p->osem_Dp);
     if (structure) {
         p->osem_struct = false;
         std::vector<float> recs((size_t)p->V * ET_VIEW_REC);
@@ -2407,15 +2430,9 @@ void yl_osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, i
                                  p->st),
                   niftyrec_error_transfergpu);
         check_hip(hipStreamSynchronize(p->st), niftyrec_error_kernel);  // (the host copies end here)
-        // every buffer the launch table refers to, before it is built
-        p->x_yf.ensure(p->yf_elems, true, p->st);
-        p->osem_meas.ensure((size_t)p->V * pe, true, p->st);
-        p->u.ensure((size_t)maxsub * p->ustride, true, p->st);
-        p->ratio.ensure((size_t)maxsub * pe, true, p->st);
-        p->sens.ensure((size_t)S * p->yf_elems, true, p->st);
         int Dmax = 1;
         for (int D : yl_chunk_candidates(p, start[1] - start[0])) Dmax = std::max(Dmax, D);
-        p->part.ensure((size_t)Dmax * maxsub * pe, false);
+        buffers(Dmax);
         int Dp = p->tune_D, Db = p->tune_D, zlen;
         yl_use_tiles(p, true);  // the tiled projector unless timing prefers the full-width one
         if (p->tune_D <= 0) {

@@ -122,3 +122,54 @@ def test_gradient_after_a_failed_allocation(model, op, spare):
     assert call(r.plan(), B) == 0
     assert got == r.tag(out)
     r.close()
+
+
+@pytest.mark.parametrize("op", ["gradient", "reference gradient", "backproject"])
+@pytest.mark.parametrize("chunks", [0, 1])
+def test_osem_after_an_operation_ran_out_of_memory(model, op, chunks):
+    """Operations share their work buffers with OSEM.  Whatever an operation that
+    found no room left of them, the next OSEM call has buffers of the size its
+    launches use."""
+    for spare in range(-1300000, 3000000, 100000):
+        r = Rig(model, 40, 20, 32, 12)
+        A, M, X, Y, S, out = r.vol(), r.vol(), r.vol(), r.vol(sino=True), r.vol(sino=True), r.vol()
+
+        def osem(h):
+            model.model_set(X, 5)
+            assert r.osem(h, X, Y, M, 3) == 0
+            return r.tag(X)
+
+        plan, fresh = r.plan(), r.plan()
+        for h in (plan, fresh):
+            assert model.et_plan_set_tuning(h, chunks, 0) == 0
+        ref = osem(fresh)
+        assert osem(plan) == ref
+        model.model_limit(max(0, model.model_used() + spare))
+        if op == "backproject":
+            r.backproject(plan, S, None, out, 1)
+        else:
+            r.gradient(plan, S, A, M, out, exact=int(op == "gradient"))
+        model.model_limit(NO_LIMIT)
+        assert osem(plan) == ref
+        assert model.model_violations() == b""
+        r.close()
+
+
+def test_scarce_memory_keeps_the_views_that_fit(model):
+    """Rotated-frame volumes for fewer views than asked for are kept from call to
+    call: no buffer is freed and asked for again."""
+    r = Rig(model, 40, 20, 32, 12)
+    S, out = r.vol(sino=True), r.vol()
+    big = r.plan()
+    before = model.model_used()
+    assert r.backproject(big, S, None, out) == 0
+    whole = model.model_used() - before
+    plan = r.plan()
+    model.model_limit(model.model_used() + whole - 400000)  # not the volumes of all 12 views
+    assert r.backproject(plan, S, None, out) == 0
+    assert model.model_count(b"fill") > 0
+    model.model_clear()
+    for _ in range(3):
+        assert r.backproject(plan, S, None, out) == 0
+    assert model.model_count(b"fill") == 0
+    r.close()
