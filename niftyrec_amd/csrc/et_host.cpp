@@ -518,7 +518,7 @@ struct et_plan {
     DevBuf fwd_part;
     int fwd_D = 0, fwd_tiles = 0;
     std::vector<struct YlLaunch> yl_launches;          // per subset: projection, ratio, backprojection, pull
-    std::vector<const void *> osem_sig;                // buffers yl_launches refer to
+    std::vector<const void *> osem_sig;                // buffers and epsilon that yl_launches refer to
     bool osem_struct = false;   // row-lane plans: records, chunking and tables are those of osem_S, osem_has_mu and
     int osem_tune_D = 0;        // tune_D = osem_tune_D (they do not depend on the map's content)
     unsigned osem_key_gen = 0;  // key_gen when the factors were last known to be the OSEM map's
@@ -2340,12 +2340,15 @@ int yl_tune_chunks(et_plan *p, int mode, int S, int nv, int Dp = 0)
     return c.first;
 }
 
-// Device buffers the row-lane OSEM launch table refers to.  A single
-// operation of the plan may grow (reallocate) some of them between OSEM calls;
-// the table is then rebuilt.
+// What the row-lane OSEM launch table was made from: device buffers, some of
+// which a single operation of the plan may reallocate between OSEM calls, and
+// the epsilon in its records.  The table is rebuilt when any of them differs.
 std::vector<const void *> yl_osem_sig(const et_plan *p)
 {
-    return {p->x_yf.p, p->osem_meas.p, p->part.p, p->ratio.p, p->u.p, p->sens.p, p->osem_recs.p, p->fac.p};
+    uint32_t eps;
+    std::memcpy(&eps, &p->osem_cur_eps, 4);
+    return {p->x_yf.p, p->osem_meas.p, p->part.p, p->ratio.p, p->u.p, p->sens.p, p->osem_recs.p, p->fac.p,
+            reinterpret_cast<const void *>((uintptr_t)eps)};
 }
 
 // Launch table of a row-lane OSEM run: per subset the sensitivity
@@ -2354,6 +2357,7 @@ std::vector<const void *> yl_osem_sig(const et_plan *p)
 void yl_osem_tables(et_plan *p, int S, const std::vector<int> &start)
 {
     const std::vector<et_plan *> one{p};
+    p->osem_sig.clear();  // (an upload that throws leaves no table)
     YlTable t;
     t.S = S;
     for (int pass = 0; pass < 2; pass++) {
@@ -2442,14 +2446,13 @@ void yl_osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, i
         yl_chunks(p, Dp, p->osem_Dp, zlen);
         yl_chunks(p, Db, p->osem_Db, zlen);
     }
-    // (a single operation may have reallocated a buffer of the table)
+    // (a single operation may have reallocated a buffer of the table; epsilon is in its records)
     if (structure || yl_osem_sig(p) != p->osem_sig) yl_osem_tables(p, S, start);
     p->osem_struct = true;
     p->osem_S = S;
     p->osem_has_mu = has_mu;
     p->osem_tune_D = p->tune_D;
     if (content) {
-        if (!structure && p->osem_eps != eps) yl_osem_tables(p, S, start);  // (epsilon is in the records)
         yl_issue(p->osem_tables.p, p->yl_launches, 0, 2 * (size_t)S, p->st, p);  // sensitivities
         p->osem_mu_key = mu_key;
         p->osem_eps = eps;

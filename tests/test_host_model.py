@@ -173,3 +173,27 @@ def test_scarce_memory_keeps_the_views_that_fit(model):
         assert r.backproject(plan, S, None, out) == 0
     assert model.model_count(b"fill") == 0
     r.close()
+
+
+@pytest.mark.parametrize("failing", ["yl_sweep", "yl_pull", "planes_t"])
+@pytest.mark.parametrize("nth", [1, 2, 3])
+def test_epsilon_after_a_failed_osem_call(model, failing, nth):
+    """An OSEM call with another epsilon that fails on its way leaves nothing of
+    that epsilon to the next call."""
+    r = Rig(model, 40, 20, 32, 6)
+    M, X, Y = r.vol(), r.vol(), r.vol(sino=True)
+
+    def osem(h, eps):
+        model.model_set(X, 5)
+        return r.osem(h, X, Y, M, 2, eps)
+
+    plan, fresh = r.plan(), r.plan()
+    assert osem(fresh, 0.5) == 0
+    ref = r.tag(X)
+    assert osem(plan, 0.5) == 0
+    model.model_fail(failing.encode(), nth)
+    osem(plan, 0.25)
+    model.model_fail(b"", 0)
+    assert osem(plan, 0.5) == 0
+    assert r.tag(X) == ref
+    r.close()
