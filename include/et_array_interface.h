@@ -237,7 +237,14 @@ int et_array_osem_ordered(float *activity_data, unsigned int size_x, unsigned in
 /* A plan holds the geometry (cameras, centres, PSF, backgrounds) on the device
  * and its own workspaces.  Array arguments below are DEVICE pointers in the
  * layouts of Part 1; `stream` is a hipStream_t (NULL: the default stream).
- * Calls on one plan must not overlap; distinct plans are independent. */
+ * Calls on one plan must not overlap; distinct plans are independent.
+ * Calls may be recorded into a HIP graph when they have nothing left to allocate:
+ * after one call of every operation that the plan is used for, for a graph holds
+ * the addresses of the plan's buffers.  A replay then does what the call does at
+ * that time: the content of the maps and activities is compared on the device.
+ * et_plan_osem can be recorded with et_plan_set_mu_check(plan, 0) where its caches
+ * are built already (otherwise it is refused), and its replays take the map to be
+ * the one they were built from. */
 typedef struct et_plan et_plan;
 
 /* Volumes up to 512 voxels wide (nx; the projection kernels hold one thread

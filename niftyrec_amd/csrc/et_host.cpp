@@ -50,6 +50,15 @@ inline void check_launch(int e)
     if (e != (int)hipSuccess) throw EtError{niftyrec_error_kernel};
 }
 
+// Whether launches on st are being recorded into a graph.
+bool is_capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &s) == hipSuccess) return s == hipStreamCaptureStatusActive;
+    (void)hipGetLastError();
+    return false;
+}
+
 // Selects the library's device; returns niftyrec_error_nogpuinstalled when
 // there is no usable HIP device.
 int select_device()
@@ -452,9 +461,13 @@ enum {
     YL_GREF = 7,        // reference attenuation gradient
     YL_PROJECT_IF = 8,  // projection that the device may skip
 };
-// Table slots of the single operations (each keeps its last upload).
-enum {
-    YL_OP_PROJECT = 0, YL_OP_BACKPROJECT = 1, YL_OP_GRADIENT = 2, YL_OP_BACKWARD = 3, YL_OP_GREF = 4, YL_OP_SLOTS = 5
+// A single operation's launch table on the device: what it holds (its bytes and
+// launches) and where.  Written once and not over again while a captured graph may
+// read it.
+struct OpTable {
+    std::vector<char> sig;
+    char *at;
+    bool stored;  // the device holds it (else: only after a replay of the graph that stores it)
 };
 
 struct et_plan {
@@ -504,19 +517,24 @@ struct et_plan {
     bool yl_ops = false;
     bool yl_osem = false;                 // OSEM on the row-lane kernels
     DevBuf fac, sino_t, op_acc, op_acc2;  // (op_acc, op_acc2: pull accumulators, YF layout)
-    DevBuf op_tables[YL_OP_SLOTS];        // per operation: its last table, and that table's bytes
-    std::vector<char> op_tables_h[YL_OP_SLOTS];
+    std::vector<OpTable> op_tables;               // the single operations' launch tables,
+    std::vector<std::unique_ptr<DevBuf>> op_mem;  // in these, op_mem_used bytes of the last
+    size_t op_mem_used = 0;
+    // this call's stream is being captured: what is issued runs at replays, if ever,
+    // so the host's flags stay as they are; and whether a captured graph uses the
+    // operations' tables / changes the keyed buffers behind the host
+    bool capturing = false, tables_captured = false, keys_captured = false;
     // content keys on the device (EtKeys), and what the host knows: key_gen the
     // operations so far, fac_built / fwd_built whether the factors / the forward
     // sums hold those of the last keys
     DevBuf keys;
     unsigned key_gen = 0;
     bool fac_built = false, fwd_built = false;
-    // the last projection's partial sums [D][V][x'][rows] (D chunks as asked of
-    // yl_chunks, the projector's tiles): an exact gradient of the same activity
-    // and map seeds its reverse sweeps from them instead of projecting again
+    // the last projection's partial sums with attenuation [D][V][x'][rows] (D chunks as
+    // asked of yl_chunks, the projector's tiles: the shape of its keys): an exact gradient
+    // of the same activity and map seeds its reverse sweeps from them instead of
+    // projecting again
     DevBuf fwd_part;
-    int fwd_D = 0, fwd_tiles = 0;
     std::vector<struct YlLaunch> yl_launches;          // per subset: projection, ratio, backprojection, pull
     std::vector<const void *> osem_sig;                // buffers and epsilon that yl_launches refer to
     bool osem_struct = false;   // row-lane plans: records, chunking and tables are those of osem_S, osem_has_mu and
@@ -1850,6 +1868,9 @@ bool yl_factor_room(et_plan *p)
     }
 }
 
+// Shape of the forward sums in D chunks (EtKeys).
+int yl_forward_shape(const et_plan *p, int D) { return D * 1024 + p->yl_tiles; }
+
 // Sources of a single operation: the YF copies of act and mu (either may be
 // null) and, with a map, the factors of every view in view order
 // ([v][z'][x'][rows], null without a map).  The factors and the forward sums are
@@ -1859,8 +1880,8 @@ bool yl_factor_room(et_plan *p)
 // on the device: the factor kernel of an unchanged map ends at once, a
 // projection that the forward sums make superfluous likewise (EtSweepArgs.skip),
 // and no call waits for the stream (32 x 24 x 32, 16 views: projection 33.6 ->
-// 19.4 us).  fwd: as EtKeys.
-const float *yl_sources(et_plan *p, const float *act, const float *mu, int fwd)
+// 19.4 us).  fwd: as EtKeys, for forward sums in D chunks; same: yl_take_forward.
+const float *yl_sources(et_plan *p, const float *act, const float *mu, int fwd, int D = 0, bool same = false)
 {
     EtPackArgs a;
     std::memset(&a, 0, sizeof(a));
@@ -1882,30 +1903,36 @@ const float *yl_sources(et_plan *p, const float *act, const float *mu, int fwd)
     if (n == 0) return nullptr;
     EtKeys k;
     std::memset(&k, 0, sizeof(k));
+    const bool fac_built = p->fac_built, fwd_built = p->fwd_built;
     if (mu) {
-        // (8-byte words: the state, which starts out unread, then the partial sums)
+        p->fac.ensure(yl_att_elems(p, p->V), false);
+        // (8-byte words: the state, then the partial sums)
         k.np = et_pack_keys_blocks(p->nx, p->ny, p->nz);
-        k.st = reinterpret_cast<unsigned long long *>(p->keys.ensure(2 * (ET_KEY_WORDS + 2 * (size_t)k.np), false));
+        k.st = reinterpret_cast<unsigned long long *>(
+            p->keys.ensure(2 * (ET_KEY_WORDS + 2 * (size_t)k.np), true, p->st));
+        a.st = k.st;
         a.parts = k.st + ET_KEY_WORDS;
         k.mu = a.parts;
         k.act = act ? a.parts + k.np : nullptr;
-        k.cur = (int)(p->key_gen & 1u);
-        k.fac_built = p->fac_built;
+        k.fac_built = fac_built;
+        k.fwd_built = fwd == 2 ? same : fwd_built;
         k.fwd = fwd;
+        k.shape = fwd ? yl_forward_shape(p, D) : 0;
+        p->keys_captured = p->keys_captured || p->capturing;
+        p->fac_built = p->fwd_built = false;  // until the launches are queued
     }
     {
         ProfScope ps(p, ET_PROF_OTHER, n * 8.0 * p->nvox);
         check_launch(et_launch_pack_keys(a, n, (et_stream_t)p->st));
     }
     if (!mu) return nullptr;
-    p->fac_built = false;  // until the launch is queued
-    p->fac.ensure(yl_att_elems(p, p->V), false);
     EtSweepArgs f = yl_sweep_args(p, p->d_recs.p, p->V, 1, p->fac.p);
     f.mu = p->mu_yf.p;
     const bool stream_out = yl_att_elems(p, p->V) * sizeof(float) > (256ull << 20);  // (the Infinity Cache)
     ProfScope ps(p, ET_PROF_OTHER, (double)p->V * 8.0 * p->nvox);
     check_launch(et_launch_yl_factors(p->yl_rpl, stream_out, f, k, (et_stream_t)p->st));
-    p->fac_built = true;
+    p->fac_built = fac_built || !p->capturing;
+    p->fwd_built = fwd_built;
     p->key_gen++;
     return p->fac.p;
 }
@@ -1917,6 +1944,7 @@ int yl_u_views(et_plan *p, int want)
 {
     const int have = (int)std::min<size_t>(p->u.n / p->ustride, want);
     if (have >= want) return want;
+    if (have > 0 && p->capturing) return have;
     int nv = want;
     if (have > 0) {
         size_t room = 0, total = 0;
@@ -1958,12 +1986,15 @@ float *yl_sino_t(et_plan *p, const float *sino)
     return t;
 }
 
-// Issues a single operation's table from its slot.  A table equal to the
-// slot's last upload (the same launches over the same buffers and sizes:
-// repeated calls) is on the device already and is not uploaded again (no
-// stream synchronisation); the comparison covers the device bytes and each
-// launch's kernel choice and offsets.
-void yl_run(et_plan *p, const YlTable &t, int slot)
+// Issues a single operation's table.  The tables of the operations that were
+// called before are on the device already (the same launches over the same
+// buffers and sizes: repeated calls); the comparison covers the device bytes and
+// each launch's kernel choice and offsets.  A new one is stored in stream order,
+// without a wait (first projection of a plan of 64^3, 64 views, without
+// attenuation: 95 us with an upload that waits, 87 without).  Every table has a
+// place of its own, because a captured graph reads the table it was captured with
+// at every replay, whatever other operations ran since.
+void yl_run(et_plan *p, const YlTable &t)
 {
     std::vector<char> sig = t.tb.bytes;
     for (const YlLaunch &l : t.L) {
@@ -1972,14 +2003,35 @@ void yl_run(et_plan *p, const YlTable &t, int slot)
         const char *c = reinterpret_cast<const char *>(f);
         sig.insert(sig.end(), c, c + sizeof(f));
     }
-    DevBuf &buf = p->op_tables[slot];
-    std::vector<char> &last = p->op_tables_h[slot];
-    if (!buf.p || last != sig) {
-        last.clear();  // (an upload that throws leaves the slot unmatched)
-        yl_upload(buf, t, p->st);
-        last.swap(sig);
+    size_t i = 0;
+    while (i < p->op_tables.size() && p->op_tables[i].sig != sig) i++;
+    if (i == p->op_tables.size()) {
+        constexpr size_t CHUNK = 64 << 10;
+        const size_t need = align256(t.tb.bytes.size());
+        auto room = [&]() { return !p->op_mem.empty() && p->op_mem_used + need <= p->op_mem.back()->n * sizeof(float); };
+        if (!room() && !p->op_mem.empty() && !p->tables_captured && !p->capturing) {
+            // full, and read by launches before this one only: start over
+            p->op_tables.clear();
+            p->op_mem_used = 0;
+        }
+        if (!room()) {
+            p->op_mem.emplace_back(new DevBuf());
+            p->op_mem_used = 0;
+            p->op_mem.back()->ensure(std::max(CHUNK, need) / sizeof(float), false);
+        }
+        p->op_tables.push_back({std::move(sig), reinterpret_cast<char *>(p->op_mem.back()->p) + p->op_mem_used, false});
+        p->op_mem_used += need;
+        i = p->op_tables.size() - 1;
     }
-    yl_issue(buf.p, t.L, 0, t.L.size(), p->st, p);
+    OpTable &o = p->op_tables[i];
+    if (!o.stored) {
+        std::vector<char> bytes = t.tb.bytes;
+        bytes.resize(align256(bytes.size()));
+        check_launch(et_launch_store(o.at, bytes.data(), bytes.size(), (et_stream_t)p->st));
+        o.stored = !p->capturing;
+    }
+    p->tables_captured = p->tables_captured || p->capturing;
+    yl_issue(reinterpret_cast<const float *>(o.at), t.L, 0, t.L.size(), p->st, p);
 }
 
 // Adds to t the pull of nv views' rotated-frame volumes (p->u) into the YF
@@ -1998,13 +2050,14 @@ void yl_pull_into(YlTable &t, et_plan *p, const float *recs, int nv, bool adjoin
                           });
 }
 
-// Adds to t the projection of every view into the forward sums p->fwd_part (D
-// chunks asked for), not done where *skip is set.
+// Adds to t the projection of every view into partial sums (D chunks asked for),
+// not done where *skip is set: with attenuation the forward sums p->fwd_part, else
+// p->part, for which there is no key.
 float *yl_forward(YlTable &t, et_plan *p, const float *fac, int D, const int *skip)
 {
     int Deff, zlen;
     yl_chunks(p, D, Deff, zlen);
-    float *part = p->fwd_part.ensure((size_t)Deff * p->V * yl_plane_elems(p), false);
+    float *part = (fac ? p->fwd_part : p->part).ensure((size_t)Deff * p->V * yl_plane_elems(p), false);
     t.grouped<EtSweepArgs>(skip ? YL_PROJECT_IF : YL_PROJECT, {p}, YlTable::project_key,
                            [&](int, int &gx, int &gy, double &bytes) {
         bytes += (double)p->V * ((fac ? 8.0 : 4.0) * p->nvox + 4.0 * p->P);
@@ -2046,23 +2099,37 @@ int yl_forward_chunks(const et_plan *p, bool mu)
     return D;
 }
 
+// Whether the device may take the forward sums in the plan for a gradient's.  They
+// count as lost from here until yl_forward_kept: yl_sources with fwd = 2 names them
+// this gradient's on the device, and what comes between (allocations, launches) may
+// throw.  Called before yl_sources.
+bool yl_take_forward(et_plan *p)
+{
+    const bool same = p->fwd_built;
+    p->fwd_built = false;
+    return same;
+}
+
+// The launches that leave this operation's forward sums are queued (under capture:
+// the plan still holds those of the call before, kept as it said).
+void yl_forward_kept(et_plan *p, bool before) { p->fwd_built = p->capturing ? before : true; }
+
 bool yl_op_project(et_plan *p, const float *act, const float *mu, float *sino, int truncate)
 {
     if (!p->yl_ops || !p->yl || !act || (mu && !yl_factor_room(p))) return false;
-    p->fwd_built = false;  // until the sums are queued
-    const float *fac = yl_sources(p, act, mu, 1);
     const int D = yl_forward_chunks(p, mu != nullptr);
+    const bool kept = p->fwd_built;
+    if (mu) p->fwd_built = false;  // until the sums are queued
+    const float *fac = yl_sources(p, act, mu, 1, D);
     int Deff, zlen;
     yl_chunks(p, D, Deff, zlen);
     YlTable t;
     const float *part = yl_forward(t, p, fac, D, nullptr);
-    yl_run(p, t, YL_OP_PROJECT);
+    yl_run(p, t);
     ProfScope ps(p, ET_PROF_OTHER, (Deff + 1.0) * 4.0 * p->V * p->P);
     check_launch(
         et_launch_yl_parts_to_sino(part, Deff, p->V, p->nx, p->ny, p->yu, truncate, sino, (et_stream_t)p->st));
-    p->fwd_built = mu != nullptr;  // (without a map there is no gradient to seed, and no key)
-    p->fwd_D = D;
-    p->fwd_tiles = p->yl_tiles;
+    if (mu) yl_forward_kept(p, kept);
     return true;
 }
 
@@ -2099,39 +2166,21 @@ bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *ou
     float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
     YlTable t;
     yl_backproject_views(t, p, fac, st, vb, adjoint, truncate != 0, acc);
-    yl_run(p, t, YL_OP_BACKPROJECT);
+    yl_run(p, t);
     ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc, out, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
     return true;
 }
 
-// Whether the forward sums kept in the plan have the chunking that a gradient in D
-// chunks asks for.  They count as lost from here until yl_forward_kept: yl_sources
-// with fwd = 2 names them this gradient's on the device, and what comes between
-// (allocations, launches) may throw.  Called before yl_sources.
-bool yl_take_forward(et_plan *p, int D)
-{
-    const bool same = p->fwd_built && p->fwd_D == D && p->fwd_tiles == p->yl_tiles;
-    p->fwd_built = false;
-    return same;
-}
-
 // Adds to t the forward sums that the gradient sweeps of this activity and map
-// start from: formed here, or (same: yl_take_forward) the last projection's where
-// the device finds its keys to be this pair's.
+// start from: formed here, or (same: yl_take_forward) those that are kept where the
+// device finds its keys to be this pair's.
 float *yl_gradient_forward(YlTable &t, et_plan *p, const float *fac, int D, bool same)
 {
     return yl_forward(t, p, fac, D,
                       same ? reinterpret_cast<const int *>(
                                  reinterpret_cast<const unsigned long long *>(p->keys.p) + ET_KEY_SKIP_FWD)
                            : nullptr);
-}
-
-void yl_forward_kept(et_plan *p, int D)
-{
-    p->fwd_built = true;
-    p->fwd_D = D;
-    p->fwd_tiles = p->yl_tiles;
 }
 
 // Adds to t the gradient of every view into acc, in batches of vb views: the sweep
@@ -2167,16 +2216,16 @@ bool yl_op_gradient(et_plan *p, const float *sino, const float *act, const float
 {
     if (!p->yl_ops || !p->yl || !act || !mu || !yl_factor_room(p)) return false;
     const int D = yl_forward_chunks(p, true);
-    const bool same = yl_take_forward(p, D);
-    const float *fac = yl_sources(p, act, mu, 2);
+    const bool same = yl_take_forward(p);
+    const float *fac = yl_sources(p, act, mu, 2, D, same);
     const float *st = yl_sino_t(p, sino);
     const int vb = yl_u_views(p, yl_gradient_batch(p));
     float *acc = p->op_acc.ensure(p->yf_elems, true, p->st);
     YlTable t;
     float *part = yl_gradient_forward(t, p, fac, D, same);
     yl_gradient_views(t, p, fac, st, part, D, vb, truncate != 0, acc);
-    yl_run(p, t, YL_OP_GRADIENT);
-    yl_forward_kept(p, D);
+    yl_run(p, t);
+    yl_forward_kept(p, same);
     ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc, out, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
     return true;
@@ -2220,7 +2269,7 @@ bool yl_op_gradient_ref(et_plan *p, const float *sino, const float *act, const f
         sweep(YL_GREF, v0, nv, YlTable::sweep_key);
         yl_pull_into(t, p, p->d_recs.p + (size_t)v0 * ET_VIEW_REC, nv, false, v0 > 0, v0 + nv >= p->V && truncate, acc);
     }
-    yl_run(p, t, YL_OP_GREF);
+    yl_run(p, t);
     ProfScope ps(p, ET_PROF_OTHER, 8.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc, out, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
     return true;
@@ -2236,8 +2285,8 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
 {
     if (!p->yl_ops || !p->yl || !act || !mu || !yl_factor_room(p)) return false;
     const int D = yl_forward_chunks(p, true);
-    const bool same = yl_take_forward(p, D);
-    const float *fac = yl_sources(p, act, mu, 2);
+    const bool same = yl_take_forward(p);
+    const float *fac = yl_sources(p, act, mu, 2, D, same);
     const float *st = yl_sino_t(p, sino);
     const int want_b = view_batch(p), want_g = yl_gradient_batch(p);
     const int room = yl_u_views(p, std::max(want_b, want_g));
@@ -2247,8 +2296,8 @@ bool yl_op_backward(et_plan *p, const float *sino, const float *act, const float
     float *part = yl_gradient_forward(t, p, fac, D, same);
     yl_backproject_views(t, p, fac, st, std::min(want_b, room), true, truncate != 0, acc_a);
     yl_gradient_views(t, p, fac, st, part, D, std::min(want_g, room), truncate != 0, acc_m);
-    yl_run(p, t, YL_OP_BACKWARD);
-    yl_forward_kept(p, D);
+    yl_run(p, t);
+    yl_forward_kept(p, same);
     ProfScope ps(p, ET_PROF_OTHER, 16.0 * p->nvox);
     check_launch(et_launch_unpack_yf(acc_a, out_act, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
     check_launch(et_launch_unpack_yf(acc_m, out_mu, p->nx, p->ny, p->nz, p->yp, p->gy, (et_stream_t)p->st));
@@ -2398,12 +2447,16 @@ void yl_osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, i
     const bool content = structure || !p->osem_valid || p->osem_mu_key != mu_key || p->osem_eps != eps;
     const size_t pe = yl_plane_elems(p);
     const int maxsub = (p->V + S - 1) / S;
+    // a rebuild belongs into no captured graph: later calls would take the caches for
+    // built, and the table is copied from host memory
+    if (content && p->capturing) throw EtError{niftyrec_error_kernel};
     p->osem_cur_eps = eps;
     p->osem_mu_yf = has_mu;
     if (content) p->osem_valid = false;  // until the rebuild is queued
     // the map's factors; after an OSEM call of the same map only if another
-    // operation has formed factors meanwhile (then it is the device that compares)
-    if (has_mu && (content || p->key_gen != p->osem_key_gen)) {
+    // operation has formed factors meanwhile, or a replay of a captured one may have
+    // (then it is the device that compares); a captured call compares at every replay
+    if (has_mu && (content || p->key_gen != p->osem_key_gen || p->keys_captured || p->capturing)) {
         yl_sources(p, nullptr, mu, 0);
         p->osem_key_gen = p->key_gen;
     }
@@ -2447,7 +2500,10 @@ void yl_osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, i
         yl_chunks(p, Db, p->osem_Db, zlen);
     }
     // (a single operation may have reallocated a buffer of the table; epsilon is in its records)
-    if (structure || yl_osem_sig(p) != p->osem_sig) yl_osem_tables(p, S, start);
+    if (structure || yl_osem_sig(p) != p->osem_sig) {
+        if (p->capturing) throw EtError{niftyrec_error_kernel};
+        yl_osem_tables(p, S, start);
+    }
     p->osem_struct = true;
     p->osem_S = S;
     p->osem_has_mu = has_mu;
@@ -3282,6 +3338,7 @@ void op_batch_osem(et_batch *b, float *const *act, const float *const *sino, con
     for (size_t i = 0; i < b->plans.size(); i++) {
         et_plan *p = b->plans[i];
         p->st = st;
+        p->capturing = is_capturing(st);
         const float *m = mu ? mu[i] : nullptr;
         mu_key_launch(p, m);
         any_fp = any_fp || (m && p->mu_check);
@@ -3989,6 +4046,7 @@ int et_plan_destroy(et_plan *plan)
     if (!plan) return niftyrec_error_parameters;                                \
     if (hipSetDevice(plan->device) != hipSuccess) return niftyrec_error_nogpuinstalled; \
     plan->st = reinterpret_cast<hipStream_t>(stream);                           \
+    plan->capturing = is_capturing(plan->st);                                   \
     return guarded([&]() -> int { body; return niftyrec_success; });
 
 int et_plan_project(et_plan *plan, const float *act, const float *mu, float *sino, int truncate, void *stream)

@@ -168,6 +168,10 @@ int et_launch_conv_axis(const float *src, float *dst, int nx, int ny, int nz, lo
                         et_stream_t stream);
 int et_launch_truncate(float *buf, size_t n, et_stream_t stream);
 int et_launch_fill(float *buf, size_t n, float value, et_stream_t stream);
+// bytes (a multiple of 16) from host memory, read before the call returns, to the
+// device address dst (16-byte aligned), in stream order: they travel as kernel
+// arguments, so nothing is waited for and a captured graph holds them.
+int et_launch_store(void *dst, const void *src, size_t bytes, et_stream_t stream);
 int et_launch_clamp_min(float *buf, size_t n, float lo, et_stream_t stream);
 int et_launch_yf_clamp_min(float *yf, int nx, int ny, int nz, int yp, int gy, float lo,
                            et_stream_t stream);
@@ -210,27 +214,52 @@ struct EtPackArgs {
     float *dst[2];
     int guard[2];
     unsigned long long *parts;
+    unsigned long long *st;  // key state that this launch opens (et_keys_begin), or null
     int nx, ny, nz, yp;
 };
 int et_pack_keys_blocks(int nx, int ny, int nz);
 int et_launch_pack_keys(const EtPackArgs &a, int n, et_stream_t stream);
 
 // Content keys of a plan's single operations, kept and compared on the device
-// (no host synchronisation).  mu, act: the operation's partial sums (np each;
-// act null when the operation reads none).  st: ET_KEY_WORDS words, two slots
-// per key; the operation reads slot cur ^ 1, which the one before it wrote, and
-// writes slot cur, so that no block of the launch reads a word that another
-// block of it writes.
-enum { ET_KEY_MU = 0, ET_KEY_FWD_MU = 2, ET_KEY_FWD_ACT = 4, ET_KEY_SKIP_FWD = 6, ET_KEY_WORDS = 8 };
+// (no host synchronisation; a captured operation compares at every replay).  mu,
+// act: the operation's partial sums (np each; act null when the operation reads
+// none).  st: ET_KEY_WORDS words, zero at first: which of two slots is open, two
+// slots per key, and the decision on the forward sums.  The pack launch opens the
+// slot that the operation before it did not write; the factor launch reads that
+// operation's slot and writes the open one, so that no block of it reads a word
+// that another block writes.
+enum {
+    ET_KEY_SLOT = 0, ET_KEY_MU = 1, ET_KEY_FWD_MU = 3, ET_KEY_FWD_ACT = 5, ET_KEY_FWD_SHAPE = 7, ET_KEY_SKIP_FWD = 9,
+    ET_KEY_WORDS = 10
+};
 struct EtKeys {
     const unsigned long long *mu, *act;
     int np;
     unsigned long long *st;
-    int cur;
-    int fac_built;  // the factor buffer holds the factors of slot cur ^ 1's map
+    int fac_built;  // the factor buffer holds the factors of the last slot's map
+    int fwd_built;  // the forward sums are those of the last slot's keys
     int fwd;        // 0: the forward sums stay as they are; 1: this operation forms them;
-                    // 2: formed again unless those of slot cur ^ 1 are this pair's (st[ET_KEY_SKIP_FWD])
+                    // 2: formed again unless they are this pair's in this shape (st[ET_KEY_SKIP_FWD])
+    int shape;      // their chunks and tiles, not 0
 };
+// (constexpr: for the kernels and for host code)
+constexpr void et_keys_begin(unsigned long long *st) { st[ET_KEY_SLOT] ^= 1; }
+constexpr bool et_keys_keep_factors(const EtKeys &k, unsigned long long km)
+{
+    return k.fac_built && k.st[ET_KEY_MU + (k.st[ET_KEY_SLOT] ^ 1)] == km;
+}
+constexpr void et_keys_end(const EtKeys &k, unsigned long long km, unsigned long long ka)
+{
+    unsigned long long *mu = k.st + ET_KEY_MU, *fm = k.st + ET_KEY_FWD_MU, *fa = k.st + ET_KEY_FWD_ACT,
+                       *fs = k.st + ET_KEY_FWD_SHAPE;
+    const int cur = (int)k.st[ET_KEY_SLOT], last = cur ^ 1;
+    mu[cur] = km;
+    k.st[ET_KEY_SKIP_FWD] =
+        k.fwd == 2 && k.fwd_built && fm[last] == km && fa[last] == ka && fs[last] == (unsigned long long)k.shape;
+    fm[cur] = k.fwd ? km : fm[last];
+    fa[cur] = k.fwd ? ka : fa[last];
+    fs[cur] = k.fwd ? (unsigned long long)k.shape : (k.fwd_built ? fs[last] : 0);
+}
 
 // Row-lane kernels of the OSEM subset loop (et_yl.h).  Grouped launches only
 // (tab as et_launch_sweep_group): sweeps kind 0 projection, 1 rotated-frame

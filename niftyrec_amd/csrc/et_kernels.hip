@@ -494,6 +494,19 @@ __global__ void __launch_bounds__(256) k_pack_yf(const float *__restrict__ abi, 
     }
 }
 
+// dst[i] = a.v[i], i < n: up to 2 KiB that travel as kernel arguments.
+constexpr int STORE_WORDS = 128;
+typedef unsigned store_word __attribute__((ext_vector_type(4)));
+struct StoreArgs {
+    store_word v[STORE_WORDS];
+};
+__global__ void __launch_bounds__(STORE_WORDS) k_store(StoreArgs a, store_word *__restrict__ dst, int n)
+{
+    // (read where the arguments lie: indexing `a` by thread would copy it first)
+    const ET_CONST_AS store_word *v = (const ET_CONST_AS store_word *)__builtin_amdgcn_kernarg_segment_ptr();
+    if ((int)threadIdx.x < n) dst[threadIdx.x] = v[threadIdx.x];
+}
+
 // k_pack_yf for up to two volumes with the fingerprints of what it reads
 // (EtPackArgs): a single operation's sources and their content keys in one
 // launch (at 32 x 24 x 32 three launches, a copy and a stream synchronisation
@@ -508,6 +521,7 @@ __global__ void __launch_bounds__(256) k_pack_keys(EtPackArgs a, int zb)
     float *__restrict__ dst = a.dst[vol];
     const int xb = blockIdx.x * 32, yb = blockIdx.y * 32, guard = a.guard[vol];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    if (a.st && threadIdx.x == 0 && blockIdx.x + blockIdx.y + blockIdx.z == 0) et_keys_begin(a.st);
     unsigned long long h = 0;
     for (int z = z0; z < a.nz; z += zb) {
         for (int k = ty; k < 32; k += 8) {
@@ -1058,6 +1072,21 @@ int et_launch_fill(float *buf, size_t n, float value, et_stream_t stream)
 {
     hipLaunchKernelGGL(k_fill, dim3(nblk(n, 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), buf, n, value);
     return (int)hipGetLastError();
+}
+
+int et_launch_store(void *dst, const void *src, size_t bytes, et_stream_t stream)
+{
+    if (bytes % 16 != 0) return (int)hipErrorInvalidValue;
+    for (size_t at = 0; at < bytes; at += sizeof(StoreArgs)) {
+        StoreArgs a;
+        const size_t n = std::min(bytes - at, sizeof(StoreArgs));
+        std::memcpy(&a, static_cast<const char *>(src) + at, n);
+        hipLaunchKernelGGL(k_store, dim3(1), dim3(STORE_WORDS), 0, reinterpret_cast<hipStream_t>(stream), a,
+                           reinterpret_cast<store_word *>(static_cast<char *>(dst) + at), (int)(n / 16));
+        const int e = (int)hipGetLastError();
+        if (e != (int)hipSuccess) return e;
+    }
+    return (int)hipSuccess;
 }
 
 int et_launch_clamp_min(float *buf, size_t n, float lo, et_stream_t stream)

@@ -1592,35 +1592,27 @@ __device__ __forceinline__ void yl_factor_body(const EtSweepArgs &a)
     }
 }
 
-// Keys of a single operation (EtKeys; the OSEM caches pass none): every block
-// adds up the map's partial fingerprints and stops if its key is the one the
-// factors were formed from; block (0, 0) writes the keys of this operation and
-// whether its forward sums are there already.  At 128^3 the launch takes about
-// 8 us where the factors stay; a host that read the keys waited for the stream.
+// Keys (EtKeys): every block adds up the map's partial fingerprints and stops if
+// its key is the one the factors were formed from; block (0, 0) writes the keys of
+// this operation and whether its forward sums are there already.  At 128^3 the
+// launch takes about 8 us where the factors stay; a host that read the keys waited
+// for the stream.
 template <int RPL, bool STREAM>
 __global__ void __launch_bounds__(256) k_yl_factors(EtSweepArgs a, EtKeys k)
 {
-    if (k.st) {
-        __shared__ unsigned long long part[4];
-        unsigned long long h = 0;
-        for (int i = threadIdx.x; i < k.np; i += 256) h += k.mu[i];
-        const unsigned long long km = block_sum_256(h, part);
-        const int prev = k.cur ^ 1;
-        if (blockIdx.x == 0 && blockIdx.y == 0) {
-            h = 0;
-            if (k.act)
-                for (int i = threadIdx.x; i < k.np; i += 256) h += k.act[i];
-            const unsigned long long ka = block_sum_256(h, part);
-            if (threadIdx.x == 0) {
-                const unsigned long long fm = k.st[ET_KEY_FWD_MU + prev], fa = k.st[ET_KEY_FWD_ACT + prev];
-                k.st[ET_KEY_MU + k.cur] = km;
-                k.st[ET_KEY_FWD_MU + k.cur] = k.fwd ? km : fm;
-                k.st[ET_KEY_FWD_ACT + k.cur] = k.fwd ? ka : fa;
-                *reinterpret_cast<int *>(k.st + ET_KEY_SKIP_FWD) = k.fwd == 2 && fm == km && fa == ka;
-            }
-        }
-        if (k.fac_built && k.st[ET_KEY_MU + prev] == km) return;
+    __shared__ unsigned long long part[4];
+    unsigned long long h = 0;
+    for (int i = threadIdx.x; i < k.np; i += 256) h += k.mu[i];
+    const unsigned long long km = block_sum_256(h, part);
+    const bool keep = et_keys_keep_factors(k, km);
+    if (blockIdx.x == 0 && blockIdx.y == 0) {
+        h = 0;
+        if (k.act)
+            for (int i = threadIdx.x; i < k.np; i += 256) h += k.act[i];
+        const unsigned long long ka = block_sum_256(h, part);
+        if (threadIdx.x == 0) et_keys_end(k, km, ka);
     }
+    if (keep) return;
     yl_factor_body<RPL, STREAM>(a);
 }
 

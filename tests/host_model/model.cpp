@@ -368,6 +368,13 @@ int et_launch_fill(float *buf, size_t n, float value, et_stream_t st)
         set_tag(buf, mix(3, v));
     });
 }
+int et_launch_store(void *dst, const void *src, size_t bytes, et_stream_t st)
+{
+    const std::string b(static_cast<const char *>(src), bytes);
+    return launch("store", st, {dst}, [=]() {
+        if (need(dst, bytes / 4, "table")) std::memcpy(dst, b.data(), bytes);
+    });
+}
 int et_launch_fingerprint(const float *p, size_t n, u64 *parts, et_stream_t st)
 {
     return launch("fingerprint", st, {p, parts}, [=]() {
@@ -391,6 +398,7 @@ int et_launch_unpack_yf(const float *yf, float *abi, int nx, int ny, int nz, int
 int et_launch_pack_keys(const EtPackArgs &a, int n, et_stream_t st)
 {
     return launch("pack_keys", st, {a.src[0], a.src[1], a.dst[0], a.dst[1]}, [=]() {
+        if (a.st && need(a.st, 2 * ET_KEY_WORDS, "keys")) et_keys_begin(a.st);
         for (int k = 0; k < n; k++) {
             if (!need(a.src[k], (size_t)a.nx * a.ny * a.nz, "volume") ||
                 !need(a.dst[k], (size_t)a.yp * (a.nx + 2) * (a.nz + 2), "YF copy"))
@@ -409,13 +417,8 @@ int et_launch_yl_factors(int, bool, const EtSweepArgs &a, const EtKeys &k, et_st
         const u64 t = sweep_reads(a, false, true, 0, 0);
         if (!need(a.att, yl_att(a), "factors") || !need(k.st, 2 * ET_KEY_WORDS, "keys")) return;
         const u64 km = k.mu[0] + k.mu[1], ka = k.act ? k.act[0] + k.act[1] : 0;
-        const int prev = k.cur ^ 1;
-        const u64 fm = k.st[ET_KEY_FWD_MU + prev], fa = k.st[ET_KEY_FWD_ACT + prev];
-        const bool keep = k.fac_built && k.st[ET_KEY_MU + prev] == km;
-        k.st[ET_KEY_MU + k.cur] = km;
-        k.st[ET_KEY_FWD_MU + k.cur] = k.fwd ? km : fm;
-        k.st[ET_KEY_FWD_ACT + k.cur] = k.fwd ? ka : fa;
-        *reinterpret_cast<int *>(k.st + ET_KEY_SKIP_FWD) = k.fwd == 2 && fm == km && fa == ka;
+        const bool keep = et_keys_keep_factors(k, km);
+        et_keys_end(k, km, ka);
         if (keep) return;
         log_.push_back("factors built");
         set_tag(a.att, t);

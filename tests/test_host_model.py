@@ -197,3 +197,156 @@ def test_epsilon_after_a_failed_osem_call(model, failing, nth):
     assert osem(plan, 0.5) == 0
     assert r.tag(X) == ref
     r.close()
+
+
+class Calls:
+    """The single operations and OSEM on one plan's buffers, and on a fresh plan
+    for comparison."""
+
+    def __init__(self, r):
+        self.r = r
+        self.A, self.B, self.M, self.N = (r.vol() for _ in range(4))
+        self.S, self.Y = r.vol(sino=True), r.vol(sino=True)
+
+    def outputs(self):
+        r = self.r
+        return dict(sino=r.vol(sino=True), img=r.vol(), img2=r.vol())
+
+    def call(self, h, op, o):
+        r = self.r
+        st = {"project A M": lambda: r.project(h, self.A, self.M, o["sino"]),
+              "project B M": lambda: r.project(h, self.B, self.M, o["sino"]),
+              "project A N": lambda: r.project(h, self.A, self.N, o["sino"]),
+              "project A": lambda: r.project(h, self.A, None, o["sino"]),
+              "adjoint": lambda: r.backproject(h, self.S, None, o["img"], 1, 0),
+              "reference": lambda: r.backproject(h, self.S, None, o["img"], 0, 1),
+              "adjoint M": lambda: r.backproject(h, self.S, self.M, o["img"], 1, 0),
+              "gradient A M": lambda: r.gradient(h, self.S, self.A, self.M, o["img"]),
+              "gradient B N": lambda: r.gradient(h, self.S, self.B, self.N, o["img"]),
+              "reference gradient": lambda: r.gradient(h, self.S, self.A, self.M, o["img"], 0),
+              "backward A M": lambda: r.backward(h, self.S, self.A, self.M, o["img"], o["img2"]),
+              "osem M": lambda: r.osem(h, o["img"], self.Y, self.M, 2),
+              "osem": lambda: r.osem(h, o["img"], self.Y, None, 2)}[op]
+        if op.startswith("osem"):
+            r.m.model_set(o["img"], 9)
+        return st()
+
+    def tags(self, o):
+        return [self.r.tag(v) for v in o.values()]
+
+    def fresh(self, op):
+        o = self.outputs()
+        for v in o.values():
+            self.r.m.model_set(v, 3)
+        assert self.call(self.r.plan(), op, o) == 0
+        return self.tags(o)
+
+
+CAPTURED = ["project A M", "project A", "adjoint", "adjoint M", "gradient A M", "reference gradient", "backward A M",
+            "osem M", "osem"]
+BETWEEN = ["project B M", "project A N", "project A", "adjoint", "reference", "gradient B N", "gradient A M",
+           "rewrite", "invalidate", "osem M"]
+
+
+@pytest.mark.parametrize("op", CAPTURED)
+def test_captured_calls(model, op):
+    """A captured call gives at every replay what the call gives on a fresh plan
+    then, whatever ran in between; so do the calls after a replay."""
+    r = Rig(model, 40, 20, 32, 6)
+    c = Calls(r)
+    plan, o, e = r.plan(), c.outputs(), c.outputs()
+    for warm in BETWEEN + [op]:  # every buffer has its size, and the caches are some other map's
+        if warm not in ("rewrite", "invalidate"):
+            assert c.call(plan, warm, e) == 0
+    if op.startswith("osem"):
+        assert c.call(plan, op, o) == 0  # (the caches are built by a call of its own)
+    model.model_begin(STREAM)
+    assert c.call(plan, op, o) == 0
+    g = model.model_end()
+
+    def replay():
+        for v in o.values():
+            model.model_set(v, 9 if op.startswith("osem") else 3)
+        model.model_replay(g)
+        got = c.tags(o)
+        ref = c.fresh(op)
+        if op.startswith("osem"):
+            got, ref = got[1:2], ref[1:2]
+        assert got == ref
+
+    replay()
+    for step, between in enumerate(BETWEEN):
+        if op.startswith("osem") and between in ("osem M", "rewrite", "invalidate"):
+            continue  # (the caller's part: the sensitivities are the captured call's)
+        if between == "rewrite":
+            model.model_set(c.M, 1000 + step)
+            model.model_set(c.A, 2000 + step)
+        elif between == "invalidate":
+            assert model.et_plan_invalidate(plan) == 0
+        else:
+            for v in e.values():
+                model.model_set(v, 3)
+            assert c.call(plan, between, e) == 0
+            got, ref = c.tags(e), c.fresh(between)
+            if between.startswith("osem"):
+                got, ref = got[1:2], ref[1:2]
+            assert got == ref, between
+        replay()
+        replay()
+    r.close()
+
+
+def test_a_captured_call_that_never_ran(model):
+    """Capturing changes nothing that later calls rely on."""
+    r = Rig(model, 40, 20, 32, 6)
+    c = Calls(r)
+    plan, e = r.plan(), c.outputs()
+    for warm in BETWEEN + ["backward A M"]:
+        if warm not in ("rewrite", "invalidate"):
+            assert c.call(plan, warm, e) == 0
+    for captured in CAPTURED[:-2]:
+        for after in ["gradient A M", "gradient B N", "project A N", "adjoint M", "osem M"]:
+            model.et_plan_invalidate(plan)
+            model.model_begin(STREAM)
+            assert c.call(plan, captured, e) == 0
+            model.model_end()
+            for v in e.values():
+                model.model_set(v, 3)
+            assert c.call(plan, after, e) == 0
+            got, ref = c.tags(e), c.fresh(after)
+            if after.startswith("osem"):
+                got, ref = got[1:2], ref[1:2]
+            assert got == ref, (captured, after)
+    r.close()
+
+
+def test_no_rebuild_is_captured(model):
+    """An OSEM call that would build its caches is refused under capture, and the
+    next call builds them."""
+    r = Rig(model, 40, 20, 32, 6)
+    c = Calls(r)
+    plan, o = r.plan(), c.outputs()
+    assert c.call(plan, "osem M", o) == 0
+    model.et_plan_invalidate(plan)
+    model.model_begin(STREAM)
+    assert c.call(plan, "osem M", o) != 0
+    model.model_end()
+    assert c.call(plan, "osem M", o) == 0
+    assert c.tags(o)[1] == c.fresh("osem M")[1]
+    r.close()
+
+
+def test_tables_are_bounded(model):
+    """Calls of ever other kinds do not pile up tables."""
+    r = Rig(model, 40, 20, 32, 6)
+    c = Calls(r)
+    plan, o = r.plan(), c.outputs()
+    for i in range(60):
+        if i == 30:
+            held = model.model_used()
+        for d in range(1, 7):
+            assert model.et_plan_set_tuning(plan, 1 + i % 8, d) == 0
+            assert c.call(plan, "adjoint", o) == 0
+            assert c.call(plan, "project A", o) == 0
+    assert model.model_used() == held
+    r.close()
