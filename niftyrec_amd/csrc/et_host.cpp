@@ -2653,6 +2653,60 @@ void op_osem(et_plan *p, float *x, const float *meas, const float *mu, int S, in
     osem_finish(p, x);
 }
 
+// ---- calls that run out of device memory ------------------------------------------
+
+// Frees what the plan keeps beyond a call's own needs: the row-lane operations'
+// factors, sums and planes, and the work buffers.  False where it holds none of
+// the former (the call has failed then), or where a captured graph uses them.
+bool give_back(et_plan *p)
+{
+    if (p->keys_captured || p->tables_captured || p->capturing) return false;
+    bool held = false;
+    for (DevBuf *b : {&p->fac, &p->fwd_part, &p->sino_t, &p->op_acc, &p->op_acc2}) {
+        held = held || b->p;
+        b->release();
+    }
+    p->u.release();
+    p->part.release();
+    p->fac_built = p->fwd_built = false;
+    p->key_gen++;  // (OSEM looks at the factors again)
+    return held;
+}
+
+// Runs a call on plans; where the device has no room for it, once more after they
+// have given back what they keep, with the single operations on the sweep kernels,
+// which need least.  (A call allocates before it writes a caller's array.)
+template <class F>
+void with_room(et_plan *const *plans, size_t n, F &&call)
+{
+    try {
+        return call();
+    } catch (const EtError &e) {
+        if (e.code != niftyrec_error_allocgpu) throw;
+        bool held = false;
+        for (size_t i = 0; i < n; i++) held = give_back(plans[i]) || held;
+        if (!held) throw;
+        (void)hipGetLastError();
+    }
+    struct Lean {
+        et_plan *const *plans;
+        size_t n;
+        std::vector<char> ops;
+        Lean(et_plan *const *q, size_t m) : plans(q), n(m), ops(m)
+        {
+            for (size_t i = 0; i < n; i++) {
+                ops[i] = plans[i]->yl_ops;
+                plans[i]->yl_ops = false;
+            }
+        }
+        ~Lean()
+        {
+            for (size_t i = 0; i < n; i++) plans[i]->yl_ops = ops[i];
+        }
+    } lean(plans, n);
+    call();
+}
+
 // ---------------------------------------------------------------------------
 // Host-pointer calls: upload, run on a private stream, download.
 // ---------------------------------------------------------------------------
@@ -4047,7 +4101,10 @@ int et_plan_destroy(et_plan *plan)
     if (hipSetDevice(plan->device) != hipSuccess) return niftyrec_error_nogpuinstalled; \
     plan->st = reinterpret_cast<hipStream_t>(stream);                           \
     plan->capturing = is_capturing(plan->st);                                   \
-    return guarded([&]() -> int { body; return niftyrec_success; });
+    return guarded([&]() -> int {                                                \
+        with_room(&plan, 1, [&]() { body; });                                   \
+        return niftyrec_success;                                                \
+    });
 
 int et_plan_project(et_plan *plan, const float *act, const float *mu, float *sino, int truncate, void *stream)
 {
@@ -4219,7 +4276,9 @@ int et_batch_osem(et_batch *batch, float *const *act, const float *const *sino, 
             check_hip(hipStreamSynchronize(nullptr), niftyrec_error_kernel);
             st = batch->own;
         }
-        op_batch_osem(batch, act, sino, mu, subsets, iterations, epsilon, use_graph != 0, st);
+        with_room(batch->plans.data(), batch->plans.size(), [&]() {
+            op_batch_osem(batch, act, sino, mu, subsets, iterations, epsilon, use_graph != 0, st);
+        });
         if (st == batch->own) check_hip(hipStreamSynchronize(st), niftyrec_error_kernel);
         return niftyrec_success;
     });
