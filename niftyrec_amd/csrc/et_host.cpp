@@ -1095,13 +1095,18 @@ void pull_fast(et_plan *p, const float *recs, int nv, const float *u, bool adjoi
 // wave on 256 CUs).  A batch of views shares every launch, with one rotated
 // copy per view.
 
+// Blocks of a launch along its second and third axis at most.
+constexpr size_t ET_GRID_YZ = 65535;
+
 // Views per batch: the rotated copies of the activity, the map and the
-// rotated-frame volume of a batch stay within 256 MiB.
+// rotated-frame volume of a batch stay within 256 MiB, and the launches over its
+// views within their grids.
 int general_batch(const et_plan *p)
 {
-    if (p->tune_vb > 0) return std::min(p->tune_vb, p->V);
+    if (p->tune_vb > 0) return (int)std::min<size_t>(std::min(p->tune_vb, p->V), ET_GRID_YZ);
     const size_t per_view = (2 * p->yf_elems + p->ustride) * sizeof(float);
-    return (int)std::max<size_t>(1, std::min<size_t>((256ull << 20) / std::max<size_t>(per_view, 1), p->V));
+    const size_t fit = std::min<size_t>((256ull << 20) / std::max<size_t>(per_view, 1), ET_GRID_YZ);
+    return (int)std::max<size_t>(1, std::min<size_t>(fit, p->V));
 }
 
 // Depth chunks of the general path's projection and backprojection: powers of
@@ -1135,12 +1140,16 @@ EtSweepArgs general_args(et_plan *p, int nv, int D, bool act, bool mu)
     return a;
 }
 
+// Whether the rotation reads a volume with background bg in the YF layout (its
+// launch has a grid axis of planes).
+bool rotates_yf(const et_plan *p, float bg) { return bg == 0.f && (size_t)p->nz <= ET_GRID_YZ; }
+
 // Source volumes of an operation in the YF layout, once per operation, where the
-// rotation reads that (zero background); the others are read as the caller's.
+// rotation reads that; the others are read as the caller's.
 void general_sources(et_plan *p, const float *act, const float *mu)
 {
-    if (act && p->bg == 0.f) pack(p, act, p->act_yf);
-    if (mu && p->bga == 0.f) pack(p, mu, p->mu_yf);
+    if (act && rotates_yf(p, p->bg)) pack(p, act, p->act_yf);
+    if (mu && rotates_yf(p, p->bga)) pack(p, mu, p->mu_yf);
 }
 
 // Rotated copies of act and mu (either may be null) for views [v0, v0 + nv) in
@@ -1153,7 +1162,7 @@ void rotate_general(et_plan *p, const float *act, const float *mu, int v0, int n
     const et_stream_t st = (et_stream_t)p->st;
     if (act) p->rot_act.ensure(nv * vs, true, p->st);
     if (mu) p->rot_mu.ensure(nv * vs, true, p->st);
-    const bool act_yf = act && p->bg == 0.f, mu_yf = mu && p->bga == 0.f;
+    const bool act_yf = act && rotates_yf(p, p->bg), mu_yf = mu && rotates_yf(p, p->bga);
     {
         ProfScope ps(p, ET_PROF_OTHER, nv * ((act ? 8.0 : 0.0) + (mu ? 8.0 : 0.0)) * p->nvox);
         if (act_yf || mu_yf)
