@@ -3104,7 +3104,9 @@ int em_driver_host(int kind, float *activity, int size_x, int size_y, const floa
                 int rc = expand_cameras(c.data(), nsub, 3, vs, cs);
                 if (rc) return rc;
                 // the same plan object each step: its workspaces are reused, its
-                // OSEM caches rebuilt for the new cameras
+                // OSEM caches rebuilt for the new cameras (off the fast path the last
+                // step's launches read the records that build_plan overwrites)
+                if (it > 0 && !plan.fast) check_hip(hipStreamSynchronize(hc.st), niftyrec_error_kernel);
                 rc = build_plan(&plan, nx, ny, nz, cs, psf, psf ? psf_h : 0, bg, bga);
                 if (rc) return rc;
                 plan.osem_valid = false;

@@ -420,3 +420,19 @@ def test_general_path_beyond_a_grid(model, dims, views):
     assert r.backproject(plan, S, None, out) == 0
     assert r.gradient(plan, S, A, A, out) == 0
     r.close()
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+def test_random_subsets_wait_for_their_records(model, axis):
+    """The random-subset driver builds its plan anew for every step: no record is
+    overwritten that a launch of the step before may still read."""
+    model.model_clear()
+    model.model_limit(NO_LIMIT)
+    n, ny, V = 8, 6, 12
+    floats = lambda k: (F * k)(*([1.0] * k))  # noqa: E731
+    x, y, mu, psf = floats(n * n * ny), floats(n * ny * V), floats(n * n * ny), floats(9 * n)
+    f = model.et_array_osem
+    f.argtypes = [P, ctypes.c_uint, ctypes.c_uint, ctypes.c_uint, P, I, F, F, ctypes.c_uint, I, I, P, I, P,
+                  ctypes.c_uint, ctypes.c_uint, F, F, F, I]
+    assert f(x, n, ny, 4, y, V, 0.0, 360.0, axis, 3, 1, mu, 1, psf, 3, 3, 0.0, 0.0, 1e-6, 1) == 0
+    assert model.model_violations() == b""
