@@ -1973,14 +1973,20 @@ int yl_u_views(et_plan *p, int want)
     }
 }
 
-// Depth chunks of a row-lane launch of `per_chunk` blocks per chunk: the fewest
-// (powers of two, chunks of at least 4 planes) that give two blocks per CU.
-int yl_op_chunks(const et_plan *p, long per_chunk)
+int device_cus()
 {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
+    return cus;
+}
+
+// Depth chunks of a row-lane launch of `per_chunk` blocks per chunk: the fewest
+// (powers of two, chunks of at least 4 planes) that give two blocks per CU.
+int yl_op_chunks(const et_plan *p, long per_chunk)
+{
+    const int cus = device_cus();
     int D = 1;
     while (D < 32 && p->nz / (2 * D) >= 4 && per_chunk * D < 2L * cus) D *= 2;
     return D;
@@ -2094,18 +2100,39 @@ int yl_gradient_batch(const et_plan *p)
 }
 
 // Depth chunks of the projection of every view (the forward sums' chunking, which
-// the gradient sweeps share).  The blocks of a tall plan have a CU to themselves,
-// so a launch of a few blocks per CU ends in a nearly empty round (256^3, 63
-// views, PSF 21, gradient sweep: 320 blocks in one chunk 5.6 ms, 4.0 ms in
-// eight); its chunks, of at least 16 planes, give eight per CU.
+// the gradient sweeps share).  The blocks of a tall plan have a CU to themselves, so
+// a launch runs in rounds of as many blocks as there are CUs, and a last round of a
+// few blocks takes as long as a full one.  Without attenuation the chunks are those
+// whose rounds pass the fewest planes, with two planes' time for a block's own start
+// (100 columns of 192 rows, 12 views, PSF 11: 115 us in four chunks, 61 in ten; over
+// 180 shapes of 65 to 256 columns and 12 to 90 views 0.3% above the best chunking on
+// average, where powers of two were 19% above it and up to 30% behind the sweep
+// kernels).  With it, chunks of at least 16 planes that give eight blocks
+// per CU (256^3, 63 views, PSF 21, gradient sweep: 320 blocks in one chunk 5.6 ms,
+// 4.0 ms in eight).
 int yl_forward_chunks(const et_plan *p, bool mu)
 {
     if (!mu && p->tune_D > 0) return p->tune_D;
     if (p->yt_L != 32) return yl_op_chunks(p, (long)p->V * p->yl_tiles);
-    const long per_chunk = (long)yl_gradient_batch(p) * p->yl_tiles;
-    int D = 1;
-    while (D < 32 && p->nz / (2 * D) >= 16 && per_chunk * D < 8L * 256) D *= 2;
-    return D;
+    const long cus = device_cus();
+    if (mu) {
+        const long per_chunk = (long)yl_gradient_batch(p) * p->yl_tiles;
+        int D = 1;
+        while (D < 32 && p->nz / (2 * D) >= 16 && per_chunk * D < 8 * cus) D *= 2;
+        return D;
+    }
+    long least = 0;
+    int best = 1;
+    for (int D = 1; D <= 32; D++) {
+        int Deff, zlen;
+        yl_chunks(p, D, Deff, zlen);
+        if (D > 1 && zlen < 4) break;
+        const long planes = ((long)p->V * p->yl_tiles * Deff + cus - 1) / cus * (zlen + 2);
+        if (D > 1 && planes >= least) continue;
+        least = planes;
+        best = Deff;
+    }
+    return best;
 }
 
 // Whether the device may take the forward sums in the plan for a gradient's.  They

@@ -37,6 +37,7 @@ std::vector<std::vector<std::function<void()>>> graphs;
 const void *capturing = nullptr;            // the captured stream
 std::string fail_name;
 int fail_at = 0;
+int sweep_blocks = 0, sweep_planes = 0;     // of the last row-lane sweep: its grid, planes per block
 
 void violation(const std::string &s) { violations += s + "\n"; }
 
@@ -335,6 +336,8 @@ int model_count(const char *name)
     for (const std::string &s : log_) n += s == name;
     return n;
 }
+int model_sweep_blocks() { return sweep_blocks; }
+int model_sweep_planes() { return sweep_planes; }
 void model_begin(void *stream)
 {
     capturing = stream;
@@ -432,6 +435,8 @@ int et_launch_yl_sweep(int kind, int R, int RPL, int NR, int nthr, size_t lds, c
         const int *t4 = static_cast<const int *>(tab);
         for (int j = 0; j < n; j++) {
             const EtSweepArgs a = args[j];
+            sweep_blocks = t4[4 * j + 1] * t4[4 * j + 2];
+            sweep_planes = a.zlen;
             const int end = j + 1 < n ? t4[4 * (j + 1)] : blocks, k = kind % ET_YL_COND;
             if (t4[4 * j] + t4[4 * j + 1] * t4[4 * j + 2] > end) violation("table: more blocks than the grid has");
             const bool grad = k == 3 || k == 4 || k == 5 || k == 8, bpu = k == 1 || k == 7;

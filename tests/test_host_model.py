@@ -436,3 +436,15 @@ def test_random_subsets_wait_for_their_records(model, axis):
                   ctypes.c_uint, ctypes.c_uint, F, F, F, I]
     assert f(x, n, ny, 4, y, V, 0.0, 360.0, axis, 3, 1, mu, 1, psf, 3, 3, 0.0, 0.0, 1e-6, 1) == 0
     assert model.model_violations() == b""
+
+
+@pytest.mark.parametrize("dims, views, planes", [((100, 192, 100), 40, 34), ((192, 200, 192), 12, 28),
+                                                 ((65, 130, 65), 40, 22), ((256, 250, 256), 90, 396)])
+def test_a_tall_projection_ends_in_full_rounds(model, dims, views, planes):
+    """The depth chunks of a tall plan's projection without attenuation (one block
+    per CU at a time): rounds of 256 blocks, times the planes of a block, are within
+    a tenth of the planes of all blocks over 256."""
+    r = Rig(model, *dims, views)
+    assert r.project(r.plan(), r.vol(), None, r.vol(sino=True)) == 0
+    assert -(-model.model_sweep_blocks() // 256) * model.model_sweep_planes() <= planes
+    r.close()
