@@ -482,6 +482,11 @@ struct et_plan {
     // layouts
     int gy = ET_GY, gmu = ET_GY, yp = 0, xp = 0, zp = 0, yu = 0, slabs = 0;
     size_t yf_elems = 0, ustride = 0, P = 0, nvox = 0;
+    // the sweep kernels' rotated-frame volumes: columns of whole 16-row slabs, in u_slab
+    // where the row-lane kernels' (yu, ustride, in u) are longer
+    int yus = 0;
+    size_t ustride_s = 0;
+    DevBuf u_slab;
     // workspaces
     DevBuf act_yf, mu_yf, rot_act, rot_mu, u, part, ratio, csum, csum_lo, astart, atot, atot_lo, tmp, tmp2, em_sino,
         em_vol, att;
@@ -726,6 +731,8 @@ int build_plan(et_plan *p, int nx, int ny, int nz, const Cameras &cams, const fl
     p->yu = rows;
     p->yf_elems = (size_t)p->yp * p->xp * p->zp;
     p->ustride = (size_t)p->yu * p->xp * p->zp;
+    p->yus = p->slabs * ET_T;
+    p->ustride_s = (size_t)p->yus * p->xp * p->zp;
     p->P = (size_t)nx * ny;
     p->nvox = (size_t)nx * ny * nz;
     // device copies
@@ -864,8 +871,8 @@ EtSweepArgs base_args(et_plan *p)
     a.xp = p->xp;
     a.gy = p->gy;
     a.gmu = p->gmu;
-    a.yu = p->yu;
-    a.ustride = (int)p->ustride;
+    a.yu = p->yus;
+    a.ustride = (int)p->ustride_s;
     a.slabs = p->slabs;
     a.K = p->K;
     a.psf = p->K > 0 ? p->d_sep.p : nullptr;
@@ -895,7 +902,7 @@ int choose_D(et_plan *p, int views)
     return D;
 }
 
-// Views per batch of a backprojection: rotated-frame volumes of at most 208 MiB, so
+// Views per batch of a backprojection on the row-lane kernels: rotated-frame volumes of at most 208 MiB, so
 // that with the volume they are added into they stay in the 256 MiB Infinity Cache
 // between the sweep that writes them and the pull that reads them; the views are
 // spread evenly over the batches.  128^3 x 120 views, PSF 11: 24 views a batch 452
@@ -909,10 +916,25 @@ int view_batch(et_plan *p)
     return (int)((p->V + nb - 1) / nb);
 }
 
+DevBuf &slab_u(et_plan *p) { return p->yus == p->yu ? p->u : p->u_slab; }
+
+// Views per batch of a backprojection on the sweep kernels: rotated-frame volumes of
+// at most 256 MiB, spread evenly over the batches.  Over 1,005 shapes (as
+// yt_backprojects') batches of at most 208 MiB cost 10 to 20% where one or two of 256
+// hold every view (up to 43%); full batches with a short last one cost 2 to 9%
+// elsewhere.
+int slab_batch(et_plan *p)
+{
+    if (p->tune_vb > 0) return std::min(p->tune_vb, p->V);
+    const long vb = std::max(1L, (long)((256ull << 20) / std::max<size_t>(p->ustride_s * sizeof(float), 1)));
+    const long nb = (p->V + vb - 1) / vb;
+    return (int)((p->V + nb - 1) / nb);
+}
+
 // Views per launch of the gradient sweeps.  They run whole rays (one depth
 // chunk: the reverse sum needs the ray's total), so a launch has only
 // slabs x views blocks: at least two per CU are taken, with rotated-frame
-// volumes of up to 4 GiB (256^3: 32 views, 2.2 GB), where view_batch would give
+// volumes of up to 4 GiB (256^3: 32 views, 2.2 GB), where slab_batch would give
 // 3 views (48 blocks).
 int grad_view_batch(et_plan *p)
 {
@@ -922,8 +944,8 @@ int grad_view_batch(et_plan *p)
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     const long want = (2L * cus + p->slabs - 1) / std::max(p->slabs, 1);
-    const long cap = (long)((4ull << 30) / std::max<size_t>(p->ustride * sizeof(float), 1));
-    const long vb = std::max<long>(view_batch(p), std::min(want, cap));
+    const long cap = (long)((4ull << 30) / std::max<size_t>(p->ustride_s * sizeof(float), 1));
+    const long vb = std::max<long>(slab_batch(p), std::min(want, cap));
     return (int)std::max(1L, std::min<long>(vb, p->V));
 }
 
@@ -974,7 +996,7 @@ void mu_prefix(et_plan *p, const float *recs, int nv, int D, const float *mu_yf,
 // Floats of the attenuation-factor buffer of nv views ([nv][nz][yu][roundup(nx, 64)]).
 size_t att_elems(const et_plan *p, int nv)
 {
-    return (size_t)nv * p->nz * p->yu * (size_t)nthreads_for(p->nx);
+    return (size_t)nv * p->nz * p->yus * (size_t)nthreads_for(p->nx);
 }
 
 // Arguments of a projection sweep of nv views into `part` ([D][nv][ny][nx]).
@@ -1061,9 +1083,9 @@ EtPullArgs pull_args(et_plan *p, const float *recs, int nv, const float *u, bool
     a.nx = p->nx;
     a.ny = p->ny;
     a.nz = p->nz;
-    a.yu = p->yu;
+    a.yu = p->yus;
     a.xp = p->xp;
-    a.ustride = (int)p->ustride;
+    a.ustride = (int)p->ustride_s;
     a.V = nv;
     a.views = recs;
     a.u = u;
@@ -1104,7 +1126,7 @@ constexpr size_t ET_GRID_YZ = 65535;
 int general_batch(const et_plan *p)
 {
     if (p->tune_vb > 0) return (int)std::min<size_t>(std::min(p->tune_vb, p->V), ET_GRID_YZ);
-    const size_t per_view = (2 * p->yf_elems + p->ustride) * sizeof(float);
+    const size_t per_view = (2 * p->yf_elems + p->ustride_s) * sizeof(float);
     const size_t fit = std::min<size_t>((256ull << 20) / std::max<size_t>(per_view, 1), ET_GRID_YZ);
     return (int)std::max<size_t>(1, std::min<size_t>(fit, p->V));
 }
@@ -1196,9 +1218,9 @@ int general_R(et_plan *p) { return p->R > ET_RMAX ? 0 : p->R; }
 void conv_u_general(et_plan *p, float *u, int nv, bool flip)
 {
     if (!(p->K > 0 && p->R > ET_RMAX)) return;
-    const size_t vs = p->ustride;
+    const size_t vs = p->ustride_s;
     p->tmp2.ensure(nv * vs, true, p->st);
-    const long sx = p->yu, sy = 1, sz = (long)p->yu * p->xp, off = (long)p->yu * (1 + p->xp);
+    const long sx = p->yus, sy = 1, sz = (long)p->yus * p->xp, off = (long)p->yus * (1 + p->xp);
     const float *sep = flip ? p->d_sep_flip.p : p->d_sep.p;
     // row pass then column pass; the transpose takes them in the other order
     check_launch(et_launch_conv_axis(u, p->tmp2.p, p->nx, p->ny, p->nz, sx, sy, sz, off, flip ? 1 : 0, sep, p->K, 0,
@@ -1296,8 +1318,8 @@ void op_backproject(et_plan *p, const float *sino, const float *mu, float *out, 
             pack(p, mu, p->mu_yf);
             mu_yf = p->mu_yf.p;
         }
-        const int vb = view_batch(p);
-        p->u.ensure((size_t)vb * p->ustride, true, p->st);
+        const int vb = slab_batch(p);
+        slab_u(p).ensure((size_t)vb * p->ustride_s, true, p->st);
         for (int v0 = 0; v0 < p->V; v0 += vb) {
             const int nv = std::min(vb, p->V - v0);
             const float *recs = p->d_recs.p + (size_t)v0 * ET_VIEW_REC;
@@ -1308,15 +1330,15 @@ void op_backproject(et_plan *p, const float *sino, const float *mu, float *out, 
                 astart = p->astart.p;
             }
             bpu_fast(p, recs, nv, mu_yf, ET_SRC_SINO, sino + (size_t)v0 * p->P, nullptr, nullptr, 0, 0.f, D, astart,
-                     adjoint, p->u.p);
+                     adjoint, slab_u(p).p);
             const bool last = v0 + nv >= p->V;
-            pull_fast(p, recs, nv, p->u.p, adjoint, ET_EPI_ABI_STORE, v0 > 0, last && truncate, out);
+            pull_fast(p, recs, nv, slab_u(p).p, adjoint, ET_EPI_ABI_STORE, v0 > 0, last && truncate, out);
         }
         return;
     }
     general_sources(p, nullptr, mu);
     const int R = general_R(p), vb = general_batch(p);
-    p->u.ensure((size_t)vb * p->ustride, true, p->st);
+    slab_u(p).ensure((size_t)vb * p->ustride_s, true, p->st);
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
         if (mu) rotate_general(p, nullptr, mu, v0, nv, false);
@@ -1326,14 +1348,14 @@ void op_backproject(et_plan *p, const float *sino, const float *mu, float *out, 
         a.astart = mu && D > 1 ? p->astart.p : nullptr;
         a.src = ET_SRC_SINO;
         a.sino = sino + (size_t)v0 * p->P;
-        a.u = p->u.p;
+        a.u = slab_u(p).p;
         if (p->K > 0) a.psf = adjoint ? p->d_sep_flip.p : p->d_sep.p;
         {
             ProfScope ps(p, ET_PROF_BPU, nv * ((mu ? 8.0 : 4.0) * p->nvox + 4.0 * p->P));
             check_launch(et_launch_sweep(ET_MODE_BPU, R, mu != nullptr, 0, a, (et_stream_t)p->st));
         }
-        conv_u_general(p, p->u.p, nv, adjoint);
-        pull_general(p, v0, nv, p->u.p, adjoint, v0 > 0, truncate && v0 + nv >= p->V, out);
+        conv_u_general(p, slab_u(p).p, nv, adjoint);
+        pull_general(p, v0, nv, slab_u(p).p, adjoint, v0 > 0, truncate && v0 + nv >= p->V, out);
     }
 }
 
@@ -1348,7 +1370,7 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
         pack(p, act, p->act_yf);
         pack(p, mu, p->mu_yf);
         const int vb = grad_view_batch(p);
-        p->u.ensure((size_t)vb * p->ustride, true, p->st);
+        slab_u(p).ensure((size_t)vb * p->ustride_s, true, p->st);
         for (int v0 = 0; v0 < p->V; v0 += vb) {
             const int nv = std::min(vb, p->V - v0);
             const float *recs = p->d_recs.p + (size_t)v0 * ET_VIEW_REC;
@@ -1362,19 +1384,19 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
             a.atot_lo = p->atot_lo.p;
             a.src = ET_SRC_SINO;
             a.sino = sino + (size_t)v0 * p->P;
-            a.u = p->u.p;
+            a.u = slab_u(p).p;
             {
                 ProfScope ps(p, ET_PROF_GRAD, (double)nv * (12.0 * p->nvox + 4.0 * p->P));
                 check_launch(et_launch_sweep(mode, p->R, 1, 1, a, (et_stream_t)p->st));
             }
             const bool last = v0 + nv >= p->V;
-            pull_fast(p, recs, nv, p->u.p, exact, ET_EPI_ABI_STORE, v0 > 0, last && truncate, out);
+            pull_fast(p, recs, nv, slab_u(p).p, exact, ET_EPI_ABI_STORE, v0 > 0, last && truncate, out);
         }
         return;
     }
     general_sources(p, act, mu);
     const int R = general_R(p), vb = general_batch(p);
-    p->u.ensure((size_t)vb * p->ustride, true, p->st);
+    slab_u(p).ensure((size_t)vb * p->ustride_s, true, p->st);
     for (int v0 = 0; v0 < p->V; v0 += vb) {
         const int nv = std::min(vb, p->V - v0);
         rotate_general(p, act, mu, v0, nv, exact);
@@ -1384,13 +1406,13 @@ void op_gradient(et_plan *p, const float *sino, const float *act, const float *m
         a.atot_lo = p->atot_lo.p;
         a.src = ET_SRC_SINO;
         a.sino = sino + (size_t)v0 * p->P;
-        a.u = p->u.p;
+        a.u = slab_u(p).p;
         {
             ProfScope ps(p, ET_PROF_GRAD, nv * (12.0 * p->nvox + 4.0 * p->P));
             check_launch(et_launch_sweep(mode, R, 1, 1, a, (et_stream_t)p->st));
         }
-        if (!exact) conv_u_general(p, p->u.p, nv, false);
-        pull_general(p, v0, nv, p->u.p, exact, v0 > 0, truncate && v0 + nv >= p->V, out);
+        if (!exact) conv_u_general(p, slab_u(p).p, nv, false);
+        pull_general(p, v0, nv, slab_u(p).p, exact, v0 > 0, truncate && v0 + nv >= p->V, out);
     }
 }
 
@@ -1439,7 +1461,7 @@ struct BlockTable {
 void em_subset_update(et_plan *p, const float *recs, int nv, float *x_yf, const float *mu_yf, const float *meas,
                       const float *sens_yf, float eps, int Dp, int Db, float *att)
 {
-    p->u.ensure((size_t)nv * p->ustride, true, p->st);
+    slab_u(p).ensure((size_t)nv * p->ustride_s, true, p->st);
     float *parts = p->part.ensure((size_t)Dp * nv * p->P, false);
     float *ratio = p->ratio.ensure((size_t)nv * p->P, false);
     project_fast(p, recs, nv, x_yf, mu_yf, nullptr, 1, Dp, nullptr, parts, att);
@@ -1447,8 +1469,8 @@ void em_subset_update(et_plan *p, const float *recs, int nv, float *x_yf, const 
         ProfScope ps(p, ET_PROF_OTHER, (Dp + 2.0) * 4.0 * nv * p->P);
         check_launch(et_launch_ratio_parts(meas, parts, Dp, (size_t)nv * p->P, eps, ratio, (et_stream_t)p->st));
     }
-    bpu_fast(p, recs, nv, mu_yf, ET_SRC_SINO, ratio, nullptr, nullptr, 0, 0.f, Db, nullptr, false, p->u.p, att);
-    pull_fast(p, recs, nv, p->u.p, false, ET_EPI_OSEM, false, false, nullptr, x_yf, sens_yf);
+    bpu_fast(p, recs, nv, mu_yf, ET_SRC_SINO, ratio, nullptr, nullptr, 0, 0.f, Db, nullptr, false, slab_u(p).p, att);
+    pull_fast(p, recs, nv, slab_u(p).p, false, ET_EPI_OSEM, false, false, nullptr, x_yf, sens_yf);
 }
 
 // Sensitivity of views [recs, nv): reference backprojection of ones, truncated,
@@ -1457,9 +1479,9 @@ void em_subset_update(et_plan *p, const float *recs, int nv, float *x_yf, const 
 void em_sensitivity(et_plan *p, const float *recs, int nv, const float *mu_yf, float eps, int D, float *att,
                     float *sens_yf)
 {
-    p->u.ensure((size_t)nv * p->ustride, true, p->st);
-    bpu_fast(p, recs, nv, mu_yf, ET_SRC_ONES, nullptr, nullptr, nullptr, 0, 0.f, D, nullptr, false, p->u.p, att);
-    pull_fast(p, recs, nv, p->u.p, false, ET_EPI_YF_STORE, false, true, sens_yf);
+    slab_u(p).ensure((size_t)nv * p->ustride_s, true, p->st);
+    bpu_fast(p, recs, nv, mu_yf, ET_SRC_ONES, nullptr, nullptr, nullptr, 0, 0.f, D, nullptr, false, slab_u(p).p, att);
+    pull_fast(p, recs, nv, slab_u(p).p, false, ET_EPI_YF_STORE, false, true, sens_yf);
     ProfScope ps(p, ET_PROF_OTHER, 0);
     check_launch(et_launch_yf_clamp_min(sens_yf, p->nx, p->ny, p->nz, p->yp, p->gy, eps, (et_stream_t)p->st));
 }
@@ -1536,7 +1558,7 @@ int tune_depth_chunks(et_plan *p, int mode, const float *recs, int nv, const flo
             const int D = cand[ci];
             const float *as = nullptr;  // both sweeps read the factors: no attenuation prefix
             float *parts = p->part.ensure((size_t)std::max(D, Dp) * nv * p->P, false);
-            p->u.ensure((size_t)nv * p->ustride, true, p->st);
+            slab_u(p).ensure((size_t)nv * p->ustride_s, true, p->st);
             // as in em_subset_update: both sweeps read the attenuation factors
             float *att = mu_yf ? p->att.ensure(att_elems(p, nv), true, p->st) : nullptr;
             float *ratio = p->ratio.ensure((size_t)nv * p->P, false);
@@ -1552,7 +1574,7 @@ int tune_depth_chunks(et_plan *p, int mode, const float *recs, int nv, const flo
                     project_fast(p, recs, nv, act, mu_yf, nullptr, 1, Dp, as, parts, att);
                     check_launch(et_launch_ratio_parts(parts, parts, Dp, (size_t)nv * p->P, 1e-6f, ratio,
                                                        (et_stream_t)p->st));
-                    bpu_fast(p, recs, nv, mu_yf, ET_SRC_SINO, ratio, nullptr, nullptr, 0, 0.f, D, as, false, p->u.p,
+                    bpu_fast(p, recs, nv, mu_yf, ET_SRC_SINO, ratio, nullptr, nullptr, 0, 0.f, D, as, false, slab_u(p).p,
                              att);
                 }
             };
@@ -1642,12 +1664,24 @@ EtSweepArgs yl_sweep_args(const et_plan *p, const float *recs, int nv, int D, co
     a.V = nv;
     a.D = Deff;
     a.zlen = zlen;
+    a.yu = p->yu;
+    a.ustride = (int)p->ustride;
     a.att = const_cast<float *>(att);
     a.att_vs = (size_t)p->nz * yl_plane_elems(p);
     a.part_V = nv;
     a.yl_nbuf = p->yl_nbuf;
     a.yt_cols = p->yt_cols;
     a.yl_tiles = p->yl_tiles;
+    return a;
+}
+
+// Arguments of a row-lane pull.
+EtPullArgs yl_pull_args(et_plan *p, const float *recs, int nv, const float *u, bool adjoint, int epi, bool accumulate,
+                        bool truncate, float *out, float *x, const float *sens)
+{
+    EtPullArgs a = pull_args(p, recs, nv, u, adjoint, epi, accumulate, truncate, out, x, sens);
+    a.yu = p->yu;
+    a.ustride = (int)p->ustride;
     return a;
 }
 
@@ -1782,9 +1816,9 @@ struct YlTable {
             et_plan *p = plans[i];
             bytes += (double)nv[i] * 4.0 * p->nvox + (sens_out ? 8.0 : 16.0) * p->nvox;
             const float *r = p->osem_recs.p + (size_t)v0[i] * ET_VIEW_REC;
-            EtPullArgs a = sens_out ? pull_args(p, r, nv[i], p->u.p, false, ET_EPI_YF_STORE, false, true,
+            EtPullArgs a = sens_out ? yl_pull_args(p, r, nv[i], p->u.p, false, ET_EPI_YF_STORE, false, true,
                                                 (*sens_out)[i], nullptr, nullptr)
-                                    : pull_args(p, r, nv[i], p->u.p, false, ET_EPI_OSEM, false, false, nullptr,
+                                    : yl_pull_args(p, r, nv[i], p->u.p, false, ET_EPI_OSEM, false, false, nullptr,
                                                 p->x_yf.p, sens[i]);
             // the sensitivity is truncated at 0, then clamped below at epsilon
             if (sens_out) a.floor = std::max(p->osem_cur_eps, 0.f);
@@ -2060,7 +2094,7 @@ void yl_pull_into(YlTable &t, et_plan *p, const float *recs, int nv, bool adjoin
                               bytes += (double)nv * 4.0 * p->nvox + (accumulate ? 8.0 : 4.0) * p->nvox;
                               gx = yl_pull_tiles(p);
                               gy = 1;
-                              return pull_args(p, recs, nv, p->u.p, adjoint, ET_EPI_YF_STORE, accumulate, truncate,
+                              return yl_pull_args(p, recs, nv, p->u.p, adjoint, ET_EPI_YF_STORE, accumulate, truncate,
                                                acc, nullptr, nullptr);
                           });
 }
@@ -2193,9 +2227,31 @@ void yl_backproject_views(YlTable &t, et_plan *p, const float *fac, const float 
     }
 }
 
+// Whether a backprojection without attenuation of a wide or tall plan takes the tile
+// kernels: by the columns x rows that they and the sweep kernels convolve per plane.
+// Tiles hold 2R halo columns and rows padded to 16 or 32 lanes, the sweep kernels'
+// blocks columns padded to waves and rows to 16.  Tiles that convolve more still gain
+// by their pull, most by the adjoint one; tall blocks, alone on a CU, gain least.
+// Timed over 525 tall shapes (65 to 256 columns, 130 to 250 rows) and 480 wide ones
+// (193 to 320, 17 to 128), PSF 0 to 21, 12 to 90 views; times of the sweep kernels
+// over those taken, on average, and shapes more than 5% behind the sweep kernels:
+//   reference, tall  1.08, 39 (tiles throughout 1.00, 221, at worst 1.8 times as long)
+//              wide  1.27, 37 (1.26, 62)
+//   adjoint,   tall  1.29, 28 (1.28, 61)
+//              wide  1.33, 18 (1.33, 22)
+// at worst 1.4 times as long.  Without a PSF tiles are faster throughout.
+bool yt_backprojects(const et_plan *p, bool adjoint)
+{
+    if (!p->yt_L || p->R == 0) return true;
+    const bool tall = p->yt_L == 32;
+    const double tiles = (double)p->yl_tiles * (p->yt_cols + 2 * p->R) * p->yu;
+    const double sweeps = (double)nthreads_for(p->nx) * p->slabs * ET_T;
+    return tiles <= sweeps * (adjoint ? (tall ? 1.45 : 1.7) : (tall ? 1.1 : 1.4));
+}
+
 bool yl_op_backproject(et_plan *p, const float *sino, const float *mu, float *out, bool adjoint, int truncate)
 {
-    if (!p->yl_ops || !p->yl || (mu && !yl_factor_room(p))) return false;
+    if (!p->yl_ops || !p->yl || (!mu && !yt_backprojects(p, adjoint)) || (mu && !yl_factor_room(p))) return false;
     const float *fac = yl_sources(p, nullptr, mu, 0);
     const float *st = yl_sino_t(p, sino);
     const int vb = yl_u_views(p, view_batch(p));
@@ -2643,7 +2699,7 @@ void osem_prepare(et_plan *p, float *x, const float *meas, const float *mu, int 
     }
     pack(p, x, p->x_yf);
     // work buffers of the largest subset (allocated here, outside any capture)
-    p->u.ensure((size_t)maxsub * p->ustride, true, p->st);
+    slab_u(p).ensure((size_t)maxsub * p->ustride_s, true, p->st);
     p->part.ensure((size_t)p->osem_Dp * maxsub * p->P, false);
     p->ratio.ensure((size_t)maxsub * p->P, false);
     p->osem_start = start;
@@ -2703,6 +2759,7 @@ bool give_back(et_plan *p)
         b->release();
     }
     p->u.release();
+    p->u_slab.release();
     p->part.release();
     p->fac_built = p->fwd_built = false;
     p->key_gen++;  // (OSEM looks at the factors again)
@@ -3214,7 +3271,7 @@ std::vector<const void *> batch_key(const et_batch *b, int S, float eps)
     std::memcpy(&e, &eps, 4);
     k.push_back(reinterpret_cast<const void *>((uintptr_t)e));
     for (const et_plan *p : b->plans) {
-        k.insert(k.end(), {p->x_yf.p, p->osem_meas.p, p->part.p, p->ratio.p, p->u.p, p->sens.p, p->osem_recs.p,
+        k.insert(k.end(), {p->x_yf.p, p->osem_meas.p, p->part.p, p->ratio.p, p->u.p, slab_u(const_cast<et_plan *>(p)).p, p->sens.p, p->osem_recs.p,
                            p->osem_E.p, p->fac.p, p->osem_cur_mu, p->d_sep.p});
         k.push_back(reinterpret_cast<const void *>((uintptr_t)(p->osem_Dp * 1024 + p->osem_Db)));
         k.push_back(reinterpret_cast<const void *>((uintptr_t)p->osem_yl));
@@ -3323,7 +3380,7 @@ void batch_build(et_batch *b, int S, hipStream_t st)
                         bt.add((p->ny + ts - 1) / ts, nv * p->osem_Dp);
                     } else {
                         args.push_back(bpu_args(p, r, nv, p->osem_cur_mu, ET_SRC_SINO, p->ratio.p, nullptr, nullptr, 0,
-                                                0.f, p->osem_Db, nullptr, false, p->u.p, osem_att(p, v0)));
+                                                0.f, p->osem_Db, nullptr, false, slab_u(p).p, osem_att(p, v0)));
                         bt.add((p->ny + ts - 1) / ts, nv * p->osem_Db);
                     }
                 }
@@ -3338,7 +3395,7 @@ void batch_build(et_batch *b, int S, hipStream_t st)
         for (et_plan *p : oldp) {
             const int v0 = p->osem_start[s], nv = p->osem_start[s + 1] - v0;
             const float *r = p->osem_recs.p + (size_t)v0 * ET_VIEW_REC;
-            pa.push_back(pull_args(p, r, nv, p->u.p, false, ET_EPI_OSEM, false, false, nullptr, p->x_yf.p,
+            pa.push_back(pull_args(p, r, nv, slab_u(p).p, false, ET_EPI_OSEM, false, false, nullptr, p->x_yf.p,
                                    p->sens.p + (size_t)s * p->yf_elems));
             bt.add((int)(((size_t)p->nx * p->nz + 255) / 256), (p->ny + ET_T - 1) / ET_T);
         }

@@ -448,3 +448,20 @@ def test_a_tall_projection_ends_in_full_rounds(model, dims, views, planes):
     assert r.project(r.plan(), r.vol(), None, r.vol(sino=True)) == 0
     assert -(-model.model_sweep_blocks() // 256) * model.model_sweep_planes() <= planes
     r.close()
+
+
+@pytest.mark.parametrize("dims, psf, tiles", [((100, 130, 100), 21, (0, 0)), ((100, 130, 100), 3, (0, 1)),
+                                              ((100, 130, 100), 0, (1, 1)), ((65, 192, 65), 11, (1, 1)),
+                                              ((192, 192, 192), 7, (1, 1)), ((192, 200, 192), 21, (0, 0)),
+                                              ((256, 40, 256), 21, (0, 0)), ((224, 64, 224), 21, (1, 1)),
+                                              ((193, 17, 193), 11, (1, 1))])
+def test_backprojections_take_the_faster_kernels(model, dims, psf, tiles):
+    """Wide and tall plans without attenuation, (reference, adjoint): tile kernels
+    or not, as timed."""
+    r = Rig(model, *dims, 2, psf=psf)
+    plan, S, out = r.plan(), r.vol(sino=True), r.vol()
+    for adjoint in (0, 1):
+        model.model_clear()
+        assert r.backproject(plan, S, None, out, adjoint) == 0
+        assert (model.model_count(b"yl_sweep") > 0) == bool(tiles[adjoint])
+    r.close()
