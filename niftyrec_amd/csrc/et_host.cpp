@@ -598,23 +598,15 @@ void yt_plan(et_plan *p)
         return;
     // Columns per tile: as few tiles as possible with two LDS planes per block, the
     // columns spread evenly over them (blocks of up to 512 threads, 16 lanes per
-    // column, share a CU by two, those of up to 1,024 have it to themselves); one
-    // plane of the widest tile where two would leave tiles narrower than 40
-    // columns.  The slots of a tile, C / 2, cover its 2R halo columns, and its
+    // column, share a CU by two, those of up to 1,024 have it to themselves; in 160
+    // KiB at least 56 columns fit, whatever the rows and the radius).  The slots of a tile, C / 2, cover its 2R halo columns, and its
     // threads are whole waves: C a multiple of 4 (L = 32) or 8, at least 4R.
     const int blocks = tall ? 1 : 2, step = 128 / L, R = p->R;
     const int least = (std::max(4 * R, step) + step - 1) / step * step;
-    auto fits = [&](int C, int nbuf) {
-        return R == 0 || nbuf * blocks * et_yt_plane_bytes(C, R, L * rpl) <= (size_t)lim;
-    };
-    int widest = ET_YL_TILE, nbuf = 2;
-    while (widest > 40 && !fits(widest, 2)) widest -= step;
-    if (!fits(widest, 2) || widest < least) {
-        widest = ET_YL_TILE;
-        nbuf = 1;
-        while (widest > least && !fits(widest, 1)) widest -= step;
-        if (!fits(widest, 1) || widest < least) return;
-    }
+    auto fits = [&](int C) { return R == 0 || 2 * blocks * et_yt_plane_bytes(C, R, L * rpl) <= (size_t)lim; };
+    int widest = ET_YL_TILE;
+    while (widest > least && !fits(widest)) widest -= step;
+    if (!fits(widest)) return;
     const int T = (nx + widest - 1) / widest;
     const int C = std::max(least, ((nx + T - 1) / T + step - 1) / step * step);
     p->yl = true;
@@ -623,8 +615,8 @@ void yt_plan(et_plan *p)
     p->yl_rpl = rpl;
     p->yl_nr = 0;
     p->yl_w = C / 2;
-    p->yl_nbuf = nbuf;
-    p->yl_lds = p->yl_lds_full = p->yl_lds_tile = p->yl_lds_bpu = R == 0 ? 0 : nbuf * et_yt_plane_bytes(C, R, L * rpl);
+    p->yl_nbuf = 2;
+    p->yl_lds = p->yl_lds_full = p->yl_lds_tile = p->yl_lds_bpu = R == 0 ? 0 : 2 * et_yt_plane_bytes(C, R, L * rpl);
     p->yl_tile_n = p->yl_tiles = (nx + C - 1) / C;
 }
 

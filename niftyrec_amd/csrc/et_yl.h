@@ -1056,7 +1056,7 @@ __device__ __forceinline__ void yl_gref_body(const EtSweepArgs &a, const Blk &b)
 // slots of L lanes own two adjacent columns each, so the x' pass reads 2R + 2 LDS
 // columns for both instead of 2 (2R + 1), and 2R slots take one halo column
 // each; the x' pass comes first, as in the tiled projector.  Two LDS planes
-// alternate (one barrier per plane) wherever a narrower tile lets them fit: the
+// alternate (one barrier per plane), in tiles narrow enough for them to fit: the
 // phases of a plane (gathers, x' pass, axial pass) are bound by HBM, the LDS and
 // the VALU in turn, and a single block of 16 waves with one plane runs them one
 // after another (256^3, PSF 21, 18 views: 1,056 us with one plane of 64 columns,
@@ -1153,13 +1153,13 @@ struct YtCtx {
         return slot < 2 * R ? x_lo + C + slot - R : -1;
     }
     __device__ __forceinline__ bool valid(int xc) const { return xc >= 0 && xc < nx; }
-    // Zeroes the LDS columns of every plane that lie outside the volume; the
+    // Zeroes the LDS columns of both planes that lie outside the volume; the
     // others are written at every plane.  (Clearing whole planes, up to 150 KB a
     // block, cost as much as two planes' work.)
-    __device__ __forceinline__ void zero_outside(float *lds, int planes) const
+    __device__ __forceinline__ void zero_outside(float *lds) const
     {
         const int lo = max(0, R - x_lo), hi = max(lo, min(C + 2 * R, nx - x_lo + R));
-        for (int p = 0; p < planes; p++)
+        for (int p = 0; p < 2; p++)
             for (int k = 4 * (int)threadIdx.x; k < PF; k += 4 * (int)blockDim.x)
                 if (k < lo * CS || k >= hi * CS)
                     *reinterpret_cast<float4 *>(lds + p * PF + k) = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1199,7 +1199,7 @@ __device__ __forceinline__ void yt_project_body(const EtSweepArgs &a, const Blk 
     const C c(a, b);
     const int dx = a.yp, dz = a.yp * a.xp, v = c.v, d = c.d, row0 = c.row0;
     const FastView fv = load_fast_view(a.views + (size_t)v * ET_VIEW_REC);
-    if constexpr (R > 0) c.zero_outside(lds, a.yl_nbuf);
+    if constexpr (R > 0) c.zero_outside(lds);
     const float *act = a.act + a.gy + row0;
     float *uv = GRAD ? a.u + (size_t)v * a.ustride : nullptr;
 
@@ -1254,7 +1254,7 @@ __device__ __forceinline__ void yt_project_body(const EtSweepArgs &a, const Blk 
 #pragma unroll
                 for (int i = 0; i < RPL; i++) e[r][i] = 1.f;
         }
-        float *plane = lds + (R > 0 && a.yl_nbuf == 2 ? (z & 1) * c.PF : 0);
+        float *plane = lds + (R > 0 ? (z & 1) * c.PF : 0);
 #pragma unroll
         for (int r = 0; r < NRR; r++) {
             const int xc = c.col(r);
@@ -1295,8 +1295,6 @@ __device__ __forceinline__ void yt_project_body(const EtSweepArgs &a, const Blk 
                 }
             }
         }
-        if constexpr (R > 0)
-            if (a.yl_nbuf == 1) __syncthreads();  // one plane: the next writes wait for these reads
     }
     if constexpr (!GRAD) {
 #pragma unroll
@@ -1323,7 +1321,7 @@ __device__ __forceinline__ void yt_bpu_body(const EtSweepArgs &a, const Blk &b)
     extern __shared__ float lds[];
     const C c(a, b);
     const int v = c.v, row0 = c.row0;
-    if constexpr (R > 0) c.zero_outside(lds, a.yl_nbuf);
+    if constexpr (R > 0) c.zero_outside(lds);
     float sv[NRR][RPL];
 #pragma unroll
     for (int r = 0; r < NRR; r++) {
@@ -1351,7 +1349,7 @@ __device__ __forceinline__ void yt_bpu_body(const EtSweepArgs &a, const Blk &b)
     load(c.zb);
     for (int z = c.zb; z < c.ze; z++) {
         const float *kz = psf_plane<R>(a.psf, z);  // never read when R == 0
-        float *plane = lds + (R > 0 && a.yl_nbuf == 2 ? (z & 1) * c.PF : 0);
+        float *plane = lds + (R > 0 ? (z & 1) * c.PF : 0);
 #pragma unroll
         for (int r = 0; r < NRR; r++) {
             const int xc = c.col(r);
@@ -1387,7 +1385,6 @@ __device__ __forceinline__ void yt_bpu_body(const EtSweepArgs &a, const Blk &b)
                         yl_istore<RPL>(uv + (size_t)rows * ((c.col(r) + 1) + (size_t)a.xp * (z + 1)), c.lane, o);
                 }
             }
-            if (a.yl_nbuf == 1) __syncthreads();  // one plane: the next writes wait for these reads
         }
     }
 }
