@@ -6,13 +6,18 @@
 // ABI layout   [nx, ny, nz] x fastest: idx = x + nx*(y + ny*z)   (caller buffers)
 // YF layout    axial-fastest, zero-padded source volumes read by the sweep kernels:
 //              idx = (gy + y) + yp*((x + 1) + xp*(z + 1)),
-//              xp = nx + 2, zp = nz + 2, yp = gy + roundup(ny, ET_T) + gy.
+//              xp = nx + 2, zp = nz + 2, yp an odd multiple of 16 floats that holds the
+//              guard rows gy and the plan's rows.
 //              Everything outside the logical volume is zero, so trilinear
 //              corners that fall one voxel outside the grid read zeros.
-// U layout     rotated-frame per-view volumes written by the sweep kernels and
-//              pulled by the backprojection kernels:
-//              idx = v*ustride + y + yu*((x' + 1) + xp*(z' + 1)), yu = roundup(ny, ET_T),
-//              with a zero border of one voxel in x' and z'.
+// U layout     rotated-frame per-view volumes written by a backprojection or gradient
+//              sweep and read by the pull of the same kind:
+//              idx = v*ustride + y + yu*((x' + 1) + xp*(z' + 1)),
+//              with a zero border of one voxel in x' and z'.  Sweep kernels: yu =
+//              roundup(ny, ET_T), rows in order.  Row-lane and tile kernels: yu = 16 or 32
+//              lanes times the rows a lane holds, each column in lane order (et_yl.h).
+// Factors      e^{-A} of a view: sweep kernels [nz][yu][roundup(nx, 64)], x' fastest;
+//              row-lane and tile kernels [nz][nx][yu], each column in lane order.
 // Sinogram     [nx, ny, V] x fastest (the ABI layout), partial projections
 //              [D][V][ny][nx].
 #pragma once
@@ -50,7 +55,7 @@ struct EtSweepArgs {
     int nx, ny, nz;
     int yp, xp, gy;          // YF layout of act (row stride, columns, guard rows)
     int gmu;                 // guard rows of mu in the same layout
-    int yu, ustride;         // U layout of the output volumes (per view stride)
+    int yu, ustride;         // U layout of the output volumes (per view stride), of the kernels' kind
     int V, D, zlen;          // views in launch, depth chunks, z' per chunk
     int slabs;               // ceil(ny / ET_T)
     const float *views;      // view v's record at views + v * rec_stride
@@ -81,7 +86,8 @@ struct EtSweepArgs {
     size_t att_vs;           // row-lane kernels
     int part_V;              // row-lane sweeps: views per depth chunk of `part` (V, or more in a view batch)
     const int *skip;         // conditional row-lane projection: nothing to do when *skip is set
-    int yl_nbuf;             // row-lane sweeps: LDS planes (2: alternate, one barrier per plane; 1: two)
+    int yl_nbuf;             // full-width row-lane sweeps: LDS planes (2: they alternate, one barrier per plane; 1:
+                             // two barriers per plane)
     int near_views;          // tiled row-lane sweeps: the views are in order (neighbouring angles), see yl_block_order
     int yt_cols;             // tile kernels of wide or tall volumes: columns per tile
     int yl_tiles;            // row-lane projector: column tiles per plane (1: the whole width per block)
@@ -214,7 +220,7 @@ struct EtPackArgs {
     float *dst[2];
     int guard[2];
     unsigned long long *parts;
-    unsigned long long *st;  // key state that this launch opens (et_keys_begin), or null
+    unsigned long long *st;  // key state whose copy this launch makes (ET_KEY_LAST), or null
     int nx, ny, nz, yp;
 };
 int et_pack_keys_blocks(int nx, int ny, int nz);
@@ -223,42 +229,41 @@ int et_launch_pack_keys(const EtPackArgs &a, int n, et_stream_t stream);
 // Content keys of a plan's single operations, kept and compared on the device
 // (no host synchronisation; a captured operation compares at every replay).  mu,
 // act: the operation's partial sums (np each; act null when the operation reads
-// none).  st: ET_KEY_WORDS words, zero at first: which of two slots is open, two
-// slots per key, and the decision on the forward sums.  The pack launch opens the
-// slot that the operation before it did not write; the factor launch reads that
-// operation's slot and writes the open one, so that no block of it reads a word
-// that another block writes.
+// none).  st: ET_KEY_WORDS words, zero at first: the keys as the last operation left
+// them, a copy, and the decision on the forward sums.  The pack launch makes the
+// copy; the factor launch reads it and writes the keys, so that no block of it reads
+// a word that another block writes.
 enum {
-    ET_KEY_SLOT = 0, ET_KEY_MU = 1, ET_KEY_FWD_MU = 3, ET_KEY_FWD_ACT = 5, ET_KEY_FWD_SHAPE = 7, ET_KEY_SKIP_FWD = 9,
+    ET_KEY_MU = 0, ET_KEY_FWD_MU = 1, ET_KEY_FWD_ACT = 2, ET_KEY_FWD_SHAPE = 3, ET_KEY_LAST = 4, ET_KEY_SKIP_FWD = 8,
     ET_KEY_WORDS = 10
 };
 struct EtKeys {
     const unsigned long long *mu, *act;
     int np;
     unsigned long long *st;
-    int fac_built;  // the factor buffer holds the factors of the last slot's map
-    int fwd_built;  // the forward sums are those of the last slot's keys
+    int fac_built;  // the factor buffer holds the factors of the last operation's map
+    int fwd_built;  // the forward sums are those of its keys
     int fwd;        // 0: the forward sums stay as they are; 1: this operation forms them;
                     // 2: formed again unless they are this pair's in this shape (st[ET_KEY_SKIP_FWD])
     int shape;      // their chunks and tiles, not 0
 };
 // (constexpr: for the kernels and for host code)
-constexpr void et_keys_begin(unsigned long long *st) { st[ET_KEY_SLOT] ^= 1; }
-constexpr bool et_keys_keep_factors(const EtKeys &k, unsigned long long km)
+// last: the copy, st + ET_KEY_LAST; km, ka: the keys of this operation's map and
+// activity.
+constexpr bool et_keys_keep_factors(const EtKeys &k, const unsigned long long *last, unsigned long long km)
 {
-    return k.fac_built && k.st[ET_KEY_MU + (k.st[ET_KEY_SLOT] ^ 1)] == km;
+    return k.fac_built && last[ET_KEY_MU] == km;
 }
-constexpr void et_keys_end(const EtKeys &k, unsigned long long km, unsigned long long ka)
+constexpr void et_keys_end(const EtKeys &k, const unsigned long long *last, unsigned long long km,
+                           unsigned long long ka)
 {
-    unsigned long long *mu = k.st + ET_KEY_MU, *fm = k.st + ET_KEY_FWD_MU, *fa = k.st + ET_KEY_FWD_ACT,
-                       *fs = k.st + ET_KEY_FWD_SHAPE;
-    const int cur = (int)k.st[ET_KEY_SLOT], last = cur ^ 1;
-    mu[cur] = km;
-    k.st[ET_KEY_SKIP_FWD] =
-        k.fwd == 2 && k.fwd_built && fm[last] == km && fa[last] == ka && fs[last] == (unsigned long long)k.shape;
-    fm[cur] = k.fwd ? km : fm[last];
-    fa[cur] = k.fwd ? ka : fa[last];
-    fs[cur] = k.fwd ? (unsigned long long)k.shape : (k.fwd_built ? fs[last] : 0);
+    const unsigned long long shape = (unsigned long long)k.shape;
+    k.st[ET_KEY_SKIP_FWD] = k.fwd == 2 && k.fwd_built && last[ET_KEY_FWD_MU] == km && last[ET_KEY_FWD_ACT] == ka &&
+                            last[ET_KEY_FWD_SHAPE] == shape;
+    k.st[ET_KEY_MU] = km;
+    k.st[ET_KEY_FWD_MU] = k.fwd ? km : last[ET_KEY_FWD_MU];
+    k.st[ET_KEY_FWD_ACT] = k.fwd ? ka : last[ET_KEY_FWD_ACT];
+    k.st[ET_KEY_FWD_SHAPE] = k.fwd ? shape : (k.fwd_built ? last[ET_KEY_FWD_SHAPE] : 0);
 }
 
 // Row-lane kernels of the OSEM subset loop (et_yl.h).  Grouped launches only

@@ -521,7 +521,9 @@ __global__ void __launch_bounds__(256) k_pack_keys(EtPackArgs a, int zb)
     float *__restrict__ dst = a.dst[vol];
     const int xb = blockIdx.x * 32, yb = blockIdx.y * 32, guard = a.guard[vol];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    if (a.st && threadIdx.x == 0 && blockIdx.x + blockIdx.y + blockIdx.z == 0) et_keys_begin(a.st);
+    // the keys' copy: loaded here, stored at the end, so that no wave waits for it
+    const bool keys = a.st && threadIdx.x < ET_KEY_LAST && blockIdx.x + blockIdx.y + blockIdx.z == 0;
+    const unsigned long long key = keys ? a.st[threadIdx.x] : 0;
     unsigned long long h = 0;
     for (int z = z0; z < a.nz; z += zb) {
         for (int k = ty; k < 32; k += 8) {
@@ -547,6 +549,7 @@ __global__ void __launch_bounds__(256) k_pack_keys(EtPackArgs a, int zb)
         if (threadIdx.x == 0)
             a.parts[blockIdx.x + (size_t)gridDim.x * (blockIdx.y + (size_t)gridDim.y * blockIdx.z)] = h;
     }
+    if (keys) a.st[ET_KEY_LAST + threadIdx.x] = key;
 }
 
 __global__ void __launch_bounds__(256) k_unpack_yf(const float *__restrict__ yf, float *__restrict__ abi,

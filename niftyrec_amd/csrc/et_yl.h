@@ -18,16 +18,18 @@
 // one block barrier per plane orders every write after the reads of the same
 // buffer (a wave reaches plane z + 2's write only after every wave has passed
 // plane z + 1's barrier, which follows its plane-z reads); with one plane
-// (a.yl_nbuf == 1, planes too large for two) a second barrier follows the
-// reads.  The backprojection always uses one plane and two barriers, so that
+// (a.yl_nbuf == 1, planes too large for two) a second barrier per plane follows
+// the reads.  The backprojection always uses one plane and two barriers, so that
 // two of its blocks fit a CU.
 //
-// Layouts (rows = 16 * RPL, y fastest everywhere):
+// Layouts (rows = 16 * RPL, 32 * RPL in the tile kernels of tall volumes; y fastest
+// everywhere):
 //   factors   att[v][z'][x'][rows]  e^{-A(x', y, z')}, A the inclusive sum of mu' (none without
 //             attenuation: att null, every factor 1), rows in lane order (yl_iload)
 //   partials  part[d][v][x'][rows]  projection of depth chunk d
 //   measured counts and ratio       [v][x'][rows]
-//   U         u + v*ustride + y + rows*((x'+1) + xp*(z'+1))  (zero border in x', z'), rows in lane order
+//   U         u + v*ustride + y + rows*((x'+1) + xp*(z'+1))  (zero border in x', z'), rows in lane order:
+//             the pulls here are its only readers
 // Activity, attenuation and sensitivity are in the YF layout of the plan, whose
 // columns hold at least `rows` rows.
 #pragma once
@@ -1598,18 +1600,20 @@ template <int RPL, bool STREAM>
 __global__ void __launch_bounds__(256) k_yl_factors(EtSweepArgs a, EtKeys k)
 {
     __shared__ unsigned long long part[4];
-    unsigned long long h = 0;
-    for (int i = threadIdx.x; i < k.np; i += 256) h += k.mu[i];
-    const unsigned long long km = block_sum_256(h, part);
-    const bool keep = et_keys_keep_factors(k, km);
-    if (blockIdx.x == 0 && blockIdx.y == 0) {
-        h = 0;
-        if (k.act)
-            for (int i = threadIdx.x; i < k.np; i += 256) h += k.act[i];
-        const unsigned long long ka = block_sum_256(h, part);
-        if (threadIdx.x == 0) et_keys_end(k, km, ka);
+    // (every load goes out before the first sum waits)
+    unsigned long long last[ET_KEY_LAST], hm = 0, ha = 0;
+#pragma unroll
+    for (int i = 0; i < ET_KEY_LAST; i++) last[i] = k.st[ET_KEY_LAST + i];
+    const bool lead = blockIdx.x == 0 && blockIdx.y == 0;
+    if (lead && k.act)
+        for (int i = threadIdx.x; i < k.np; i += 256) ha += k.act[i];
+    for (int i = threadIdx.x; i < k.np; i += 256) hm += k.mu[i];
+    const unsigned long long km = block_sum_256(hm, part);
+    if (lead) {
+        const unsigned long long ka = block_sum_256(ha, part);
+        if (threadIdx.x == 0) et_keys_end(k, last, km, ka);
     }
-    if (keep) return;
+    if (et_keys_keep_factors(k, last, km)) return;
     yl_factor_body<RPL, STREAM>(a);
 }
 
@@ -1696,7 +1700,7 @@ __device__ __forceinline__ void yl_pull_body(const EtPullArgs &a, const Blk &b)
 // popcount), and the row takes them four at a time, the four loads in flight
 // together.  Stores as ET_EPI_YF_STORE (accumulate, truncate; rows below ny).
 // Block: a 4 x 4 tile of image columns (x fastest), as the reference pull's.
-// 256 threads; grid ceil(nx/4) * ceil(nz/4).
+// 256 threads; grid as the reference pull's.
 // ------------------------------------------------------------------------------
 template <int RPL>
 __device__ __forceinline__ void yl_pull_adj_body(const EtPullArgs &a, const Blk &b)

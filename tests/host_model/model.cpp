@@ -401,7 +401,7 @@ int et_launch_unpack_yf(const float *yf, float *abi, int nx, int ny, int nz, int
 int et_launch_pack_keys(const EtPackArgs &a, int n, et_stream_t st)
 {
     return launch("pack_keys", st, {a.src[0], a.src[1], a.dst[0], a.dst[1]}, [=]() {
-        if (a.st && need(a.st, 2 * ET_KEY_WORDS, "keys")) et_keys_begin(a.st);
+        if (a.st && need(a.st, 2 * ET_KEY_WORDS, "keys")) std::copy(a.st, a.st + ET_KEY_LAST, a.st + ET_KEY_LAST);
         for (int k = 0; k < n; k++) {
             if (!need(a.src[k], (size_t)a.nx * a.ny * a.nz, "volume") ||
                 !need(a.dst[k], (size_t)a.yp * (a.nx + 2) * (a.nz + 2), "YF copy"))
@@ -420,8 +420,9 @@ int et_launch_yl_factors(int, bool, const EtSweepArgs &a, const EtKeys &k, et_st
         const u64 t = sweep_reads(a, false, true, 0, 0);
         if (!need(a.att, yl_att(a), "factors") || !need(k.st, 2 * ET_KEY_WORDS, "keys")) return;
         const u64 km = k.mu[0] + k.mu[1], ka = k.act ? k.act[0] + k.act[1] : 0;
-        const bool keep = et_keys_keep_factors(k, km);
-        et_keys_end(k, km, ka);
+        const u64 *last = k.st + ET_KEY_LAST;
+        const bool keep = et_keys_keep_factors(k, last, km);
+        et_keys_end(k, last, km, ka);
         if (keep) return;
         log_.push_back("factors built");
         set_tag(a.att, t);
