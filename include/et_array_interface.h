@@ -268,9 +268,9 @@ int et_plan_project(et_plan *plan, const float *act, const float *mu, float *sin
  * GPU, held until the process ends; plans whose copies exceed it return
  * niftyrec_error_parameters (each copy holds (nx+2)(nz+2) padded columns of
  * about ny + 16 floats: 128^3 and 160x96x160 fit with mu, 256^3 does not).
- * One depth chunk per view: the same kernels and results as et_plan_project
- * after et_plan_set_tuning(plan, 1, 0).  Calls share the array: calls that
- * overlap on one GPU race. */
+ * One depth chunk per view, on the sweep kernels, whatever kernels
+ * et_plan_project takes: results agree with its within rounding.  Calls share
+ * the array: calls that overlap on one GPU race. */
 int et_plan_project_noalloc(et_plan *plan, const float *act, const float *mu, float *sino,
                             int truncate, void *stream);
 /* adjoint = 0: the reference backprojector; 1: exact transpose of et_plan_project. */

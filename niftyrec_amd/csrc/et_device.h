@@ -413,6 +413,7 @@ __device__ __forceinline__ Samp fast_sample(const FastView &fv, float fxp, int z
 // 64-bit mix of one element of a content fingerprint (bits in the upper half,
 // index times an odd constant folded in): the fingerprint of an array is the sum
 // modulo 2^64 over its elements, so any partition into blocks gives the same key.
+// The mix is MurmurHash3's 64-bit finaliser (Austin Appleby, public domain).
 __device__ __forceinline__ unsigned long long fp_mix(unsigned long long h)
 {
     h ^= h >> 33;

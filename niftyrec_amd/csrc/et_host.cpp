@@ -506,7 +506,8 @@ struct et_plan {
     float osem_eps = 0.f;
     int mu_check = 1;               // 1: fingerprint mu's content on every OSEM call
     // row-lane OSEM kernels (et_yl.h): fast-path plans whose
-    // rotated plane fits the LDS of one block; rows = yu = 16 * yl_rpl
+    // rotated plane fits the LDS of one block; rows = yu = 16 * yl_rpl (tile
+    // kernels: yt_L * yl_rpl)
     bool yl = false;
     int yl_rpl = 0, yl_nr = 0, yl_w = 0, yl_nbuf = 0;  // rows per lane, column rounds, columns per round, LDS planes
     size_t yl_lds = 0, yl_lds_bpu = 0;                 // LDS bytes of a projector / backprojection block
@@ -1877,14 +1878,13 @@ void yl_upload(DevBuf &buf, const YlTable &t, hipStream_t st)
 
 // ---- row-lane single operations -------------------------------------------------
 // A created plan on the row-lane kernels projects, backprojects (reference or
-// exact adjoint) and forms the exact attenuation gradient with them.  Without
-// attenuation they run on no factors: 64^3 x 64 views, PSF 7, projects in 27.5
+// exact adjoint) and forms both attenuation gradients with them.  Without
+// attenuation they run on no factors: 64^3 x 64 views, PSF 7, projects in 27.8
 // us (56.1 us with the sweep kernels, whose 16-row slabs gather 2 R4 halo rows
-// each) and 128^3 x 120 views, PSF 11, backprojects in 499 us (615 us).  With
-// attenuation the factors e^{-A} of every view are cached (on the
-// attenuation map's key, as the OSEM caches), the activity is gathered by the
-// projector, and the rotated-frame volumes go to the sweep kernels' pulls
-// (same u layout).
+// each) and 128^3 x 120 views, PSF 11, backprojects in 452 us (615 us).  With
+// attenuation the factors e^{-A} of every view are kept, by the map's content.
+// The rotated-frame volumes are in lane order (et_yl.h), which only the row-lane
+// pulls read: a sweep kernel's pull of them would permute rows without an error.
 
 // Whether the device has room for the factors of every view (4 bytes per voxel
 // and view: 12 GB at 256^3 x 180 views); a single operation falls back to the
@@ -2037,10 +2037,12 @@ float *yl_sino_t(et_plan *p, const float *sino)
 // at every replay, whatever other operations ran since.
 void yl_run(et_plan *p, const YlTable &t)
 {
-    std::vector<char> sig = t.tb.bytes;
+    std::vector<char> sig;
+    sig.reserve(t.tb.bytes.size() + t.L.size() * 10 * sizeof(long long));
+    sig = t.tb.bytes;
     for (const YlLaunch &l : t.L) {
-        const long long f[] = {l.kind, l.R, l.RPL, l.NR, l.nthr, (long long)l.lds, (long long)l.args_off,
-                               (long long)l.tab_off, l.n, l.blocks};
+        const long long f[10] = {l.kind, l.R, l.RPL, l.NR, l.nthr, (long long)l.lds, (long long)l.args_off,
+                                 (long long)l.tab_off, l.n, l.blocks};
         const char *c = reinterpret_cast<const char *>(f);
         sig.insert(sig.end(), c, c + sizeof(f));
     }

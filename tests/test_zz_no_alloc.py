@@ -97,3 +97,23 @@ def test_noalloc_refusals():
     assert st == 2
     plan.close()
     plan2.close()
+
+
+@pytest.mark.parametrize("shape, K", [((72, 20, 72), 5), ((130, 24, 130), 11)])
+def test_noalloc_against_the_tiled_projector(shape, K):
+    """Without attenuation et_plan_project runs on the row-lane kernels, above 64
+    columns on tiles, whose PSF passes run in the other order: equal within
+    rounding (the bound of the plan's own path above), at one depth chunk too."""
+    from niftyrec_amd.api import Plan
+    act_np, _, cams, psf = _problem(shape, 6, K, seed=73)
+    plan = Plan(act_np.shape, cams, psf)
+    act = _t(act_np)
+    st, got = _noalloc(plan, act, None)
+    assert st == 0
+    for chunks in (0, 1):
+        plan.set_tuning(chunks, 0)
+        ref = plan.project(act)
+        torch.cuda.synchronize()
+        g, r = got.cpu().numpy(), ref.cpu().numpy()
+        assert rel_l2(g, r) <= 1e-6 and max_rel(g, r) <= 1e-5
+    plan.close()
