@@ -600,8 +600,9 @@ void yt_plan(et_plan *p)
     // Columns per tile: as few tiles as possible with two LDS planes per block, the
     // columns spread evenly over them (blocks of up to 512 threads, 16 lanes per
     // column, share a CU by two, those of up to 1,024 have it to themselves; in 160
-    // KiB at least 56 columns fit, whatever the rows and the radius).  The slots of a tile, C / 2, cover its 2R halo columns, and its
-    // threads are whole waves: C a multiple of 4 (L = 32) or 8, at least 4R.
+    // KiB at least 56 columns fit, whatever the rows and the radius).  The slots of a
+    // tile, C / 2, cover its 2R halo columns, and its threads are whole waves: C a
+    // multiple of 4 (L = 32) or 8, at least 4R.
     const int blocks = tall ? 1 : 2, step = 128 / L, R = p->R;
     const int least = (std::max(4 * R, step) + step - 1) / step * step;
     auto fits = [&](int C) { return R == 0 || 2 * blocks * et_yt_plane_bytes(C, R, L * rpl) <= (size_t)lim; };
@@ -895,10 +896,10 @@ int choose_D(et_plan *p, int views)
     return D;
 }
 
-// Views per batch of a backprojection on the row-lane kernels: rotated-frame volumes of at most 208 MiB, so
-// that with the volume they are added into they stay in the 256 MiB Infinity Cache
-// between the sweep that writes them and the pull that reads them; the views are
-// spread evenly over the batches.  128^3 x 120 views, PSF 11: 24 views a batch 452
+// Views per batch of a backprojection on the row-lane kernels: rotated-frame volumes
+// of at most 208 MiB, so that with the volume they are added into they stay in the
+// 256 MiB Infinity Cache between the sweep that writes them and the pull that reads
+// them; the views are spread evenly over the batches.  128^3 x 120 views, PSF 11: 24 views a batch 452
 // us, 15 494, 30 500, all at once 529; 96^3 x 120, PSF 7: 40 a batch 233, 64 246.
 int view_batch(et_plan *p)
 {
@@ -1130,7 +1131,7 @@ int general_batch(const et_plan *p)
 // takes them, would leave a quarter of that.
 int general_D(const et_plan *p, int nv)
 {
-    if (p->tune_D > 0) return std::min(p->tune_D, p->nz);
+    if (p->tune_D > 0) return std::max(1, std::min({p->tune_D, p->nz, (int)(ET_GRID_YZ / (size_t)nv)}));
     const long waves = (long)p->slabs * nv * (nthreads_for(p->nx) / 64);
     int D = 1;
     while (D < 32 && waves * D < 4096 && p->nz / (2 * D) >= 4) D *= 2;

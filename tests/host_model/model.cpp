@@ -512,6 +512,7 @@ int et_launch_yl_parts_to_sino(const float *part, int D, int V, int nx, int ny, 
 int et_launch_sweep(int mode, int R, int has_mu, int has_act, const EtSweepArgs &a, et_stream_t st)
 {
     const size_t P = (size_t)a.nx * a.ny, nthr = (a.nx + 63) / 64 * 64;
+    if ((size_t)a.V * a.D > 65535) return (int)hipErrorInvalidConfiguration;
     return launch("sweep", st, {a.act, a.mu, a.views, a.part, a.u, a.sino, a.att}, [=]() {
         u64 t = sweep_reads(a, mode != ET_MODE_BPU && mode != ET_MODE_MUSUM && has_act, has_mu == 1,
                             has_mu == 3 ? (size_t)a.V * a.nz * a.yu * nthr : 0,

@@ -410,12 +410,13 @@ def test_kept_buffers_give_way(model, first, op):
     r.close()
 
 
-@pytest.mark.parametrize("dims, views", [((1, 1, 1), 70000), ((2, 1, 66000), 2)])
-def test_general_path_beyond_a_grid(model, dims, views):
-    """More views, or planes, than a launch has blocks along an axis."""
+@pytest.mark.parametrize("dims, views, chunks", [((1, 1, 1), 70000, 0), ((2, 1, 66000), 2, 0), ((1, 1, 8), 40000, 4)])
+def test_general_path_beyond_a_grid(model, dims, views, chunks):
+    """More views, planes, or views in chunks than a launch has blocks along an axis."""
     r = Rig(model, *dims, views, cols=3)
     A, S, out = r.vol(), r.vol(sino=True), r.vol()
     plan = r.plan()
+    assert model.et_plan_set_tuning(plan, chunks, 0) == 0
     assert r.project(plan, A, A, S) == 0
     assert r.backproject(plan, S, None, out) == 0
     assert r.gradient(plan, S, A, A, out) == 0
